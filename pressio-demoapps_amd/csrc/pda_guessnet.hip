@@ -42,6 +42,7 @@
 // lane group g = lane/16 and element j.  The output layout used is the
 // 16x16 MFMA's: lane l holds D[4*(l/16) + i][l%16], i = 0..3; A row = l%16,
 // B column = l%16.
+#include <algorithm>
 #include <cmath>
 
 #include "pda_internal.hpp"
@@ -70,14 +71,6 @@ __device__ __forceinline__ float silu(float z) { return z / (1.f + __expf(-z)); 
 __device__ __forceinline__ float dsilu(float z) {
   const float s = 1.f / (1.f + __expf(-z));
   return s * (1.f + z * (1.f - s));
-}
-
-__device__ __forceinline__ int64_t shifted(int64_t p, int tap, int H, int W) {
-  const int y = int(p / W), x = int(p - int64_t(y) * W);
-  int yy = y + tap / 3 - 1, xx = x + tap % 3 - 1;
-  yy = yy < 0 ? yy + H : (yy >= H ? yy - H : yy);
-  xx = xx < 0 ? xx + W : (xx >= W ? xx - W : xx);
-  return int64_t(yy) * W + xx;
 }
 
 // A operand: 8 bf16 of the pixel at row y, column x for K step s, lane
@@ -181,92 +174,192 @@ __global__ void __launch_bounds__(64) k_conv(const __bf16 *__restrict__ X, const
   }
 }
 
-// Backward-weight: partial dW[tap][cout][cin] over a chunk of 32*KCH pixels,
-// as MFMAs with M = cout, N = cin, K = pixels.  dZ (bf16 [p][32], zero
-// beyond the layer's outputs) and X (bf16 [p][CIN]) tiles of 32 pixels are
-// staged in LDS so that each lane gathers 8 consecutive pixels of one
-// channel.
-constexpr int KCH = 16; // 32-pixel K steps per chunk
+// Backward-weight of a hidden layer: dW[tap][cout][cin] = sum_p dZ[p][cout]
+// X[p + tap][cin] and db[cout] = sum_p dZ[p][cout], as MFMAs with M = cout,
+// N = cin, K = pixels.  A workgroup takes a band of WG_SEG columns and marches
+// up its share of the grid rows, WG_ROWS rows at a time: those rows of dZ and
+// the WG_ROWS + 2 rows of X that the taps read are staged in LDS once, in the
+// layout they have in memory ([pixel][channel]), and the operands, which need
+// the 8 pixels of one channel, come from the transposing LDS reads
+// (ds_read_b64_tr_b16: the 16 lanes of a group read 4 pixels x 16 channels,
+// every lane getting the 4 pixels of its channel).  A tap's shift in x is a
+// pixel more in the read's address; each of the three waves has one row of
+// taps, so a wave keeps 3 x 2 x 2 accumulators and no sum crosses waves.
+// Pixels past the grid's edge are staged as zeros.  The workgroup's sums leave
+// in accumulator order, part[wg][wave][dx][mt][nt][i][lane] and then db, for
+// k_wgrad_reduce; db is a product with ones.
+// Bound by the staging loads' latency (33.5 MB per layer at 512 x 512, 7 us at
+// the copy rate) and by the partial sums (18.9 MB out and in again); at
+// 512 x 512 21.6 us per 32-channel layer (12.7 us the 8-channel one), where
+// one workgroup per tap and 512 pixels, gathering the operands from LDS two
+// bytes at a time, took 158 us (63 us), and db, 32 blocks over all pixels,
+// another 324 us.
+constexpr int WG_SEG = 64, WG_ROWS = 4, WG_MAX = 512; // columns, rows a step, most workgroups
+constexpr int WG_THREADS = 192;
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+
+// the 4 pixels of this lane's channel: p = the lane's own 8 bytes of the tile
+__device__ __forceinline__ s16x4 lds_tr(const __bf16 *p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+      (__attribute__((address_space(3))) s16x4 *)(reinterpret_cast<const s16x4 *>(p)));
+}
+__device__ __forceinline__ bf16x8 join(s16x4 lo, s16x4 hi) {
+  typedef short s16x8 __attribute__((ext_vector_type(8)));
+  const s16x8 v = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+  return __builtin_bit_cast(bf16x8, v);
+}
+
+// 16-wide N tiles of a wave's three taps: 2 of one tap's 32 channels, or two
+// taps of 8 channels side by side (the fourth tap repeats the third, unused)
+__host__ __device__ constexpr int wg_ntiles(int cin) { return cin == C ? 6 : 2; }
+// sums of one workgroup: 3 waves x tiles x 2 (mt) x 256, and db
+__host__ __device__ constexpr int wg_sums(int cin) { return 3 * wg_ntiles(cin) * 2 * 256 + C; }
+
+struct WgradGrid {
+  int nseg, rows_per_wg, nwg; // bands, grid rows of a workgroup, workgroups
+};
+inline WgradGrid wgrad_grid(int H, int W) {
+  WgradGrid G;
+  G.nseg = (W + WG_SEG - 1) / WG_SEG;
+  const int per = std::max(1, WG_MAX / G.nseg);           // workgroups a band may take
+  G.rows_per_wg = ((H + per - 1) / per + WG_ROWS - 1) / WG_ROWS * WG_ROWS;
+  G.nwg = G.nseg * ((H + G.rows_per_wg - 1) / G.rows_per_wg);
+  return G;
+}
 
 template <int CIN>
-__global__ void __launch_bounds__(64) k_conv_wgrad(const __bf16 *__restrict__ dZ, const __bf16 *__restrict__ X,
-                                                    int H, int W, int coutp, float *__restrict__ part) {
-  constexpr int NTN = CIN == C ? 2 : 1; // 16-wide cin tiles
-  __shared__ __bf16 sz[32][C + 2];
-  __shared__ __bf16 sx[32][CIN + 2];
-  const int lane = threadIdx.x, r = lane & 15, g = lane >> 4;
-  const int tap = blockIdx.y, chunk = blockIdx.x;
-  const int MTN = coutp / 16; // 16-wide cout tiles
-  f32x4 acc[2][NTN];
-#pragma unroll
-  for (int a = 0; a < 2; ++a)
-#pragma unroll
-    for (int b = 0; b < NTN; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int ks = 0; ks < KCH; ++ks) {
-    const int64_t pb = (int64_t(chunk) * KCH + ks) * 32;
-    // stage dZ[pb .. pb+31][0..31] and X[shift(pb + i, tap)][0..CIN-1]
-    for (int q = lane; q < 32 * C; q += 64) sz[q / C][q % C] = dZ[(pb + q / C) * C + q % C];
-    for (int q = lane; q < 32 * CIN; q += 64)
-      sx[q / CIN][q % CIN] = X[shifted(pb + q / CIN, tap, H, W) * CIN + q % CIN];
-    __syncthreads();
-#pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
-      if (mt >= MTN) break;
-      bf16x8 a;
-#pragma unroll
-      for (int j = 0; j < 8; ++j) a[j] = sz[8 * g + j][16 * mt + r];
-#pragma unroll
-      for (int nt = 0; nt < NTN; ++nt) {
-        bf16x8 b;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const int cin = 16 * nt + r;
-          b[j] = cin < CIN ? sx[8 * g + j][cin < CIN ? cin : 0] : __bf16(0.f);
-        }
-        acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[mt][nt], 0, 0, 0);
-      }
-    }
-    __syncthreads();
-  }
-  // part[chunk][tap][cout][cin]
-  float *dst = part + (int64_t(chunk) * 9 + tap) * (C * C);
+__global__ void __launch_bounds__(WG_THREADS) k_conv_wgrad(const __bf16 *__restrict__ dZ,
+                                                          const __bf16 *__restrict__ X, int H, int W,
+                                                          int nseg, int rows_per_wg, float *__restrict__ part) {
+  constexpr int NT = wg_ntiles(CIN);
+  __shared__ __align__(16) __bf16 sz[WG_ROWS * WG_SEG * C];
+  __shared__ __align__(16) __bf16 sx[(WG_ROWS + 2) * (WG_SEG + 2) * CIN];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int g = lane >> 4, i16 = lane & 15;
+  const int x0 = (int(blockIdx.x) % nseg) * WG_SEG;
+  const int yb = (int(blockIdx.x) / nseg) * rows_per_wg;
+  const int ye = yb + rows_per_wg < H ? yb + rows_per_wg : H;
+  f32x4 acc[NT][2], accb[2];
 #pragma unroll
   for (int mt = 0; mt < 2; ++mt) {
-    if (mt >= MTN) break;
+    accb[mt] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int nt = 0; nt < NTN; ++nt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int cout = 16 * mt + 4 * g + i, cin = 16 * nt + r;
-        if (cin < CIN) dst[cout * C + cin] = acc[mt][nt][i];
-      }
+    for (int nt = 0; nt < NT; ++nt) acc[nt][mt] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
-}
-
-// sum of the partials over chunks -> dW[tap][cout][cin] (FP32); bias
-// gradient db[cout] = sum_p dZ[p][cout]
-__global__ void k_wgrad_reduce(const float *__restrict__ part, int nchunk, int cin, int cout,
-                               float *__restrict__ dW) {
-  const int e = blockIdx.x * blockDim.x + threadIdx.x; // tap*cout*cin
-  if (e >= 9 * cout * cin) return;
-  const int tap = e / (cout * cin), co = (e / cin) % cout, ci = e % cin;
-  float s = 0.f;
-  for (int c = 0; c < nchunk; ++c) s += part[(int64_t(c) * 9 + tap) * (C * C) + co * C + ci];
-  dW[e] = s;
-}
-
-__global__ void k_bias_grad(const __bf16 *__restrict__ dZ, int64_t npix, int cout, float *__restrict__ db) {
-  __shared__ float sh[256];
-  const int c = blockIdx.x;
-  float s = 0.f;
-  for (int64_t p = threadIdx.x; p < npix; p += 256) s += float(dZ[p * C + c]);
-  sh[threadIdx.x] = s;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
+  bf16x8 ones, zero;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    ones[j] = __bf16(1.f);
+    zero[j] = __bf16(0.f);
+  }
+  for (int y0 = yb; y0 < ye; y0 += WG_ROWS) {
+    constexpr int ZV = WG_ROWS * WG_SEG * (C / 8), XW = WG_SEG + 2, XV = (WG_ROWS + 2) * XW * (CIN / 8);
+    for (int q = tid; q < ZV; q += WG_THREADS) {
+      const int v = q % (C / 8), px = q / (C / 8) % WG_SEG, row = q / (C / 8 * WG_SEG);
+      const int x = x0 + px, y = y0 + row;
+      bf16x8 d = zero;
+      if (x < W && y < ye) d = *reinterpret_cast<const bf16x8 *>(dZ + (int64_t(y) * W + x) * C + 8 * v);
+      *reinterpret_cast<bf16x8 *>(sz + (row * WG_SEG + px) * C + 8 * v) = d;
+    }
+    for (int q = tid; q < XV; q += WG_THREADS) {
+      const int v = q % (CIN / 8), px = q / (CIN / 8) % XW, row = q / (CIN / 8 * XW);
+      int x = x0 - 1 + px, y = y0 - 1 + row;
+      bf16x8 d = zero;
+      if (x <= W && y <= H) { // W, H: the wrapped neighbours of the last column and row
+        x = x < 0 ? x + W : (x >= W ? x - W : x);
+        y = y < 0 ? y + H : (y >= H ? y - H : y);
+        d = *reinterpret_cast<const bf16x8 *>(X + (int64_t(y) * W + x) * CIN + 8 * v);
+      }
+      *reinterpret_cast<bf16x8 *>(sx + (row * XW + px) * CIN + 8 * v) = d;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int row = 0; row < WG_ROWS; ++row)
+#pragma unroll
+      for (int ks = 0; ks < WG_SEG / 32; ++ks) {
+        const int px = 32 * ks + 8 * g + (i16 >> 2); // this lane's pixel of the first 4 of 8
+        bf16x8 a[2];
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) {
+          const __bf16 *pz = sz + (row * WG_SEG + px) * C + 16 * mt + 4 * (i16 & 3);
+          a[mt] = join(lds_tr(pz), lds_tr(pz + 4 * C));
+          if (wave == 0) accb[mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt], ones, accb[mt], 0, 0, 0);
+        }
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) {
+          int dx, ch;
+          if constexpr (CIN == C) {
+            dx = nt / 2;
+            ch = 16 * (nt & 1) + 4 * (i16 & 3);
+          } else {
+            dx = 2 * nt + ((i16 & 3) >> 1);
+            dx = dx < 3 ? dx : 2;
+            ch = 4 * (i16 & 1);
+          }
+          const __bf16 *px_ = sx + ((row + wave) * XW + px + dx) * CIN + ch;
+          const bf16x8 b = join(lds_tr(px_), lds_tr(px_ + 4 * CIN));
+#pragma unroll
+          for (int mt = 0; mt < 2; ++mt)
+            acc[nt][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[mt], b, acc[nt][mt], 0, 0, 0);
+        }
+      }
     __syncthreads();
   }
-  if (threadIdx.x == 0) db[c] = sh[0];
+  float *dst = part + int64_t(blockIdx.x) * wg_sums(CIN);
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dst[(((wave * NT + nt) * 2 + mt) * 4 + i) * 64 + lane] = acc[nt][mt][i];
+  if (wave == 0 && i16 == 0) {
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) dst[wg_sums(CIN) - C + 16 * mt + 4 * g + i] = accb[mt][i];
+  }
+}
+
+// dW and db of the three hidden layers from their workgroups' sums: a block
+// sums 64 elements, 16 slices of the workgroups at a time (1024 threads, so
+// that a slice is 32 loads long; one thread per element walking every partial
+// took 121 us per layer, this 8.4 us for the three), then the slices in order.
+struct WgradLayers {
+  const float *part[NL - 1];
+  float *gw[NL - 1]; // dW of the layer, db behind it
+  int nwg;
+};
+constexpr int WR_SLICES = 16;
+
+__global__ void __launch_bounds__(64 * WR_SLICES) k_wgrad_reduce(WgradLayers L) {
+  __shared__ float sh[WR_SLICES][64];
+  const int l = blockIdx.y, cin = cin_of(l), n = wg_sums(cin);
+  const int e0 = blockIdx.x * 64;
+  if (e0 >= n) return; // the whole block: the 8-channel layer has fewer sums
+  const int k = threadIdx.x & 63, sl = threadIdx.x >> 6, e = e0 + k;
+  const float *part = l == 0 ? L.part[0] : (l == 1 ? L.part[1] : L.part[2]);
+  float *gw = l == 0 ? L.gw[0] : (l == 1 ? L.gw[1] : L.gw[2]);
+  float s = 0.f;
+  if (e < n)
+#pragma unroll 8
+    for (int w = sl; w < L.nwg; w += WR_SLICES) s += part[int64_t(w) * n + e];
+  sh[sl][k] = s;
+  __syncthreads();
+  if (sl != 0 || e >= n) return;
+  s = 0.f;
+  for (int q = 0; q < WR_SLICES; ++q) s += sh[q][k];
+  if (e >= n - C) {
+    gw[9 * cin * C + (e - (n - C))] = s;
+    return;
+  }
+  // accumulator order -> dW[tap][cout][cin]
+  const int lane = e & 63, i = (e >> 6) & 3, mt = (e >> 8) & 1, t = e >> 9;
+  const int NT = wg_ntiles(cin), wave = t / NT, nt = t % NT;
+  const int cout = 16 * mt + 4 * (lane >> 4) + i, col = lane & 15;
+  const int dx = cin == C ? nt / 2 : 2 * nt + (col >> 3);
+  const int ci = cin == C ? 16 * (nt & 1) + col : col & 7;
+  if (dx < 3) gw[((3 * wave + dx) * C + cout) * cin + ci] = s;
 }
 
 // the velocities the predictors read: f[0] = f(y_n), ..., f[4] = f(y_{n-4})
@@ -400,15 +493,39 @@ __global__ void k_guess(const double *__restrict__ un, const double *__restrict_
   guess[i] = (4. / 3.) * un[i] - (1. / 3.) * unm1[i] + ((2. / 3.) * dt) * E;
 }
 
-// dZ of the output layer: d loss / d out[p][c] = (d loss / d m_c) / npix
-// for every pixel (the logits are means over the pixels), zero beyond NOUT
-__global__ void k_dz_uniform(const double *__restrict__ lg, int64_t npix, __bf16 *__restrict__ dZ) {
-  const int64_t p = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (p >= npix) return;
-  const double inv = 1. / double(npix);
+// Backward of the output layer.  The loss reads its grid means alone, so
+// d loss / d out[p][c] = (d loss / d m_c) / npix = dz_c at every pixel (held in
+// BF16 as every dZ), and with the periodic padding
+//   dW[tap][c][i] = dz_c sum_p Y[p][i]  (the channel sums of the policy),
+//   db[c] = dz_c npix,
+//   d loss / d Y[p][i] = sum_c dz_c Weff[c][i] = dy[i], the same at every pixel:
+// one block per tap instead of three passes over the pixels.
+__global__ void __launch_bounds__(256) k_out_backward(const double *__restrict__ lg, const double *__restrict__ sums,
+                                                      const float *__restrict__ weff, double npix,
+                                                      float *__restrict__ gw, float *__restrict__ dy) {
+  const int tap = blockIdx.x, e = threadIdx.x;
+  auto dz = [&](int c) { return double(float(__bf16(float(lg[1 + c] / npix)))); };
+  if (e < NOUT * C) gw[tap * NOUT * C + e] = float(dz(e / C) * sums[e % C]);
+  if (tap != 0) return;
+  if (e < NOUT) gw[9 * NOUT * C + e] = float(dz(e) * npix);
+  if (e < C) {
+    double v = 0.;
+    for (int c = 0; c < NOUT; ++c) v += dz(c) * double(weff[c * C + e]);
+    dy[e] = float(v);
+  }
+}
+
+// dZ of the last hidden layer: dy[c] SiLU'(Z[p][c]), 8 channels per thread
+__global__ void __launch_bounds__(256) k_dz_hidden(const float *__restrict__ dy, const float *__restrict__ Z,
+                                                   int64_t npix, __bf16 *__restrict__ dZ) {
+  const int64_t q = int64_t(blockIdx.x) * 256 + threadIdx.x;
+  if (q >= npix * (C / 8)) return;
+  const int c0 = 8 * int(q % (C / 8));
+  const f32x4 z0 = *reinterpret_cast<const f32x4 *>(Z + 8 * q), z1 = *reinterpret_cast<const f32x4 *>(Z + 8 * q + 4);
+  bf16x8 d;
 #pragma unroll
-  for (int c = 0; c < NOUT; ++c) dZ[p * C + c] = __bf16(float(lg[1 + c] * inv));
-  for (int c = NOUT; c < C; ++c) dZ[p * C + c] = __bf16(0.f);
+  for (int j = 0; j < 8; ++j) d[j] = __bf16(dy[c0 + j] * dsilu(j < 4 ? z0[j & 3] : z1[j & 3]));
+  *reinterpret_cast<bf16x8 *>(dZ + 8 * q) = d;
 }
 
 // Adam on the FP32 master parameters
@@ -482,6 +599,7 @@ struct pda_guessnet_s {
   pda::DevBuf csum, sums, weff;      // last hidden layer's channel sums; output tap sums
   pda::DevBuf pol;                   // the last forward's policy: p, t, weights of P(t)
   pda::DevBuf lg;                    // expected cost, its derivatives w.r.t. the NOUT logits
+  pda::DevBuf dy;                    // d loss / d Y of the last hidden layer, per channel
   int adam_t = 0;
 };
 
@@ -559,29 +677,36 @@ int forward(pda_guessnet_s &net, bool keep_z, bool full_out, hipStream_t st) {
   return PDA_OK;
 }
 
-// Gradients (into net.g) of the loss whose output-layer dZ is in dZa.
-// Layer l: dW_l from (dZ_l, input_l); dZ_{l-1} = (dZ_l conv flipped
-// transposed W_l) * SiLU'(Z_{l-1}), alternating between dZa and dZb.
+// Gradients (into net.g) of the loss whose derivatives w.r.t. the output
+// means are in net.lg.  The output layer's follow from the channel sums.
+// Hidden layer l: the sums of dW_l from (dZ_l, input_l); dZ_{l-1} = (dZ_l
+// conv flipped transposed W_l) * SiLU'(Z_{l-1}), alternating between dZa and
+// dZb; the sums of the three layers are reduced together at the end.
 int backward(pda_guessnet_s &net, hipStream_t st) {
   const unsigned grid = unsigned(net.npix / (16 * MT));
-  const int nchunk = int(net.npix / (32 * KCH));
+  const WgradGrid G = wgrad_grid(net.H, net.W);
   float *gW = net.g.as<float>();
   const __bf16 *Wb = net.Wb.as<__bf16>();
   __bf16 *dz = net.dZa.as<__bf16>(), *dz_next = net.dZb.as<__bf16>();
-  for (int l = NL - 1; l >= 0; --l) {
-    const int cin = cin_of(l), cout = cout_of(l), coutp = cout == NOUT ? 16 : C;
-    const __bf16 *Xin = l == 0 ? net.X0.as<__bf16>() : net.Y[l - 1].as<__bf16>();
+  hipLaunchKernelGGL(k_out_backward, dim3(9), dim3(256), 0, st, net.lg.as<double>(), net.sums.as<double>(),
+                     net.weff.as<float>(), double(net.npix), gW + net.woff[NL - 1], net.dy.as<float>());
+  hipLaunchKernelGGL(k_dz_hidden, dim3(unsigned((net.npix * (C / 8) + 255) / 256)), dim3(256), 0, st,
+                     net.dy.as<float>(), net.Z[NL - 2].as<float>(), net.npix, dz);
+  PDA_HIP_CHECK(hipGetLastError());
+  WgradLayers L{};
+  L.nwg = G.nwg;
+  float *part = net.part.as<float>();
+  for (int l = NL - 2; l >= 0; --l) {
+    const int cin = cin_of(l);
+    L.part[l] = part;
+    L.gw[l] = gW + net.woff[l];
     if (cin == C)
-      hipLaunchKernelGGL((k_conv_wgrad<C>), dim3(nchunk, 9), dim3(64), 0, st, dz, Xin, net.H, net.W, coutp,
-                         net.part.as<float>());
+      hipLaunchKernelGGL((k_conv_wgrad<C>), dim3(G.nwg), dim3(WG_THREADS), 0, st, dz, net.Y[l - 1].as<__bf16>(),
+                         net.H, net.W, G.nseg, G.rows_per_wg, part);
     else
-      hipLaunchKernelGGL((k_conv_wgrad<CIN0>), dim3(nchunk, 9), dim3(64), 0, st, dz, Xin, net.H, net.W,
-                         coutp, net.part.as<float>());
-    const int ne = 9 * cout * cin;
-    hipLaunchKernelGGL(k_wgrad_reduce, dim3((ne + 255) / 256), dim3(256), 0, st, net.part.as<float>(), nchunk,
-                       cin, cout, gW + net.woff[l]);
-    hipLaunchKernelGGL(k_bias_grad, dim3(cout), dim3(256), 0, st, dz, net.npix, cout,
-                       gW + net.woff[l] + 9 * cin * cout);
+      hipLaunchKernelGGL((k_conv_wgrad<CIN0>), dim3(G.nwg), dim3(WG_THREADS), 0, st, dz, net.X0.as<__bf16>(),
+                         net.H, net.W, G.nseg, G.rows_per_wg, part);
+    part += int64_t(G.nwg) * wg_sums(cin);
     PDA_HIP_CHECK(hipGetLastError());
     if (l == 0) break;
     hipLaunchKernelGGL((k_conv<C, 2, MODE_BWD>), dim3(grid), dim3(64), 0, st, dz, Wb + net.boff[l], nullptr,
@@ -589,20 +714,18 @@ int backward(pda_guessnet_s &net, hipStream_t st) {
     PDA_HIP_CHECK(hipGetLastError());
     std::swap(dz, dz_next);
   }
+  hipLaunchKernelGGL(k_wgrad_reduce, dim3((wg_sums(C) + 63) / 64, NL - 1), dim3(64 * WR_SLICES), 0, st, L);
+  PDA_HIP_CHECK(hipGetLastError());
   return PDA_OK;
 }
 
 // loss of the current forward's cost estimates against a sample's costs;
-// leaves the output dZ in dZa
+// leaves its derivatives w.r.t. the output means in net.lg
 int loss(pda_guessnet_s &net, const double *costs, float *lval, hipStream_t st) {
   Costs c;
   for (int j = 0; j < NOUT; ++j) c.c[j] = costs[j];
   int rc = policy(net, &c, st);
   if (rc) return rc;
-  const int nb = int((net.npix + 255) / 256);
-  hipLaunchKernelGGL(k_dz_uniform, dim3(unsigned(nb)), dim3(256), 0, st, net.lg.as<double>(), net.npix,
-                     net.dZa.as<__bf16>());
-  PDA_HIP_CHECK(hipGetLastError());
   if (lval) {
     double l = 0.;
     PDA_HIP_CHECK(hipMemcpyAsync(&l, net.lg.ptr, sizeof(double), hipMemcpyDeviceToHost, st));
@@ -630,7 +753,7 @@ int check_costs(const double *costs, const char *who) {
 extern "C" {
 
 int pda_guessnet_create(int nx, int ny, pda_guessnet *out) {
-  if (!out || nx < 4 || ny < 4 || (int64_t(nx) * ny) % (32 * KCH) != 0 || int64_t(nx) * ny > (int64_t(1) << 30)) {
+  if (!out || nx < 4 || ny < 4 || (int64_t(nx) * ny) % 512 != 0 || int64_t(nx) * ny > (int64_t(1) << 30)) {
     set_error("pda_guessnet_create: need nx, ny >= 4 and nx*ny a multiple of 512, at most 2^30");
     return PDA_E_INVALID_ARG;
   }
@@ -668,12 +791,14 @@ int pda_guessnet_create(int nx, int ny, pda_guessnet *out) {
   if (e == hipSuccess) e = net->dZa.alloc(sizeof(__bf16) * np * C);
   if (e == hipSuccess) e = net->dZb.alloc(sizeof(__bf16) * np * C);
   if (e == hipSuccess) e = net->out.alloc(sizeof(float) * np * NOUT);
-  if (e == hipSuccess) e = net->part.alloc(sizeof(float) * (np / (32 * KCH)) * 9 * C * C);
+  if (e == hipSuccess)
+    e = net->part.alloc(sizeof(float) * size_t(wgrad_grid(ny, nx).nwg) * (wg_sums(CIN0) + (NL - 2) * wg_sums(C)));
   if (e == hipSuccess) e = net->csum.alloc(sizeof(float) * (np / (16 * MT)) * C);
   if (e == hipSuccess) e = net->sums.alloc(sizeof(double) * C);
   if (e == hipSuccess) e = net->weff.alloc(sizeof(float) * NOUT * C);
   if (e == hipSuccess) e = net->pol.alloc(sizeof(double) * POL_LEN);
   if (e == hipSuccess) e = net->lg.alloc(sizeof(double) * (1 + NOUT));
+  if (e == hipSuccess) e = net->dy.alloc(sizeof(float) * C);
   if (e == hipSuccess) e = hipMemset(net->pol.ptr, 0, sizeof(double) * POL_LEN);
   if (e == hipSuccess) e = hipMemset(net->w.ptr, 0, sizeof(float) * wo);
   if (e == hipSuccess) e = hipMemset(net->m1.ptr, 0, sizeof(float) * wo);

@@ -175,3 +175,24 @@ def test_batch_autotune_validates_state(torch):
         b.autotune(torch.zeros(b.total // 2, dtype=torch.float64, device="cuda"))
     with pytest.raises(pda.PdaError):
         b.autotune(torch.zeros(b.total, dtype=torch.float32, device="cuda"))
+
+
+@pytest.mark.parametrize("W,H", [(4, 128), (128, 4), (64, 8), (100, 128), (72, 64), (65 * 8, 64)])
+def test_gradients_on_ragged_grids(torch, W, H):
+    """The backward-weight kernel's bands of 64 columns and groups of 4 rows:
+    partial bands, fewer rows than a group, several workgroups per band.
+    Tolerances as in test_forward_and_gradients_match_oracle (BF16)."""
+    print(f"[gpu-nn] gradients, {W}x{H}", flush=True)
+    rng = np.random.default_rng(W * H)
+    net = pda.GuessNet(W, H)
+    w = _weights(rng, net.nparams, 0.15)
+    net.set_params(w)
+    un, unm1, f = _fields(rng, H, W)
+    net.set_scales(*_scales(f))
+    loss, g, out = net.gradients([torch.from_numpy(x).cuda() for x in f], 0.004, COSTS)
+    lo, oo, go = G.loss_and_grad(w.astype(np.float64), f, 0.004, COSTS, H, W, *_scales(f), bf=True)
+    o = 0
+    for li, (ci, co) in enumerate(G.LAYERS):
+        nW = 9 * ci * co
+        assert rel(g[o:o + nW], go[o:o + nW]) <= 3e-2 and rel(g[o + nW:o + nW + co], go[o + nW:o + nW + co]) <= 3e-2, li
+        o += nW + co
