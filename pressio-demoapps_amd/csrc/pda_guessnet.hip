@@ -35,7 +35,7 @@
 //                    |dt D^4 f| / s_4 (f = the problem's velocity, FP64)
 //   L1 8->32 SiLU, L2 32->32 SiLU, L3 32->32 SiLU, L4 32->7 (linear)
 //   (periodic padding)
-// Every convolution is an implicit GEMM: D[pixel][cout] += A[pixel][k] B[k][cout]
+// Every convolution is an implicit GEMM: D[cout][pixel] += A[cout][k] B[k][pixel]
 // over K = taps x input channels, 32 K per MFMA.  An MFMA pairs A's and B's K
 // elements by register position, so any consistent assignment of K to
 // (lane group, register element) is valid; the kernels use K = 8*g + j for
@@ -58,7 +58,6 @@ constexpr int CIN0 = 8;    // feature channels (7 used)
 constexpr int NOUT = 7;    // output channels: logits of the orders 1, 1.5, ..., 4
 constexpr int NCOMP = 2;   // field components per pixel
 constexpr int NL = 4;      // layers
-constexpr int MT = 4;      // 16-pixel M tiles per wavefront in the forward kernels
 
 // layer geometry: input channels, output channels
 __host__ __device__ constexpr int cin_of(int l) { return l == 0 ? CIN0 : C; }
@@ -67,111 +66,228 @@ __host__ __device__ constexpr int cout_of(int l) { return l == NL - 1 ? NOUT : C
 // channels packed four taps per step
 __host__ __device__ constexpr int ksteps(int cin) { return cin == C ? 9 : 3; }
 
-__device__ __forceinline__ float silu(float z) { return z / (1.f + __expf(-z)); }
+// 1 / (1 + exp(-z)): the hardware reciprocal and one Newton step (exp's own
+// error is the larger; the IEEE division is three times the instructions, a
+// third of a hidden layer's vector work).  z is kept above -87, where the
+// value is 1e-38, so that exp stays finite and the step defined.
+__device__ __forceinline__ float sigmoid(float z) {
+  const float d = 1.f + __expf(-fmaxf(z, -87.f));
+  const float r = __builtin_amdgcn_rcpf(d);
+  return __fmaf_rn(r, __fmaf_rn(-d, r, 1.f), r);
+}
+__device__ __forceinline__ float silu(float z) { return z * sigmoid(z); }
 __device__ __forceinline__ float dsilu(float z) {
-  const float s = 1.f / (1.f + __expf(-z));
+  const float s = sigmoid(z);
   return s * (1.f + z * (1.f - s));
 }
 
-// A operand: 8 bf16 of the pixel at row y, column x for K step s, lane
-// group g (the tap's neighbour, periodic)
-template <int CIN>
-__device__ __forceinline__ bf16x8 load_a(const __bf16 *__restrict__ X, int y, int x, int s, int g, int H, int W) {
-  const int tap = CIN == C ? s : 4 * s + g;
-  if (CIN != C && tap >= 9) {
-    bf16x8 z;
+// the velocities the predictors read: f[0] = f(y_n), ..., f[4] = f(y_{n-4})
+struct FHist {
+  const double *f[5];
+};
+
+// features of pixel p: dt D^k f / s_k (k = 1, 2, 3; 2 channels each), nu_hat,
+// |dt D^4 f| / s_4
+struct Features {
+  FHist F;
+  double c[4], nu_hat;
+};
+__device__ __forceinline__ bf16x8 features(const Features &T, int64_t p) {
+  bf16x8 x;
+  double n4 = 0.;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) z[j] = __bf16(0.f);
-    return z;
+  for (int c = 0; c < 2; ++c) {
+    const int64_t i = 2 * p + c;
+    const double f0 = T.F.f[0][i], f1 = T.F.f[1][i], f2 = T.F.f[2][i], f3 = T.F.f[3][i], f4 = T.F.f[4][i];
+    const double d1 = f0 - f1, d2 = f0 - 2. * f1 + f2, d3 = f0 - 3. * f1 + 3. * f2 - f3;
+    const double d4 = f0 - 4. * f1 + 6. * f2 - 4. * f3 + f4;
+    x[c] = __bf16(float(d1 * T.c[0]));
+    x[2 + c] = __bf16(float(d2 * T.c[1]));
+    x[4 + c] = __bf16(float(d3 * T.c[2]));
+    n4 += (d4 * T.c[3]) * (d4 * T.c[3]);
   }
-  int yy = y + tap / 3 - 1, xx = x + tap % 3 - 1;
-  yy = yy < 0 ? yy + H : (yy >= H ? yy - H : yy);
-  xx = xx < 0 ? xx + W : (xx >= W ? xx - W : xx);
-  const int64_t q = int64_t(yy) * W + xx;
-  return *reinterpret_cast<const bf16x8 *>(X + q * CIN + (CIN == C ? 8 * g : 0));
+  x[6] = __bf16(float(T.nu_hat));
+  x[7] = __bf16(float(sqrt(n4)));
+  return x;
 }
 
 // Forward convolution (and, with MODE_BWD, the backward-data convolution).
-//   Wp: packed weights [kstep][ncout_pad][32] bf16 (B operand rows)
+//   Wp: packed weights [kstep][ncout_pad][32] bf16 (A operand rows)
+//   MODE_FIRST:  as MODE_HIDDEN on the 8 features, formed from the velocity
+//                history while the tile is staged and, with X0, kept for the
+//                backward
 //   MODE_HIDDEN: Z = acc + bias (FP32, kept for the backward; not stored
 //                when Z is null, as in inference), Y = SiLU(Z) (bf16); with
 //                csum, also the block's per-channel sums of Y (FP32,
 //                csum[c][block])
 //   MODE_OUT:    out[p][c] = acc + bias for c < NOUT (FP32)
 //   MODE_BWD:    dZprev[p][c] = acc * SiLU'(Zprev[p][c]) (bf16), no bias
-enum { MODE_HIDDEN = 0, MODE_OUT = 1, MODE_BWD = 2 };
+// A workgroup of four waves owns a tile of CT_W columns x 4 RW rows (RW rows
+// per wave).  The tile and its halo are staged in LDS once, [pixel][channel]
+// as in memory, so a pixel operand is one 16-byte LDS read for every tap and
+// no lane computes addresses or wraps per tap; the layer's weights stay in
+// registers.  M = output channels and N = pixels, so that a lane ends with
+// four consecutive channels of one pixel: 8-byte (Y) and 16-byte (Z) accesses
+// instead of one per value.  At 512 x 512 a hidden layer takes 16.3 us (33.5 MB
+// in and out: 7 us at the copy rate; SiLU's vector instructions: 4 us; the two
+// phases overlap little, as all 512 workgroups run at once), 24.2 us when
+// every lane gathered its pixels per tap from memory.  Loading the tile in a
+// loop that waits for each 16 bytes took 17.4 us.
+enum { MODE_FIRST = 0, MODE_HIDDEN = 1, MODE_OUT = 2, MODE_BWD = 3 };
+constexpr int CT_W = 32; // columns of a tile
 
-template <int CIN, int NT, int MODE>
-__global__ void __launch_bounds__(64) k_conv(const __bf16 *__restrict__ X, const __bf16 *__restrict__ Wp,
-                                              const float *__restrict__ bias, int H, int W,
-                                              float *__restrict__ Z, __bf16 *__restrict__ Y,
-                                              float *__restrict__ out, const float *__restrict__ Zprev,
-                                              float *__restrict__ csum) {
-  const int lane = threadIdx.x, r = lane & 15, g = lane >> 4;
-  const int64_t p0 = int64_t(blockIdx.x) * (16 * MT);
-  f32x4 acc[MT][NT];
+struct ConvArgs {
+  const __bf16 *X, *Wp;
+  const float *bias;
+  int H, W, ntx;          // grid, tiles across
+  float *Z;
+  __bf16 *Y, *X0;
+  float *out;
+  const float *Zprev;
+  float *csum;
+};
+
+template <int MODE, int RW>
+__global__ void __launch_bounds__(256) k_conv(ConvArgs A, Features T) {
+  constexpr int CIN = MODE == MODE_FIRST ? CIN0 : C, NT = MODE == MODE_OUT ? 1 : 2, KS = ksteps(CIN);
+  constexpr int TR = 4 * RW, XW = CT_W + 2, NV = CIN / 8, NPT = CT_W / 16;
+  __shared__ __align__(16) __bf16 sx[(TR + 2) * XW * CIN];
+  __shared__ float ssum[4][C];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, g = lane >> 4;
+  const int H = A.H, W = A.W;
+  const int x0 = (int(blockIdx.x) % A.ntx) * CT_W, y0 = (int(blockIdx.x) / A.ntx) * TR;
+  // every load of the tile in flight before the first LDS store
+  constexpr int TOT = (TR + 2) * XW * NV, PER = (TOT + 255) / 256;
+  bf16x8 stg[PER];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt) acc[mt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // the row and column of this lane's A-row pixel in each M tile
-  int py[MT], px[MT];
-#pragma unroll
-  for (int mt = 0; mt < MT; ++mt) {
-    const int p = int(p0) + 16 * mt + r;
-    py[mt] = p / W;
-    px[mt] = p - py[mt] * W;
-  }
-  constexpr int KS = ksteps(CIN);
-#pragma unroll
-  for (int s = 0; s < KS; ++s) {
-    bf16x8 b[NT];
-#pragma unroll
-    for (int nt = 0; nt < NT; ++nt)
-      b[nt] = *reinterpret_cast<const bf16x8 *>(Wp + (int64_t(s) * (16 * NT) + 16 * nt + r) * 32 + 8 * g);
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt) {
-      const bf16x8 a = load_a<CIN>(X, py[mt], px[mt], s, g, H, W);
-#pragma unroll
-      for (int nt = 0; nt < NT; ++nt)
-        acc[mt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[nt], acc[mt][nt], 0, 0, 0);
+  for (int k = 0; k < PER; ++k) {
+    const int q = tid + 256 * k < TOT ? tid + 256 * k : TOT - 1;
+    const int v = q % NV, px = q / NV % XW, row = q / (NV * XW);
+    int x = x0 - 1 + px, y = y0 - 1 + row;
+    // columns past W and rows past H only feed pixels that are not stored
+    x = x < 0 ? x + W : (x >= W ? (x == W ? 0 : W - 1) : x);
+    y = y < 0 ? y + H : (y >= H ? (y == H ? 0 : H - 1) : y);
+    const int64_t p = int64_t(y) * W + x;
+    if constexpr (MODE == MODE_FIRST) {
+      stg[k] = features(T, p);
+      if (A.X0 && px >= 1 && px <= CT_W && row >= 1 && row <= TR && x0 - 1 + px < W && y0 - 1 + row < H)
+        *reinterpret_cast<bf16x8 *>(A.X0 + p * CIN) = stg[k];
+    } else {
+      stg[k] = *reinterpret_cast<const bf16x8 *>(A.X + p * CIN + 8 * v);
     }
   }
-  float ysum[NT];
 #pragma unroll
-  for (int nt = 0; nt < NT; ++nt) ysum[nt] = 0.f;
+  for (int k = 0; k < PER; ++k)
+    if (tid + 256 * k < TOT) *reinterpret_cast<bf16x8 *>(sx + 8 * (tid + 256 * k)) = stg[k];
+  bf16x8 w[KS][NT];
 #pragma unroll
-  for (int mt = 0; mt < MT; ++mt)
+  for (int s = 0; s < KS; ++s)
+#pragma unroll
+    for (int nt = 0; nt < NT; ++nt)
+      w[s][nt] = *reinterpret_cast<const bf16x8 *>(A.Wp + (int64_t(s) * (16 * NT) + 16 * nt + r) * 32 + 8 * g);
+  f32x4 bias[NT];
+  if constexpr (MODE != MODE_BWD) {
 #pragma unroll
     for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const int64_t p = p0 + 16 * mt + 4 * g + i;
-        const int c = 16 * nt + r;
-        if constexpr (MODE == MODE_HIDDEN) {
-          const float z = acc[mt][nt][i] + bias[c];
-          if (Z) Z[p * C + c] = z;
-          const __bf16 y = __bf16(silu(z));
-          Y[p * C + c] = y;
-          ysum[nt] += float(y);
-        } else if constexpr (MODE == MODE_OUT) {
-          if (c < NOUT) out[p * NOUT + c] = acc[mt][nt][i] + bias[c];
-        } else {
-          Y[p * C + c] = __bf16(acc[mt][nt][i] * dsilu(Zprev[p * C + c]));
-        }
+        const int c = 16 * nt + 4 * g + i;
+        bias[nt][i] = MODE != MODE_OUT || c < NOUT ? A.bias[c] : 0.f;
       }
-  if constexpr (MODE == MODE_HIDDEN) {
-    if (csum) {
-      // channel c = 16 nt + r is held by the four lane groups g: sum them
+  }
+  f32x4 ysum[NT];
+#pragma unroll
+  for (int nt = 0; nt < NT; ++nt) ysum[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+  __syncthreads();
+#pragma unroll 1
+  for (int rr = 0; rr < RW; ++rr) {
+    const int row = wave * RW + rr, y = y0 + row;
+    f32x4 acc[NPT][NT];
+#pragma unroll
+    for (int pt = 0; pt < NPT; ++pt)
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt) acc[pt][nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      // the taps of this K step: one of 32 channels, or four of 8 channels,
+      // one per lane group (past the ninth: zeros)
+      const int tap = CIN == C ? s : (4 * s + g < 9 ? 4 * s + g : 8);
+#pragma unroll
+      for (int pt = 0; pt < NPT; ++pt) {
+        const int px = 16 * pt + r;
+        bf16x8 a = *reinterpret_cast<const bf16x8 *>(sx + ((row + tap / 3) * XW + px + tap % 3) * CIN +
+                                                     (CIN == C ? 8 * g : 0));
+        if constexpr (CIN != C) {
+          if (4 * s + g >= 9)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) a[j] = __bf16(0.f);
+        }
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt)
+          acc[pt][nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[s][nt], a, acc[pt][nt], 0, 0, 0);
+      }
+    }
+#pragma unroll
+    for (int pt = 0; pt < NPT; ++pt) {
+      const int x = x0 + 16 * pt + r;
+      if (x >= W || y >= H) continue;
+      const int64_t p = int64_t(y) * W + x;
 #pragma unroll
       for (int nt = 0; nt < NT; ++nt) {
-        float v = ysum[nt];
-        v += __shfl_xor(v, 16);
-        v += __shfl_xor(v, 32);
-        if (g == 0) csum[int64_t(16 * nt + r) * gridDim.x + blockIdx.x] = v;
+        const int c = 16 * nt + 4 * g;
+        f32x4 z = acc[pt][nt];
+        typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+        bf16x4 o;
+        if constexpr (MODE == MODE_OUT) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            if (c + i < NOUT) A.out[p * NOUT + c + i] = z[i] + bias[nt][i];
+        } else if constexpr (MODE == MODE_BWD) {
+          const f32x4 zp = *reinterpret_cast<const f32x4 *>(A.Zprev + p * C + c);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) o[i] = __bf16(z[i] * dsilu(zp[i]));
+          *reinterpret_cast<bf16x4 *>(A.Y + p * C + c) = o;
+        } else {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            z[i] += bias[nt][i];
+            o[i] = __bf16(silu(z[i]));
+            ysum[nt][i] += float(o[i]);
+          }
+          if (A.Z) *reinterpret_cast<f32x4 *>(A.Z + p * C + c) = z;
+          *reinterpret_cast<bf16x4 *>(A.Y + p * C + c) = o;
+        }
       }
     }
   }
+  if constexpr (MODE == MODE_HIDDEN) {
+    if (A.csum) { // sum over the 16 pixels of a lane group, then the waves
+#pragma unroll
+      for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          float v = ysum[nt][i];
+#pragma unroll
+          for (int o = 1; o < 16; o <<= 1) v += __shfl_xor(v, o);
+          if (r == 0) ssum[wave][16 * nt + 4 * g + i] = v;
+        }
+      __syncthreads();
+      if (tid < C)
+        A.csum[int64_t(tid) * gridDim.x + blockIdx.x] = (ssum[0][tid] + ssum[1][tid]) + (ssum[2][tid] + ssum[3][tid]);
+    }
+  }
+}
+
+// rows per wave: 4 where that still gives the chip a workgroup per CU (fewer
+// halo pixels, 1.20 times the tile against 1.59, and the weights loaded for
+// more pixels: a hidden layer at 512 x 512 takes 16.3 us with 4 rows, 16.9 with
+// 2, 18.0 with 1), else 1
+inline int conv_rows(int H, int W) {
+  return int64_t((W + CT_W - 1) / CT_W) * ((H + 15) / 16) >= 256 ? 4 : 1;
+}
+inline int conv_blocks(int H, int W) {
+  const int tr = 4 * conv_rows(H, W);
+  return ((W + CT_W - 1) / CT_W) * ((H + tr - 1) / tr);
 }
 
 // Backward-weight of a hidden layer: dW[tap][cout][cin] = sum_p dZ[p][cout]
@@ -190,7 +306,8 @@ __global__ void __launch_bounds__(64) k_conv(const __bf16 *__restrict__ X, const
 // k_wgrad_reduce; db is a product with ones.
 // Bound by the staging loads' latency (33.5 MB per layer at 512 x 512, 7 us at
 // the copy rate) and by the partial sums (18.9 MB out and in again); at
-// 512 x 512 21.6 us per 32-channel layer (12.7 us the 8-channel one), where
+// 512 x 512 16.7 us per 32-channel layer (10.5 us the 8-channel one; 21.6 and
+// 12.7 us with each staging load waited for), where
 // one workgroup per tap and 512 pixels, gathering the operands from LDS two
 // bytes at a time, took 158 us (63 us), and db, 32 blocks over all pixels,
 // another 324 us.
@@ -255,24 +372,35 @@ __global__ void __launch_bounds__(WG_THREADS) k_conv_wgrad(const __bf16 *__restr
   }
   for (int y0 = yb; y0 < ye; y0 += WG_ROWS) {
     constexpr int ZV = WG_ROWS * WG_SEG * (C / 8), XW = WG_SEG + 2, XV = (WG_ROWS + 2) * XW * (CIN / 8);
-    for (int q = tid; q < ZV; q += WG_THREADS) {
+    constexpr int ZP = (ZV + WG_THREADS - 1) / WG_THREADS, XP = (XV + WG_THREADS - 1) / WG_THREADS;
+    bf16x8 dz[ZP], dx[XP]; // every load in flight before the first LDS store
+#pragma unroll
+    for (int k = 0; k < ZP; ++k) {
+      const int q = tid + WG_THREADS * k;
       const int v = q % (C / 8), px = q / (C / 8) % WG_SEG, row = q / (C / 8 * WG_SEG);
       const int x = x0 + px, y = y0 + row;
-      bf16x8 d = zero;
-      if (x < W && y < ye) d = *reinterpret_cast<const bf16x8 *>(dZ + (int64_t(y) * W + x) * C + 8 * v);
-      *reinterpret_cast<bf16x8 *>(sz + (row * WG_SEG + px) * C + 8 * v) = d;
+      dz[k] = zero;
+      if (q < ZV && x < W && y < ye)
+        dz[k] = *reinterpret_cast<const bf16x8 *>(dZ + (int64_t(y) * W + x) * C + 8 * v);
     }
-    for (int q = tid; q < XV; q += WG_THREADS) {
+#pragma unroll
+    for (int k = 0; k < XP; ++k) {
+      const int q = tid + WG_THREADS * k;
       const int v = q % (CIN / 8), px = q / (CIN / 8) % XW, row = q / (CIN / 8 * XW);
       int x = x0 - 1 + px, y = y0 - 1 + row;
-      bf16x8 d = zero;
-      if (x <= W && y <= H) { // W, H: the wrapped neighbours of the last column and row
+      dx[k] = zero;
+      if (q < XV && x <= W && y <= H) { // W, H: the wrapped neighbours of the last column and row
         x = x < 0 ? x + W : (x >= W ? x - W : x);
         y = y < 0 ? y + H : (y >= H ? y - H : y);
-        d = *reinterpret_cast<const bf16x8 *>(X + (int64_t(y) * W + x) * CIN + 8 * v);
+        dx[k] = *reinterpret_cast<const bf16x8 *>(X + (int64_t(y) * W + x) * CIN + 8 * v);
       }
-      *reinterpret_cast<bf16x8 *>(sx + (row * XW + px) * CIN + 8 * v) = d;
     }
+#pragma unroll
+    for (int k = 0; k < ZP; ++k)
+      if (tid + WG_THREADS * k < ZV) *reinterpret_cast<bf16x8 *>(sz + 8 * (tid + WG_THREADS * k)) = dz[k];
+#pragma unroll
+    for (int k = 0; k < XP; ++k)
+      if (tid + WG_THREADS * k < XV) *reinterpret_cast<bf16x8 *>(sx + 8 * (tid + WG_THREADS * k)) = dx[k];
     __syncthreads();
 #pragma unroll
     for (int row = 0; row < WG_ROWS; ++row)
@@ -362,51 +490,6 @@ __global__ void __launch_bounds__(64 * WR_SLICES) k_wgrad_reduce(WgradLayers L) 
   if (dx < 3) gw[((3 * wave + dx) * C + cout) * cin + ci] = s;
 }
 
-// the velocities the predictors read: f[0] = f(y_n), ..., f[4] = f(y_{n-4})
-struct FHist {
-  const double *f[5];
-};
-
-// features: dt D^k f / s_k (k = 1, 2, 3; 2 channels each), nu_hat,
-// |dt D^4 f| / s_4
-__global__ void k_features(FHist F, double c1, double c2, double c3, double c4, double nu_hat, int64_t npix,
-                           __bf16 *__restrict__ X0) {
-  const int64_t p = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (p >= npix) return;
-  __bf16 *x = X0 + p * CIN0;
-  double n4 = 0.;
-#pragma unroll
-  for (int c = 0; c < 2; ++c) {
-    const int64_t i = 2 * p + c;
-    const double f0 = F.f[0][i], f1 = F.f[1][i], f2 = F.f[2][i], f3 = F.f[3][i], f4 = F.f[4][i];
-    const double d1 = f0 - f1, d2 = f0 - 2. * f1 + f2, d3 = f0 - 3. * f1 + 3. * f2 - f3;
-    const double d4 = f0 - 4. * f1 + 6. * f2 - 4. * f3 + f4;
-    x[c] = __bf16(float(d1 * c1));
-    x[2 + c] = __bf16(float(d2 * c2));
-    x[4 + c] = __bf16(float(d3 * c3));
-    n4 += (d4 * c4) * (d4 * c4);
-  }
-  x[6] = __bf16(float(nu_hat));
-  x[7] = __bf16(float(sqrt(n4)));
-}
-
-// sums over the blocks of the last hidden layer's per-block channel sums:
-// one block per channel
-__global__ void __launch_bounds__(256) k_chan_sums(const float *__restrict__ csum, int nblk,
-                                                   double *__restrict__ sums) {
-  __shared__ double sh[256];
-  const int c = blockIdx.x;
-  double v = 0.;
-  for (int b = threadIdx.x; b < nblk; b += 256) v += double(csum[int64_t(c) * nblk + b]);
-  sh[threadIdx.x] = v;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if (int(threadIdx.x) < o) sh[threadIdx.x] += sh[threadIdx.x + o];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) sums[c] = sh[0];
-}
-
 // a sample's costs at the orders T_j = 1 + j/2, by value
 struct Costs {
   double c[NOUT];
@@ -435,21 +518,39 @@ __device__ __forceinline__ double extrap_weight(int k, int j) {
 // (the BF16 weights the MFMAs use), from the channel sums of the last
 // hidden layer; p = softmax(-m / kTau), t = sum_j p_j T_j, the weights of
 // P(t) and m into pol; with costs c, also lg[0] = sum_j (m_j - (c_j -
-// mean c))^2 / NOUT and lg[1 + j] = d lg[0] / d m_j.  One thread.
-__global__ void k_policy(const double *__restrict__ sums, const float *__restrict__ weff,
-                         const float *__restrict__ bias, double inv_npix, Costs costs, int with_costs,
-                         double *__restrict__ pol, double *__restrict__ lg) {
-  if (threadIdx.x != 0) return;
-  double m[NOUT], mn = 1e300;
+// mean c))^2 / NOUT and lg[1 + j] = d lg[0] / d m_j.  One workgroup: 32
+// lanes per channel add the blocks' sums (FP64), 32 per output its products;
+// one thread the seven-term rest.  Latency-bound, one launch.
+__global__ void __launch_bounds__(1024) k_policy(const float *__restrict__ csum, int nblk, double *__restrict__ sums,
+                                                 const float *__restrict__ weff, const float *__restrict__ bias,
+                                                 double inv_npix, Costs costs, int with_costs,
+                                                 double *__restrict__ pol, double *__restrict__ lg) {
+  __shared__ double sc[C], m[NOUT];
+  const int ch = threadIdx.x >> 5, l = threadIdx.x & 31;
+  double v = 0.;
+#pragma unroll 4
+  for (int b = l; b < nblk; b += 32) v += double(csum[int64_t(ch) * nblk + b]);
 #pragma unroll
-  for (int c = 0; c < NOUT; ++c) {
-    double v = 0.;
-    for (int i = 0; i < C; ++i) v += double(weff[c * C + i]) * sums[i];
-    m[c] = double(bias[c]) + v * inv_npix;
-    pol[POL_M + c] = m[c];
-    mn = fmin(mn, m[c]);
+  for (int o = 16; o > 0; o >>= 1) v += __shfl_xor(v, o, 32);
+  if (l == 0) {
+    sc[ch] = v;
+    sums[ch] = v;
   }
-  double z = 0., t = 0., e[NOUT];
+  __syncthreads();
+  if (ch < NOUT) {
+    double w = double(weff[ch * C + l]) * sc[l];
+#pragma unroll
+    for (int o = 16; o > 0; o >>= 1) w += __shfl_xor(w, o, 32);
+    if (l == 0) {
+      m[ch] = double(bias[ch]) + w * inv_npix;
+      pol[POL_M + ch] = m[ch];
+    }
+  }
+  __syncthreads();
+  if (threadIdx.x != 0) return;
+  double mn = 1e300, z = 0., t = 0., e[NOUT];
+#pragma unroll
+  for (int c = 0; c < NOUT; ++c) mn = fmin(mn, m[c]);
 #pragma unroll
   for (int c = 0; c < NOUT; ++c) {
     e[c] = exp(-(m[c] - mn) / kTau);
@@ -468,17 +569,17 @@ __global__ void k_policy(const double *__restrict__ sums, const float *__restric
 #pragma unroll
   for (int j = 0; j < 5; ++j) pol[POL_E + j] = (1. - w) * extrap_weight(k, j) + w * extrap_weight(k + 1, j);
   if (with_costs) {
-    double cbar = 0., l = 0.;
+    double cbar = 0., ls = 0.;
 #pragma unroll
     for (int c = 0; c < NOUT; ++c) cbar += costs.c[c];
     cbar /= NOUT;
 #pragma unroll
     for (int c = 0; c < NOUT; ++c) {
       const double r = m[c] - (costs.c[c] - cbar);
-      l += r * r;
+      ls += r * r;
       lg[1 + c] = 2. * r / NOUT;
     }
-    lg[0] = l / NOUT;
+    lg[0] = ls / NOUT;
   }
 }
 
@@ -635,44 +736,61 @@ int history(const double *const *f, FHist *F, const char *who) {
   return PDA_OK;
 }
 
-int features(pda_guessnet_s &net, const FHist &F, double nu, hipStream_t st) {
-  hipLaunchKernelGGL(k_features, dim3(unsigned((net.npix + 255) / 256)), dim3(256), 0, st, F,
-                     net.dt / net.s[0], net.dt / net.s[1], net.dt / net.s[2], net.dt / net.s[3],
-                     (nu - net.nu_mean) / net.nu_scale, net.npix, net.X0.as<__bf16>());
-  PDA_HIP_CHECK(hipGetLastError());
-  return PDA_OK;
+Features feature_args(const pda_guessnet_s &net, const FHist &F, double nu) {
+  Features T;
+  T.F = F;
+  for (int k = 0; k < 4; ++k) T.c[k] = net.dt / net.s[k];
+  T.nu_hat = (nu - net.nu_mean) / net.nu_scale;
+  return T;
 }
 
 // the order policy of the last forward into net.pol; with costs, the
 // cost-estimate loss and its derivatives into net.lg
 int policy(pda_guessnet_s &net, const Costs *costs, hipStream_t st) {
-  const int nblk = int(net.npix / (16 * MT));
-  hipLaunchKernelGGL(k_chan_sums, dim3(C), dim3(256), 0, st, net.csum.as<float>(), nblk, net.sums.as<double>());
-  hipLaunchKernelGGL(k_policy, dim3(1), dim3(64), 0, st, net.sums.as<double>(), net.weff.as<float>(),
-                     bias_of(net, NL - 1), 1. / double(net.npix), costs ? *costs : Costs{}, costs ? 1 : 0,
-                     net.pol.as<double>(), net.lg.as<double>());
+  hipLaunchKernelGGL(k_policy, dim3(1), dim3(1024), 0, st, net.csum.as<float>(), conv_blocks(net.H, net.W),
+                     net.sums.as<double>(), net.weff.as<float>(), bias_of(net, NL - 1), 1. / double(net.npix),
+                     costs ? *costs : Costs{}, costs ? 1 : 0, net.pol.as<double>(), net.lg.as<double>());
   PDA_HIP_CHECK(hipGetLastError());
   return PDA_OK;
 }
 
-// forward through the hidden layers from the features in X0, with the
+template <int MODE>
+void conv(const pda_guessnet_s &net, ConvArgs A, const Features &T, hipStream_t st) {
+  A.H = net.H;
+  A.W = net.W;
+  A.ntx = (net.W + CT_W - 1) / CT_W;
+  const dim3 grid{unsigned(conv_blocks(net.H, net.W)), 1, 1};
+  if (conv_rows(net.H, net.W) == 4) hipLaunchKernelGGL((k_conv<MODE, 4>), grid, dim3(256), 0, st, A, T);
+  else hipLaunchKernelGGL((k_conv<MODE, 1>), grid, dim3(256), 0, st, A, T);
+}
+
+// forward through the hidden layers from the velocity history, with the
 // last one's channel sums (all the policy needs: the output layer is
-// linear); the pre-activations Z only when a backward follows; with
-// full_out, the output layer too, out = L4 (FP32 [p][NOUT])
-int forward(pda_guessnet_s &net, bool keep_z, bool full_out, hipStream_t st) {
-  const unsigned grid = unsigned(net.npix / (16 * MT));
-  const __bf16 *Wf = net.Wf.as<__bf16>();
-  hipLaunchKernelGGL((k_conv<CIN0, 2, MODE_HIDDEN>), dim3(grid), dim3(64), 0, st, net.X0.as<__bf16>(),
-                     Wf + net.foff[0], bias_of(net, 0), net.H, net.W, keep_z ? net.Z[0].as<float>() : nullptr,
-                     net.Y[0].as<__bf16>(), nullptr, nullptr, nullptr);
-  for (int l = 1; l < NL - 1; ++l)
-    hipLaunchKernelGGL((k_conv<C, 2, MODE_HIDDEN>), dim3(grid), dim3(64), 0, st, net.Y[l - 1].as<__bf16>(),
-                       Wf + net.foff[l], bias_of(net, l), net.H, net.W, keep_z ? net.Z[l].as<float>() : nullptr,
-                       net.Y[l].as<__bf16>(), nullptr, nullptr, l == NL - 2 ? net.csum.as<float>() : nullptr);
-  if (full_out)
-    hipLaunchKernelGGL((k_conv<C, 1, MODE_OUT>), dim3(grid), dim3(64), 0, st, net.Y[NL - 2].as<__bf16>(),
-                       Wf + net.foff[NL - 1], bias_of(net, NL - 1), net.H, net.W, nullptr, nullptr,
-                       net.out.as<float>(), nullptr, nullptr);
+// linear); the features and the pre-activations Z are kept only when a
+// backward follows; with full_out, the output layer too, out = L4 (FP32
+// [p][NOUT])
+int forward(pda_guessnet_s &net, const Features &T, bool keep, bool full_out, hipStream_t st) {
+  for (int l = 0; l < NL; ++l) {
+    if (l == NL - 1 && !full_out) break;
+    ConvArgs A{};
+    A.X = l == 0 ? nullptr : net.Y[l - 1].as<__bf16>();
+    A.Wp = net.Wf.as<__bf16>() + net.foff[l];
+    A.bias = bias_of(net, l);
+    if (l == NL - 1) {
+      A.out = net.out.as<float>();
+      conv<MODE_OUT>(net, A, T, st);
+      break;
+    }
+    A.Z = keep ? net.Z[l].as<float>() : nullptr;
+    A.Y = net.Y[l].as<__bf16>();
+    A.csum = l == NL - 2 ? net.csum.as<float>() : nullptr;
+    if (l == 0) {
+      A.X0 = keep ? net.X0.as<__bf16>() : nullptr;
+      conv<MODE_FIRST>(net, A, T, st);
+    } else {
+      conv<MODE_HIDDEN>(net, A, T, st);
+    }
+  }
   PDA_HIP_CHECK(hipGetLastError());
   return PDA_OK;
 }
@@ -683,7 +801,6 @@ int forward(pda_guessnet_s &net, bool keep_z, bool full_out, hipStream_t st) {
 // conv flipped transposed W_l) * SiLU'(Z_{l-1}), alternating between dZa and
 // dZb; the sums of the three layers are reduced together at the end.
 int backward(pda_guessnet_s &net, hipStream_t st) {
-  const unsigned grid = unsigned(net.npix / (16 * MT));
   const WgradGrid G = wgrad_grid(net.H, net.W);
   float *gW = net.g.as<float>();
   const __bf16 *Wb = net.Wb.as<__bf16>();
@@ -709,8 +826,12 @@ int backward(pda_guessnet_s &net, hipStream_t st) {
     part += int64_t(G.nwg) * wg_sums(cin);
     PDA_HIP_CHECK(hipGetLastError());
     if (l == 0) break;
-    hipLaunchKernelGGL((k_conv<C, 2, MODE_BWD>), dim3(grid), dim3(64), 0, st, dz, Wb + net.boff[l], nullptr,
-                       net.H, net.W, nullptr, dz_next, nullptr, net.Z[l - 1].as<float>(), nullptr);
+    ConvArgs A{};
+    A.X = dz;
+    A.Wp = Wb + net.boff[l];
+    A.Y = dz_next;
+    A.Zprev = net.Z[l - 1].as<float>();
+    conv<MODE_BWD>(net, A, Features{}, st);
     PDA_HIP_CHECK(hipGetLastError());
     std::swap(dz, dz_next);
   }
@@ -793,7 +914,7 @@ int pda_guessnet_create(int nx, int ny, pda_guessnet *out) {
   if (e == hipSuccess) e = net->out.alloc(sizeof(float) * np * NOUT);
   if (e == hipSuccess)
     e = net->part.alloc(sizeof(float) * size_t(wgrad_grid(ny, nx).nwg) * (wg_sums(CIN0) + (NL - 2) * wg_sums(C)));
-  if (e == hipSuccess) e = net->csum.alloc(sizeof(float) * (np / (16 * MT)) * C);
+  if (e == hipSuccess) e = net->csum.alloc(sizeof(float) * size_t(conv_blocks(ny, nx)) * C);
   if (e == hipSuccess) e = net->sums.alloc(sizeof(double) * C);
   if (e == hipSuccess) e = net->weff.alloc(sizeof(float) * NOUT * C);
   if (e == hipSuccess) e = net->pol.alloc(sizeof(double) * POL_LEN);
@@ -868,8 +989,7 @@ int pda_guessnet_predict(pda_guessnet net, const double *d_un, const double *d_u
   int rc = history(d_f, &F, "pda_guessnet_predict");
   if (rc) return rc;
   hipStream_t st = hipStream_t(stream);
-  rc = features(*net, F, nu, st);
-  if (!rc) rc = forward(*net, false, false, st);
+  rc = forward(*net, feature_args(*net, F, nu), false, false, st);
   if (!rc) rc = policy(*net, nullptr, st);
   if (rc) return rc;
   const int64_t n = net->npix * NCOMP;
@@ -905,8 +1025,7 @@ int pda_guessnet_gradients(pda_guessnet net, const double *const *d_f, double nu
   if (!rc) rc = check_costs(costs, "pda_guessnet_gradients");
   if (rc) return rc;
   hipStream_t st = hipStream_t(stream);
-  rc = features(*net, F, nu, st);
-  if (!rc) rc = forward(*net, true, outv != nullptr, st);
+  rc = forward(*net, feature_args(*net, F, nu), true, outv != nullptr, st);
   if (!rc) rc = loss(*net, costs, lossv, st);
   if (!rc) rc = backward(*net, st);
   if (rc) return rc;
@@ -929,8 +1048,7 @@ int pda_guessnet_train_step(pda_guessnet net, const double *const *d_f, double n
   if (!rc) rc = check_costs(costs, "pda_guessnet_train_step");
   if (rc) return rc;
   hipStream_t st = hipStream_t(stream);
-  rc = features(*net, F, nu, st);
-  if (!rc) rc = forward(*net, true, false, st);
+  rc = forward(*net, feature_args(*net, F, nu), true, false, st);
   if (!rc) rc = loss(*net, costs, lossv, st);
   if (!rc) rc = backward(*net, st);
   if (rc) return rc;

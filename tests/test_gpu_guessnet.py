@@ -177,7 +177,7 @@ def test_batch_autotune_validates_state(torch):
         b.autotune(torch.zeros(b.total, dtype=torch.float32, device="cuda"))
 
 
-@pytest.mark.parametrize("W,H", [(4, 128), (128, 4), (64, 8), (100, 128), (72, 64), (65 * 8, 64)])
+@pytest.mark.parametrize("W,H", [(4, 128), (128, 4), (64, 8), (100, 128), (72, 64), (65 * 8, 64), (33 * 16, 256)])
 def test_gradients_on_ragged_grids(torch, W, H):
     """The backward-weight kernel's bands of 64 columns and groups of 4 rows:
     partial bands, fewer rows than a group, several workgroups per band.
