@@ -27,7 +27,7 @@ COMMON = [
     "-Wall", "-Wno-unused-function", "-Wno-unused-variable",
 ]
 
-SOURCES = ["pda_mesh.cpp", "pda_problem.cpp", "pda_kernels.hip", "pda_box_kernels.hip",
+SOURCES = ["pda_mesh.cpp", "pda_problem.cpp", "pda_kernels.hip", "pda_box_kernels.hip", "pda_apply.hip",
            "pda_stepper.hip", "pda_implicit.hip",
            "pda_guessnet.hip", "pda_batch.hip", "pda_noalloc.hip"]
 

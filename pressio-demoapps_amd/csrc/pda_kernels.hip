@@ -1,8 +1,8 @@
 // pda_kernels.hip -- generic kernels of the finite-volume hot path (any
-// mesh: full, sample/stencil, 1D/2D/3D): velocity (residual), Jacobian
-// assembly into the fixed CSR pattern, and the Jacobian action, plus the
-// launch logic that pairs them with the structured box kernels.  The per-row
-// device code is in pda_rows.hpp.
+// mesh: full, sample/stencil, 1D/2D/3D): velocity (residual) and Jacobian
+// assembly into the fixed CSR pattern, plus the launch logic that pairs them
+// with the structured box kernels.  The per-row device code is in
+// pda_rows.hpp.
 #include "pda_rows.hpp"
 
 namespace pda {
@@ -935,25 +935,6 @@ int jac_weno_tiled(const View &v, const Box &B, int w, const double *U, double *
   return w == 2 ? launch_jac_weno_tiled<Ph, 2>(v, B, U, V, J, s) : launch_jac_weno_tiled<Ph, 3>(v, B, U, V, J, s);
 }
 
-// ------------------------------------------------- Jacobian action (SpMM)
-// AJ = J * B.  One thread per (scalar row, column of B).
-__global__ void k_apply(const int64_t *__restrict__ rowptr, const int32_t *__restrict__ col,
-                        const double *__restrict__ J, const double *__restrict__ B,
-                        int64_t nrows, int64_t ncolsB, int64_t ldB_rows, int layout,
-                        double *__restrict__ AJ) {
-  const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= nrows * ncolsB) return;
-  const int64_t row = layout == 0 ? t % nrows : t / ncolsB;
-  const int64_t c = layout == 0 ? t / nrows : t % ncolsB;
-  double s = 0.;
-  for (int64_t e = rowptr[row]; e < rowptr[row + 1]; ++e) {
-    const int64_t bi = col[e];
-    s += J[e] * (layout == 0 ? B[c * ldB_rows + bi] : B[bi * ncolsB + c]);
-  }
-  if (layout == 0) AJ[c * nrows + row] = s;
-  else AJ[row * ncolsB + c] = s;
-}
-
 }  // namespace
 
 template <class Ph>
@@ -1291,20 +1272,6 @@ int launch_jacobian(const pda_problem_s &p, const double *U, double, double *J, 
   int rc = launch_jacobian_box(p, U, J, V, s, &rest_done);
   if (rc || rest_done || p.h_rem_rows.empty()) return rc;
   return jac_generic(generic_view(p, &p.d_rem_rows, int64_t(p.h_rem_rows.size())), p, U, V, J, s);
-}
-
-int launch_apply(const pda_problem_s &p, const double *J, const double *B, int64_t ncols,
-                 int layout, double *AJ, hipStream_t s) {
-  const int64_t nrows = p.view.nrows * p.m;
-  const int64_t ldb = p.mesh->n_stencil * p.m;
-  const int64_t n = nrows * ncols;
-  if (n == 0) return PDA_OK;
-  const int bs = 256;
-  hipLaunchKernelGGL(k_apply, dim3(unsigned((n + bs - 1) / bs)), dim3(bs), 0, s,
-                     p.d_rowptr.as<int64_t>(), p.d_colidx.as<int32_t>(), J, B, nrows, ncols, ldb,
-                     layout, AJ);
-  PDA_HIP_CHECK(hipGetLastError());
-  return PDA_OK;
 }
 
 }  // namespace pda

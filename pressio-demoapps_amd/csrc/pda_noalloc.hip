@@ -63,9 +63,9 @@ int pda_apply_jacobian_noalloc(pda_problem p, const double *d_U, double t, const
               " this entry point holds; use pda_apply_jacobian");
     return PDA_E_INVALID_ARG;
   }
-  // the problem's index tables and scalar CSR pattern are uploaded by the
-  // allocating entry points on first use; this one only reads them
-  if (!p->on_device || !p->d_rowptr.ptr) {
+  // the problem's index tables are uploaded by the allocating entry points on
+  // first use; this one only reads them
+  if (!p->on_device || !(p->d_rowptr.ptr || p->applied)) {
     set_error("pda_apply_jacobian_noalloc: the problem's device tables are not built; call "
               "pda_jacobian_pattern (or pda_apply_jacobian) once before");
     return PDA_E_STATE;

@@ -756,8 +756,11 @@ int pda_apply_jacobian(pda_problem p, const double *d_U, double t, const double 
     set_error("pda_apply_jacobian: invalid argument");
     return PDA_E_INVALID_ARG;
   }
-  int rc = ensure_scalar_pattern(*p);
+  // the block tables are enough: the scalar pattern (12 bytes a nonzero, built
+  // on the host) is not made for this
+  int rc = ensure_device(*p);
   if (rc) return rc;
+  p->applied = true;
   if (p->d_scratch_v.bytes < sizeof(double) * size_t(p->nnz))
     PDA_HIP_CHECK(p->d_scratch_v.alloc(sizeof(double) * size_t(p->nnz)));
   rc = launch_jacobian(*p, d_U, t, p->d_scratch_v.as<double>(), nullptr, hipStream_t(stream));
