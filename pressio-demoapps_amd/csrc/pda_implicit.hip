@@ -24,11 +24,15 @@ namespace pda {
 namespace {
 
 constexpr int TB = 256; // threads per block of the vector kernels
+constexpr int MAXB = 1024; // most blocks (partial sums) of the reducing kernels
 
-// scalar slots of the Krylov solver
+// Device scalars of the Krylov solver.  Each is written by the first block of
+// one kernel and read by the kernels after it (never by the one that writes
+// it): the search kernel writes RHO_NEXT, RR and DONE_NEXT, the
+// preconditioned-residual kernel RHO, ALPHA and DONE, the update kernel W and
+// NITER.
 enum {
-  S_RHO = 0, S_RHO_OLD, S_ALPHA, S_W, S_BETA, S_R0V, S_TS, S_TT, S_RR, S_BB, S_TOL2, S_DONE,
-  S_NITER, S_COUNT
+  S_RHO = 0, S_RHO_NEXT, S_ALPHA, S_W, S_RR, S_BB, S_TOL2, S_DONE, S_DONE_NEXT, S_NITER, S_CF, S_CNP1, S_COUNT
 };
 
 __device__ __forceinline__ double block_sum(double v, double *sh) {
@@ -38,21 +42,25 @@ __device__ __forceinline__ double block_sum(double v, double *sh) {
   if (l == 0) sh[w] = v;
   __syncthreads();
   double s = 0.;
-  if (threadIdx.x == 0)
-    for (int i = 0; i < int(blockDim.x >> 6); ++i) s += sh[i];
-  return s; // valid in thread 0
+  for (int i = 0; i < TB / 64; ++i) s += sh[i];
+  return s; // the same in every thread
 }
 
-// partial dot products (a.b, c.d) per block; part[2*blk], part[2*blk+1]
-__global__ void __launch_bounds__(TB) k_dot2(const double *__restrict__ a, const double *__restrict__ b,
-                                              const double *__restrict__ c, const double *__restrict__ d,
-                                              int64_t n, double *__restrict__ part) {
-  __shared__ double sh[TB / 64];
-  double s1 = 0., s2 = 0.;
-  for (int64_t i = int64_t(blockIdx.x) * TB + threadIdx.x; i < n; i += int64_t(gridDim.x) * TB) {
-    s1 += a[i] * b[i];
-    if (c) s2 += c[i] * d[i];
+// The sums of n pairs of partial sums, in a fixed order, the same in every
+// thread of every block: a kernel that needs a dot product reduces the
+// partial sums of the kernel that formed it by itself (16 KB from L2, about
+// 1.5 us), where a launch of one block to do it took 4.6 us and a gap.
+__device__ __forceinline__ void sum_pairs(const double *__restrict__ part, int n, double *sh, double &s1, double &s2) {
+  double a = 0., b = 0.;
+  for (int i = threadIdx.x; i < n; i += TB) {
+    a += part[2 * i];
+    b += part[2 * i + 1];
   }
+  s1 = block_sum(a, sh);
+  s2 = block_sum(b, sh);
+}
+
+__device__ __forceinline__ void put_pair(double *part, double s1, double s2, double *sh) {
   s1 = block_sum(s1, sh);
   s2 = block_sum(s2, sh);
   if (threadIdx.x == 0) {
@@ -61,114 +69,153 @@ __global__ void __launch_bounds__(TB) k_dot2(const double *__restrict__ a, const
   }
 }
 
-// y = A x (scalar CSR) with LPR lanes per row: the lanes of a row read its
-// values and column indices as contiguous runs; a row's sum is reduced with
-// lane shuffles.  Grid-stride over row groups (at most MAXB blocks), with
-// optional per-block partial dots (d1 . y) and (y . y).  (Reading one column
-// index per m x m block instead of one per value measured no faster.)
-constexpr int MAXB = 2048;
-
-template <int LPR>
-__global__ void __launch_bounds__(TB) k_spmv(const int64_t *__restrict__ rp, const int32_t *__restrict__ ci,
-                                              const double *__restrict__ A, const double *__restrict__ x,
-                                              double *__restrict__ y, int64_t n,
-                                              const double *__restrict__ d1, int want_yy,
-                                              double *__restrict__ part, const double *__restrict__ scal) {
+// partial sums of a.a (the second of the pair unused)
+__global__ void __launch_bounds__(TB) k_norm(const double *__restrict__ a, int64_t n, double *__restrict__ part) {
   __shared__ double sh[TB / 64];
-  constexpr int RPB = TB / LPR; // rows per block pass
-  const bool done = scal && scal[S_DONE] != 0.;
-  const int g = threadIdx.x / LPR, l = threadIdx.x % LPR;
+  double s = 0.;
+  for (int64_t i = int64_t(blockIdx.x) * TB + threadIdx.x; i < n; i += int64_t(gridDim.x) * TB) s += a[i] * a[i];
+  put_pair(part, s, 0., sh);
+}
+
+// the norms of up to two vectors from their partial sums, into host memory
+__global__ void __launch_bounds__(TB) k_norms_out(const double *__restrict__ pa, const double *__restrict__ pb, int n,
+                                                  double *__restrict__ host) {
+  __shared__ double sh[TB / 64];
+  double s1, s2;
+  sum_pairs(pa, n, sh, s1, s2);
+  if (threadIdx.x == 0) host[0] = sqrt(s1);
+  if (!pb) return;
+  sum_pairs(pb, n, sh, s1, s2);
+  if (threadIdx.x == 0) host[1] = sqrt(s1);
+}
+
+// sum over the 16 (or 8) lanes of a DPP row, in every lane of it
+template <int CTRL> __device__ __forceinline__ double dpp_add(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, int(b), CTRL, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, int(b >> 32), CTRL, 0xf, 0xf, false);
+  return v + __longlong_as_double((long long)(unsigned(lo)) | ((long long)hi << 32));
+}
+template <int L> __device__ __forceinline__ double lanes_sum(double v) {
+  static_assert(L == 8 || L == 16, "half a DPP row or one");
+  v = dpp_add<0xB1>(v);  // quad_perm 1,0,3,2
+  v = dpp_add<0x4E>(v);  // quad_perm 2,3,0,1
+  v = dpp_add<0x141>(v); // row_half_mirror
+  if constexpr (L == 16) v = dpp_add<0x140>(v); // row_mirror
+  return v;
+}
+
+// The index tables of the Jacobian's blocks
+struct Blocks {
+  const int64_t *rowbase;
+  const int32_t *nblk, *bcol;
+  const int64_t *diag; // first value of the diagonal block, per cell
+  int maxb;
+  int64_t ncell;
+};
+
+// y = (cnp1 I + cf J) x by blocks: L lanes per cell, a lane per M x M block
+// (its M rows of M values and the M values of x they multiply, one column-cell
+// index for all of them), the lanes' sums added by DPP.  The Newton matrix is
+// not formed: cf and cnp1 enter here.  A block of threads takes a contiguous
+// range of cells, and the ranges of one XCD are neighbours, so that x is read
+// into each L2 once; several cells' loads are in flight per lane.  Bound by the
+// matrix: 512 x 512 Burgers (13 2 x 2 blocks a cell, 109 MB of values and 14 MB
+// of indices) 23.8 us (5.2 TB/s), 47.2 us walking the scalar CSR with 32 lanes a row (164 MB).
+// Partial sums of (d1 . y) and, with want_yy, (y . y).
+template <int M> constexpr int spmv_cells() { return M <= 2 ? 4 : M <= 4 ? 2 : 1; } // in flight per lane
+
+template <int M, int L>
+__global__ void __launch_bounds__(TB) k_spmv(Blocks K, const double *__restrict__ J, const double *__restrict__ x,
+                                             double *__restrict__ y, int64_t per_block,
+                                             const double *__restrict__ d1, int want_yy, double *__restrict__ part,
+                                             const double *__restrict__ scal) {
+  __shared__ double sh[TB / 64];
+  constexpr int CPB = TB / L, NU = spmv_cells<M>();
+  if (scal[S_DONE_NEXT] != 0.) return;
+  const double cf = scal[S_CF], cnp1 = scal[S_CNP1];
+  const int l = threadIdx.x % L, g = threadIdx.x / L;
+  // block -> range: the blocks of XCD b % 8 take neighbouring ranges
+  const int nbk = gridDim.x, q = nbk / 8, rem = nbk % 8, xcd = int(blockIdx.x) % 8, kk = int(blockIdx.x) / 8;
+  const int64_t range = int64_t(xcd) * q + (xcd < rem ? xcd : rem) + kk;
+  const int64_t c_lo = range * per_block, c_hi = c_lo + per_block < K.ncell ? c_lo + per_block : K.ncell;
   double s1 = 0., s2 = 0.;
-  if (!done) {
-    for (int64_t base = int64_t(blockIdx.x) * RPB; base < n; base += int64_t(gridDim.x) * RPB) {
-      const int64_t i = base + g;
-      double acc = 0.;
-      if (i < n)
-        for (int64_t j = rp[i] + l; j < rp[i + 1]; j += LPR) acc += A[j] * x[ci[j]];
+  for (int64_t base = c_lo; base < c_hi; base += CPB * NU) {
+    double acc[NU][M];
+    int64_t cell[NU], rb[NU];
+    int nb[NU];
 #pragma unroll
-      for (int o = LPR / 2; o > 0; o >>= 1) acc += __shfl_xor(acc, o, LPR);
-      if (i < n && l == 0) {
-        y[i] = acc;
-        if (d1) s1 += d1[i] * acc;
-        if (want_yy) s2 += acc * acc;
+    for (int u = 0; u < NU; ++u) {
+      const int64_t c = base + u * CPB + g;
+      cell[u] = c < c_hi ? c : c_hi - 1;
+      nb[u] = c < c_hi ? K.nblk[cell[u]] : 0;
+      rb[u] = K.rowbase[cell[u]];
+#pragma unroll
+      for (int k = 0; k < M; ++k) acc[u][k] = 0.;
+    }
+    for (int s0 = 0; s0 < K.maxb; s0 += L) {
+      const int s = s0 + l;
+      double a[NU][M * M], v[NU][M];
+#pragma unroll
+      for (int u = 0; u < NU; ++u) {
+        const bool on = s < nb[u];
+        const int ss = on ? s : 0;
+        const double *xc = x + int64_t(K.bcol[cell[u] * K.maxb + ss]) * M;
+        const double *Jr = J + rb[u] + ss * M;
+#pragma unroll
+        for (int k = 0; k < M; ++k)
+#pragma unroll
+          for (int j = 0; j < M; ++j) a[u][k * M + j] = Jr[int64_t(k) * nb[u] * M + j];
+#pragma unroll
+        for (int j = 0; j < M; ++j) v[u][j] = on ? xc[j] : 0.;
+      }
+#pragma unroll
+      for (int u = 0; u < NU; ++u) {
+        const bool on = s < nb[u];
+#pragma unroll
+        for (int k = 0; k < M; ++k) {
+          double t = 0.;
+#pragma unroll
+          for (int j = 0; j < M; ++j) t += a[u][k * M + j] * v[u][j];
+          acc[u][k] += on ? t : 0.;
+        }
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      double mine = 0.;
+#pragma unroll
+      for (int k = 0; k < M; ++k) {
+        const double t = lanes_sum<L>(acc[u][k]);
+        if (l == k) mine = t;
+      }
+      if (l < M && base + u * CPB + g < c_hi) {
+        const int64_t i = cell[u] * M + l;
+        const double yi = cf * mine + cnp1 * x[i];
+        y[i] = yi;
+        s1 += d1[i] * yi;
+        if (want_yy) s2 += yi * yi;
       }
     }
   }
-  if (part) {
-    s1 = block_sum(s1, sh);
-    s2 = block_sum(s2, sh);
-    if (threadIdx.x == 0) {
-      part[2 * blockIdx.x] = s1;
-      part[2 * blockIdx.x + 1] = s2;
-    }
-  }
+  put_pair(part, s1, s2, sh);
 }
 
-// Reduce the block partials (deterministic order) and advance the solver's
-// scalars.  stage 0: after r changed (rr, rho, beta, convergence);
-// 1: alpha = rho / (r0.v); 2: w = (t.s)/(t.t); 3: initial (bb, tol2).
-__global__ void __launch_bounds__(TB) k_finish(const double *__restrict__ part, int nblk, int stage,
-                                                double *__restrict__ scal, double rtol) {
-  __shared__ double sh[TB / 64];
-  double s1 = 0., s2 = 0.;
-  for (int i = threadIdx.x; i < nblk; i += TB) {
-    s1 += part[2 * i];
-    s2 += part[2 * i + 1];
-  }
-  s1 = block_sum(s1, sh);
-  s2 = block_sum(s2, sh);
-  if (threadIdx.x != 0) return;
-  if (stage == 3) {
-    // s1 = r0.r = b.b (x0 = 0)
-    scal[S_BB] = s1;
-    scal[S_TOL2] = rtol * rtol * s1;
-    scal[S_RHO] = 1.;
-    scal[S_ALPHA] = 1.;
-    scal[S_W] = 1.;
-    scal[S_NITER] = 0.;
-    scal[S_DONE] = (s1 == 0.) ? 1. : 0.;
-    return;
-  }
-  if (scal[S_DONE] != 0.) return;
-  if (stage == 0) {
-    // s1 = r0.r, s2 = r.r; a non-finite reduction (a breakdown, or NaN in
-    // the system) also ends the solve, whose result the Newton loop rejects
-    scal[S_RR] = s2;
-    if (s2 <= scal[S_TOL2] || !isfinite(s1) || !isfinite(s2)) {
-      scal[S_DONE] = 1.;
-      return;
-    }
-    scal[S_RHO_OLD] = scal[S_RHO];
-    scal[S_RHO] = s1;
-    scal[S_BETA] = (s1 / scal[S_RHO_OLD]) * (scal[S_ALPHA] / scal[S_W]);
-    scal[S_NITER] += 1.;
-  } else if (stage == 1) {
-    scal[S_R0V] = s1;
-    scal[S_ALPHA] = scal[S_RHO] / s1;
-  } else {
-    scal[S_TS] = s1;
-    scal[S_TT] = s2;
-    scal[S_W] = s2 > 0. ? s1 / s2 : 0.;
-  }
-}
-
-// Inverse of the m x m diagonal block of every cell (Gauss-Jordan with
-// partial pivoting); in each of the cell's scalar rows the block is the m
-// consecutive values starting at column cell*m.
+// Inverse of the m x m diagonal block of cnp1 I + cf J of every cell
+// (Gauss-Jordan with partial pivoting)
 template <int M>
-__global__ void __launch_bounds__(TB) k_block_inv(const int64_t *__restrict__ diag,
-                                                   const double *__restrict__ A, int64_t ncell,
+__global__ void __launch_bounds__(TB) k_block_inv(Blocks K, const double *__restrict__ J, double cf, double cnp1,
                                                    double *__restrict__ Minv) {
   const int64_t c = int64_t(blockIdx.x) * TB + threadIdx.x;
-  if (c >= ncell) return;
+  if (c >= K.ncell) return;
   double a[M][2 * M];
+  const int64_t pos = K.diag[c];
+  const int rs = K.nblk[c] * M;
 #pragma unroll
   for (int k = 0; k < M; ++k) {
-    // the diagonal block's row k starts k entries before the diagonal entry
-    const int64_t pos = diag[c * M + k] - k;
 #pragma unroll
     for (int j = 0; j < M; ++j) {
-      a[k][j] = A[pos + j];
+      a[k][j] = cf * J[pos + int64_t(k) * rs + j] + (j == k ? cnp1 : 0.);
       a[k][M + j] = (j == k) ? 1. : 0.;
     }
   }
@@ -208,15 +255,69 @@ __global__ void __launch_bounds__(TB) k_block_inv(const int64_t *__restrict__ di
     for (int j = 0; j < M; ++j) Minv[(c * M + k) * M + j] = a[k][M + j];
 }
 
-// p = r + beta (p - w v); y = Minv p          (per cell)
+// start of a solve: x = 0, r = r0 = -R; partial sums of r0 . r twice (r0 . r
+// and r . r); the matrix's coefficients and cleared flags for the iterations
+__global__ void __launch_bounds__(TB) k_start(const double *__restrict__ R, double *__restrict__ x,
+                                              double *__restrict__ r, double *__restrict__ r0, int64_t n, double cf,
+                                              double cnp1, double *__restrict__ part, double *__restrict__ scal) {
+  __shared__ double sh[TB / 64];
+  double s = 0.;
+  for (int64_t i = int64_t(blockIdx.x) * TB + threadIdx.x; i < n; i += int64_t(gridDim.x) * TB) {
+    const double b = -R[i];
+    x[i] = 0.;
+    r[i] = b;
+    r0[i] = b;
+    s += b * b;
+  }
+  put_pair(part, s, s, sh);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    scal[S_RHO] = 1.;
+    scal[S_ALPHA] = 1.;
+    scal[S_W] = 1.;
+    scal[S_NITER] = 0.;
+    scal[S_DONE] = 0.;
+    scal[S_DONE_NEXT] = 0.;
+    scal[S_CF] = cf;
+    scal[S_CNP1] = cnp1;
+  }
+}
+
+// whether a residual with (r0.r, r.r) = (s1, s2) ends the solve: converged, or
+// a non-finite reduction (a breakdown, or NaN in the system), whose result
+// the Newton loop rejects
+__device__ __forceinline__ bool ends(double s1, double s2, double tol2) {
+  return s2 <= tol2 || !isfinite(s1) || !isfinite(s2);
+}
+
+// The search direction: beta from the partial sums of (r0 . r, r . r), or, in
+// the first iteration, the tolerance from those of b . b;
+// p = r + beta (p - w v), y = Minv p          (per cell)
 template <int M>
 __global__ void __launch_bounds__(TB) k_p_prec(const double *__restrict__ r, double *__restrict__ p,
                                                 const double *__restrict__ v, const double *__restrict__ Minv,
                                                 double *__restrict__ y, int64_t ncell,
-                                                const double *__restrict__ scal, int first) {
+                                                const double *__restrict__ part, int npart, double *__restrict__ scal,
+                                                int first, double rtol) {
+  __shared__ double sh[TB / 64];
+  if (scal[S_DONE] != 0.) return; // written by earlier kernels: the same in every block
+  const double alpha = scal[S_ALPHA], w = scal[S_W], rho = scal[S_RHO];
+  double s1, s2;
+  sum_pairs(part, npart, sh, s1, s2);
+  const double tol2 = first ? rtol * rtol * s1 : scal[S_TOL2];
+  const bool done = ends(s1, s2, tol2) || (first && s1 == 0.);
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    if (first) {
+      scal[S_BB] = s1;
+      scal[S_TOL2] = tol2;
+    }
+    scal[S_RR] = s2;
+    scal[S_RHO_NEXT] = s1;
+    scal[S_DONE_NEXT] = done ? 1. : 0.;
+  }
+  if (done) return;
+  const double beta = (s1 / rho) * (alpha / w);
   const int64_t c = int64_t(blockIdx.x) * TB + threadIdx.x;
-  if (c >= ncell || scal[S_DONE] != 0.) return;
-  const double beta = scal[S_BETA], w = scal[S_W];
+  if (c >= ncell) return;
   double pc[M];
 #pragma unroll
   for (int k = 0; k < M; ++k) {
@@ -233,15 +334,29 @@ __global__ void __launch_bounds__(TB) k_p_prec(const double *__restrict__ r, dou
   }
 }
 
-// s = r - alpha v; z = Minv s                 (per cell)
+// alpha = rho / (r0 . v) from its partial sums; s = r - alpha v; z = Minv s
 template <int M>
 __global__ void __launch_bounds__(TB) k_s_prec(const double *__restrict__ r, const double *__restrict__ v,
                                                 const double *__restrict__ Minv, double *__restrict__ s,
                                                 double *__restrict__ z, int64_t ncell,
-                                                const double *__restrict__ scal) {
+                                                const double *__restrict__ part, int npart,
+                                                double *__restrict__ scal) {
+  __shared__ double sh[TB / 64];
+  const double dn = scal[S_DONE_NEXT], rho = scal[S_RHO_NEXT];
+  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+  if (dn != 0.) {
+    if (lead) scal[S_DONE] = 1.;
+    return;
+  }
+  double s1, s2;
+  sum_pairs(part, npart, sh, s1, s2);
+  const double alpha = rho / s1;
+  if (lead) {
+    scal[S_RHO] = rho;
+    scal[S_ALPHA] = alpha;
+  }
   const int64_t c = int64_t(blockIdx.x) * TB + threadIdx.x;
-  if (c >= ncell || scal[S_DONE] != 0.) return;
-  const double alpha = scal[S_ALPHA];
+  if (c >= ncell) return;
   double sc[M];
 #pragma unroll
   for (int k = 0; k < M; ++k) {
@@ -258,56 +373,79 @@ __global__ void __launch_bounds__(TB) k_s_prec(const double *__restrict__ r, con
   }
 }
 
-// x += alpha y + w z; r = s - w t; partial dots (r0.r, r.r)
+// w = (t . s) / (t . t) from their partial sums; x += alpha y + w z;
+// r = s - w t; partial sums of (r0 . r, r . r)
 __global__ void __launch_bounds__(TB) k_xr(double *__restrict__ x, double *__restrict__ r,
                                             const double *__restrict__ y, const double *__restrict__ z,
                                             const double *__restrict__ s, const double *__restrict__ t,
                                             const double *__restrict__ r0, int64_t n,
-                                            double *__restrict__ part, const double *__restrict__ scal) {
+                                            const double *__restrict__ part_in, int npart,
+                                            double *__restrict__ part, double *__restrict__ scal) {
   __shared__ double sh[TB / 64];
-  const bool done = scal[S_DONE] != 0.;
+  if (scal[S_DONE_NEXT] != 0.) return; // the last residual's partial sums stay
+  const double alpha = scal[S_ALPHA];
+  double ts, tt;
+  sum_pairs(part_in, npart, sh, ts, tt);
+  const double w = tt > 0. ? ts / tt : 0.;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    scal[S_W] = w;
+    scal[S_NITER] += 1.; // read by no other block
+  }
   double s1 = 0., s2 = 0.;
-  if (!done) {
-    const double alpha = scal[S_ALPHA], w = scal[S_W];
-    for (int64_t i = int64_t(blockIdx.x) * TB + threadIdx.x; i < n; i += int64_t(gridDim.x) * TB) {
-      x[i] += alpha * y[i] + w * z[i];
-      const double ri = s[i] - w * t[i];
-      r[i] = ri;
-      s1 += r0[i] * ri;
-      s2 += ri * ri;
-    }
-  }
-  s1 = block_sum(s1, sh);
-  s2 = block_sum(s2, sh);
-  if (threadIdx.x == 0) {
-    part[2 * blockIdx.x] = s1;
-    part[2 * blockIdx.x + 1] = s2;
-  }
-}
-
-// A = cf * J + cnp1 * I in place: scale every value, then add cnp1 at the
-// diagonal positions
-__global__ void __launch_bounds__(TB) k_scale(double *__restrict__ A, int64_t nnz, double cf) {
-  for (int64_t j = int64_t(blockIdx.x) * TB + threadIdx.x; j < nnz; j += int64_t(gridDim.x) * TB)
-    A[j] = cf * A[j];
-}
-__global__ void __launch_bounds__(TB) k_add_diag(double *__restrict__ A, const int64_t *__restrict__ diag,
-                                                  int64_t n, double cnp1) {
-  for (int64_t i = int64_t(blockIdx.x) * TB + threadIdx.x; i < n; i += int64_t(gridDim.x) * TB)
-    A[diag[i]] += cnp1;
-}
-
-// out = sum_k c_k x_k (up to 4 terms, null x skipped)
-__global__ void __launch_bounds__(TB) k_comb(double *out, const double *x0, double c0, const double *x1,
-                                              double c1, const double *x2, double c2, const double *x3,
-                                              double c3, int64_t n) {
   for (int64_t i = int64_t(blockIdx.x) * TB + threadIdx.x; i < n; i += int64_t(gridDim.x) * TB) {
-    double v = c0 * x0[i];
-    if (x1) v += c1 * x1[i];
-    if (x2) v += c2 * x2[i];
-    if (x3) v += c3 * x3[i];
-    out[i] = v;
+    x[i] += alpha * y[i] + w * z[i];
+    const double ri = s[i] - w * t[i];
+    r[i] = ri;
+    s1 += r0[i] * ri;
+    s2 += ri * ri;
   }
+  put_pair(part, s1, s2, sh);
+}
+
+// the state of the solve after the last update, into host memory
+enum { H_DONE = 0, H_NITER, H_RR, H_BB, H_COUNT };
+__global__ void __launch_bounds__(TB) k_check(const double *__restrict__ part, int npart,
+                                              const double *__restrict__ scal, double *__restrict__ host) {
+  __shared__ double sh[TB / 64];
+  double s1, s2;
+  sum_pairs(part, npart, sh, s1, s2);
+  if (threadIdx.x != 0) return;
+  host[H_DONE] = scal[S_DONE_NEXT] != 0. || ends(s1, s2, scal[S_TOL2]) ? 1. : 0.;
+  host[H_NITER] = scal[S_NITER];
+  host[H_RR] = s2;
+  host[H_BB] = scal[S_BB];
+}
+
+// R = cnp1 y + cn y_n + c2 x2 + cf f, with partial sums of R . R
+__global__ void __launch_bounds__(TB) k_residual(double *__restrict__ R, const double *__restrict__ Y, double cnp1,
+                                                 const double *__restrict__ Yn, double cn,
+                                                 const double *__restrict__ x2, double c2,
+                                                 const double *__restrict__ F, double cf, int64_t n,
+                                                 double *__restrict__ part) {
+  __shared__ double sh[TB / 64];
+  double s = 0.;
+  for (int64_t i = int64_t(blockIdx.x) * TB + threadIdx.x; i < n; i += int64_t(gridDim.x) * TB) {
+    double v = cnp1 * Y[i];
+    v += cn * Yn[i];
+    if (x2) v += c2 * x2[i];
+    v += cf * F[i];
+    R[i] = v;
+    s += v * v;
+  }
+  put_pair(part, s, 0., sh);
+}
+
+// Y += dx, with partial sums of dx . dx
+__global__ void __launch_bounds__(TB) k_correct(double *__restrict__ Y, const double *__restrict__ dx, int64_t n,
+                                                double *__restrict__ part) {
+  __shared__ double sh[TB / 64];
+  double s = 0.;
+  for (int64_t i = int64_t(blockIdx.x) * TB + threadIdx.x; i < n; i += int64_t(gridDim.x) * TB) {
+    const double d = dx[i];
+    Y[i] += d;
+    s += d * d;
+  }
+  put_pair(part, s, 0., sh);
 }
 
 unsigned grid_of(int64_t n) { return unsigned(std::max<int64_t>(1, (n + TB - 1) / TB)); }
@@ -325,113 +463,112 @@ struct pda_implicit_s {
   int max_newton = 100;
   double lin_rtol = 1e-14;
   int lin_max = 0;          // 0: 2 * unknowns (Eigen's default)
-  int check_every = 4;      // iterations between convergence polls
-  pda::DevBuf J, F, Fn, R, Y, Yn, dx, r, r0, p, v, s, t, y, z, Minv, part, scal;
-  pda::DevBuf diag;         // position of the diagonal entry of every scalar row
-  int lpr = 32;             // SpMV lanes per row (power of two >= mean row length)
+  int check_every = 4;      // iterations of the recorded graph
+  pda::DevBuf J, F, Fn, R, Y, Yn, dx, r, r0, p, v, s, t, y, z, Minv, scal;
+  pda::DevBuf part[5];      // partial sums: r0.v, (t.s, t.t), (r0.r, r.r), R.R, dx.dx
+  pda::DevBuf diag;         // first value of every cell's diagonal block
+  double *host = nullptr;   // pinned: what the host reads after a synchronization
+  // linear iterations of the last step's first, second, ... Newton iteration
+  int guess_iters[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   pda_implicit_stats last{};
   // check_every BiCGSTAB iterations recorded once as a graph (their kernel
   // arguments are the same for every solve of this stepper)
   hipStream_t cap = nullptr;
   hipGraph_t lin_graph = nullptr;
   hipGraphExec_t lin_exec = nullptr;
-  const double *lin_x = nullptr;    // the solution vector the graph writes
   ~pda_implicit_s() {
     if (lin_exec) (void)hipGraphExecDestroy(lin_exec);
     if (lin_graph) (void)hipGraphDestroy(lin_graph);
     if (cap) (void)hipStreamDestroy(cap);
+    if (host) (void)hipHostFree(host);
   }
 };
 
 namespace {
 using namespace pda;
 
-// y = A x with the solver's lanes-per-row; returns the number of blocks
-// (the count of partial sums written when part != null)
-int spmv(const pda_implicit_s &ip, const double *A, const double *x, double *y, const double *d1, int want_yy,
-         double *part, const double *scal, hipStream_t st) {
+enum { P_R0V = 0, P_TS, P_RR, P_RES, P_DX };
+
+Blocks blocks_of(const pda_implicit_s &ip) {
   const pda_problem_s &p = *ip.prob;
-  const int64_t *rp = p.d_rowptr.as<int64_t>();
-  const int32_t *ci = p.d_colidx.as<int32_t>();
-  const int64_t n = ip.n;
-  const int64_t rows_per_block = TB / ip.lpr;
-  const unsigned g = unsigned(std::max<int64_t>(1, std::min<int64_t>((n + rows_per_block - 1) / rows_per_block, MAXB)));
-  switch (ip.lpr) {
-    case 4: hipLaunchKernelGGL(k_spmv<4>, dim3(g), dim3(TB), 0, st, rp, ci, A, x, y, n, d1, want_yy, part, scal); break;
-    case 8: hipLaunchKernelGGL(k_spmv<8>, dim3(g), dim3(TB), 0, st, rp, ci, A, x, y, n, d1, want_yy, part, scal); break;
-    case 16: hipLaunchKernelGGL(k_spmv<16>, dim3(g), dim3(TB), 0, st, rp, ci, A, x, y, n, d1, want_yy, part, scal); break;
-    case 32: hipLaunchKernelGGL(k_spmv<32>, dim3(g), dim3(TB), 0, st, rp, ci, A, x, y, n, d1, want_yy, part, scal); break;
-    default: hipLaunchKernelGGL(k_spmv<64>, dim3(g), dim3(TB), 0, st, rp, ci, A, x, y, n, d1, want_yy, part, scal); break;
-  }
+  Blocks K;
+  K.rowbase = p.view.rowbase;
+  K.nblk = p.view.nblk;
+  K.bcol = p.d_bcol.as<int32_t>();
+  K.diag = ip.diag.as<int64_t>();
+  K.maxb = p.maxb;
+  K.ncell = ip.ncell;
+  return K;
+}
+
+// y = (cnp1 I + cf J) x; returns the number of partial sums
+template <int M, int L>
+int spmv_l(const pda_implicit_s &ip, const double *x, double *y, const double *d1, int want_yy, double *part,
+           hipStream_t st) {
+  // cells of a block: whole passes of the lanes, at most MAXB blocks
+  constexpr int64_t pass = (TB / L) * spmv_cells<M>();
+  const int64_t per = ((ip.ncell + MAXB - 1) / MAXB + pass - 1) / pass * pass;
+  const unsigned g = unsigned((ip.ncell + per - 1) / per);
+  hipLaunchKernelGGL((k_spmv<M, L>), dim3(g), dim3(TB), 0, st, blocks_of(ip), ip.J.as<double>(), x, y, per, d1,
+                     want_yy, part, ip.scal.as<double>());
   return int(g);
+}
+template <int M>
+int spmv(const pda_implicit_s &ip, const double *x, double *y, const double *d1, int want_yy, double *part,
+         hipStream_t st) {
+  return ip.prob->maxb <= 8 ? spmv_l<M, 8>(ip, x, y, d1, want_yy, part, st)
+                            : spmv_l<M, 16>(ip, x, y, d1, want_yy, part, st);
 }
 
 // one BiCGSTAB iteration (preconditioned right: y = M^-1 p, z = M^-1 s);
 // every kernel is a no-op once the convergence flag is set
 template <int M>
-void bicgstab_iteration(pda_implicit_s &ip, double *x, hipStream_t st, bool first) {
+void bicgstab_iteration(pda_implicit_s &ip, hipStream_t st, bool first, double rtol) {
   const int64_t n = ip.n, nc = ip.ncell;
-  const double *A = ip.J.as<double>();
   double *r = ip.r.as<double>(), *r0 = ip.r0.as<double>(), *pp = ip.p.as<double>();
   double *v = ip.v.as<double>(), *s = ip.s.as<double>(), *t = ip.t.as<double>();
   double *y = ip.y.as<double>(), *z = ip.z.as<double>(), *Mi = ip.Minv.as<double>();
-  double *part = ip.part.as<double>(), *scal = ip.scal.as<double>();
+  double *scal = ip.scal.as<double>();
+  double *pr0v = ip.part[P_R0V].as<double>(), *pts = ip.part[P_TS].as<double>(), *prr = ip.part[P_RR].as<double>();
   const unsigned gv = grid_strided(n), gc = grid_of(nc);
-  const int nb = int(gv);
-  hipLaunchKernelGGL((k_p_prec<M>), dim3(gc), dim3(TB), 0, st, r, pp, v, Mi, y, nc, scal, first ? 1 : 0);
-  int ns = spmv(ip, A, y, v, r0, 0, part, scal, st);
-  hipLaunchKernelGGL(k_finish, dim3(1), dim3(TB), 0, st, part, ns, 1, scal, 0.);
-  hipLaunchKernelGGL((k_s_prec<M>), dim3(gc), dim3(TB), 0, st, r, v, Mi, s, z, nc, scal);
-  ns = spmv(ip, A, z, t, s, 1, part, scal, st);
-  hipLaunchKernelGGL(k_finish, dim3(1), dim3(TB), 0, st, part, ns, 2, scal, 0.);
-  hipLaunchKernelGGL(k_xr, dim3(gv), dim3(TB), 0, st, x, r, y, z, s, t, r0, n, part, scal);
-  hipLaunchKernelGGL(k_finish, dim3(1), dim3(TB), 0, st, part, nb, 0, scal, 0.);
+  hipLaunchKernelGGL((k_p_prec<M>), dim3(gc), dim3(TB), 0, st, r, pp, v, Mi, y, nc, prr, int(gv), scal,
+                     first ? 1 : 0, rtol);
+  int ns = spmv<M>(ip, y, v, r0, 0, pr0v, st);
+  hipLaunchKernelGGL((k_s_prec<M>), dim3(gc), dim3(TB), 0, st, r, v, Mi, s, z, nc, pr0v, ns, scal);
+  ns = spmv<M>(ip, z, t, s, 1, pts, st);
+  hipLaunchKernelGGL(k_xr, dim3(gv), dim3(TB), 0, st, ip.dx.as<double>(), r, y, z, s, t, r0, n, pts, ns, prr, scal);
 }
 
+// (cnp1 I + cf J) dx = -R.  newton: index of the Newton iteration, whose
+// linear iterations in the step before decide how many run before the first
+// poll (the kernels stop by themselves at convergence, so this moves no value)
 template <int M>
-int bicgstab_m(pda_implicit_s &ip, const double *b, double *x, hipStream_t st, double rtol,
-               int *iters, double *rel_res) {
+int bicgstab_m(pda_implicit_s &ip, double cf, double cnp1, hipStream_t st, double rtol, int newton, int *iters,
+               double *rel_res) {
   const int64_t n = ip.n, nc = ip.ncell;
-  const double *A = ip.J.as<double>();
-  double *r = ip.r.as<double>(), *r0 = ip.r0.as<double>(), *Mi = ip.Minv.as<double>();
-  double *part = ip.part.as<double>(), *scal = ip.scal.as<double>();
+  double *prr = ip.part[P_RR].as<double>(), *scal = ip.scal.as<double>(), *h = ip.host;
   const unsigned gv = grid_strided(n), gc = grid_of(nc);
-  const int nb = int(gv);
-  // preconditioner
-  hipLaunchKernelGGL((k_block_inv<M>), dim3(gc), dim3(TB), 0, st, ip.diag.as<int64_t>(), A, nc, Mi);
-  // x = 0, r = r0 = b
-  hipLaunchKernelGGL(k_comb, dim3(grid_strided(n)), dim3(TB), 0, st, x, b, 0., nullptr, 0., nullptr, 0.,
-                     nullptr, 0., n);
-  hipLaunchKernelGGL(k_comb, dim3(grid_strided(n)), dim3(TB), 0, st, r, b, 1., nullptr, 0., nullptr, 0.,
-                     nullptr, 0., n);
-  hipLaunchKernelGGL(k_comb, dim3(grid_strided(n)), dim3(TB), 0, st, r0, b, 1., nullptr, 0., nullptr, 0.,
-                     nullptr, 0., n);
-  hipLaunchKernelGGL(k_dot2, dim3(gv), dim3(TB), 0, st, r0, r, r, r, n, part);
-  hipLaunchKernelGGL(k_finish, dim3(1), dim3(TB), 0, st, part, nb, 3, scal, rtol);
-  hipLaunchKernelGGL(k_finish, dim3(1), dim3(TB), 0, st, part, nb, 0, scal, rtol);
+  hipLaunchKernelGGL((k_block_inv<M>), dim3(gc), dim3(TB), 0, st, blocks_of(ip), ip.J.as<double>(), cf, cnp1,
+                     ip.Minv.as<double>());
+  hipLaunchKernelGGL(k_start, dim3(gv), dim3(TB), 0, st, ip.R.as<double>(), ip.dx.as<double>(), ip.r.as<double>(),
+                     ip.r0.as<double>(), n, cf, cnp1, prr, scal);
   PDA_HIP_CHECK(hipGetLastError());
   const int64_t maxit = ip.lin_max > 0 ? ip.lin_max : 2 * n;
-  const int K = ip.check_every;
-  double h[S_COUNT];
+  const int K = ip.check_every, slot = newton < 8 ? newton : 7;
   // iteration 0 (p = r) eagerly, then chunks of K iterations replayed from
-  // one graph, polling the convergence flag after each chunk; a tail shorter
-  // than K runs eagerly so that maxit is exact
-  bicgstab_iteration<M>(ip, x, st, true);
+  // one graph, polling the convergence flag after each chunk from about the
+  // last step's count on; a tail shorter than K runs eagerly so that maxit is
+  // exact
+  bicgstab_iteration<M>(ip, st, true, rtol);
   PDA_HIP_CHECK(hipGetLastError());
-  int64_t it = 1;
+  int64_t it = 1, unpolled = ip.guess_iters[slot] - 1 - K;
   bool done = false;
-  while (it < maxit && !done) {
+  while (!done) {
     if (maxit - it >= K) {
-      if (ip.lin_exec && ip.lin_x != x) {
-        (void)hipGraphExecDestroy(ip.lin_exec);
-        (void)hipGraphDestroy(ip.lin_graph);
-        ip.lin_exec = nullptr;
-        ip.lin_graph = nullptr;
-      }
       if (!ip.lin_exec) {
         if (!ip.cap) PDA_HIP_CHECK(hipStreamCreateWithFlags(&ip.cap, hipStreamNonBlocking));
         PDA_HIP_CHECK(hipStreamBeginCapture(ip.cap, hipStreamCaptureModeThreadLocal));
-        for (int k = 0; k < K; ++k) bicgstab_iteration<M>(ip, x, ip.cap, false);
+        for (int k = 0; k < K; ++k) bicgstab_iteration<M>(ip, ip.cap, false, 0.);
         hipGraph_t g = nullptr;
         const hipError_t e = hipStreamEndCapture(ip.cap, &g);
         if (e != hipSuccess || !g) {
@@ -447,51 +584,39 @@ int bicgstab_m(pda_implicit_s &ip, const double *b, double *x, hipStream_t st, d
           return PDA_E_HIP;
         }
         ip.lin_graph = g;
-        ip.lin_x = x;
       }
       PDA_HIP_CHECK(hipGraphLaunch(ip.lin_exec, st));
       it += K;
+      unpolled -= K;
+      if (unpolled > 0 && maxit - it >= K) continue;
     } else {
-      for (; it < maxit; ++it) bicgstab_iteration<M>(ip, x, st, false);
+      for (; it < maxit; ++it) bicgstab_iteration<M>(ip, st, false, 0.);
       PDA_HIP_CHECK(hipGetLastError());
     }
-    PDA_HIP_CHECK(hipMemcpyAsync(h, scal, sizeof(h), hipMemcpyDeviceToHost, st));
+    hipLaunchKernelGGL(k_check, dim3(1), dim3(TB), 0, st, prr, int(gv), scal, h);
+    PDA_HIP_CHECK(hipGetLastError());
     PDA_HIP_CHECK(hipStreamSynchronize(st));
-    done = h[S_DONE] != 0.;
+    done = h[H_DONE] != 0. || it >= maxit;
   }
-  PDA_HIP_CHECK(hipMemcpyAsync(h, scal, sizeof(h), hipMemcpyDeviceToHost, st));
-  PDA_HIP_CHECK(hipStreamSynchronize(st));
-  *iters = int(h[S_NITER]);
-  *rel_res = h[S_BB] > 0. ? std::sqrt(h[S_RR] / h[S_BB]) : 0.;
+  *iters = int(h[H_NITER]) + (h[H_DONE] == 0. ? 1 : 0); // at the limit the unmet check counts too
+  *rel_res = h[H_BB] > 0. ? std::sqrt(h[H_RR] / h[H_BB]) : 0.;
+  ip.guess_iters[slot] = *iters;
   // a solve that stops at the iteration limit is reported through rel_res;
   // the Newton loop's own stop rule decides
   return PDA_OK;
 }
 
-int bicgstab(pda_implicit_s &ip, const double *b, double *x, hipStream_t st, double rtol, int *iters,
+int bicgstab(pda_implicit_s &ip, double cf, double cnp1, hipStream_t st, double rtol, int newton, int *iters,
              double *rel) {
   switch (ip.prob->m) {
-    case 1: return bicgstab_m<1>(ip, b, x, st, rtol, iters, rel);
-    case 2: return bicgstab_m<2>(ip, b, x, st, rtol, iters, rel);
-    case 3: return bicgstab_m<3>(ip, b, x, st, rtol, iters, rel);
-    case 4: return bicgstab_m<4>(ip, b, x, st, rtol, iters, rel);
-    case 5: return bicgstab_m<5>(ip, b, x, st, rtol, iters, rel);
+    case 1: return bicgstab_m<1>(ip, cf, cnp1, st, rtol, newton, iters, rel);
+    case 2: return bicgstab_m<2>(ip, cf, cnp1, st, rtol, newton, iters, rel);
+    case 3: return bicgstab_m<3>(ip, cf, cnp1, st, rtol, newton, iters, rel);
+    case 4: return bicgstab_m<4>(ip, cf, cnp1, st, rtol, newton, iters, rel);
+    case 5: return bicgstab_m<5>(ip, cf, cnp1, st, rtol, newton, iters, rel);
   }
   set_error("implicit: unsupported block size");
   return PDA_E_UNSUPPORTED;
-}
-
-double norm2(pda_implicit_s &ip, const double *a, hipStream_t st) {
-  const unsigned g = grid_strided(ip.n);
-  double *part = ip.part.as<double>();
-  hipLaunchKernelGGL(k_dot2, dim3(g), dim3(TB), 0, st, a, a, nullptr, nullptr, ip.n, part);
-  std::vector<double> h(2 * g);
-  if (hipMemcpyAsync(h.data(), part, sizeof(double) * h.size(), hipMemcpyDeviceToHost, st) != hipSuccess)
-    return NAN;
-  if (hipStreamSynchronize(st) != hipSuccess) return NAN;
-  double s = 0.;
-  for (unsigned i = 0; i < g; ++i) s += h[2 * i];
-  return std::sqrt(s);
 }
 
 }  // namespace
@@ -513,13 +638,6 @@ int pda_implicit_create(pda_problem p, int scheme, pda_implicit *out) {
   }
   int rc = ensure_device(*p);
   if (rc) return rc;
-  // the Newton matrix and the Krylov solver work on the scalar CSR pattern
-  rc = ensure_pattern_device(*p);
-  if (rc) return rc;
-  if (!p->d_rowptr.ptr || !p->d_colidx.ptr) {
-    set_error("pda_implicit_create: Jacobian pattern not on the device");
-    return PDA_E_STATE;
-  }
   auto *ip = new pda_implicit_s();
   ip->prob = p;
   ip->scheme = scheme;
@@ -532,26 +650,22 @@ int pda_implicit_create(pda_problem p, int scheme, pda_implicit *out) {
   for (auto *d : vecs)
     if (e == hipSuccess) e = d->alloc(vb);
   if (e == hipSuccess) e = ip->Minv.alloc(sizeof(double) * size_t(ip->ncell) * p->m * p->m);
-  if (e == hipSuccess) e = ip->part.alloc(sizeof(double) * 2 * pda::MAXB);
+  for (auto &d : ip->part)
+    if (e == hipSuccess) e = d.alloc(sizeof(double) * 2 * pda::MAXB);
+  if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void **>(&ip->host), sizeof(double) * 8, hipHostMallocDefault);
   if (e == hipSuccess) {
-    // diagonal position of every scalar row (full mesh: row i's diagonal is column i)
-    std::vector<int64_t> dg(size_t(ip->n), -1);
-    for (int64_t i = 0; i < ip->n; ++i)
-      for (int64_t j = p->rowptr[i]; j < p->rowptr[i + 1]; ++j)
-        if (p->colidx[j] == int32_t(i)) {
-          dg[i] = j;
-          break;
-        }
-    for (int64_t i = 0; i < ip->n; ++i)
-      if (dg[i] < 0 || dg[i] - i % p->m < p->rowptr[i] || dg[i] - i % p->m + p->m > p->rowptr[i + 1]) {
+    // the diagonal block of every cell (full mesh: cell c's column is c)
+    std::vector<int64_t> dg(size_t(ip->ncell), -1);
+    for (int64_t c = 0; c < ip->ncell; ++c)
+      for (int s = 0; s < p->h_nblk[c]; ++s)
+        if (p->h_bcol[size_t(c) * p->maxb + s] == int32_t(c)) dg[c] = p->h_rowbase[c] + int64_t(s) * p->m;
+    for (int64_t c = 0; c < ip->ncell; ++c)
+      if (dg[c] < 0) {
         set_error("pda_implicit_create: Jacobian pattern lacks a contiguous diagonal block");
         delete ip;
         return PDA_E_STATE;
       }
     e = ip->diag.upload(dg);
-    const double mean = double(p->nnz) / double(std::max<int64_t>(ip->n, 1));
-    ip->lpr = 4;
-    while (ip->lpr < 64 && ip->lpr < mean) ip->lpr *= 2;
   }
   if (e == hipSuccess) e = ip->scal.alloc(sizeof(double) * pda::S_COUNT);
   if (e != hipSuccess) {
@@ -559,6 +673,7 @@ int pda_implicit_create(pda_problem p, int scheme, pda_implicit *out) {
     delete ip;
     return PDA_E_HIP;
   }
+  p->applied = true; // pda_apply_jacobian_noalloc may follow
   *out = ip;
   return PDA_OK;
 }
@@ -589,7 +704,7 @@ int pda_implicit_step(pda_implicit ip, double *d_U, const double *d_Uprev, const
   hipStream_t st = hipStream_t(stream);
   pda_problem_s &p = *ip->prob;
   const int64_t n = ip->n;
-  if (!p.d_rowptr.ptr || !p.d_colidx.ptr || !p.on_device) {
+  if (!p.on_device) {
     set_error("pda_implicit_step: problem tables not on the device");
     return PDA_E_STATE;
   }
@@ -618,55 +733,54 @@ int pda_implicit_step(pda_implicit ip, double *d_U, const double *d_Uprev, const
   }
   pda_implicit_stats S{};
   S.converged = 0;
+  double *pres = ip->part[P_RES].as<double>(), *pdx = ip->part[P_DX].as<double>(), *h = ip->host;
+  const double *Rx2 = scheme == PDA_BDF2 ? d_Uprev : (scheme == PDA_CRANK_NICOLSON ? Fn : nullptr);
+  const double c2 = scheme == PDA_BDF2 ? cnm1 : cfn;
+  const bool by_residual = ip->stop == PDA_STOP_RESIDUAL;
+  // R(Y) and its partial sums.  Residual rule: from the velocity alone, the
+  // Jacobian only when another Newton correction is needed; correction rule:
+  // f(y) and df/dy from one evaluation (the Jacobian path's velocity, as
+  // pressio's residual-and-Jacobian call)
+  auto evaluate = [&]() -> int {
+    const int e = by_residual ? launch_velocity(p, Y, t + dt, F, st) : launch_jacobian(p, Y, t + dt, J, F, st);
+    if (e) return e;
+    hipLaunchKernelGGL(k_residual, dim3(gs), dim3(TB), 0, st, R, Y, cnp1, Yn, cn, Rx2, c2, F, cf, n, pres);
+    PDA_HIP_CHECK(hipGetLastError());
+    return PDA_OK;
+  };
+  // the norms of the given partial sums on the host
+  auto norms = [&](const double *a, const double *b) -> int {
+    hipLaunchKernelGGL(k_norms_out, dim3(1), dim3(TB), 0, st, a, b, int(gs), h);
+    PDA_HIP_CHECK(hipGetLastError());
+    PDA_HIP_CHECK(hipStreamSynchronize(st));
+    return PDA_OK;
+  };
+  auto fail = [&](const char *what) -> int {
+    // pressio: ResidualHasNans -> NonlinearSolveFailure, the stepper
+    // restores y_n (solvers_nonlinear/impl/root_finder.cpp:60-70,
+    // ode/impl/ode_implicit_stepper_standard.hpp:213-225); d_U has not
+    // been written yet
+    ip->last = S;
+    if (stats) *stats = S;
+    set_error(std::string("pda_implicit_step: ") + what);
+    return PDA_E_STATE;
+  };
+  rc = evaluate();
+  if (!rc) rc = norms(pres, nullptr);
+  if (rc) return rc;
+  double rnorm = h[0];
   for (int it = 0; it < ip->max_newton; ++it) {
-    const double *Rx2 = scheme == PDA_BDF2 ? d_Uprev : (scheme == PDA_CRANK_NICOLSON ? Fn : nullptr);
-    const double c2 = scheme == PDA_BDF2 ? cnm1 : cfn;
-    if (ip->stop == PDA_STOP_RESIDUAL) {
-      // residual from the velocity alone; the Jacobian only when another
-      // Newton correction is needed
-      rc = launch_velocity(p, Y, t + dt, F, st);
-      if (rc) return rc;
-      hipLaunchKernelGGL(k_comb, dim3(gs), dim3(TB), 0, st, R, Y, cnp1, Yn, cn, Rx2, c2, F, cf, n);
-      PDA_HIP_CHECK(hipGetLastError());
-      S.residual_norm = norm2(*ip, R, st);
-      if (it == 0) S.initial_residual_norm = S.residual_norm;
-      if (!std::isfinite(S.residual_norm)) {
-        // pressio: ResidualHasNans -> NonlinearSolveFailure, the stepper
-        // restores y_n (solvers_nonlinear/impl/root_finder.cpp:60-70,
-        // ode/impl/ode_implicit_stepper_standard.hpp:213-225); d_U has not
-        // been written yet
-        ip->last = S;
-        if (stats) *stats = S;
-        set_error("pda_implicit_step: residual is not finite");
-        return PDA_E_STATE;
-      }
-      if (S.residual_norm <= ip->tol) {
+    S.residual_norm = rnorm;
+    if (it == 0) S.initial_residual_norm = rnorm;
+    if (!std::isfinite(rnorm)) return fail("residual is not finite");
+    if (by_residual) {
+      if (rnorm <= ip->tol) {
         S.converged = 1;
         break;
       }
       rc = launch_jacobian(p, Y, t + dt, J, nullptr, st);
       if (rc) return rc;
-    } else {
-      // f(y) and df/dy from one evaluation (the Jacobian path's velocity,
-      // as pressio's residual-and-Jacobian call)
-      rc = launch_jacobian(p, Y, t + dt, J, F, st);
-      if (rc) return rc;
-      hipLaunchKernelGGL(k_comb, dim3(gs), dim3(TB), 0, st, R, Y, cnp1, Yn, cn, Rx2, c2, F, cf, n);
-      PDA_HIP_CHECK(hipGetLastError());
-      S.residual_norm = norm2(*ip, R, st);
-      if (it == 0) S.initial_residual_norm = S.residual_norm;
-      if (!std::isfinite(S.residual_norm)) {
-        ip->last = S;
-        if (stats) *stats = S;
-        set_error("pda_implicit_step: residual is not finite");
-        return PDA_E_STATE;
-      }
     }
-    // A = cnp1 I + cf df/dy; solve A dx = -R
-    hipLaunchKernelGGL(k_scale, dim3(grid_strided(p.nnz)), dim3(TB), 0, st, J, p.nnz, cf);
-    hipLaunchKernelGGL(k_add_diag, dim3(grid_strided(n)), dim3(TB), 0, st, J, ip->diag.as<int64_t>(), n, cnp1);
-    hipLaunchKernelGGL(k_comb, dim3(gs), dim3(TB), 0, st, R, R, -1., nullptr, 0., nullptr, 0., nullptr, 0., n);
-    PDA_HIP_CHECK(hipGetLastError());
     int li = 0;
     double lr = 0.;
     // residual rule: inexact Newton, the linear residual only needs to fall
@@ -674,26 +788,43 @@ int pda_implicit_step(pda_implicit ip, double *d_U, const double *d_Uprev, const
     // [lin_rtol, 0.1]); correction rule: solve to lin_rtol (pressio's
     // BiCGSTAB runs to machine precision)
     double rtol = ip->lin_rtol;
-    if (ip->stop == PDA_STOP_RESIDUAL && S.residual_norm > 0.)
-      rtol = std::min(0.1, std::max(ip->lin_rtol, 0.1 * ip->tol / S.residual_norm));
-    rc = bicgstab(*ip, ip->R.as<double>(), dx, st, rtol, &li, &lr);
+    if (by_residual && rnorm > 0.) rtol = std::min(0.1, std::max(ip->lin_rtol, 0.1 * ip->tol / rnorm));
+    rc = bicgstab(*ip, cf, cnp1, st, rtol, it, &li, &lr);
     if (rc) return rc;
     S.linear_iters += li;
     S.last_linear_rel_residual = lr;
     S.newton_iters = it + 1;
-    S.correction_norm = norm2(*ip, dx, st);
-    if (!std::isfinite(S.correction_norm)) {
-      ip->last = S;
-      if (stats) *stats = S;
-      set_error("pda_implicit_step: Newton correction is not finite");
-      return PDA_E_STATE;
+    const bool more = it + 1 < ip->max_newton;
+    if (by_residual) {
+      // the correction, the next residual and both norms in one go: a
+      // non-finite correction is found before d_U is written
+      hipLaunchKernelGGL(k_correct, dim3(gs), dim3(TB), 0, st, Y, dx, n, pdx);
+      PDA_HIP_CHECK(hipGetLastError());
+      if (more) rc = evaluate();
+      if (!rc) rc = norms(pdx, more ? pres : nullptr);
+      if (rc) return rc;
+      S.correction_norm = h[0];
+      if (!std::isfinite(S.correction_norm)) return fail("Newton correction is not finite");
+      if (more) rnorm = h[1];
+    } else {
+      hipLaunchKernelGGL(k_norm, dim3(gs), dim3(TB), 0, st, dx, n, pdx);
+      PDA_HIP_CHECK(hipGetLastError());
+      rc = norms(pdx, nullptr);
+      if (rc) return rc;
+      S.correction_norm = h[0];
+      if (!std::isfinite(S.correction_norm)) return fail("Newton correction is not finite");
+      if (S.correction_norm < ip->tol) {
+        S.converged = 1;
+        break;
+      }
+      hipLaunchKernelGGL(k_correct, dim3(gs), dim3(TB), 0, st, Y, dx, n, pdx);
+      PDA_HIP_CHECK(hipGetLastError());
+      if (!more) break;
+      rc = evaluate();
+      if (!rc) rc = norms(pres, nullptr);
+      if (rc) return rc;
+      rnorm = h[0];
     }
-    if (ip->stop == PDA_STOP_CORRECTION && S.correction_norm < ip->tol) {
-      S.converged = 1;
-      break;
-    }
-    hipLaunchKernelGGL(k_comb, dim3(gs), dim3(TB), 0, st, Y, Y, 1., dx, 1., nullptr, 0., nullptr, 0., n);
-    PDA_HIP_CHECK(hipGetLastError());
   }
   PDA_HIP_CHECK(hipMemcpyAsync(d_U, Y, sizeof(double) * n, hipMemcpyDeviceToDevice, st));
   PDA_HIP_CHECK(hipStreamSynchronize(st));
