@@ -259,6 +259,42 @@ template <> struct AxisTerms<PhBurgers> {
   }
 };
 
+// ---------------------------------------------------------- axis as a value
+// For Euler, shallow water and Burgers the flux along axis a is the flux along
+// x of the state with two dofs exchanged, exchanged back, so a lane that works
+// on an axis of its own runs the x-face code on the exchanged state.
+template <class Ph> struct AxisPerm {
+  // Euler, SWE: (rho u) <-> (rho u_a)
+  __host__ __device__ static constexpr int p(int k, int a) { return k == 1 ? 1 + a : (k == 1 + a ? 1 : k); }
+};
+template <> struct AxisPerm<PhBurgers> {
+  __host__ __device__ static constexpr int p(int k, int a) { return k == 0 ? a : (k == a ? 0 : k); } // u <-> u_a
+};
+
+// value of the axis-a frame array x at the index of dof k of the
+// physical frame: x[p_a(k)], selected among the D compile-time candidates
+// (a is the lane's axis), so every index stays a compile-time constant
+template <class Ph, class X>
+__device__ __forceinline__ double perm_pick(const X &x, int a, int k) {
+  double v = x(AxisPerm<Ph>::p(k, 0));
+  if constexpr (Ph::DIM > 1) v = a == 1 ? x(AxisPerm<Ph>::p(k, 1)) : v;
+  if constexpr (Ph::DIM > 2) v = a == 2 ? x(AxisPerm<Ph>::p(k, 2)) : v;
+  return v;
+}
+
+// flux of a face along axis a from states in the axis frame, in that frame
+template <class Ph>
+__device__ __forceinline__ void axis_flux(const View &P, int, const double *l, const double *r, double *F) {
+  Ph::template flux<0>(P, l, r, F);
+}
+template <>
+__device__ __forceinline__ void axis_flux<PhAdr>(const View &P, int a, const double *l, const double *, double *F) {
+  F[0] = l[0] * (a == 0 ? P.p[0] : P.p[1]);
+}
+template <> struct AxisPerm<PhAdr> {
+  __host__ __device__ static constexpr int p(int k, int) { return k; }
+};
+
 // ------------------------------------------------------------------ helpers
 // LDS hand-off inside one wavefront (the workgroup is a single wave): LDS
 // instructions of a wave execute in order, so only the compiler must be kept
@@ -287,40 +323,88 @@ __device__ __forceinline__ int colof(int a, int side, int L) {
   return a == 0 ? base + (side ? 2 : 0) : a == 1 ? base + (side ? 1 : 3) : base + (side ? 5 : 4);
 }
 
-__device__ __forceinline__ const double *ghost_ptr(const View &P, int a, int side, int64_t g,
-                                                   int wm) {
-  return P.ghost + ((int64_t(a) * 2 + side) * P.n_near + g) * wm;
-}
-
-// st[p][k], p = 0..2W, centre at W.  Missing neighbours (graph -1) of a
-// near-boundary row are read from its ghost layers, as
-// impl/functor_fill_stencil.hpp does.  GW is the ghost-layer width the ghost
-// arrays were filled with (the scheme's), W the width gathered.
-template <class Ph, int W, int A>
-__device__ __forceinline__ void gather(const View &P, const int32_t *gr, int64_t g, int GW,
-                                       const double *__restrict__ U, double st[][Ph::M]) {
-  constexpr int M = Ph::M;
-  const int64_t self = gr[0];
+// Source cells of the 2W+1 stencil points of a row along axis a (centre at W):
+// the graph's neighbours, and for a missing one (graph -1, near-boundary rows)
+// the cell that its ghost layer copies, with a bit of `minus` or `plus` set
+// for the point.  Layer 0 copies the cell itself; for layer L>0 the source
+// follows the family's rule:
+//   GHOST_OPPOSITE: the opposite layer-(L-1) neighbour
+//     (impl/euler_1d_ghost_filler.hpp:104-143, impl/euler_3d_ghost_filler_sedov.hpp:184-236,
+//      impl/advection_diffusion_reaction_2d_ghost_filler_problemA.hpp:106-133);
+//   GHOST_MIRROR: the mirror image about the boundary
+//     (impl/euler_2d_ghost_filler_neumann.hpp:163-279,
+//      impl/swe_2d_ghost_filler_inviscid_wall.hpp:160-270).
+// A ghost value is the side's sign (gsign: reflective walls, Dirichlet) times
+// the source cell's.  (No ghost values are stored: a row's own lanes would
+// write and read them back through memory.)
+template <int DIM, int W>
+__device__ __forceinline__ void stencil_cells(const View &P, const int32_t *gr, int a, int32_t (&src)[2 * W + 1],
+                                              int &minus, int &plus) {
+  const int om = colof<DIM>(a, 0, 0), op = colof<DIM>(a, 1, 0);
+  int32_t nb[2][W]; // [side][layer]
 #pragma unroll
-  for (int k = 0; k < M; ++k) st[W][k] = U[self * M + k];
+  for (int L = 0; L < W; ++L) {
+    nb[0][L] = gr[om + 2 * DIM * L];
+    nb[1][L] = gr[op + 2 * DIM * L];
+  }
+  const int32_t self = gr[0];
+  src[W] = self;
+  minus = 0;
+  plus = 0;
 #pragma unroll
   for (int side = 0; side < 2; ++side)
 #pragma unroll
     for (int L = 0; L < W; ++L) {
-      const int32_t nb = gr[colof<Ph::DIM>(A, side, L)];
       const int p = side ? W + 1 + L : W - 1 - L;
-      if (nb >= 0) {
-#pragma unroll
-        for (int k = 0; k < M; ++k) st[p][k] = U[int64_t(nb) * M + k];
-      } else {
-        const double *gp = ghost_ptr(P, A, side, g, GW * M) + L * M;
-#pragma unroll
-        for (int k = 0; k < M; ++k) st[p][k] = gp[k];
+      int32_t c = nb[side][L];
+      if (c < 0) {
+        c = self;
+        if (L > 0) {
+          if (P.ghost_rule == GHOST_OPPOSITE) {
+            c = nb[1 - side][L > 0 ? L - 1 : 0];
+          } else if (L == 1) {
+            c = nb[side][0] < 0 ? nb[1 - side][0] : nb[side][0];
+          } else {
+            const int32_t n0 = nb[side][0], n1 = nb[side][W > 1 ? 1 : 0], o1 = nb[1 - side][W > 1 ? 1 : 0];
+            if (n1 >= 0 && n0 >= 0) c = n1;
+            if (n1 < 0 && n0 < 0) c = o1;
+          }
+        }
+        if (c < 0) c = self; // degenerate meshes narrower than the stencil
+        if (side) plus |= 1 << p;
+        else minus |= 1 << p;
       }
+      src[p] = c;
     }
 }
 
-// face states of the cell's left (minus) and right (plus) faces
+// st[p][k], p = 0..2W, centre at W: the states of the row's stencil along A
+template <class Ph, int W, int A>
+__device__ __forceinline__ void gather(const View &P, const int32_t *gr, const double *__restrict__ U,
+                                       double st[][Ph::M]) {
+  constexpr int M = Ph::M;
+  int32_t src[2 * W + 1];
+  int minus, plus;
+  stencil_cells<Ph::DIM, W>(P, gr, A, src, minus, plus);
+#pragma unroll
+  for (int p = 0; p <= 2 * W; ++p) {
+#pragma unroll
+    for (int k = 0; k < M; ++k) st[p][k] = U[int64_t(src[p]) * M + k];
+  }
+  if (minus | plus) {
+#pragma unroll
+    for (int p = 0; p <= 2 * W; ++p)
+#pragma unroll
+      for (int k = 0; k < M; ++k) {
+        if (minus >> p & 1) st[p][k] = P.gsign[A][0][k] * st[p][k];
+        if (plus >> p & 1) st[p][k] = P.gsign[A][1][k] * st[p][k];
+      }
+  }
+}
+
+// face states of the cell's left (minus) and right (plus) faces: the box
+// kernels' forms of the weights (one division each, the cell's own two values
+// sharing their windows), equal to theirs bit for bit where the stencils are
 template <int M, int W>
 struct Faces {
   double lm[M], lp[M], rm[M], rp[M];
@@ -340,11 +424,14 @@ __device__ __forceinline__ void reconstruct(const double st[][M], Faces<M, W> &f
     if constexpr (W == 1) {
       f.lm[k] = q[0]; f.lp[k] = q[1]; f.rm[k] = q[1]; f.rp[k] = q[2];
     } else if constexpr (W == 2) {
-      phys::weno3(q, f.lm[k], f.lp[k]);
-      phys::weno3(q + 1, f.rm[k], f.rp[k]);
+      double un, up;
+      phys::weno3_1div(q, f.lm[k], up);
+      phys::weno3_cell_1div(q[1], q[2], q[3], f.rm[k], f.lp[k]);
+      phys::weno3_1div(q + 1, un, f.rp[k]);
     } else {
-      phys::weno5(q, f.lm[k], f.lp[k]);
-      phys::weno5(q + 1, f.rm[k], f.rp[k]);
+      f.lm[k] = phys::weno5_side_1div(q[0], q[1], q[2], q[3], q[4]);
+      phys::weno5_cell_1div(q[1], q[2], q[3], q[4], q[5], f.rm[k], f.lp[k]);
+      f.rp[k] = phys::weno5_side_1div(q[6], q[5], q[4], q[3], q[2]);
     }
   }
 }

@@ -110,7 +110,6 @@ struct View {
   const int32_t *ghost_row = nullptr; // per graph row: near-boundary index or -1
   const int32_t *near_rows = nullptr; // graph rows of near-boundary cells
   int64_t n_near = 0;
-  double *ghost = nullptr;            // [axis][side][n_near][w*m]
   const double *bcf = nullptr;        // [n_near][dim][m] Jacobian BC factors
   const int64_t *rowbase = nullptr;   // per graph row: first CSR value of dof 0
   const int32_t *nblk = nullptr;      // per graph row: number of column blocks
@@ -202,7 +201,7 @@ struct pda_problem_s {
   int vel_rps = 0;                   // velocity march strip height (0: from the grid size)
   int jac_rps = 0;                   // first-order 2D/3D Euler Jacobian strip height (0: from the grid size)
   pda::View view;
-  pda::DevBuf d_graph, d_ghost_row, d_near_rows, d_ghost, d_bcf;
+  pda::DevBuf d_graph, d_ghost_row, d_near_rows, d_bcf;
   pda::DevBuf d_rowptr, d_colidx, d_rowbase, d_nblk, d_slot, d_bcol;
   pda::DevBuf d_scratch_v;           // Jacobian values for applyJacobian()
 };

@@ -12,20 +12,27 @@ using namespace fam;
 template <class Ph, int W>
 __global__ void __launch_bounds__(64) k_velocity(View P, const double *__restrict__ U,
                                                    double *__restrict__ V) {
-  rows::velocity_row<Ph, W>(P, int64_t(blockIdx.x) * blockDim.x + threadIdx.x, U, V);
+  constexpr int M = Ph::M, D = Ph::DIM;
+  double acc[M];
+  const int64_t r = rows::velocity_lanes<Ph, W>(P, int64_t(blockIdx.x), U, acc);
+  if (r < 0) return;
+  const int a = int(threadIdx.x) % D; // the row's lanes share its stores
+#pragma unroll
+  for (int k = 0; k < M; ++k)
+    if (k % D == a) V[r * M + k] = acc[k];
 }
 
 // velocity with an explicit stage fused into the store (RkStage)
 template <class Ph, int W>
 __global__ void __launch_bounds__(64) k_velocity_stage(View P, const double *__restrict__ U, RkStage S) {
-  constexpr int M = Ph::M;
-  const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (t >= P.nvisit) return;
-  const int64_t r = P.rows ? P.rows[t] : t;
+  constexpr int M = Ph::M, D = Ph::DIM;
   double acc[M];
-  rows::velocity_acc<Ph, W>(P, r, U, acc);
+  const int64_t r = rows::velocity_lanes<Ph, W>(P, int64_t(blockIdx.x), U, acc);
+  if (r < 0) return;
+  const int a = int(threadIdx.x) % D;
 #pragma unroll
   for (int k = 0; k < M; ++k) {
+    if (k % D != a) continue;
     const int64_t e = r * M + k;
     if (S.kout) S.kout[e] = acc[k];
     double o = S.c[0] * S.x[0][e];
@@ -390,25 +397,6 @@ __global__ void __launch_bounds__(64) k_jac_fo_euler_staged(View P, const double
 // generic kernel.  The per-lane live set is one face's gradients and
 // Jacobians (2 M (2W) + 2 M^2 doubles), where one thread per row holds all
 // faces of all axes and spills.
-template <class Ph> struct AxisPerm {
-  // Euler, SWE: (rho u) <-> (rho u_a)
-  __host__ __device__ static constexpr int p(int k, int a) { return k == 1 ? 1 + a : (k == 1 + a ? 1 : k); }
-};
-template <> struct AxisPerm<PhBurgers> {
-  __host__ __device__ static constexpr int p(int k, int a) { return k == 0 ? a : (k == a ? 0 : k); } // u <-> u_a
-};
-
-// value of the axis-a frame array x at the index of dof k of the
-// physical frame: x[p_a(k)], selected among the D compile-time candidates
-// (a is the lane's axis), so every index stays a compile-time constant
-template <class Ph, class X>
-__device__ __forceinline__ double perm_pick(const X &x, int a, int k) {
-  double v = x(AxisPerm<Ph>::p(k, 0));
-  if constexpr (Ph::DIM > 1) v = a == 1 ? x(AxisPerm<Ph>::p(k, 1)) : v;
-  if constexpr (Ph::DIM > 2) v = a == 2 ? x(AxisPerm<Ph>::p(k, 2)) : v;
-  return v;
-}
-
 // store (or add) the axis-frame block b at dst (row stride RS) in the
 // physical frame: dst[K][J] = b[p_a(K)][p_a(J)] (p_a is an involution)
 template <class Ph, int RS, bool ADD>
@@ -941,7 +929,8 @@ template <class Ph>
 static int vel_dispatch(const View &v, int w, const double *U, double *V, hipStream_t s) {
   const int bs = 64; // one-wave groups fit next to the structured kernels
   if (v.nvisit == 0) return PDA_OK;
-  const unsigned nb = unsigned((v.nvisit + bs - 1) / bs);
+  constexpr int RPW = rows::vel_rows<Ph::DIM>();
+  const unsigned nb = unsigned((v.nvisit + RPW - 1) / RPW);
   if (w == 1) hipLaunchKernelGGL((k_velocity<Ph, 1>), dim3(nb), dim3(bs), 0, s, v, U, V);
   else if (w == 2) hipLaunchKernelGGL((k_velocity<Ph, 2>), dim3(nb), dim3(bs), 0, s, v, U, V);
   else hipLaunchKernelGGL((k_velocity<Ph, 3>), dim3(nb), dim3(bs), 0, s, v, U, V);
@@ -953,7 +942,8 @@ template <class Ph>
 static int vel_stage_dispatch(const View &v, int w, const double *U, const RkStage &S, hipStream_t s) {
   const int bs = 64;
   if (v.nvisit == 0) return PDA_OK;
-  const unsigned nb = unsigned((v.nvisit + bs - 1) / bs);
+  constexpr int RPW = rows::vel_rows<Ph::DIM>();
+  const unsigned nb = unsigned((v.nvisit + RPW - 1) / RPW);
   if (w == 1) hipLaunchKernelGGL((k_velocity_stage<Ph, 1>), dim3(nb), dim3(bs), 0, s, v, U, S);
   else if (w == 2) hipLaunchKernelGGL((k_velocity_stage<Ph, 2>), dim3(nb), dim3(bs), 0, s, v, U, S);
   else hipLaunchKernelGGL((k_velocity_stage<Ph, 3>), dim3(nb), dim3(bs), 0, s, v, U, S);

@@ -26,31 +26,6 @@ __device__ __forceinline__ double fdiv(double n, double d) {
 }
 
 // ---------------------------------------------------------------- WENO3
-// impl/weno3.hpp:56-132.  q = {q_{i-1}, q_i, q_{i+1}, q_{i+2}}
-__device__ __forceinline__ void weno3(const double *q, double &un, double &up) {
-  constexpr double eps = 1.e-6, c13 = 1. / 3., c23 = 2. / 3.;
-  {
-    const double p0 = (-q[0] + 3. * q[1]) * 0.5;
-    const double p1 = (q[1] + q[2]) * 0.5;
-    const double B0 = (q[0] - q[1]) * (q[0] - q[1]);
-    const double B1 = (q[1] - q[2]) * (q[1] - q[2]);
-    const double a0 = c13 / (eps * eps + 2. * eps * B0 + B0 * B0);
-    const double a1 = c23 / (eps * eps + 2. * eps * B1 + B1 * B1);
-    const double s = 1. / (a0 + a1);
-    un = (a0 * s) * p0 + (a1 * s) * p1;
-  }
-  {
-    const double p0 = (q[1] + q[2]) * 0.5;
-    const double p1 = (3. * q[2] - q[3]) * 0.5;
-    const double B0 = (q[1] - q[2]) * (q[1] - q[2]);
-    const double B1 = (q[2] - q[3]) * (q[2] - q[3]);
-    const double a0 = c23 / (eps * eps + 2. * eps * B0 + B0 * B0);
-    const double a1 = c13 / (eps * eps + 2. * eps * B1 + B1 * B1);
-    const double s = 1. / (a0 + a1);
-    up = (a0 * s) * p0 + (a1 * s) * p1;
-  }
-}
-
 // impl/weno3.hpp:134-246: values plus d(face)/d(q_j), j = 0..3
 __device__ __forceinline__ void weno3_grad(const double *q, double &un, double &up,
                                            double *gn, double *gp) {
@@ -113,47 +88,11 @@ __device__ __forceinline__ void weno3_grad(const double *q, double &un, double &
 }
 
 // ---------------------------------------------------------------- WENO5
-// impl/weno5.hpp:56-178.  q = {q_{i-2}, ..., q_{i+3}}
-__device__ __forceinline__ void weno5(const double *q, double &un, double &up) {
-  constexpr double eps = 1.e-6, c1312 = 13. / 12., c16 = 1. / 6.;
-  {
-    const double p0 = (2. * q[0] - 7. * q[1] + 11. * q[2]) * c16;
-    const double p1 = (-q[1] + 5. * q[2] + 2. * q[3]) * c16;
-    const double p2 = (2. * q[2] + 5. * q[3] - q[4]) * c16;
-    const double t0 = q[0] - 2. * q[1] + q[2], s0 = q[0] - 4. * q[1] + 3. * q[2];
-    const double t1 = q[1] - 2. * q[2] + q[3], s1 = q[1] - q[3];
-    const double t2 = q[2] - 2. * q[3] + q[4], s2 = 3. * q[2] - 4. * q[3] + q[4];
-    const double B0 = c1312 * t0 * t0 + 0.25 * s0 * s0;
-    const double B1 = c1312 * t1 * t1 + 0.25 * s1 * s1;
-    const double B2 = c1312 * t2 * t2 + 0.25 * s2 * s2;
-    const double a0 = 0.1 / (eps * eps + 2. * eps * B0 + B0 * B0);
-    const double a1 = 0.6 / (eps * eps + 2. * eps * B1 + B1 * B1);
-    const double a2 = 0.3 / (eps * eps + 2. * eps * B2 + B2 * B2);
-    const double s = 1. / (a0 + a1 + a2);
-    un = (a0 * s) * p0 + (a1 * s) * p1 + (a2 * s) * p2;
-  }
-  {
-    const double p0 = (-q[1] + 5. * q[2] + 2. * q[3]) * c16;
-    const double p1 = (2. * q[2] + 5. * q[3] - q[4]) * c16;
-    const double p2 = (11. * q[3] - 7. * q[4] + 2. * q[5]) * c16;
-    const double t0 = q[1] - 2. * q[2] + q[3], s0 = q[1] - 4. * q[2] + 3. * q[3];
-    const double t1 = q[2] - 2. * q[3] + q[4], s1 = q[2] - q[4];
-    const double t2 = q[3] - 2. * q[4] + q[5], s2 = 3. * q[3] - 4. * q[4] + q[5];
-    const double B0 = c1312 * t0 * t0 + 0.25 * s0 * s0;
-    const double B1 = c1312 * t1 * t1 + 0.25 * s1 * s1;
-    const double B2 = c1312 * t2 * t2 + 0.25 * s2 * s2;
-    const double a0 = 0.3 / (eps * eps + 2. * eps * B0 + B0 * B0);
-    const double a1 = 0.6 / (eps * eps + 2. * eps * B1 + B1 * B1);
-    const double a2 = 0.1 / (eps * eps + 2. * eps * B2 + B2 * B2);
-    const double s = 1. / (a0 + a1 + a2);
-    up = (a0 * s) * p0 + (a1 * s) * p1 + (a2 * s) * p2;
-  }
-}
-
-// Same reconstruction with the normalised weights formed with one division:
-// alpha_k / sum(alpha) = N_k / sum(N) with N_k = d_k * prod_{j != k} D_j and
-// D_k = eps^2 + 2 eps B_k + B_k^2 (the reference's denominator).  Equal to
-// weno5() in exact arithmetic; the results differ by a few ulps.
+// Reconstruction (impl/weno5.hpp:56-178) with the normalised weights formed
+// with one division: alpha_k / sum(alpha) = N_k / sum(N) with N_k = d_k *
+// prod_{j != k} D_j and D_k = eps^2 + 2 eps B_k + B_k^2 (the reference's
+// denominator).  Equal to the reference's four divisions in exact arithmetic;
+// the results differ by a few ulps.
 //
 // D of a side window (far, mid, near), near = the reconstructed cell:
 // B = 13/12 (far - 2 mid + near)^2 + 1/4 (far - 4 mid + 3 near)^2.  The

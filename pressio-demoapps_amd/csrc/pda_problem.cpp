@@ -483,15 +483,10 @@ int ensure_device(pda_problem_s &p) {
   PDA_HIP_CHECK(p.d_bcol.upload(p.h_bcol));
   PDA_HIP_CHECK(p.d_rem_rows.upload(p.h_rem_rows));
   PDA_HIP_CHECK(p.d_vrem_rows.upload(p.h_vrem_rows));
-  const size_t gn = size_t(2 * p.dim) * size_t(std::max<int64_t>(p.n_near, 1)) * p.w * p.m;
-  // unused ghost slots hold numeric_limits<double>::min(),
-  // impl/euler_2d_prob_class.hpp:1266-1270
-  PDA_HIP_CHECK(p.d_ghost.upload(std::vector<double>(gn, 2.2250738585072014e-308)));
   View &v = p.view;
   v.graph = p.d_graph.as<int32_t>();
   v.ghost_row = p.d_ghost_row.as<int32_t>();
   v.near_rows = p.d_near_rows.as<int32_t>();
-  v.ghost = p.d_ghost.as<double>();
   v.bcf = p.d_bcf.as<double>();
   v.rowbase = p.d_rowbase.as<int64_t>();
   v.nblk = p.d_nblk.as<int32_t>();

@@ -1,7 +1,7 @@
-// pda_rows.hpp -- per-row device code of the generic kernels: one thread
-// owns one graph row (one sample-mesh cell) and produces all of its V
-// entries and its whole Jacobian block-row, so every output value is written
-// exactly once with plain stores (no atomics, no zero-fill pass).  The
+// pda_rows.hpp -- per-row device code of the generic kernels: the lanes of one
+// graph row (one sample-mesh cell) produce all of its V entries, one thread its
+// whole Jacobian block-row, so every output value is written exactly once with
+// plain stores (no atomics, no zero-fill pass).  The
 // per-entry accumulation order follows the reference:
 //   - V: x, then y, then z axis, then sources
 //     (impl/mixin_directional_flux_balance.hpp:68-84);
@@ -17,113 +17,103 @@ namespace pda {
 namespace rows {
 using namespace fam;
 
-// ---------------------------------------------------------------- ghosts
-// Ghost layers of every near-boundary row.  Layer 0 copies the cell itself;
-// for layer L>0 the source cell follows the family's rule:
-//   GHOST_OPPOSITE: the opposite layer-(L-1) neighbour
-//     (impl/euler_1d_ghost_filler.hpp:104-143, impl/euler_3d_ghost_filler_sedov.hpp:184-236,
-//      impl/advection_diffusion_reaction_2d_ghost_filler_problemA.hpp:106-133);
-//   GHOST_MIRROR: the mirror image about the boundary
-//     (impl/euler_2d_ghost_filler_neumann.hpp:163-279,
-//      impl/swe_2d_ghost_filler_inviscid_wall.hpp:160-270);
-// each value is multiplied by the side's sign pattern (reflective walls,
-// Dirichlet negation).  A slot is written only when its neighbour is -1,
-// the same condition under which the stencil reads it.
-template <int DIM, int M>
-__device__ __forceinline__ void fill_row_ghosts(const View &P, int W, int64_t g,
-                                                const int32_t *gr, const double *__restrict__ U) {
-  const int32_t self = gr[0];
-  for (int a = 0; a < DIM; ++a)
-    for (int side = 0; side < 2; ++side) {
-      double *dst = P.ghost + ((int64_t(a) * 2 + side) * P.n_near + g) * (W * M);
-      const double *sg = P.gsign[a][side];
-      for (int L = 0; L < W; ++L) {
-        const int32_t nL = gr[colof<DIM>(a, side, L)];
-        if (nL != -1) continue;
-        int32_t src = self;
-        if (L > 0) {
-          if (P.ghost_rule == GHOST_OPPOSITE) {
-            src = gr[colof<DIM>(a, 1 - side, L - 1)];
-          } else {
-            const int32_t n0 = gr[colof<DIM>(a, side, 0)];
-            const int32_t o0 = gr[colof<DIM>(a, 1 - side, 0)];
-            if (L == 1) {
-              src = n0 == -1 ? o0 : n0;
-            } else {
-              const int32_t n1 = gr[colof<DIM>(a, side, 1)];
-              const int32_t o1 = gr[colof<DIM>(a, 1 - side, 1)];
-              if (n1 != -1 && n0 != -1) src = n1;
-              if (n1 == -1 && n0 != -1) src = self;
-              if (n1 == -1 && n0 == -1) src = o1;
-            }
-          }
-        }
-        if (src < 0) src = self; // degenerate meshes narrower than the stencil
-        for (int k = 0; k < M; ++k) dst[L * M + k] = sg[k] * U[int64_t(src) * M + k];
-      }
-    }
-}
-
-// The row kernels fill the ghost slots of their own near-boundary row before
-// reading them (the slots of a row are read by that row only), so no
-// separate ghost pass runs ahead of an evaluation.
-
 // ---------------------------------------------------------------- velocity
-template <class Ph, int W, int A>
-__device__ __forceinline__ void velocity_axis(const View &P, const int32_t *gr, int64_t g,
-                                              const double *__restrict__ U, double *acc) {
+// A row is evaluated by DIM lanes, lane a forming axis a's part on states in
+// the axis frame (one instruction stream for the axes); the parts are then
+// added in axis order, every lane of the row ending with the sum.  One lane
+// per row walked its axes one after the other, and a mesh of 10^5 rows gave
+// the chip 1.6 waves per SIMD: 3D WENO5 velocity of the 5 % sample mesh of
+// 128^3 42.6 us, 55.9 us with one lane (64.5 us
+// with the reference's four divisions per WENO5 weight set and ghost layers
+// written to memory and read back); its near-boundary rows of the full mesh
+// 138 -> 72 us.
+template <int DIM> constexpr int vel_rows() { return 64 / DIM; } // rows per wavefront
+
+// axis a's part of the velocity of graph row r
+template <class Ph, int W>
+__device__ __forceinline__ void velocity_axis(const View &P, const int32_t *gr, bool near, int a,
+                                              const double *__restrict__ U, double (&acc)[Ph::M]) {
   constexpr int M = Ph::M;
   double st[2 * W + 1][M];
-  gather<Ph, W, A>(P, gr, g, W, U, st);
+  {
+    int32_t src[2 * W + 1];
+    int minus, plus;
+    stencil_cells<Ph::DIM, W>(P, gr, a, src, minus, plus);
+#pragma unroll
+    for (int p = 0; p <= 2 * W; ++p) {
+      double u[M];
+#pragma unroll
+      for (int k = 0; k < M; ++k) u[k] = U[int64_t(src[p]) * M + k];
+#pragma unroll
+      for (int k = 0; k < M; ++k) st[p][k] = perm_pick<Ph>([&](int x) { return u[x]; }, a, k);
+    }
+    if (minus | plus) {
+      double sg[2][M]; // the sides' signs in the axis frame
+#pragma unroll
+      for (int side = 0; side < 2; ++side)
+#pragma unroll
+        for (int k = 0; k < M; ++k) {
+          double v = P.gsign[0][side][AxisPerm<Ph>::p(k, 0)];
+          if constexpr (Ph::DIM > 1) v = a == 1 ? P.gsign[1][side][AxisPerm<Ph>::p(k, 1)] : v;
+          if constexpr (Ph::DIM > 2) v = a == 2 ? P.gsign[2][side][AxisPerm<Ph>::p(k, 2)] : v;
+          sg[side][k] = v;
+        }
+#pragma unroll
+      for (int p = 0; p <= 2 * W; ++p)
+#pragma unroll
+        for (int k = 0; k < M; ++k) {
+          if (minus >> p & 1) st[p][k] = sg[0][k] * st[p][k];
+          if (plus >> p & 1) st[p][k] = sg[1][k] * st[p][k];
+        }
+    }
+  }
   Faces<M, W> f;
   reconstruct<M, W>(st, f);
-  double FL[M], FR[M];
-  Ph::template flux<A>(P, f.lm, f.lp, FL);
-  Ph::template flux<A>(P, f.rm, f.rp, FR);
-  const double h = P.hinv[A];
+  double FL[M], FR[M], F[M];
+  axis_flux<Ph>(P, a, f.lm, f.lp, FL);
+  axis_flux<Ph>(P, a, f.rm, f.rp, FR);
+  double h = P.hinv[0];
+  if constexpr (Ph::DIM > 1) h = a == 1 ? P.hinv[1] : h;
+  if constexpr (Ph::DIM > 2) h = a == 2 ? P.hinv[2] : h;
 #pragma unroll
-  for (int k = 0; k < M; ++k) acc[k] += h * (FL[k] - FR[k]);
+  for (int k = 0; k < M; ++k) F[k] = h * (FL[k] - FR[k]);
+#pragma unroll
+  for (int k = 0; k < M; ++k) acc[k] = perm_pick<Ph>([&](int x) { return F[x]; }, a, k);
+  if (near) {
+    if (Ph::DIM == 1 || a == 0) AxisTerms<Ph>::template velocity<0>(P, gr, U, acc);
+    else if (Ph::DIM == 2 || a == 1) AxisTerms<Ph>::template velocity<1>(P, gr, U, acc);
+    else AxisTerms<Ph>::template velocity<2>(P, gr, U, acc);
+  }
 }
 
-// velocity of graph row r into acc
+// The velocity of the visited row of this lane of a wavefront (workgroup wg's
+// rows, DIM lanes each) into acc, in every lane of the row; returns the row,
+// or -1 for a lane without one.  The whole wavefront takes part.
 template <class Ph, int W>
-__device__ __forceinline__ void velocity_acc(const View &P, int64_t r, const double *__restrict__ U,
-                                             double (&acc)[Ph::M]) {
-  constexpr int M = Ph::M;
-  const int32_t *gr = P.graph + r * P.ncols;
-  const int64_t g = P.ghost_row[r];
-  if (g >= 0) fill_row_ghosts<Ph::DIM, M>(P, W, g, gr, U);
+__device__ __forceinline__ int64_t velocity_lanes(const View &P, int64_t wg, const double *__restrict__ U,
+                                                  double (&acc)[Ph::M]) {
+  constexpr int M = Ph::M, D = Ph::DIM, RPW = vel_rows<D>();
+  const int lane = threadIdx.x & 63, g = lane / D, a = lane % D;
+  const int64_t t = wg * RPW + g;
+  int64_t r = -1;
+  bool near = false;
 #pragma unroll
   for (int k = 0; k < M; ++k) acc[k] = 0.;
-  velocity_axis<Ph, W, 0>(P, gr, g, U, acc);
-  if (g >= 0) AxisTerms<Ph>::template velocity<0>(P, gr, U, acc);
-  if constexpr (Ph::DIM > 1) {
-    // one axis at a time: its gathered stencil and temporaries are dead
-    // before the next axis loads (the 3D WENO5 row otherwise holds all
-    // three axes' stencils and runs at one wave per SIMD)
-    __builtin_amdgcn_sched_barrier(0);
-    velocity_axis<Ph, W, 1>(P, gr, g, U, acc);
-    if (g >= 0) AxisTerms<Ph>::template velocity<1>(P, gr, U, acc);
+  if (g < RPW && t < P.nvisit) {
+    r = P.rows ? P.rows[t] : t;
+    near = P.ghost_row[r] >= 0;
+    velocity_axis<Ph, W>(P, P.graph + r * P.ncols, near, a, U, acc);
   }
-  if constexpr (Ph::DIM > 2) {
-    __builtin_amdgcn_sched_barrier(0);
-    velocity_axis<Ph, W, 2>(P, gr, g, U, acc);
-    if (g >= 0) AxisTerms<Ph>::template velocity<2>(P, gr, U, acc);
-  }
-  Sources<Ph>::apply(P, r, g >= 0, U, gr[0], acc, nullptr);
-}
-
-// velocity of visited row t (row P.rows[t], or t when the list is absent)
-template <class Ph, int W>
-__device__ __forceinline__ void velocity_row(const View &P, int64_t t, const double *__restrict__ U,
-                                             double *__restrict__ V) {
-  constexpr int M = Ph::M;
-  if (t >= P.nvisit) return;
-  const int64_t r = P.rows ? P.rows[t] : t;
-  double acc[M];
-  velocity_acc<Ph, W>(P, r, U, acc);
+  if constexpr (D > 1) {
 #pragma unroll
-  for (int k = 0; k < M; ++k) V[r * M + k] = acc[k];
+    for (int k = 0; k < M; ++k) {
+      double s = __shfl(acc[k], g * D, 64) + __shfl(acc[k], g * D + 1, 64);
+      if constexpr (D > 2) s += __shfl(acc[k], (g * D + 2) & 63, 64);
+      acc[k] = s;
+    }
+  }
+  if (r >= 0) Sources<Ph>::apply(P, r, near, U, P.graph[r * P.ncols], acc, nullptr);
+  return r;
 }
 
 // ---------------------------------------------------------------- jacobian
@@ -135,7 +125,7 @@ __device__ __forceinline__ void jac_axis_inner(const View &P, const int32_t *gr,
                                                double *__restrict__ J, int64_t base, int rs) {
   constexpr int M = Ph::M;
   double st[2 * W + 1][M];
-  gather<Ph, W, A>(P, gr, -1, W, U, st);
+  gather<Ph, W, A>(P, gr, U, st);
   Faces<M, W> f;
   double FL[M], FR[M];
   double JLn[M * M], JLp[M * M], JRn[M * M], JRp[M * M];
@@ -219,7 +209,7 @@ __device__ __forceinline__ void jac_axis_near(const View &P, const int32_t *gr, 
   const double h = P.hinv[A];
   double FL[M], FR[M];
   double st1[3][M];
-  gather<Ph, 1, A>(P, gr, g, W, U, st1);
+  gather<Ph, 1, A>(P, gr, U, st1);
   Faces<M, 1> f1;
   reconstruct<M, 1>(st1, f1);
   if constexpr (WV) {
@@ -228,7 +218,7 @@ __device__ __forceinline__ void jac_axis_near(const View &P, const int32_t *gr, 
       Ph::template flux<A>(P, f1.rm, f1.rp, FR);
     } else {
       double st[2 * W + 1][M];
-      gather<Ph, W, A>(P, gr, g, W, U, st);
+      gather<Ph, W, A>(P, gr, U, st);
       Faces<M, W> f;
       reconstruct<M, W>(st, f);
       Ph::template flux<A>(P, f.lm, f.lp, FL);
@@ -308,7 +298,6 @@ __device__ __forceinline__ void jacobian_row(const View &P, int64_t t, const dou
     if constexpr (Ph::DIM > 1) jac_axis_inner<Ph, W, 1, WV>(P, gr, sl, U, acc, self, J, base, rs);
     if constexpr (Ph::DIM > 2) jac_axis_inner<Ph, W, 2, WV>(P, gr, sl, U, acc, self, J, base, rs);
   } else {
-    fill_row_ghosts<Ph::DIM, M>(P, W, g, gr, U);
     jac_axis_near<Ph, W, 0, WV>(P, gr, g, sl, U, acc, self, J, base, rs);
     if constexpr (WV) AxisTerms<Ph>::template velocity<0>(P, gr, U, acc);
     if constexpr (Ph::DIM > 1) {
