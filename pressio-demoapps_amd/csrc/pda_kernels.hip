@@ -217,7 +217,12 @@ __global__ void __launch_bounds__(64) k_jacobian(View P, const double *__restric
 // row would scatter every store over 64 rows); 16 rows consecutive in the
 // CSR leave as one range of 16-byte stores.  Used where no structured box
 // kernel applies (sample meshes, 2D meshes given as a graph) and for the
-// boundary rows of a structured 3D full mesh.  Near-boundary rows: a
+// boundary rows of a structured 3D full mesh.  Bound by latency: a wavefront
+// alone takes 11 us (three dependent loads, two faces of divisions and square
+// roots, the stage, the copy) and the stage's 23 KB leave 7 of them per CU; 5 %
+// sample mesh of 128^3 50.6 us (147 MB of values), 61.7 us with a ghost branch
+// per block entry and the rows' CSR offsets fetched one by one at the copy.
+// Near-boundary rows: a
 // missing neighbour along axis a reads the ghost state sign_k U_k of the row's own cell (the first
 // ghost layer of every ghost rule), writes no block, and adds fac_j JL (left
 // side) or -fac_j JR (right side) of that face, times h, to the axis's
@@ -243,7 +248,8 @@ __global__ void __launch_bounds__(64) k_jac_fo_euler_staged(View P, const double
   using Ph = PhEuler<D>;
   constexpr int M = D + 2, NB = 1 + 2 * D, RS = NB * M, PER = M * RS;
   __shared__ double stage[SJ_ROWS * PER];
-  __shared__ int64_t row_of[SJ_ROWS];
+  __shared__ int64_t base_of[SJ_ROWS]; // first CSR value of the row, -1: no row
+  __shared__ int blk_of[SJ_ROWS];      // its column blocks
   const int lane = threadIdx.x, g = lane / SJ_LANES, a = lane % SJ_LANES;
   const int64_t t = int64_t(blockIdx.x) * SJ_ROWS + g;
   int64_t r = -1;
@@ -251,7 +257,13 @@ __global__ void __launch_bounds__(64) k_jac_fo_euler_staged(View P, const double
     const int64_t rr = P.rows ? P.rows[t] : t;
     r = rr;
   }
-  if (a == 0) row_of[g] = r;
+  // the row's place in the CSR, in each of its lanes
+  const int64_t base = r >= 0 ? P.rowbase[r] : -1;
+  const int nblk = r >= 0 ? P.nblk[r] : 0;
+  if (a == 0) {
+    base_of[g] = base;
+    blk_of[g] = nblk;
+  }
   const bool act = r >= 0 && a < D;
   double *st = stage + g * PER;
   typename Ph::Side Ln, Lp, Rn, Rp;
@@ -299,16 +311,17 @@ __global__ void __launch_bounds__(64) k_jac_fo_euler_staged(View P, const double
   // a fence between the face math and the stage stores keeps the entry
   // evaluations from being hoisted into it (2D: 148 -> 126 registers)
   wave_sync();
-  if (act) {
+  auto put = [&](int slot, const typename Ph::Side &S, bool minus) {
 #pragma unroll
     for (int k = 0; k < M; ++k)
 #pragma unroll
       for (int j = 0; j < M; ++j) {
-        const int o = exch(k, a) * RS + exch(j, a);
-        if (!gl) st[o + sL * M] = 0. + Ph::template entry<0>(P, Ln, k, j) * h;
-        if (!gr_) st[o + sR * M] = 0. + (-Ph::template entry<0>(P, Rp, k, j)) * h;
+        const double v = Ph::template entry<0>(P, S, k, j);
+        st[exch(k, a) * RS + exch(j, a) + slot * M] = 0. + (minus ? -v : v) * h;
       }
-  }
+  };
+  if (act && !gl) put(sL, Ln, false);
+  if (act && !gr_) put(sR, Rp, true);
   // every lane forms its axis's part of the diagonal block at once; the
   // axes then add their parts in order, one axis at a time, in LDS
   double dg[M][M];
@@ -317,11 +330,20 @@ __global__ void __launch_bounds__(64) k_jac_fo_euler_staged(View P, const double
 #pragma unroll
     for (int k = 0; k < M; ++k)
 #pragma unroll
-      for (int j = 0; j < M; ++j) {
+      for (int j = 0; j < M; ++j)
         dg[k][j] = (Ph::template entry<0>(P, Lp, k, j) - Ph::template entry<0>(P, Rn, k, j)) * h;
-        if (gl) dg[k][j] += (fac[j] * Ph::template entry<0>(P, Ln, k, j)) * h;
-        if (gr_) dg[k][j] += (fac[j] * -Ph::template entry<0>(P, Rp, k, j)) * h;
-      }
+  }
+  if (act && gl) {
+#pragma unroll
+    for (int k = 0; k < M; ++k)
+#pragma unroll
+      for (int j = 0; j < M; ++j) dg[k][j] += (fac[j] * Ph::template entry<0>(P, Ln, k, j)) * h;
+  }
+  if (act && gr_) {
+#pragma unroll
+    for (int k = 0; k < M; ++k)
+#pragma unroll
+      for (int j = 0; j < M; ++j) dg[k][j] += (fac[j] * -Ph::template entry<0>(P, Rp, k, j)) * h;
   }
 #pragma unroll
   for (int ax = 0; ax < D; ++ax) {
@@ -337,37 +359,52 @@ __global__ void __launch_bounds__(64) k_jac_fo_euler_staged(View P, const double
     }
   }
   wave_sync();
-  // rows consecutive in the CSR (a run along x): the stage is their values
-  // in order, copied as one range with 16-byte stores
-  const int64_t r0 = row_of[0], rl = row_of[SJ_ROWS - 1];
-  bool run = r0 >= 0;
-#pragma unroll
-  for (int gg = 1; gg < SJ_ROWS; ++gg) run = run && row_of[gg] == r0 + gg;
-  int64_t rb0 = 0;
-  if (run) {
-    rb0 = P.rowbase[r0];
-    run = P.rowbase[rl] == rb0 + int64_t(SJ_ROWS - 1) * PER;
-    run = run && P.nblk[rl] == NB;
-  }
-  if (run) {
+  // Copy-out from the row table in LDS alone: the rows' CSR offsets were
+  // loaded with their states (not here, one row after the other).  Whole
+  // rows leave as one flattened loop over their values: 16-byte stores where
+  // every row starts on an even value (2D, and 3D rows consecutive in the CSR
+  // after a leading value), else 8-byte ones.
+  const int64_t rb0 = base_of[0];
+  const bool whole = __all(base >= 0 && nblk == NB);
+  const bool run = __all(base == rb0 + int64_t(g) * PER);
+  if (whole && run) {
     constexpr int TOT = SJ_ROWS * PER;
     const int head = int(rb0 & 1); // a leading value that is not 16-byte aligned
     double *dst = J + rb0;
     if (head && lane == 0) store_stream(dst, stage[0]);
     const int npairs = (TOT - head) / 2;
     double2 *d2 = reinterpret_cast<double2 *>(dst + head);
+#pragma unroll 4
     for (int q = lane; q < npairs; q += 64)
       store_stream(d2 + q, make_double2(stage[head + 2 * q], stage[head + 2 * q + 1]));
     if (((TOT - head) & 1) && lane == 0) store_stream(dst + TOT - 1, stage[TOT - 1]);
     return;
   }
+  if (whole) {
+    if constexpr (PER % 2 == 0) {
+#pragma unroll 4
+      for (int q = lane; q < SJ_ROWS * (PER / 2); q += 64) {
+        const int gg = q / (PER / 2), e = 2 * (q - gg * (PER / 2));
+        const double *src = stage + gg * PER + e;
+        store_stream(reinterpret_cast<double2 *>(J + base_of[gg] + e), make_double2(src[0], src[1]));
+      }
+    } else {
+#pragma unroll 4
+      for (int q = lane; q < SJ_ROWS * PER; q += 64) {
+        const int gg = q / PER;
+        store_stream(J + base_of[gg] + (q - gg * PER), stage[q]);
+      }
+    }
+    return;
+  }
+#pragma clang loop unroll(disable)
   for (int gg = 0; gg < SJ_ROWS; ++gg) {
-    const int64_t rg = row_of[gg];
-    if (rg < 0) continue;
-    double *dst = J + P.rowbase[rg];
+    const int64_t rb = base_of[gg];
+    if (rb < 0) continue;
+    double *dst = J + rb;
     const double *src = stage + gg * PER;
     // a near-boundary row holds nblk of the NB block slots per scalar row
-    const int rs = P.nblk[rg] * M;
+    const int rs = blk_of[gg] * M;
     for (int e = lane; e < M * rs; e += 64) {
       int k = 0;
 #pragma unroll
