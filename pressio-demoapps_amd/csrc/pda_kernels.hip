@@ -43,41 +43,56 @@ __global__ void __launch_bounds__(64) k_velocity_stage(View P, const double *__r
 }
 
 // ----------------------------------------------- 1D steps in one launch
-// A small 1D problem is bound by launch latency: an SSPRK3 step is three
-// velocity launches of a few waves each.  k_steps1d advances several steps
-// in one launch.  Workgroup b owns cells [own b, own b + own) and holds them
+// A small 1D problem is bound by latency: an SSPRK3 step was three velocity
+// launches of a few waves each.  k_steps1d advances several steps in one
+// launch.  Workgroup b owns cells [own b, own b + own) and holds them
 // in LDS with H cells on each side, H = W x the number of stages it runs:
 // each stage's values are valid on a region W cells narrower per side than
-// the stage before, so after the last stage the owned cells are exact.  The
-// region is 128 rows (256 lanes, one wave per SIMD of the workgroup's CU:
-// a stage is one dependent chain of face arithmetic per lane, so a second
-// wave per SIMD would double it).  Two lanes per row evaluate its left and
-// right faces (the generic row code's stencil and ghost rule, the
-// one-division WENO weights of the 2D march, the same flux) and exchange
-// the fluxes; the row's velocity and its stage combination are formed as
-// k_velocity_stage forms them, term by term.  Ghosts: the
-// opposite rule (a row reads position g - d < 0 as cell g + d - 1, g + d
-// >= n as g - d + 1, times the side's sign), or periodic wrap.  The state
-// is read from Uin and written to Uout (workgroups read each other's cells).
-constexpr int S1_ROWS = 128;
+// the stage before, so after the last stage the owned cells are exact.  A
+// stage is one dependent chain per lane with little beside it on the CU, so
+// it is spread thin: four lanes per row, lane (f, s) reconstructing side s
+// (0 minus, 1 plus) of face f (0 left, 1 right) of the row with the generic
+// row code's stencil and ghost rule (the plus side is the minus side of the
+// reversed stencil, so the lanes share one instruction stream); the pair
+// exchanges its sides and the faces their fluxes by DPP, and lane q < M forms
+// dof q of the stage, as k_velocity_stage does, term by term.  Where a lane
+// reads does not change from stage to stage: its cells' places in LDS are
+// found once per launch.  Ghosts: the opposite rule (a row reads position
+// g - d < 0 as cell g + d - 1, g + d >= n as g - d + 1; the 1D problems have no
+// sign to apply), or periodic wrap.  The state is read from Uin and
+// written to Uout (workgroups read each other's cells).  The region is 128
+// rows (two waves per SIMD of the CU).  1000 cells, WENO5, SSPRK3: 4.8 us per
+// step, 8.6 us with two lanes per row that each reconstructed both sides of
+// a face and looked up every cell's place in every stage.
+constexpr int S1_ROWS = 128, S1_LPR = 4;
 
 struct Steps1dCoef {
   double c[4][4];  // per stage: coefficients of the stage's terms
   double cv[4];    // per stage: coefficient of the velocity
 };
 
+// value of the lane whose index differs in bit 0 (quad_perm 1,0,3,2) or bit 1
+// (quad_perm 2,3,0,1)
+template <int CTRL> __device__ __forceinline__ double quad_swap(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, int(b), CTRL, 0xf, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, int(b >> 32), CTRL, 0xf, 0xf, false);
+  return __longlong_as_double((long long)(unsigned(lo)) | ((long long)hi << 32));
+}
+
 template <class Ph, int W, int SCHEME>
-__global__ void __launch_bounds__(2 * S1_ROWS) k_steps1d(View P, int64_t n, int periodic, int own, int H,
-                                                        int nsteps, const double *__restrict__ Uin,
-                                                        double *__restrict__ Uout, Steps1dCoef C) {
-  constexpr int M = Ph::M;
+__global__ void __launch_bounds__(S1_LPR * S1_ROWS) k_steps1d(View P, int64_t n, int periodic, int own, int H,
+                                                             int nsteps, const double *__restrict__ Uin,
+                                                             double *__restrict__ Uout, Steps1dCoef C) {
+  constexpr int M = Ph::M, R = S1_ROWS, NP = 2 * W - 1;
+  static_assert(M <= S1_LPR, "a lane per dof");
   extern __shared__ double lds[];
-  const int R = own + 2 * H;
   const int64_t a0 = int64_t(blockIdx.x) * own, base = a0 - H;
-  // buffers of R x M doubles: 0 the step's state, 1 and 2 stage states,
-  // 3..5 the RK4 stage velocities
-  auto buf = [&](int b) { return lds + int64_t(b) * R * M; };
-  for (int e = threadIdx.x; e < R * M; e += blockDim.x) {
+  const int rows = own + 2 * H; // <= R
+  // buffers of M x R doubles ([dof][row]): 0 the step's state, 1 and 2 stage
+  // states, 3..5 the RK4 stage velocities
+  auto buf = [&](int b) { return lds + b * (R * M); };
+  for (int e = threadIdx.x; e < rows * M; e += blockDim.x) {
     const int i = e / M, k = e - i * M;
     int64_t g = base + i;
     double v = 0.;
@@ -88,113 +103,105 @@ __global__ void __launch_bounds__(2 * S1_ROWS) k_steps1d(View P, int64_t n, int 
     } else if (g >= 0 && g < n) {
       v = Uin[g * M + k];
     }
-    buf(0)[e] = v;
+    buf(0)[k * R + i] = v;
+  }
+  const int i = int(threadIdx.x) / S1_LPR, q4 = int(threadIdx.x) % S1_LPR, f = q4 >> 1, sd = q4 & 1;
+  const int64_t g = base + i;
+  const bool store = i < rows && (periodic || (g >= 0 && g < n)) && q4 < M;
+  const int kq = q4 < M ? q4 : 0; // this lane's dof
+  const double hf = f ? -P.hinv[0] : P.hinv[0];
+  // the lane's 2W-1 cells, from the one upwind of the face's farthest on
+  int at[NP];
+#pragma unroll
+  for (int j = 0; j < NP; ++j) {
+    const int p = sd ? 2 * W - 1 - j : j; // point of the face's 2W cells
+    int64_t src = g + f - W + p;
+    if (!periodic) src = src < 0 ? 2 * g - src - 1 : (src >= n ? 2 * g - src + 1 : src);
+    const int64_t li = src - base;
+    at[j] = int(li < 0 ? 0 : (li >= rows ? rows - 1 : li));
   }
   __syncthreads();
-  const int i = int(threadIdx.x) >> 1, f = int(threadIdx.x) & 1;
-  const int64_t g = base + i;
-  const bool row = i < R && (periodic || (g >= 0 && g < n));
-  const bool store = row && f == 0;
-  const double h = P.hinv[0];
-  // velocity of row i from state X (every lane takes part in the exchange)
-  auto vel = [&](const double *X, double (&acc)[M]) {
-    double q[M][2 * W];
+  // dof kq of the velocity of row i from state X (every lane takes part in
+  // the exchanges)
+  auto vel = [&](const double *X) {
+    double q[M][NP];
 #pragma unroll
-    for (int p = 0; p < 2 * W; ++p) {
-      int64_t src = g + f - W + p;
-      int side = -1;
-      if (!periodic) {
-        if (src < 0) {
-          src = 2 * g - src - 1;
-          side = 0;
-        } else if (src >= n) {
-          src = 2 * g - src + 1;
-          side = 1;
-        }
-      }
-      int64_t li = src - base;
-      li = li < 0 ? 0 : (li >= R ? R - 1 : li);
+    for (int k = 0; k < M; ++k)
 #pragma unroll
-      for (int k = 0; k < M; ++k) {
-        const double v = X[li * M + k];
-        q[k][p] = side < 0 ? v : P.gsign[0][side][k] * v;
-      }
-    }
+      for (int j = 0; j < NP; ++j) q[k][j] = X[k * R + at[j]];
     double um[M], up[M], F[M];
 #pragma unroll
     for (int k = 0; k < M; ++k) {
+      double v;
       if constexpr (W == 1) {
-        um[k] = q[k][0];
-        up[k] = q[k][1];
+        v = q[k][0];
       } else if constexpr (W == 2) {
-        phys::weno3_1div(q[k], um[k], up[k]);
+        v = phys::w3_hi(q[k][0], q[k][1], q[k][2], phys::w3_d(q[k][0], q[k][1]), phys::w3_d(q[k][1], q[k][2]));
       } else {
-        phys::weno5_1div(q[k], um[k], up[k]);
+        v = phys::weno5_side_1div(q[k][0], q[k][1], q[k][2], q[k][3], q[k][4]);
       }
+      const double o = quad_swap<0xB1>(v);
+      um[k] = sd ? o : v;
+      up[k] = sd ? v : o;
     }
     Ph::template flux<0>(P, um, up, F);
+    // left minus right flux: this lane's face minus the other, turned round in
+    // the lanes of the right face
+    double acc = 0.;
 #pragma unroll
     for (int k = 0; k < M; ++k) {
-      const double o = __shfl_xor(F[k], 1);
-      const double FL = f ? o : F[k], FR = f ? F[k] : o;
-      acc[k] = 0.;
-      acc[k] += h * (FL - FR);
+      const double d = F[k] - quad_swap<0x4E>(F[k]);
+      acc = k == kq ? d : acc;
     }
+    acc = 0. + hf * acc;
+    return acc;
   };
+  const int e = kq * R + (i < rows ? i : 0);
   // out = c0 x0 + ... + cv v, the terms in k_velocity_stage's order
   auto comb = [&](double *out, int st, int nx, const double *x0, const double *x1, const double *x2,
-                  const double *x3, const double (&acc)[M]) {
+                  const double *x3, double acc) {
     if (!store) return;
-#pragma unroll
-    for (int k = 0; k < M; ++k) {
-      const int e = i * M + k;
-      double o = C.c[st][0] * x0[e];
-      if (nx > 1) o += C.c[st][1] * x1[e];
-      if (nx > 2) o += C.c[st][2] * x2[e];
-      if (nx > 3) o += C.c[st][3] * x3[e];
-      o += C.cv[st] * acc[k];
-      out[e] = o;
-    }
+    double o = C.c[st][0] * x0[e];
+    if (nx > 1) o += C.c[st][1] * x1[e];
+    if (nx > 2) o += C.c[st][2] * x2[e];
+    if (nx > 3) o += C.c[st][3] * x3[e];
+    o += C.cv[st] * acc;
+    out[e] = o;
   };
-  auto keep = [&](double *kb, const double (&acc)[M]) {
-    if (!store) return;
-#pragma unroll
-    for (int k = 0; k < M; ++k) kb[i * M + k] = acc[k];
+  auto keep = [&](double *kb, double acc) {
+    if (store) kb[e] = acc;
   };
   for (int s = 0; s < nsteps; ++s) {
-    double acc[M];
+    double acc;
     if constexpr (SCHEME == PDA_SSPRK3) {
-      vel(buf(0), acc);  // u1 = u + dt f(u)
+      acc = vel(buf(0));  // u1 = u + dt f(u)
       comb(buf(1), 0, 1, buf(0), nullptr, nullptr, nullptr, acc);
       __syncthreads();
-      vel(buf(1), acc);  // u2 = 1/4 u1 + 3/4 u + 1/4 dt f(u1)
+      acc = vel(buf(1));  // u2 = 1/4 u1 + 3/4 u + 1/4 dt f(u1)
       comb(buf(2), 1, 2, buf(1), buf(0), nullptr, nullptr, acc);
       __syncthreads();
-      vel(buf(2), acc);  // u = 1/3 u + 2/3 u2 + 2/3 dt f(u2)
+      acc = vel(buf(2));  // u = 1/3 u + 2/3 u2 + 2/3 dt f(u2)
       comb(buf(0), 2, 2, buf(0), buf(2), nullptr, nullptr, acc);
       __syncthreads();
     } else {
-      vel(buf(0), acc);  // k1; y1 = u + dt/2 k1
+      acc = vel(buf(0));  // k1; y1 = u + dt/2 k1
       keep(buf(3), acc);
       comb(buf(1), 0, 1, buf(0), nullptr, nullptr, nullptr, acc);
       __syncthreads();
-      vel(buf(1), acc);  // k2; y2 = u + dt/2 k2
+      acc = vel(buf(1));  // k2; y2 = u + dt/2 k2
       keep(buf(4), acc);
       comb(buf(2), 1, 1, buf(0), nullptr, nullptr, nullptr, acc);
       __syncthreads();
-      vel(buf(2), acc);  // k3; y3 = u + dt k3
+      acc = vel(buf(2));  // k3; y3 = u + dt k3
       keep(buf(5), acc);
       comb(buf(1), 2, 1, buf(0), nullptr, nullptr, nullptr, acc);
       __syncthreads();
-      vel(buf(1), acc);  // u = u + dt/6 k1 + dt/3 k2 + dt/3 k3 + dt/6 k4
+      acc = vel(buf(1));  // u = u + dt/6 k1 + dt/3 k2 + dt/3 k3 + dt/6 k4
       comb(buf(0), 3, 4, buf(0), buf(3), buf(4), buf(5), acc);
       __syncthreads();
     }
   }
-  if (store && i >= H && i < H + own && g < n) {
-#pragma unroll
-    for (int k = 0; k < M; ++k) Uout[g * M + k] = buf(0)[i * M + k];
-  }
+  if (store && i >= H && i < H + own && g < n) Uout[g * M + kq] = buf(0)[e];
 }
 
 template <class Ph, int W, bool WV>
@@ -1134,15 +1141,31 @@ bool steps1d_fits(const pda_problem_s &p, int scheme, bool *periodic_out) {
   }
   *periodic_out = periodic;
   if (periodic) return true;
+  for (int s = 0; s < 2; ++s)
+    for (int k = 0; k < p.m; ++k) open = open && p.view.gsign[0][s][k] == 1.;
   return open && p.view.ghost_rule == GHOST_OPPOSITE;
 }
 
-// steps per launch: the most that leave at least 32 owned rows of the
-// 128-row region (SSPRK3 WENO5: 5 steps, 38 owned rows)
+// Steps per launch: more steps pay the launch (about 5 us, against 1.1 us for a
+// stage) less often, but leave a workgroup fewer owned rows of its 128 (SSPRK3
+// WENO5: 6 steps, 20 owned rows), so more workgroups.  The least time per
+// step, with the workgroups running in rounds of two per CU: the most steps
+// up to about 10^4 cells, fewer beyond.
 int steps1d_per_launch(const pda_problem_s &p, int scheme) {
-  const int per = (scheme == PDA_RK4 ? 4 : 3) * p.w;  // halo rows per side per step
-  const int k = (S1_ROWS - 32) / (2 * per);
-  return k < 1 ? 1 : (k > STEPS1D_MAX ? STEPS1D_MAX : k);
+  const int nst = scheme == PDA_RK4 ? 4 : 3;
+  int best = 1;
+  double best_cost = 1e300;
+  for (int k = 1; k <= STEPS1D_MAX; ++k) {
+    const int own = S1_ROWS - 2 * nst * p.w * k;
+    if (own < 16 && k > 1) break;
+    const int64_t nwg = (p.mesh->n_sample + own - 1) / own;
+    const double cost = double((nwg + 511) / 512) * (5. + 1.1 * nst * k) / k;
+    if (cost < best_cost) {
+      best_cost = cost;
+      best = k;
+    }
+  }
+  return best;
 }
 
 int launch_steps1d(const pda_problem_s &p, int scheme, const double *Uin, double *Uout, int nsteps, double dt,
@@ -1156,7 +1179,7 @@ int launch_steps1d(const pda_problem_s &p, int scheme, const double *Uin, double
   const int H = nst * p.w * kmax, own = S1_ROWS - 2 * H;
   const int64_t n = p.mesh->n_sample;
   constexpr int M = PhEuler1::M;
-  const unsigned threads = 2 * S1_ROWS;
+  const unsigned threads = S1_LPR * S1_ROWS;
   const size_t lds = sizeof(double) * size_t(nbuf) * size_t(S1_ROWS) * M;
   const dim3 grid{unsigned((n + own - 1) / own), 1, 1};
   if (own < 1 || lds > 64 * 1024) {

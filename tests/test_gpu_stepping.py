@@ -239,3 +239,41 @@ def test_1d_steps_per_launch(case, scheme, oracle, torch):
     err = cases.rel_err(Ua.cpu().numpy(), ref)
     print(f"[gpu-step] 1d {case[0]} {scheme}: vs oracle run {err:.2e}", flush=True)
     assert err <= 1e-11
+
+
+@pytest.mark.parametrize("scheme", ["SSPRK3", "RK4"])
+def test_1d_steps_per_launch_of_large_grids(scheme, torch):
+    """Grids where a launch takes fewer steps (its workgroups run in several
+    rounds): 9 steps in one call and in calls of 2 and 7 agree bit for bit, and
+    match the stage formulas on the problem's velocity (12 roundings a stage
+    apart, 40 stages)."""
+    print(f"[gpu-step] 1d large {scheme}", flush=True)
+    mesh = pda.create_structured_mesh((30011,), (-0.5, 0.5), 7)
+    prob = pda.create_problem(mesh, pda.Euler1d.Sod, S.Weno5)
+    dt = 1e-6
+    U0 = prob.initialCondition()
+    U0 *= 1 + 0.01 * torch.sin(torch.arange(U0.numel(), dtype=torch.float64, device="cuda"))
+    Ua, Ub = U0.clone(), U0.clone()
+    pda.ExplicitStepper(prob, pda.StepScheme[scheme]).advance(Ua, dt, 9)
+    st = pda.ExplicitStepper(prob, pda.StepScheme[scheme])
+    st.advance(Ub, dt, 2)
+    st.advance(Ub, dt, 7)
+    assert torch.equal(Ua, Ub)
+
+    def f(y):
+        v = prob.createRightHandSide()
+        prob.rightHandSide(y, 0.0, v)
+        return v
+
+    y = U0.clone()
+    for _ in range(9):
+        if scheme == "SSPRK3":
+            u1 = y + dt * f(y)
+            u2 = 0.75 * y + 0.25 * (u1 + dt * f(u1))
+            y = y / 3 + 2 / 3 * (u2 + dt * f(u2))
+        else:
+            k1 = f(y)
+            k2 = f(y + 0.5 * dt * k1)
+            k3 = f(y + 0.5 * dt * k2)
+            y = y + dt / 6 * (k1 + 2 * k2 + 2 * k3 + f(y + dt * k3))
+    assert cases.rel_err(Ua.cpu().numpy(), y.cpu().numpy()) <= 40 * 12 * 2.3e-16
