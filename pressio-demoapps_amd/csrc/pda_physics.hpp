@@ -12,17 +12,36 @@ namespace phys {
 
 constexpr double kEs = 1.e-30;
 
-// n / d from the hardware reciprocal estimate refined by two Newton steps
-// and one residual correction: within an ulp of the rounded quotient for d
-// and n / d in the normal range (the WENO weight sums, the densities and the
-// Roe factors of the velocity's fluxes), without the IEEE division
-// sequence's scaling for denormal and infinite operands.
+// 1 / d from the hardware estimate (2^-24) and one third-order step: within an
+// ulp for d and 1 / d in the normal range
+__device__ __forceinline__ double frcp(double d) {
+  const double r = __builtin_amdgcn_rcp(d);
+  const double e = __fma_rn(-d, r, 1.);
+  return __fma_rn(r, __fma_rn(e, e, e), r);
+}
+
+// n / d from that and one residual correction: within an ulp of the rounded
+// quotient for d and n / d in the normal range (the densities and the Roe
+// factors of the velocity's fluxes), without the IEEE division sequence's
+// scaling for denormal and infinite operands.
 __device__ __forceinline__ double fdiv(double n, double d) {
-  double r = __builtin_amdgcn_rcp(d);
-  r = __fma_rn(r, __fma_rn(-d, r, 1.), r);
-  r = __fma_rn(r, __fma_rn(-d, r, 1.), r);
+  const double r = frcp(d);
   const double q = n * r;
   return __fma_rn(r, __fma_rn(-d, q, n), q);
+}
+
+// sqrt(x) from the hardware reciprocal root, one Goldschmidt step and two
+// residual corrections: the library's sequence without its scaling for
+// denormal arguments.  The addend keeps 0 (a state at rest) from giving 0 * inf
+// and is lost in every x above 1e-284; x < 0 gives NaN.
+__device__ __forceinline__ double fsqrt(double x) {
+  const double y = __builtin_amdgcn_rsq(x + 1e-300);
+  double g = x * y, h = 0.5 * y;
+  const double r = __fma_rn(-h, g, 0.5);
+  g = __fma_rn(g, r, g);
+  h = __fma_rn(h, r, h);
+  g = __fma_rn(__fma_rn(-g, g, x), h, g);
+  return __fma_rn(__fma_rn(-g, g, x), h, g);
 }
 
 // ---------------------------------------------------------------- WENO3
@@ -88,47 +107,64 @@ __device__ __forceinline__ void weno3_grad(const double *q, double &un, double &
 }
 
 // ---------------------------------------------------------------- WENO5
-// Reconstruction (impl/weno5.hpp:56-178) with the normalised weights formed
-// with one division: alpha_k / sum(alpha) = N_k / sum(N) with N_k = d_k *
-// prod_{j != k} D_j and D_k = eps^2 + 2 eps B_k + B_k^2 (the reference's
-// denominator).  Equal to the reference's four divisions in exact arithmetic;
-// the results differ by a few ulps.
-//
-// D of a side window (far, mid, near), near = the reconstructed cell:
-// B = 13/12 (far - 2 mid + near)^2 + 1/4 (far - 4 mid + 3 near)^2.  The
-// operations are fixed (explicit FMAs, far + near summed first), so that a
-// window gives the same D whichever of its two cells' reconstructions reads
-// it: the low-side and high-side values of a cell share their windows.
-__device__ __forceinline__ double w5_dside(double far, double mid, double near) {
-  constexpr double eps = 1.e-6, c1312 = 13. / 12.;
-  const double t = __fma_rn(-2., mid, far + near);
-  const double s = __fma_rn(-4., mid, __fma_rn(3., near, far));
-  const double B = __fma_rn(c1312 * t, t, (0.25 * s) * s);
-  return __fma_rn(B, B, __fma_rn(2. * eps, B, eps * eps));
+// Reconstruction (impl/weno5.hpp:56-178) as a correction to the cell's value.
+// With the differences e_k = q_k - q_{k-1} of the cells q_0 .. q_4 about cell
+// q_2, the candidates at the face towards q_3 are
+//   p_0 = q_2 + (5 e_2 - 2 e_1) / 6, p_1 = q_2 + (e_2 + 2 e_3) / 6,
+//   p_2 = q_2 + (4 e_3 - e_4) / 6,
+// and with E_k = 4 (eps + B_k) the weights d_k / (eps + B_k)^2 are as
+// d_k Prod_{j != k} E_j^2: one division per value, of the correction only, so
+// that its rounding (a few ulps) counts in the correction's size, not the
+// value's.  4 B = 13/3 t^2 + s^2 with t the second difference of the window
+// and s its first (centred or one-sided).  Equal to the reference's weighted
+// sum in exact arithmetic.  The operations are fixed (explicit FMAs) and the
+// same for a window read from either side, so a face value does not depend on
+// which of the forms below gives it.  58 operations for the two values of a cell
+// (85 as weighted candidates with the B's and their squares formed apart).
+struct W5 {
+  double e1, e2, e3, e4; // the differences
+  double s0, s1, s2;     // Prod E^2 without window 0, 6 times without 1, without 2
+};
+__device__ __forceinline__ W5 w5_window(double q0, double q1, double q2, double q3, double q4) {
+  constexpr double eps4 = 4.e-6, c133 = 13. / 3.;
+  W5 w;
+  w.e1 = q1 - q0;
+  w.e2 = q2 - q1;
+  w.e3 = q3 - q2;
+  w.e4 = q4 - q3;
+  const double t0 = w.e2 - w.e1, t1 = w.e3 - w.e2, t2 = w.e4 - w.e3;
+  const double a0 = __fma_rn(2., w.e2, t0), a1 = w.e2 + w.e3, a2 = __fma_rn(-2., w.e3, t2);
+  const double E0 = __fma_rn(c133 * t0, t0, __fma_rn(a0, a0, eps4));
+  const double E1 = __fma_rn(c133 * t1, t1, __fma_rn(a1, a1, eps4));
+  const double E2 = __fma_rn(c133 * t2, t2, __fma_rn(a2, a2, eps4));
+  const double p0 = E1 * E2, p1 = E0 * E2, p2 = E0 * E1;
+  w.s0 = p0 * p0;
+  w.s1 = 6. * (p1 * p1);
+  w.s2 = p2 * p2;
+  return w;
 }
-// D of the centred window (lo, mid, hi): B = 13/12 (lo - 2 mid + hi)^2 +
-// 1/4 (lo - hi)^2, the same for the window read in either direction
-__device__ __forceinline__ double w5_dmid(double lo, double mid, double hi) {
-  constexpr double eps = 1.e-6, c1312 = 13. / 12.;
-  const double t = __fma_rn(-2., mid, lo + hi);
-  const double s = lo - hi;
-  const double B = __fma_rn(c1312 * t, t, (0.25 * s) * s);
-  return __fma_rn(B, B, __fma_rn(2. * eps, B, eps * eps));
-}
-// reconstruction at the face of cell q2 towards q3 from the windows' D
-__device__ __forceinline__ double w5_value(double q0, double q1, double q2, double q3, double q4,
-                                           double D0, double D1, double D2) {
+// n / d for the correction: within two ulps
+__device__ __forceinline__ double w_quot(double n, double d) { return n * frcp(d); }
+// value of cell q2 at the face towards q3
+__device__ __forceinline__ double w5_hi(const W5 &w, double q2) {
   constexpr double c16 = 1. / 6.;
-  const double p0 = (2. * q0 - 7. * q1 + 11. * q2) * c16;
-  const double p1 = (-q1 + 5. * q2 + 2. * q3) * c16;
-  const double p2 = (2. * q2 + 5. * q3 - q4) * c16;
-  const double n0 = 0.1 * (D1 * D2), n1 = 0.6 * (D0 * D2), n2 = 0.3 * (D0 * D1);
-  return fdiv(n0 * p0 + n1 * p1 + n2 * p2, n0 + n1 + n2);
+  const double m2 = 3. * w.s2;
+  const double n = __fma_rn(m2, __fma_rn(4., w.e3, -w.e4),
+                            __fma_rn(w.s1, __fma_rn(2., w.e3, w.e2), w.s0 * __fma_rn(5., w.e2, -2. * w.e1)));
+  return __fma_rn(c16, w_quot(n, (w.s0 + w.s1) + m2), q2);
 }
+// value of cell q2 at the face towards q1: w5_hi of the reversed cells
+__device__ __forceinline__ double w5_lo(const W5 &w, double q2) {
+  constexpr double c16 = 1. / 6.;
+  const double m0 = 3. * w.s0;
+  const double n = __fma_rn(m0, __fma_rn(4., w.e2, -w.e1),
+                            __fma_rn(w.s1, __fma_rn(2., w.e2, w.e3), w.s2 * __fma_rn(5., w.e3, -2. * w.e4)));
+  return __fma_rn(-c16, w_quot(n, (w.s2 + w.s1) + m0), q2);
+}
+// the left-biased value: of cell q2 at the face towards q3
 __device__ __forceinline__ double weno5_side_1div(double q0, double q1, double q2, double q3,
                                                   double q4) {
-  return w5_value(q0, q1, q2, q3, q4, w5_dside(q0, q1, q2), w5_dmid(q1, q2, q3),
-                  w5_dside(q4, q3, q2));
+  return w5_hi(w5_window(q0, q1, q2, q3, q4), q2);
 }
 
 // q = {q_{i-2}, ..., q_{i+3}}; un, up: left and right states of face i+1/2
@@ -141,35 +177,32 @@ __device__ __forceinline__ void weno5_1div(const double *q, double &un, double &
 
 // Both face values of one cell from q = cells i-2 .. i+2: hi = the left
 // state of face i+1/2, lo = the right state of face i-1/2.  Bit-identical to
-// the two weno5_side_1div calls of weno5_1div at those faces; the three
-// windows' D are formed once.
+// the two weno5_side_1div calls of weno5_1div at those faces; the windows are
+// formed once.
 __device__ __forceinline__ void weno5_cell_1div(double q0, double q1, double q2, double q3,
                                                 double q4, double &hi, double &lo) {
-  const double D0 = w5_dside(q0, q1, q2), D1 = w5_dmid(q1, q2, q3), D2 = w5_dside(q4, q3, q2);
-  hi = w5_value(q0, q1, q2, q3, q4, D0, D1, D2);
-  lo = w5_value(q4, q3, q2, q1, q0, D2, D1, D0);
+  const W5 w = w5_window(q0, q1, q2, q3, q4);
+  hi = w5_hi(w, q2);
+  lo = w5_lo(w, q2);
 }
 
-// WENO3 counterpart of weno5_1div (impl/weno3.hpp:56-132).  D of the
-// two-cell window (a, b): B = (a - b)^2, the same in either direction.
+// WENO3 counterparts (impl/weno3.hpp:56-132): D = (eps + B)^2 of the two-cell
+// window (a, b) with B = (a - b)^2, the same in either direction, and the
+// values as corrections: the candidates at the face of b towards c are
+// b + (b - a) / 2 and b + (c - b) / 2 with weights 1/3 and 2/3.
 __device__ __forceinline__ double w3_d(double a, double b) {
   constexpr double eps = 1.e-6;
-  const double B = (a - b) * (a - b);
-  return __fma_rn(B, B, __fma_rn(2. * eps, B, eps * eps));
+  const double d = a - b, E = __fma_rn(d, d, eps);
+  return E * E;
 }
 // the face values of cell b (neighbours a below, c above) from the windows'
 // D: hi at the face towards c, lo at the face towards a
 __device__ __forceinline__ double w3_hi(double a, double b, double c, double Dab, double Dbc) {
-  constexpr double c13 = 1. / 3., c23 = 2. / 3.;
-  const double p0 = (-a + 3. * b) * 0.5, p1 = (b + c) * 0.5;
-  const double n0 = c13 * Dbc, n1 = c23 * Dab;
-  return fdiv(n0 * p0 + n1 * p1, n0 + n1);
+  const double m = 2. * Dab;
+  return __fma_rn(0.5, w_quot(__fma_rn(m, c - b, Dbc * (b - a)), Dbc + m), b);
 }
 __device__ __forceinline__ double w3_lo(double a, double b, double c, double Dab, double Dbc) {
-  constexpr double c13 = 1. / 3., c23 = 2. / 3.;
-  const double p0 = (a + b) * 0.5, p1 = (3. * b - c) * 0.5;
-  const double n0 = c23 * Dbc, n1 = c13 * Dab;
-  return fdiv(n0 * p0 + n1 * p1, n0 + n1);
+  return w3_hi(c, b, a, Dbc, Dab);
 }
 __device__ __forceinline__ void weno3_1div(const double *q, double &un, double &up) {
   un = w3_hi(q[0], q[1], q[2], w3_d(q[0], q[1]), w3_d(q[1], q[2]));
@@ -309,16 +342,16 @@ __device__ __forceinline__ void euler_flux(const double *qL, const double *qR, d
   }
   FL[M - 1] = rL * unL * HL;
   FR[M - 1] = rR * unR * HR;
-  const double RT = sqrt(fdiv(rR, rL));
-  const double inv = fdiv(1., 1. + RT);
+  const double RT = fsqrt(rR * iL);
+  const double inv = frcp(1. + RT);
   double vr2 = 0.;
   for (int d = 0; d < DIM; ++d) {
     const double v = (velL[d] + RT * velR[d]) * inv;
     vr2 += v * v;
   }
   const double H = (HL + RT * HR) * inv;
-  const double a = sqrt((g - 1.) * (H - half * vr2));
-  const double smax = (DIM == 1 ? fabs((velL[0] + RT * velR[0]) * inv) : sqrt(vr2)) + a;
+  const double a = fsqrt((g - 1.) * (H - half * vr2));
+  const double smax = (DIM == 1 ? fabs((velL[0] + RT * velR[0]) * inv) : fsqrt(vr2)) + a;
   for (int i = 0; i < M; ++i) F[i] = half * (FL[i] + FR[i] + smax * (qL[i] - qR[i]));
 }
 
@@ -455,17 +488,18 @@ __device__ __forceinline__ void euler_fjac(const double *qL, const double *qR, d
 // impl/swe_rusanov_flux_values_function.hpp:54-97
 template <int A>
 __device__ __forceinline__ void swe_flux(const double *qL, const double *qR, double g, double *F) {
-  const double hL = qL[0], uL = fdiv(qL[1], hL + kEs), vL = fdiv(qL[2], hL + kEs);
-  const double hR = qR[0], uR = fdiv(qR[1], hR + kEs), vR = fdiv(qR[2], hR + kEs);
+  // one reciprocal per side (the reference divides per component)
+  const double hL = qL[0], iL = fdiv(1., hL + kEs), uL = qL[1] * iL, vL = qL[2] * iL;
+  const double hR = qR[0], iR = fdiv(1., hR + kEs), uR = qR[1] * iR, vR = qR[2] * iR;
   const double unL = A == 0 ? uL : vL, unR = A == 0 ? uR : vR;
   const double pL = 0.5 * g * hL * hL, pR = 0.5 * g * hR * hR;
   double FL[3], FR[3];
   FL[0] = hL * unL; FL[1] = hL * unL * uL + (A == 0 ? pL : 0.); FL[2] = hL * unL * vL + (A == 1 ? pL : 0.);
   FR[0] = hR * unR; FR[1] = hR * unR * uR + (A == 0 ? pR : 0.); FR[2] = hR * unR * vR + (A == 1 ? pR : 0.);
   const double hm = 0.5 * (hL + hR);
-  const double sL = sqrt(hL), sR = sqrt(hR);
+  const double sL = fsqrt(hL), sR = fsqrt(hR);
   const double um = fdiv(unL * sL + unR * sR, sL + sR + kEs);
-  const double c = sqrt(g * hm);
+  const double c = fsqrt(g * hm);
   // sqrt(x * x) is |x| exactly in IEEE arithmetic (no overflow here)
   const double smax = fabs(um) + fabs(c);
   for (int i = 0; i < 3; ++i) F[i] = 0.5 * (FL[i] + FR[i] + smax * (qL[i] - qR[i]));
