@@ -6,7 +6,9 @@
 // pressio/solvers_nonlinear/impl/nonlinear_least_squares.hpp:14-118) with a
 // device BiCGSTAB (the iteration of Eigen's BiCGSTAB, which pressio's
 // default linear solver wraps, solvers_linear_traits.hpp:95-105) and a
-// block-Jacobi preconditioner (the m x m diagonal blocks, inverted per cell).
+// block-Jacobi preconditioner (the m x m diagonal blocks, inverted per cell),
+// applied from the right: the matrix of the iteration is I + B with the blocks
+// B_ij = cf J_ij (cf J_jj + cnp1 I)^-1, formed once per Newton iteration.
 //
 // Stop rules:
 //   PDA_STOP_CORRECTION -- pressio's default: stop when the l2 norm of the
@@ -28,12 +30,9 @@ constexpr int MAXB = 1024; // most blocks (partial sums) of the reducing kernels
 
 // Device scalars of the Krylov solver.  Each is written by the first block of
 // one kernel and read by the kernels after it (never by the one that writes
-// it): the search kernel writes RHO_NEXT, RR and DONE_NEXT, the
-// preconditioned-residual kernel RHO, ALPHA and DONE, the update kernel W and
-// NITER.
-enum {
-  S_RHO = 0, S_RHO_NEXT, S_ALPHA, S_W, S_RR, S_BB, S_TOL2, S_DONE, S_DONE_NEXT, S_NITER, S_CF, S_CNP1, S_COUNT
-};
+// it): the search kernel writes RHO_NEXT, RR and DONE_NEXT, the second product
+// RHO, ALPHA and DONE, the update kernel W and NITER.
+enum { S_RHO = 0, S_RHO_NEXT, S_ALPHA, S_W, S_RR, S_BB, S_TOL2, S_DONE, S_DONE_NEXT, S_NITER, S_COUNT };
 
 __device__ __forceinline__ double block_sum(double v, double *sh) {
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -69,14 +68,6 @@ __device__ __forceinline__ void put_pair(double *part, double s1, double s2, dou
   }
 }
 
-// partial sums of a.a (the second of the pair unused)
-__global__ void __launch_bounds__(TB) k_norm(const double *__restrict__ a, int64_t n, double *__restrict__ part) {
-  __shared__ double sh[TB / 64];
-  double s = 0.;
-  for (int64_t i = int64_t(blockIdx.x) * TB + threadIdx.x; i < n; i += int64_t(gridDim.x) * TB) s += a[i] * a[i];
-  put_pair(part, s, 0., sh);
-}
-
 // the norms of up to two vectors from their partial sums, into host memory
 __global__ void __launch_bounds__(TB) k_norms_out(const double *__restrict__ pa, const double *__restrict__ pb, int n,
                                                   double *__restrict__ host) {
@@ -89,22 +80,6 @@ __global__ void __launch_bounds__(TB) k_norms_out(const double *__restrict__ pa,
   if (threadIdx.x == 0) host[1] = sqrt(s1);
 }
 
-// sum over the 16 (or 8) lanes of a DPP row, in every lane of it
-template <int CTRL> __device__ __forceinline__ double dpp_add(double v) {
-  const long long b = __double_as_longlong(v);
-  const int lo = __builtin_amdgcn_update_dpp(0, int(b), CTRL, 0xf, 0xf, false);
-  const int hi = __builtin_amdgcn_update_dpp(0, int(b >> 32), CTRL, 0xf, 0xf, false);
-  return v + __longlong_as_double((long long)(unsigned(lo)) | ((long long)hi << 32));
-}
-template <int L> __device__ __forceinline__ double lanes_sum(double v) {
-  static_assert(L == 8 || L == 16, "half a DPP row or one");
-  v = dpp_add<0xB1>(v);  // quad_perm 1,0,3,2
-  v = dpp_add<0x4E>(v);  // quad_perm 2,3,0,1
-  v = dpp_add<0x141>(v); // row_half_mirror
-  if constexpr (L == 16) v = dpp_add<0x140>(v); // row_mirror
-  return v;
-}
-
 // The index tables of the Jacobian's blocks
 struct Blocks {
   const int64_t *rowbase;
@@ -114,87 +89,144 @@ struct Blocks {
   int64_t ncell;
 };
 
-// y = (cnp1 I + cf J) x by blocks: L lanes per cell, a lane per M x M block
-// (its M rows of M values and the M values of x they multiply, one column-cell
-// index for all of them), the lanes' sums added by DPP.  The Newton matrix is
-// not formed: cf and cnp1 enter here.  A block of threads takes a contiguous
-// range of cells, and the ranges of one XCD are neighbours, so that x is read
-// into each L2 once; several cells' loads are in flight per lane.  Bound by the
-// matrix: 512 x 512 Burgers (13 2 x 2 blocks a cell, 109 MB of values and 14 MB
-// of indices) 23.8 us (5.2 TB/s), 47.2 us walking the scalar CSR with 32 lanes a row (164 MB).
-// Partial sums of (d1 . y) and, with want_yy, (y . y).
-template <int M> constexpr int spmv_cells() { return M <= 2 ? 4 : M <= 4 ? 2 : 1; } // in flight per lane
+// The iteration's matrix I + B, slot by slot: entry pair h (a value where M is
+// odd) of off-diagonal block e of cell c at ((e PAIRS + h) ncell + c) V, and the
+// block's column cell at e ncell + c.  Rows with fewer blocks than the widest
+// have zero blocks on their own cell.
+template <int M> struct Ell {
+  static constexpr int V = M % 2 == 0 ? 2 : 1, PAIRS = M * M / V;
+};
 
-template <int M, int L>
-__global__ void __launch_bounds__(TB) k_spmv(Blocks K, const double *__restrict__ J, const double *__restrict__ x,
+// the column cells of the off-diagonal blocks, lane per cell
+__global__ void __launch_bounds__(TB) k_ell_cols(Blocks K, int M, int32_t *__restrict__ col) {
+  const int64_t c = int64_t(blockIdx.x) * TB + threadIdx.x;
+  if (c >= K.ncell) return;
+  const int nb = K.nblk[c], d = int((K.diag[c] - K.rowbase[c]) / M);
+  for (int e = 0; e + 1 < K.maxb; ++e) {
+    const int b = e < d ? e : e + 1;
+    col[e * K.ncell + c] = b < nb ? K.bcol[c * K.maxb + b] : int32_t(c);
+  }
+}
+
+// B's blocks from the Jacobian's and the inverted diagonal blocks: 16 lanes per
+// cell, a lane per block, so that a cell's values are read as they lie; a block
+// of threads writes 16 consecutive cells of every slot.  Bound by the matrix
+// read and written: 512 x 512 Burgers (222 MB) 54 us, repaid within three iterations.
+constexpr int FL = 16;
+template <int M>
+__global__ void __launch_bounds__(TB) k_form(Blocks K, const double *__restrict__ J, double cf,
+                                             const double *__restrict__ Minv, double *__restrict__ A) {
+  constexpr int V = Ell<M>::V, PAIRS = Ell<M>::PAIRS;
+  const int64_t c = (int64_t(blockIdx.x) * TB + threadIdx.x) / FL;
+  if (c >= K.ncell) return;
+  const int nb = K.nblk[c];
+  const int64_t rb = K.rowbase[c];
+  const int d = int((K.diag[c] - rb) / M);
+  for (int e = threadIdx.x % FL; e + 1 < K.maxb; e += FL) {
+    const int b = e < d ? e : e + 1;
+    double o[M * M];
+#pragma unroll
+    for (int k = 0; k < M * M; ++k) o[k] = 0.;
+    if (b < nb) {
+      const double *Jr = J + rb + b * M;
+      const double *Mi = Minv + int64_t(K.bcol[c * K.maxb + b]) * M * M;
+#pragma unroll
+      for (int k = 0; k < M; ++k) {
+        double a[M];
+#pragma unroll
+        for (int j = 0; j < M; ++j) a[j] = cf * Jr[int64_t(k) * nb * M + j];
+#pragma unroll
+        for (int j = 0; j < M; ++j)
+#pragma unroll
+          for (int i = 0; i < M; ++i) o[k * M + j] += a[i] * Mi[i * M + j];
+      }
+    }
+#pragma unroll
+    for (int h = 0; h < PAIRS; ++h)
+#pragma unroll
+      for (int v = 0; v < V; ++v) A[((int64_t(e) * PAIRS + h) * K.ncell + c) * V + v] = o[h * V + v];
+  }
+}
+
+// y = (I + B) x, a lane per cell: every load of the matrix, its columns and
+// (but for the grid's edges) of x is one contiguous run of the wave, all of a
+// cell's loads are in flight together and no sum crosses lanes.  A block of
+// threads takes a contiguous range of cells, and the ranges of one XCD are
+// neighbours, so that x is read into each L2 once.  SECOND: alpha = rho /
+// (r0 . v) from its partial sums, and x = r - alpha v is formed as it is
+// gathered, for 50 MB more from L2 but without a launch and a vector for it.
+// Bound by the matrix, which stays in the last-level cache: 512 x 512 Burgers
+// (12 2 x 2 blocks a cell, 113 MB with their columns) 17.1 us (7.3 TB/s) and
+// 19.3 SECOND; 16 lanes per cell over the Jacobian's own CSR blocks 23.8, with
+// 14.4 us of launches that applied Minv beside each product.
+// Partial sums of (r0 . y), or with SECOND of (y . x, y . y).
+template <int M, bool SECOND>
+__global__ void __launch_bounds__(TB) k_spmv(const double *__restrict__ A, const int32_t *__restrict__ col,
+                                             int slots, int64_t ncell, const double *__restrict__ x,
+                                             const double *__restrict__ xv, const double *__restrict__ r0,
                                              double *__restrict__ y, int64_t per_block,
-                                             const double *__restrict__ d1, int want_yy, double *__restrict__ part,
-                                             const double *__restrict__ scal) {
+                                             const double *__restrict__ part_in, int npart,
+                                             double *__restrict__ part, double *__restrict__ scal) {
   __shared__ double sh[TB / 64];
-  constexpr int CPB = TB / L, NU = spmv_cells<M>();
-  if (scal[S_DONE_NEXT] != 0.) return;
-  const double cf = scal[S_CF], cnp1 = scal[S_CNP1];
-  const int l = threadIdx.x % L, g = threadIdx.x / L;
+  constexpr int V = Ell<M>::V, PAIRS = Ell<M>::PAIRS;
+  double alpha = 0.;
+  if constexpr (SECOND) {
+    const double dn = scal[S_DONE_NEXT], rho = scal[S_RHO_NEXT];
+    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
+    if (dn != 0.) {
+      if (lead) scal[S_DONE] = 1.;
+      return;
+    }
+    double s1, s2;
+    sum_pairs(part_in, npart, sh, s1, s2);
+    alpha = rho / s1;
+    if (lead) {
+      scal[S_RHO] = rho;
+      scal[S_ALPHA] = alpha;
+    }
+  } else if (scal[S_DONE_NEXT] != 0.) {
+    return;
+  }
   // block -> range: the blocks of XCD b % 8 take neighbouring ranges
   const int nbk = gridDim.x, q = nbk / 8, rem = nbk % 8, xcd = int(blockIdx.x) % 8, kk = int(blockIdx.x) / 8;
   const int64_t range = int64_t(xcd) * q + (xcd < rem ? xcd : rem) + kk;
-  const int64_t c_lo = range * per_block, c_hi = c_lo + per_block < K.ncell ? c_lo + per_block : K.ncell;
+  const int64_t c_lo = range * per_block, c_hi = c_lo + per_block < ncell ? c_lo + per_block : ncell;
   double s1 = 0., s2 = 0.;
-  for (int64_t base = c_lo; base < c_hi; base += CPB * NU) {
-    double acc[NU][M];
-    int64_t cell[NU], rb[NU];
-    int nb[NU];
+  for (int64_t c = c_lo + threadIdx.x; c < c_hi; c += TB) {
+    double acc[M], own[M];
 #pragma unroll
-    for (int u = 0; u < NU; ++u) {
-      const int64_t c = base + u * CPB + g;
-      cell[u] = c < c_hi ? c : c_hi - 1;
-      nb[u] = c < c_hi ? K.nblk[cell[u]] : 0;
-      rb[u] = K.rowbase[cell[u]];
-#pragma unroll
-      for (int k = 0; k < M; ++k) acc[u][k] = 0.;
+    for (int k = 0; k < M; ++k) {
+      own[k] = x[c * M + k];
+      if constexpr (SECOND) own[k] -= alpha * xv[c * M + k];
+      acc[k] = own[k];
     }
-    for (int s0 = 0; s0 < K.maxb; s0 += L) {
-      const int s = s0 + l;
-      double a[NU][M * M], v[NU][M];
+#pragma unroll 4
+    for (int e = 0; e < slots; ++e) {
+      const int64_t j = int64_t(col[e * ncell + c]) * M;
+      const double *a = A + (int64_t(e) * PAIRS * ncell + c) * V;
+      double u[M], b[M * M];
 #pragma unroll
-      for (int u = 0; u < NU; ++u) {
-        const bool on = s < nb[u];
-        const int ss = on ? s : 0;
-        const double *xc = x + int64_t(K.bcol[cell[u] * K.maxb + ss]) * M;
-        const double *Jr = J + rb[u] + ss * M;
+      for (int h = 0; h < PAIRS; ++h)
 #pragma unroll
-        for (int k = 0; k < M; ++k)
-#pragma unroll
-          for (int j = 0; j < M; ++j) a[u][k * M + j] = Jr[int64_t(k) * nb[u] * M + j];
-#pragma unroll
-        for (int j = 0; j < M; ++j) v[u][j] = on ? xc[j] : 0.;
-      }
-#pragma unroll
-      for (int u = 0; u < NU; ++u) {
-        const bool on = s < nb[u];
-#pragma unroll
-        for (int k = 0; k < M; ++k) {
-          double t = 0.;
-#pragma unroll
-          for (int j = 0; j < M; ++j) t += a[u][k * M + j] * v[u][j];
-          acc[u][k] += on ? t : 0.;
-        }
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < NU; ++u) {
-      double mine = 0.;
+        for (int v = 0; v < V; ++v) b[h * V + v] = a[h * ncell * V + v];
 #pragma unroll
       for (int k = 0; k < M; ++k) {
-        const double t = lanes_sum<L>(acc[u][k]);
-        if (l == k) mine = t;
+        u[k] = x[j + k];
+        if constexpr (SECOND) u[k] -= alpha * xv[j + k];
       }
-      if (l < M && base + u * CPB + g < c_hi) {
-        const int64_t i = cell[u] * M + l;
-        const double yi = cf * mine + cnp1 * x[i];
-        y[i] = yi;
-        s1 += d1[i] * yi;
-        if (want_yy) s2 += yi * yi;
+#pragma unroll
+      for (int k = 0; k < M; ++k)
+#pragma unroll
+        for (int i = 0; i < M; ++i) acc[k] += b[k * M + i] * u[i];
+    }
+#pragma unroll
+    for (int k = 0; k < M; ++k) {
+      y[c * M + k] = acc[k];
+      if constexpr (SECOND) {
+        s1 += acc[k] * own[k];
+        s2 += acc[k] * acc[k];
+      } else {
+        s1 += r0[c * M + k] * acc[k];
       }
     }
   }
@@ -256,10 +288,10 @@ __global__ void __launch_bounds__(TB) k_block_inv(Blocks K, const double *__rest
 }
 
 // start of a solve: x = 0, r = r0 = -R; partial sums of r0 . r twice (r0 . r
-// and r . r); the matrix's coefficients and cleared flags for the iterations
+// and r . r); cleared flags for the iterations
 __global__ void __launch_bounds__(TB) k_start(const double *__restrict__ R, double *__restrict__ x,
-                                              double *__restrict__ r, double *__restrict__ r0, int64_t n, double cf,
-                                              double cnp1, double *__restrict__ part, double *__restrict__ scal) {
+                                              double *__restrict__ r, double *__restrict__ r0, int64_t n,
+                                              double *__restrict__ part, double *__restrict__ scal) {
   __shared__ double sh[TB / 64];
   double s = 0.;
   for (int64_t i = int64_t(blockIdx.x) * TB + threadIdx.x; i < n; i += int64_t(gridDim.x) * TB) {
@@ -277,8 +309,6 @@ __global__ void __launch_bounds__(TB) k_start(const double *__restrict__ R, doub
     scal[S_NITER] = 0.;
     scal[S_DONE] = 0.;
     scal[S_DONE_NEXT] = 0.;
-    scal[S_CF] = cf;
-    scal[S_CNP1] = cnp1;
   }
 }
 
@@ -291,13 +321,11 @@ __device__ __forceinline__ bool ends(double s1, double s2, double tol2) {
 
 // The search direction: beta from the partial sums of (r0 . r, r . r), or, in
 // the first iteration, the tolerance from those of b . b;
-// p = r + beta (p - w v), y = Minv p          (per cell)
-template <int M>
-__global__ void __launch_bounds__(TB) k_p_prec(const double *__restrict__ r, double *__restrict__ p,
-                                                const double *__restrict__ v, const double *__restrict__ Minv,
-                                                double *__restrict__ y, int64_t ncell,
-                                                const double *__restrict__ part, int npart, double *__restrict__ scal,
-                                                int first, double rtol) {
+// p = r + beta (p - w v)
+__global__ void __launch_bounds__(TB) k_p(const double *__restrict__ r, double *__restrict__ p,
+                                           const double *__restrict__ v, int64_t n,
+                                           const double *__restrict__ part, int npart, double *__restrict__ scal,
+                                           int first, double rtol) {
   __shared__ double sh[TB / 64];
   if (scal[S_DONE] != 0.) return; // written by earlier kernels: the same in every block
   const double alpha = scal[S_ALPHA], w = scal[S_W], rho = scal[S_RHO];
@@ -316,69 +344,15 @@ __global__ void __launch_bounds__(TB) k_p_prec(const double *__restrict__ r, dou
   }
   if (done) return;
   const double beta = (s1 / rho) * (alpha / w);
-  const int64_t c = int64_t(blockIdx.x) * TB + threadIdx.x;
-  if (c >= ncell) return;
-  double pc[M];
-#pragma unroll
-  for (int k = 0; k < M; ++k) {
-    const int64_t i = c * M + k;
-    pc[k] = first ? r[i] : r[i] + beta * (p[i] - w * v[i]);
-    p[i] = pc[k];
-  }
-#pragma unroll
-  for (int k = 0; k < M; ++k) {
-    double s = 0.;
-#pragma unroll
-    for (int j = 0; j < M; ++j) s += Minv[(c * M + k) * M + j] * pc[j];
-    y[c * M + k] = s;
-  }
+  for (int64_t i = int64_t(blockIdx.x) * TB + threadIdx.x; i < n; i += int64_t(gridDim.x) * TB)
+    p[i] = first ? r[i] : r[i] + beta * (p[i] - w * v[i]);
 }
 
-// alpha = rho / (r0 . v) from its partial sums; s = r - alpha v; z = Minv s
-template <int M>
-__global__ void __launch_bounds__(TB) k_s_prec(const double *__restrict__ r, const double *__restrict__ v,
-                                                const double *__restrict__ Minv, double *__restrict__ s,
-                                                double *__restrict__ z, int64_t ncell,
-                                                const double *__restrict__ part, int npart,
-                                                double *__restrict__ scal) {
-  __shared__ double sh[TB / 64];
-  const double dn = scal[S_DONE_NEXT], rho = scal[S_RHO_NEXT];
-  const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
-  if (dn != 0.) {
-    if (lead) scal[S_DONE] = 1.;
-    return;
-  }
-  double s1, s2;
-  sum_pairs(part, npart, sh, s1, s2);
-  const double alpha = rho / s1;
-  if (lead) {
-    scal[S_RHO] = rho;
-    scal[S_ALPHA] = alpha;
-  }
-  const int64_t c = int64_t(blockIdx.x) * TB + threadIdx.x;
-  if (c >= ncell) return;
-  double sc[M];
-#pragma unroll
-  for (int k = 0; k < M; ++k) {
-    const int64_t i = c * M + k;
-    sc[k] = r[i] - alpha * v[i];
-    s[i] = sc[k];
-  }
-#pragma unroll
-  for (int k = 0; k < M; ++k) {
-    double t = 0.;
-#pragma unroll
-    for (int j = 0; j < M; ++j) t += Minv[(c * M + k) * M + j] * sc[j];
-    z[c * M + k] = t;
-  }
-}
-
-// w = (t . s) / (t . t) from their partial sums; x += alpha y + w z;
-// r = s - w t; partial sums of (r0 . r, r . r)
+// w = (t . s) / (t . t) from their partial sums; s = r - alpha v;
+// x += alpha p + w s; r = s - w t; partial sums of (r0 . r, r . r)
 __global__ void __launch_bounds__(TB) k_xr(double *__restrict__ x, double *__restrict__ r,
-                                            const double *__restrict__ y, const double *__restrict__ z,
-                                            const double *__restrict__ s, const double *__restrict__ t,
-                                            const double *__restrict__ r0, int64_t n,
+                                            const double *__restrict__ p, const double *__restrict__ v,
+                                            const double *__restrict__ t, const double *__restrict__ r0, int64_t n,
                                             const double *__restrict__ part_in, int npart,
                                             double *__restrict__ part, double *__restrict__ scal) {
   __shared__ double sh[TB / 64];
@@ -393,8 +367,9 @@ __global__ void __launch_bounds__(TB) k_xr(double *__restrict__ x, double *__res
   }
   double s1 = 0., s2 = 0.;
   for (int64_t i = int64_t(blockIdx.x) * TB + threadIdx.x; i < n; i += int64_t(gridDim.x) * TB) {
-    x[i] += alpha * y[i] + w * z[i];
-    const double ri = s[i] - w * t[i];
+    const double si = r[i] - alpha * v[i];
+    x[i] += alpha * p[i] + w * si;
+    const double ri = si - w * t[i];
     r[i] = ri;
     s1 += r0[i] * ri;
     s2 += ri * ri;
@@ -435,17 +410,32 @@ __global__ void __launch_bounds__(TB) k_residual(double *__restrict__ R, const d
   put_pair(part, s, 0., sh);
 }
 
-// Y += dx, with partial sums of dx . dx
-__global__ void __launch_bounds__(TB) k_correct(double *__restrict__ Y, const double *__restrict__ dx, int64_t n,
+// dx = Minv x, the correction from the preconditioned unknowns, with partial
+// sums of dx . dx; Y += dx where Y is given
+template <int M>
+__global__ void __launch_bounds__(TB) k_unscale(const double *__restrict__ Minv, const double *__restrict__ x,
+                                                double *__restrict__ dx, double *__restrict__ Y, int64_t ncell,
                                                 double *__restrict__ part) {
   __shared__ double sh[TB / 64];
   double s = 0.;
-  for (int64_t i = int64_t(blockIdx.x) * TB + threadIdx.x; i < n; i += int64_t(gridDim.x) * TB) {
-    const double d = dx[i];
-    Y[i] += d;
-    s += d * d;
+  for (int64_t c = int64_t(blockIdx.x) * TB + threadIdx.x; c < ncell; c += int64_t(gridDim.x) * TB) {
+#pragma unroll
+    for (int k = 0; k < M; ++k) {
+      double d = 0.;
+#pragma unroll
+      for (int j = 0; j < M; ++j) d += Minv[(c * M + k) * M + j] * x[c * M + j];
+      dx[c * M + k] = d;
+      if (Y) Y[c * M + k] += d;
+      s += d * d;
+    }
   }
   put_pair(part, s, 0., sh);
+}
+
+// Y += dx
+__global__ void __launch_bounds__(TB) k_correct(double *__restrict__ Y, const double *__restrict__ dx, int64_t n) {
+  const int64_t i = int64_t(blockIdx.x) * TB + threadIdx.x;
+  if (i < n) Y[i] += dx[i];
 }
 
 unsigned grid_of(int64_t n) { return unsigned(std::max<int64_t>(1, (n + TB - 1) / TB)); }
@@ -464,7 +454,8 @@ struct pda_implicit_s {
   double lin_rtol = 1e-14;
   int lin_max = 0;          // 0: 2 * unknowns (Eigen's default)
   int check_every = 4;      // iterations of the recorded graph
-  pda::DevBuf J, F, Fn, R, Y, Yn, dx, r, r0, p, v, s, t, y, z, Minv, scal;
+  pda::DevBuf J, F, Fn, R, Y, Yn, dx, x, r, r0, p, v, t, Minv, scal;
+  pda::DevBuf ell, ellcol;  // the iteration's matrix and its column cells
   pda::DevBuf part[5];      // partial sums: r0.v, (t.s, t.t), (r0.r, r.r), R.R, dx.dx
   pda::DevBuf diag;         // first value of every cell's diagonal block
   double *host = nullptr;   // pinned: what the host reads after a synchronization
@@ -501,57 +492,42 @@ Blocks blocks_of(const pda_implicit_s &ip) {
   return K;
 }
 
-// y = (cnp1 I + cf J) x; returns the number of partial sums
-template <int M, int L>
-int spmv_l(const pda_implicit_s &ip, const double *x, double *y, const double *d1, int want_yy, double *part,
-           hipStream_t st) {
-  // cells of a block: whole passes of the lanes, at most MAXB blocks
-  constexpr int64_t pass = (TB / L) * spmv_cells<M>();
-  const int64_t per = ((ip.ncell + MAXB - 1) / MAXB + pass - 1) / pass * pass;
-  const unsigned g = unsigned((ip.ncell + per - 1) / per);
-  hipLaunchKernelGGL((k_spmv<M, L>), dim3(g), dim3(TB), 0, st, blocks_of(ip), ip.J.as<double>(), x, y, per, d1,
-                     want_yy, part, ip.scal.as<double>());
-  return int(g);
-}
-template <int M>
-int spmv(const pda_implicit_s &ip, const double *x, double *y, const double *d1, int want_yy, double *part,
-         hipStream_t st) {
-  return ip.prob->maxb <= 8 ? spmv_l<M, 8>(ip, x, y, d1, want_yy, part, st)
-                            : spmv_l<M, 16>(ip, x, y, d1, want_yy, part, st);
-}
-
-// one BiCGSTAB iteration (preconditioned right: y = M^-1 p, z = M^-1 s);
-// every kernel is a no-op once the convergence flag is set
-template <int M>
-void bicgstab_iteration(pda_implicit_s &ip, hipStream_t st, bool first, double rtol) {
+// one BiCGSTAB iteration; every kernel is a no-op once the convergence flag is set
+template <int M> void bicgstab_iteration(pda_implicit_s &ip, hipStream_t st, bool first, double rtol) {
   const int64_t n = ip.n, nc = ip.ncell;
+  const int slots = ip.prob->maxb - 1;
   double *r = ip.r.as<double>(), *r0 = ip.r0.as<double>(), *pp = ip.p.as<double>();
-  double *v = ip.v.as<double>(), *s = ip.s.as<double>(), *t = ip.t.as<double>();
-  double *y = ip.y.as<double>(), *z = ip.z.as<double>(), *Mi = ip.Minv.as<double>();
-  double *scal = ip.scal.as<double>();
+  double *v = ip.v.as<double>(), *t = ip.t.as<double>(), *scal = ip.scal.as<double>();
+  const double *A = ip.ell.as<double>();
+  const int32_t *col = ip.ellcol.as<int32_t>();
   double *pr0v = ip.part[P_R0V].as<double>(), *pts = ip.part[P_TS].as<double>(), *prr = ip.part[P_RR].as<double>();
-  const unsigned gv = grid_strided(n), gc = grid_of(nc);
-  hipLaunchKernelGGL((k_p_prec<M>), dim3(gc), dim3(TB), 0, st, r, pp, v, Mi, y, nc, prr, int(gv), scal,
-                     first ? 1 : 0, rtol);
-  int ns = spmv<M>(ip, y, v, r0, 0, pr0v, st);
-  hipLaunchKernelGGL((k_s_prec<M>), dim3(gc), dim3(TB), 0, st, r, v, Mi, s, z, nc, pr0v, ns, scal);
-  ns = spmv<M>(ip, z, t, s, 1, pts, st);
-  hipLaunchKernelGGL(k_xr, dim3(gv), dim3(TB), 0, st, ip.dx.as<double>(), r, y, z, s, t, r0, n, pts, ns, prr, scal);
+  const unsigned gv = grid_strided(n);
+  // cells of a block of the products: whole passes of its lanes, at most MAXB blocks
+  const int64_t per = ((nc + MAXB - 1) / MAXB + TB - 1) / TB * TB;
+  const unsigned gs = unsigned((nc + per - 1) / per);
+  hipLaunchKernelGGL(k_p, dim3(gv), dim3(TB), 0, st, r, pp, v, n, prr, int(gv), scal, first ? 1 : 0, rtol);
+  hipLaunchKernelGGL((k_spmv<M, false>), dim3(gs), dim3(TB), 0, st, A, col, slots, nc, pp, nullptr, r0, v, per,
+                     nullptr, 0, pr0v, scal);
+  hipLaunchKernelGGL((k_spmv<M, true>), dim3(gs), dim3(TB), 0, st, A, col, slots, nc, r, v, nullptr, t, per, pr0v,
+                     int(gs), pts, scal);
+  hipLaunchKernelGGL(k_xr, dim3(gv), dim3(TB), 0, st, ip.x.as<double>(), r, pp, v, t, r0, n, pts, int(gs), prr, scal);
 }
 
-// (cnp1 I + cf J) dx = -R.  newton: index of the Newton iteration, whose
+// (cnp1 I + cf J) dx = -R, Y += dx where Y is given, partial sums of dx . dx.  newton: index of the Newton iteration, whose
 // linear iterations in the step before decide how many run before the first
 // poll (the kernels stop by themselves at convergence, so this moves no value)
 template <int M>
-int bicgstab_m(pda_implicit_s &ip, double cf, double cnp1, hipStream_t st, double rtol, int newton, int *iters,
-               double *rel_res) {
+int bicgstab_m(pda_implicit_s &ip, double cf, double cnp1, double *Y, hipStream_t st, double rtol, int newton,
+               int *iters, double *rel_res) {
   const int64_t n = ip.n, nc = ip.ncell;
   double *prr = ip.part[P_RR].as<double>(), *scal = ip.scal.as<double>(), *h = ip.host;
   const unsigned gv = grid_strided(n), gc = grid_of(nc);
   hipLaunchKernelGGL((k_block_inv<M>), dim3(gc), dim3(TB), 0, st, blocks_of(ip), ip.J.as<double>(), cf, cnp1,
                      ip.Minv.as<double>());
-  hipLaunchKernelGGL(k_start, dim3(gv), dim3(TB), 0, st, ip.R.as<double>(), ip.dx.as<double>(), ip.r.as<double>(),
-                     ip.r0.as<double>(), n, cf, cnp1, prr, scal);
+  hipLaunchKernelGGL((k_form<M>), dim3(grid_of(nc * FL)), dim3(TB), 0, st, blocks_of(ip), ip.J.as<double>(), cf,
+                     ip.Minv.as<double>(), ip.ell.as<double>());
+  hipLaunchKernelGGL(k_start, dim3(gv), dim3(TB), 0, st, ip.R.as<double>(), ip.x.as<double>(), ip.r.as<double>(),
+                     ip.r0.as<double>(), n, prr, scal);
   PDA_HIP_CHECK(hipGetLastError());
   const int64_t maxit = ip.lin_max > 0 ? ip.lin_max : 2 * n;
   const int K = ip.check_every, slot = newton < 8 ? newton : 7;
@@ -598,6 +574,9 @@ int bicgstab_m(pda_implicit_s &ip, double cf, double cnp1, hipStream_t st, doubl
     PDA_HIP_CHECK(hipStreamSynchronize(st));
     done = h[H_DONE] != 0. || it >= maxit;
   }
+  hipLaunchKernelGGL((k_unscale<M>), dim3(gv), dim3(TB), 0, st, ip.Minv.as<double>(),
+                     ip.x.as<double>(), ip.dx.as<double>(), Y, nc, ip.part[P_DX].as<double>());
+  PDA_HIP_CHECK(hipGetLastError());
   *iters = int(h[H_NITER]) + (h[H_DONE] == 0. ? 1 : 0); // at the limit the unmet check counts too
   *rel_res = h[H_BB] > 0. ? std::sqrt(h[H_RR] / h[H_BB]) : 0.;
   ip.guess_iters[slot] = *iters;
@@ -606,14 +585,14 @@ int bicgstab_m(pda_implicit_s &ip, double cf, double cnp1, hipStream_t st, doubl
   return PDA_OK;
 }
 
-int bicgstab(pda_implicit_s &ip, double cf, double cnp1, hipStream_t st, double rtol, int newton, int *iters,
-             double *rel) {
+int bicgstab(pda_implicit_s &ip, double cf, double cnp1, double *Y, hipStream_t st, double rtol, int newton,
+             int *iters, double *rel) {
   switch (ip.prob->m) {
-    case 1: return bicgstab_m<1>(ip, cf, cnp1, st, rtol, newton, iters, rel);
-    case 2: return bicgstab_m<2>(ip, cf, cnp1, st, rtol, newton, iters, rel);
-    case 3: return bicgstab_m<3>(ip, cf, cnp1, st, rtol, newton, iters, rel);
-    case 4: return bicgstab_m<4>(ip, cf, cnp1, st, rtol, newton, iters, rel);
-    case 5: return bicgstab_m<5>(ip, cf, cnp1, st, rtol, newton, iters, rel);
+    case 1: return bicgstab_m<1>(ip, cf, cnp1, Y, st, rtol, newton, iters, rel);
+    case 2: return bicgstab_m<2>(ip, cf, cnp1, Y, st, rtol, newton, iters, rel);
+    case 3: return bicgstab_m<3>(ip, cf, cnp1, Y, st, rtol, newton, iters, rel);
+    case 4: return bicgstab_m<4>(ip, cf, cnp1, Y, st, rtol, newton, iters, rel);
+    case 5: return bicgstab_m<5>(ip, cf, cnp1, Y, st, rtol, newton, iters, rel);
   }
   set_error("implicit: unsupported block size");
   return PDA_E_UNSUPPORTED;
@@ -645,11 +624,14 @@ int pda_implicit_create(pda_problem p, int scheme, pda_implicit *out) {
   ip->ncell = p->mesh->n_stencil;
   const size_t vb = sizeof(double) * size_t(ip->n);
   hipError_t e = ip->J.alloc(sizeof(double) * size_t(p->nnz));
-  pda::DevBuf *vecs[] = {&ip->F, &ip->Fn, &ip->R, &ip->Y, &ip->Yn, &ip->dx, &ip->r, &ip->r0,
-                         &ip->p, &ip->v, &ip->s, &ip->t, &ip->y, &ip->z};
+  pda::DevBuf *vecs[] = {&ip->F, &ip->Fn, &ip->R, &ip->Y, &ip->Yn, &ip->dx, &ip->x, &ip->r, &ip->r0,
+                         &ip->p, &ip->v, &ip->t};
   for (auto *d : vecs)
     if (e == hipSuccess) e = d->alloc(vb);
   if (e == hipSuccess) e = ip->Minv.alloc(sizeof(double) * size_t(ip->ncell) * p->m * p->m);
+  const size_t blocks = size_t(ip->ncell) * size_t(std::max(1, p->maxb - 1));
+  if (e == hipSuccess) e = ip->ell.alloc(sizeof(double) * blocks * p->m * p->m);
+  if (e == hipSuccess) e = ip->ellcol.alloc(sizeof(int32_t) * blocks);
   for (auto &d : ip->part)
     if (e == hipSuccess) e = d.alloc(sizeof(double) * 2 * pda::MAXB);
   if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void **>(&ip->host), sizeof(double) * 8, hipHostMallocDefault);
@@ -666,6 +648,12 @@ int pda_implicit_create(pda_problem p, int scheme, pda_implicit *out) {
         return PDA_E_STATE;
       }
     e = ip->diag.upload(dg);
+    if (e == hipSuccess) {
+      hipLaunchKernelGGL(k_ell_cols, dim3(grid_of(ip->ncell)), dim3(TB), 0, nullptr, blocks_of(*ip), p->m,
+                         ip->ellcol.as<int32_t>());
+      e = hipGetLastError();
+    }
+    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
   }
   if (e == hipSuccess) e = ip->scal.alloc(sizeof(double) * pda::S_COUNT);
   if (e != hipSuccess) {
@@ -709,7 +697,7 @@ int pda_implicit_step(pda_implicit ip, double *d_U, const double *d_Uprev, const
     return PDA_E_STATE;
   }
   double *J = ip->J.as<double>(), *F = ip->F.as<double>(), *R = ip->R.as<double>();
-  double *Y = ip->Y.as<double>(), *Yn = ip->Yn.as<double>(), *dx = ip->dx.as<double>();
+  double *Y = ip->Y.as<double>(), *Yn = ip->Yn.as<double>();
   double *Fn = ip->Fn.as<double>();
   const unsigned gs = grid_strided(n);
   // residual coefficients R = cnp1 y + cn y_n + cnm1 y_{n-1} + cf f(y) [+ cfn f(y_n)]
@@ -789,17 +777,16 @@ int pda_implicit_step(pda_implicit ip, double *d_U, const double *d_Uprev, const
     // BiCGSTAB runs to machine precision)
     double rtol = ip->lin_rtol;
     if (by_residual && rnorm > 0.) rtol = std::min(0.1, std::max(ip->lin_rtol, 0.1 * ip->tol / rnorm));
-    rc = bicgstab(*ip, cf, cnp1, st, rtol, it, &li, &lr);
+    // by residual the correction is applied with its norm's partial sums
+    rc = bicgstab(*ip, cf, cnp1, by_residual ? Y : nullptr, st, rtol, it, &li, &lr);
     if (rc) return rc;
     S.linear_iters += li;
     S.last_linear_rel_residual = lr;
     S.newton_iters = it + 1;
     const bool more = it + 1 < ip->max_newton;
     if (by_residual) {
-      // the correction, the next residual and both norms in one go: a
-      // non-finite correction is found before d_U is written
-      hipLaunchKernelGGL(k_correct, dim3(gs), dim3(TB), 0, st, Y, dx, n, pdx);
-      PDA_HIP_CHECK(hipGetLastError());
+      // the next residual and both norms in one go: a non-finite correction
+      // is found before d_U is written
       if (more) rc = evaluate();
       if (!rc) rc = norms(pdx, more ? pres : nullptr);
       if (rc) return rc;
@@ -807,8 +794,6 @@ int pda_implicit_step(pda_implicit ip, double *d_U, const double *d_Uprev, const
       if (!std::isfinite(S.correction_norm)) return fail("Newton correction is not finite");
       if (more) rnorm = h[1];
     } else {
-      hipLaunchKernelGGL(k_norm, dim3(gs), dim3(TB), 0, st, dx, n, pdx);
-      PDA_HIP_CHECK(hipGetLastError());
       rc = norms(pdx, nullptr);
       if (rc) return rc;
       S.correction_norm = h[0];
@@ -817,7 +802,7 @@ int pda_implicit_step(pda_implicit ip, double *d_U, const double *d_Uprev, const
         S.converged = 1;
         break;
       }
-      hipLaunchKernelGGL(k_correct, dim3(gs), dim3(TB), 0, st, Y, dx, n, pdx);
+      hipLaunchKernelGGL(k_correct, dim3(grid_of(n)), dim3(TB), 0, st, Y, ip->dx.as<double>(), n);
       PDA_HIP_CHECK(hipGetLastError());
       if (!more) break;
       rc = evaluate();

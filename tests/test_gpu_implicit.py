@@ -151,3 +151,33 @@ def test_nonfinite_state_leaves_yn(stop, torch):
     torch.cuda.synchronize()
     assert torch.equal(torch.isnan(U), torch.isnan(U0))
     assert torch.equal(torch.nan_to_num(U), torch.nan_to_num(U0))
+
+
+@pytest.mark.parametrize("enum,n,bounds,ic,st", [
+    (pda.Euler3d.SedovSymmetry, (9, 8, 7), (0.0, 1.2) * 3, None, 3),  # five values a cell, rows of 4 to 7 blocks
+    (pda.Swe2d.SlipWall, (33, 31), (-5.0, 5.0) * 2, 1, 5),            # three
+    (pda.AdvectionDiffusion2d.BurgersPeriodic, (5, 5), (-1.0, 1.0) * 2, 1, 5),      # stencils as wide as the grid
+    (pda.AdvectionDiffusion2d.BurgersPeriodic, (601, 437), (-1.0, 1.0) * 2, 1, 3),  # several cells a lane
+])
+def test_linear_solve_over_block_sizes_and_grids(enum, n, bounds, ic, st, torch):
+    """One BDF1 step to ||R|| <= 1e-9: Newton on the exact Jacobian meets it in
+    a few iterations only if every linear solve does, and the returned state's
+    residual, formed here from rightHandSide, is within it (twice, for the
+    rounding of the sums)."""
+    print(f"[gpu-implicit] linear solve {enum} {n}", flush=True)
+    mesh = pda.create_structured_mesh(n, bounds, st, True if enum == pda.AdvectionDiffusion2d.BurgersPeriodic else ())
+    scheme = {3: S.FirstOrder, 5: S.Weno3}[st]
+    args = (mesh, enum, scheme) if ic is None else (mesh, enum, scheme, ic)
+    prob = pda.create_problem(*args)
+    dt = 2e-3
+    ip = pda.ImplicitStepper(prob, pda.ImplicitScheme.BDF1)
+    ip.set_options(pda.StopRule.Residual, 1e-9, 12, 1e-12, 0)
+    yn = prob.initialCondition()
+    U = yn.clone()
+    stats = ip.step(U, 0.0, dt)
+    V = prob.createRightHandSide()
+    prob.rightHandSide(U, dt, V)
+    r = float(torch.linalg.vector_norm(U - yn - dt * V))
+    print(f"[gpu-implicit] newton {stats['newton_iters']} linear {stats['linear_iters']} residual {r:.1e}", flush=True)
+    assert stats["newton_iters"] <= 8 and not torch.equal(U, yn)
+    assert r <= 2e-9
