@@ -29,134 +29,6 @@ __device__ __forceinline__ int64_t xcd_contiguous(int64_t b, int64_t n) {
   return x * q + (x < r ? x : r) + k;
 }
 
-// ------------------------------------------------ velocity 2D, row marching
-// A wavefront owns a segment of up to 63 consecutive box cells of a grid row
-// and marches up a strip of rows.  Lane l evaluates the x face on the left
-// of cell l (lane 63 the face on the right of cell 62) and the y face above
-// cell l; the x face on the right comes from lane l+1 by a lane shuffle and
-// the y face below is the one evaluated for the previous row, carried in
-// registers.  Every face is reconstructed once (plus one row of y faces per
-// strip) and no workgroup barrier is needed.
-constexpr int VSEG = 63;
-
-// state of cell (i, j, k) with the index along axis A possibly outside
-// [0, n): periodic wrap, or the mirror cell times the side's ghost sign (the
-// GHOST_MIRROR rule, whose ghost values do not depend on the reading row)
-template <int M, int A>
-__device__ __forceinline__ void load_cell_mapped(const View &P, const Box &B, const double *__restrict__ U,
-                                                 int64_t i, int64_t j, int64_t k, double *q) {
-  int64_t c = A == 0 ? i : (A == 1 ? j : k);
-  const int64_t n = B.n[A];
-  int side = -1;
-  if (c < 0) {
-    if (B.mode[A] == 1) c += n;
-    else { c = -1 - c; side = 0; }
-  } else if (c >= n) {
-    if (B.mode[A] == 1) c -= n;
-    else { c = 2 * n - 1 - c; side = 1; }
-  }
-  const int64_t ii = A == 0 ? c : i, jj = A == 1 ? c : j, kk = A == 2 ? c : k;
-  const int64_t cell = (kk * B.n[1] + jj) * B.n[0] + ii;
-#pragma unroll
-  for (int k = 0; k < M; ++k) {
-    const double v = U[cell * M + k];
-    q[k] = side < 0 ? v : P.gsign[A][side][k] * v;
-  }
-}
-
-// flux of the face on the low side (along A) of cell (i, j, k)
-template <class Ph, int W, int A>
-__device__ __forceinline__ void face_flux_fast(const View &P, const Box &B, const double *__restrict__ U,
-                                               int64_t i, int64_t j, int64_t k, double *F) {
-  constexpr int M = Ph::M;
-  double st[2 * W][M];
-#pragma unroll
-  for (int p = 0; p < 2 * W; ++p)
-    load_cell_mapped<M, A>(P, B, U, A == 0 ? i + p - W : i, A == 1 ? j + p - W : j, A == 2 ? k + p - W : k,
-                           st[p]);
-  double qm[M], qp[M];
-#pragma unroll
-  for (int k = 0; k < M; ++k) {
-    double v[2 * W];
-#pragma unroll
-    for (int p = 0; p < 2 * W; ++p) v[p] = st[p][k];
-    if constexpr (W == 1) {
-      qm[k] = v[0];
-      qp[k] = v[1];
-    } else if constexpr (W == 2) {
-      phys::weno3_1div(v, qm[k], qp[k]);
-    } else {
-      phys::weno5_1div(v, qm[k], qp[k]);
-    }
-  }
-  Ph::template flux<A>(P, qm, qp, F);
-}
-
-template <class Ph, int W>
-__device__ __forceinline__ void vel_march_body(const View &P, const Box &B, int rows_per_strip, int64_t bid,
-                                               const double *__restrict__ U, double *__restrict__ V) {
-  constexpr int M = Ph::M;
-  const int lane = threadIdx.x;
-  const int64_t nx = B.n[0], ny = B.n[1];
-  const int64_t bw = B.hi[0] - B.lo[0];
-  const int64_t nseg = (bw + VSEG - 1) / VSEG;
-  const int64_t nstrip = (B.hi[1] - B.lo[1] + rows_per_strip - 1) / rows_per_strip;
-  // workgroup -> (plane, strip, segment); one plane in 2D
-  const int64_t plane = bid / (nseg * nstrip), rem = bid - plane * nseg * nstrip;
-  const int64_t seg = rem % nseg, strip = rem / nseg;
-  const int64_t kz = B.lo[2] + plane;
-  const int64_t iseg = B.lo[0] + seg * VSEG;
-  const int ncell = int(bw - seg * VSEG < VSEG ? bw - seg * VSEG : VSEG);
-  const int64_t j0 = B.lo[1] + strip * rows_per_strip;
-  const int64_t j1 = j0 + rows_per_strip < B.hi[1] ? j0 + rows_per_strip : B.hi[1];
-  // Lane l evaluates the x face on the left of column i = iseg + l; lane
-  // ncell (and the idle lanes after it) the face on the right of the last
-  // cell, i = iseg + ncell <= B.hi[0].  With a full-grid box that column is
-  // n, outside the grid: x stencils there are mapped by the axis mode, and
-  // everything else those lanes compute (y faces, sources; never stored)
-  // uses the last column ic instead.
-  const int64_t i = iseg + (lane <= ncell ? lane : ncell);
-  const int64_t ic = i < nx ? i : nx - 1;
-  const bool own = lane < ncell;
-  const double hx = P.hinv[0], hy = P.hinv[1], hz = P.hinv[2];
-  // one call site per face kind, so that every face value is the same
-  // whatever the strip height (the first pass only evaluates the face below
-  // the strip)
-  double fyb[M];
-  for (int64_t j = j0 - 1; j < j1; ++j) {
-    double fy[M];
-    face_flux_fast<Ph, W, 1>(P, B, U, ic, j + 1, kz, fy);
-    if (j < j0) {
-#pragma unroll
-      for (int k = 0; k < M; ++k) fyb[k] = fy[k];
-      continue;
-    }
-    const int64_t c = (kz * ny + j) * nx + ic;
-    double fx[M], acc[M];
-    face_flux_fast<Ph, W, 0>(P, B, U, i, j, kz, fx);
-#pragma unroll
-    for (int k = 0; k < M; ++k) {
-      const double fr = __shfl_down(fx[k], 1, 64);
-      acc[k] = 0. + hx * (fx[k] - fr);
-      acc[k] += hy * (fyb[k] - fy[k]);
-      fyb[k] = fy[k];
-    }
-    if constexpr (Ph::DIM == 3) {
-      // z faces below and above the cell (no carry across planes)
-      double fzb[M], fza[M];
-      face_flux_fast<Ph, W, 2>(P, B, U, ic, j, kz, fzb);
-      face_flux_fast<Ph, W, 2>(P, B, U, ic, j, kz + 1, fza);
-#pragma unroll
-      for (int k = 0; k < M; ++k) acc[k] += hz * (fzb[k] - fza[k]);
-    }
-    Sources<Ph>::apply(P, c, false, U, int32_t(c), acc, nullptr);
-    if (own) {
-#pragma unroll
-      for (int k = 0; k < M; ++k) V[c * M + k] = acc[k];
-    }
-  }
-}
-
 // ------------------------------------------ velocity 2D, cell-centred march
 // A wavefront holds 64 consecutive columns of a grid row, the 64 - 2W box
 // cells it owns and W columns on each side, and marches up a strip of rows
@@ -168,11 +40,13 @@ __device__ __forceinline__ void vel_march_body(const View &P, const Box &B, int 
 // stencil being the neighbouring lanes' row values (DPP wavefront shifts,
 // no LDS); the face on the high side is lane l + 1's.  The y face above row r takes the high-side
 // value of row r, carried from the previous step, and the low-side value of
-// row r + 1.  Every face value equals the face-by-face march's bit for bit.
+// row r + 1.
 template <int W> __host__ __device__ constexpr int vcc_width() { return 64 - 2 * W; }
 
 // state of cell (i, j) of a 2D grid, each index possibly outside the grid
-// and mapped along its axis as load_cell_mapped maps it
+// and mapped along its axis: periodic wrap, or the mirror cell times the side's
+// ghost sign (the GHOST_MIRROR rule, whose ghost values do not depend on the
+// reading row)
 template <int M>
 __device__ __forceinline__ void load_cell_mapped2(const View &P, const Box &B, const double *__restrict__ U,
                                                   int64_t i, int64_t j, double *q) {
@@ -342,6 +216,186 @@ __device__ __forceinline__ void vel_cc_body(const View &P, const Box &B, int row
   }
 }
 
+// ------------------------------------------ velocity 3D, cell-centred march
+// The 2D march's scheme with z faces added.  The box's x lines, each with one
+// more cell at either end, are laid end to end over the planes, and a wavefront
+// takes 64 consecutive cells of that sequence (the outer two overlap the
+// neighbouring wavefronts'), so that no width of the grid leaves lanes idle
+// but for the line ends.  It marches in y over a strip of rows with the 2W - 1
+// rows a y reconstruction reads in registers; the x and z stencils are loaded
+// (they are in the caches: the neighbouring lanes' and wavefronts' rows).  A
+// cell is reconstructed once per axis; the z faces take one more one-sided
+// value from the cell below and from the cell above, as planes are not carried.
+// Bound by FP64 issue: 1,750 FP64 instructions a row of 62 cells against 5,300
+// evaluating every face's two sides by themselves; WENO5 at 128^3 179 us (244).
+constexpr int V3OWN = 62; // cells a wavefront owns of its 64
+
+// cell index c along axis A, wrapped where the box covers a periodic axis whole
+// (the box keeps every stencil inside the grid otherwise)
+template <int A> __device__ __forceinline__ int wrap_axis(const Box &B, int c) {
+  const int n = int(B.n[A]);
+  if (B.mode[A] != 1) return c;
+  return c < 0 ? c + n : (c >= n ? c - n : c);
+}
+
+// forms x here: neither postponed towards its use nor kept as what it is made of
+__device__ __forceinline__ void pin(double &x) { asm volatile("" : "+v"(x)); }
+
+template <class Ph, int W>
+__device__ __forceinline__ void vel_cc3_body(const View &P, const Box &B, int rows_per_strip, int64_t bid,
+                                             const double *__restrict__ U, double *__restrict__ V) {
+  static_assert(Ph::DIM == 3, "3D march");
+  constexpr int M = Ph::M, NR = 2 * W - 1;
+  const int lane = threadIdx.x;
+  const int nx = int(B.n[0]), ny = int(B.n[1]);
+  const int bw = int(B.hi[0] - B.lo[0]), line = bw + 2;
+  const int64_t ncell = int64_t(line) * (B.hi[2] - B.lo[2]);
+  const int64_t nwave = (ncell - 2 + V3OWN - 1) / V3OWN;
+  const int64_t strip = bid / nwave, wave = bid - strip * nwave;
+  const int j0 = int(B.lo[1] + strip * rows_per_strip);
+  const int j1 = j0 + rows_per_strip < int(B.hi[1]) ? j0 + rows_per_strip : int(B.hi[1]);
+  const int64_t s0 = wave * V3OWN + lane, s = s0 < ncell ? s0 : ncell - 1;
+  const int plane = int(s / line), e = int(s - int64_t(plane) * line);
+  const int i = int(B.lo[0]) + e - 1, kz = int(B.lo[2]) + plane;
+  const bool own = lane >= 1 && lane <= V3OWN && s0 < ncell && e >= 1 && e <= bw;
+  const double hx = P.hinv[0], hy = P.hinv[1], hz = P.hinv[2];
+  // places of the x and z stencils relative to the lane's cell of the row, in cells
+  const int ic = wrap_axis<0>(B, i);
+  int dx[NR];
+  int dz[2 * W + 1];
+#pragma unroll
+  for (int p = 0; p < NR; ++p) dx[p] = wrap_axis<0>(B, i + p - (W - 1)) - ic;
+#pragma unroll
+  for (int p = 0; p <= 2 * W; ++p) dz[p] = (wrap_axis<2>(B, kz + p - W) - kz) * nx * ny;
+  const double *col = U + (int64_t(kz) * nx * ny + ic) * M; // row 0 of the lane's column
+  const int64_t row = int64_t(nx) * M;
+  auto load = [&](const double *u, double (&q)[M]) {
+#pragma unroll
+    for (int k = 0; k < M; ++k) q[k] = u[k];
+  };
+  // win[p] = row r + 2 - W + p at step r (W = 1: row r + 1); nxt = the row
+  // that enters the window at the next step
+  double win[NR][M], nxt[M];
+  auto next_row = [&](int r) { // what step r + 1 shifts in
+    if (r + 1 < j1) load(col + wrap_axis<1>(B, r + 1 + W) * row, nxt);
+  };
+#pragma unroll
+  for (int p = 0; p < NR; ++p) load(col + wrap_axis<1>(B, j0 - W + p) * row, win[p]);
+  double qhi[M], fb[M]; // high-side y value of row r; flux of the face below row r
+  // Neither unrolled nor peeled, as the 2D march's loop.  Two wavefronts a SIMD
+  // leave 256 registers, so the parts of a step (y, x, z) are kept apart: the x
+  // stencil's loads are issued before the y part, the z stencil's before the x
+  // flux and the next row's before the z fluxes (all at once, with the
+  // compiler's order of their uses, spilled 660 bytes: 500 us).
+#pragma clang loop unroll(disable)
+  for (int r = j0 - 2; r < j1; ++r) {
+    if (r > j0 - 2) {
+#pragma unroll
+      for (int p = 0; p + 1 < NR; ++p)
+#pragma unroll
+        for (int k = 0; k < M; ++k) win[p][k] = win[p + 1][k];
+#pragma unroll
+      for (int k = 0; k < M; ++k) win[NR - 1][k] = nxt[k];
+    }
+    const double *at = col + r * row;
+    double xs[NR][M], zs[2 * W + 1][M];
+    if (r < j0) {
+      next_row(r);
+    } else {
+#pragma unroll
+      for (int p = 0; p < NR; ++p)
+        if (p != W - 1) load(at + int64_t(dx[p]) * M, xs[p]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    double yhi[M], ylo[M]; // y face values of cell (i, r + 1)
+#pragma unroll
+    for (int k = 0; k < M; ++k) {
+      double c[NR];
+#pragma unroll
+      for (int p = 0; p < NR; ++p) c[p] = win[p][k];
+      recon_cell<W>(c, yhi[k], ylo[k]);
+      pin(yhi[k]);
+      pin(ylo[k]);
+    }
+    if (r >= j0 - 1) {
+      double fa[M]; // the face above row r
+      Ph::template flux<1>(P, qhi, ylo, fa);
+#pragma unroll
+      for (int k = 0; k < M; ++k) pin(fa[k]);
+      if (r >= j0) {
+        double acc[M], fx[M];
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < M; ++k) xs[W - 1][k] = zs[W][k] = W >= 2 ? win[W >= 2 ? W - 2 : 0][k] : qhi[k];
+        {
+          double xhi[M], xlo[M], ql[M];
+#pragma unroll
+          for (int k = 0; k < M; ++k) {
+            double c[NR];
+#pragma unroll
+            for (int p = 0; p < NR; ++p) c[p] = xs[p][k];
+            recon_cell<W>(c, xhi[k], xlo[k]);
+            ql[k] = lane_prev(xhi[k]);
+            pin(ql[k]);
+            pin(xlo[k]);
+          }
+          __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+          for (int p = 0; p <= 2 * W; ++p)
+            if (p != W) load(at + int64_t(dz[p]) * M, zs[p]);
+          Ph::template flux<0>(P, ql, xlo, fx);
+        }
+#pragma unroll
+        for (int k = 0; k < M; ++k) {
+          acc[k] = 0. + hx * (fx[k] - lane_next(fx[k]));
+          acc[k] += hy * (fb[k] - fa[k]);
+          pin(acc[k]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        {
+          double zhi[M], zlo[M], below[M], above[M], fzb[M], fza[M];
+#pragma unroll
+          for (int k = 0; k < M; ++k) {
+            double c[2 * W + 1];
+#pragma unroll
+            for (int p = 0; p <= 2 * W; ++p) c[p] = zs[p][k];
+            recon_cell<W>(c + 1, zhi[k], zlo[k]);
+            if constexpr (W == 1) {
+              below[k] = c[0];
+              above[k] = c[2];
+            } else if constexpr (W == 2) {
+              below[k] = phys::w3_hi(c[0], c[1], c[2], phys::w3_d(c[0], c[1]), phys::w3_d(c[1], c[2]));
+              above[k] = phys::w3_lo(c[2], c[3], c[4], phys::w3_d(c[2], c[3]), phys::w3_d(c[3], c[4]));
+            } else {
+              below[k] = phys::weno5_side_1div(c[0], c[1], c[2], c[3], c[4]);
+              above[k] = phys::weno5_side_1div(c[6], c[5], c[4], c[3], c[2]);
+            }
+            pin(zhi[k]);
+            pin(zlo[k]);
+            pin(below[k]);
+            pin(above[k]);
+          }
+          next_row(r);
+          Ph::template flux<2>(P, below, zlo, fzb);
+          Ph::template flux<2>(P, zhi, above, fza);
+#pragma unroll
+          for (int k = 0; k < M; ++k) acc[k] += hz * (fzb[k] - fza[k]);
+        }
+        if (own) {
+          const int64_t c = (int64_t(kz) * ny + r) * nx + i;
+          Sources<Ph>::apply(P, c, false, U, int32_t(c), acc, nullptr);
+#pragma unroll
+          for (int k = 0; k < M; ++k) V[c * M + k] = acc[k];
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < M; ++k) fb[k] = fa[k];
+    }
+#pragma unroll
+    for (int k = 0; k < M; ++k) qhi[k] = yhi[k];
+  }
+}
+
 // waves per SIMD the 2D march is compiled for: 3 (up to 168 registers)
 // where the rows of a WENO window of three or more dofs do not fit 128
 // registers without spilling
@@ -355,10 +409,9 @@ __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(vcc_wav
 }
 
 template <class Ph, int W>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(Ph::DIM == 3 ? 2 : 4))) k_vel_march(View P, Box B, int rows_per_strip,
-                                                     const double *__restrict__ U,
-                                                     double *__restrict__ V) {
-  vel_march_body<Ph, W>(P, B, rows_per_strip, xcd_contiguous(int64_t(blockIdx.x), int64_t(gridDim.x)), U, V);
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+k_vel_cc3(View P, Box B, int rows_per_strip, const double *__restrict__ U, double *__restrict__ V) {
+  vel_cc3_body<Ph, W>(P, B, rows_per_strip, xcd_contiguous(int64_t(blockIdx.x), int64_t(gridDim.x)), U, V);
 }
 
 // many independent instances (same family and scheme, each with its own
@@ -876,9 +929,9 @@ static int vel_box(const pda_problem_s &p, const double *U, double *V, hipStream
     else if (p.w == 2) hipLaunchKernelGGL((k_vel_cc<Ph, 2, false>), grid, dim3(64), 0, s, p.view, B, int(rps), U, V, S);
     else hipLaunchKernelGGL((k_vel_cc<Ph, 3, false>), grid, dim3(64), 0, s, p.view, B, int(rps), U, V, S);
   } else {
-    if (p.w == 1) hipLaunchKernelGGL((k_vel_march<Ph, 1>), grid, dim3(64), 0, s, p.view, B, int(rps), U, V);
-    else if (p.w == 2) hipLaunchKernelGGL((k_vel_march<Ph, 2>), grid, dim3(64), 0, s, p.view, B, int(rps), U, V);
-    else hipLaunchKernelGGL((k_vel_march<Ph, 3>), grid, dim3(64), 0, s, p.view, B, int(rps), U, V);
+    if (p.w == 1) hipLaunchKernelGGL((k_vel_cc3<Ph, 1>), grid, dim3(64), 0, s, p.view, B, int(rps), U, V);
+    else if (p.w == 2) hipLaunchKernelGGL((k_vel_cc3<Ph, 2>), grid, dim3(64), 0, s, p.view, B, int(rps), U, V);
+    else hipLaunchKernelGGL((k_vel_cc3<Ph, 3>), grid, dim3(64), 0, s, p.view, B, int(rps), U, V);
   }
   PDA_HIP_CHECK(hipGetLastError());
   return PDA_OK;
@@ -960,21 +1013,35 @@ int launch_jacobian_box(const pda_problem_s &p, const double *U, double *J, doub
   return PDA_E_UNSUPPORTED;
 }
 
-// cells of a row that one velocity wavefront owns
-static int64_t velocity_segment(int dim, int w) {
-  return dim == 2 ? (w == 1 ? vcc_width<1>() : (w == 2 ? vcc_width<2>() : vcc_width<3>())) : VSEG;
+// wavefronts that hold one row of the box (2D), or one row of all its planes
+static int64_t velocity_waves(const Box &B, int dim, int w) {
+  const int64_t bw = B.hi[0] - B.lo[0];
+  if (dim == 3) return ((bw + 2) * (B.hi[2] - B.lo[2]) - 2 + V3OWN - 1) / V3OWN;
+  const int64_t seg = w == 1 ? vcc_width<1>() : (w == 2 ? vcc_width<2>() : vcc_width<3>());
+  return (bw + seg - 1) / seg;
 }
 
 // default strip height of the single-problem velocity march.  Each strip
 // evaluates extra rows of y values, so taller strips do less work but
 // give fewer waves; 2D grids aim at ~3 waves per SIMD (1024^2: 6 rows,
-// 3,078 waves on 1,024 SIMDs), 3D grids at ~20 strips per plane (the
-// measured best: 12 rows at 256^3, 5 at 128^3).
+// 3,078 waves on 1,024 SIMDs).  3D waves run two to a SIMD for the same time
+// each, so the height is the one with the fewest rows (a strip's own and half
+// a row for the values before its first) over the rounds of 2,048 waves (128^3:
+// 16 rows, 1,952 waves, 152 us; 150 to 190 at the others from 2 to 18, 217 at 24).
 int64_t velocity_strip_height(const Box &B, int dim, int w) {
-  const int64_t seg = velocity_segment(dim, w);
-  const int64_t nseg = (B.hi[0] - B.lo[0] + seg - 1) / seg;
-  const int64_t bh = B.hi[1] - B.lo[1];
-  int64_t rps = dim == 3 ? bh / 20 : (bh * nseg + 3071) / 3072;
+  const int64_t nw = velocity_waves(B, dim, w), bh = B.hi[1] - B.lo[1];
+  if (dim == 3) {
+    int64_t best = 1, cost = INT64_MAX;
+    for (int64_t h = 1; h <= 64 && h <= bh; ++h) {
+      const int64_t rounds = (nw * ((bh + h - 1) / h) + 2047) / 2048, c = rounds * (2 * h + 1);
+      if (c < cost) {
+        cost = c;
+        best = h;
+      }
+    }
+    return best;
+  }
+  const int64_t rps = (bh * nw + 3071) / 3072;
   return rps < 1 ? 1 : (rps > 64 ? 64 : rps);
 }
 
@@ -1016,10 +1083,8 @@ int launch_jacobian_fo_euler3d_box(const pda_problem_s &p, const double *U, doub
 
 // number of one-wave groups the velocity march uses for a box
 int64_t velocity_march_blocks(const Box &B, int dim, int w, int rows_per_strip) {
-  const int64_t seg = velocity_segment(dim, w);
-  const int64_t nseg = (B.hi[0] - B.lo[0] + seg - 1) / seg;
   const int64_t bh = B.hi[1] - B.lo[1];
-  return nseg * ((bh + rows_per_strip - 1) / rows_per_strip) * (B.hi[2] - B.lo[2]);
+  return velocity_waves(B, dim, w) * ((bh + rows_per_strip - 1) / rows_per_strip);
 }
 
 template <class Ph, bool STG>

@@ -380,7 +380,7 @@ int build(pda_problem_s &p) {
         const bool per = (M.periodic_mask >> a) & 1;
         const bool big = M.n[a] >= 2 * w + 1;
         if (big && per) p.vbox.mode[a] = 1;
-        else if (big && !per && p.view.ghost_rule == GHOST_MIRROR && p.family != PDA_BURGERS2D)
+        else if (big && !per && dim == 2 && p.view.ghost_rule == GHOST_MIRROR && p.family != PDA_BURGERS2D)
           p.vbox.mode[a] = 2;
         if (p.vbox.mode[a]) {
           p.vbox.lo[a] = 0;

@@ -201,6 +201,41 @@ def test_velocity_march_3d_strip_heights(oracle, torch):
     assert err <= TOL, err
 
 
+# the 3D march lays the box's x lines end to end, 62 owned cells a wavefront:
+# lines that end one cell before, at and after a wavefront's share (60, 61, 62
+# box cells and a cell at either end), the narrowest periodic grids, boxes of
+# one cell, every stencil width
+MARCH_3D_CASES = (
+    [(f"periodic-{nx}x{ny}x{nz}-{s.name}", pda.Euler3d.PeriodicSmooth, s, (nx, ny, nz), True)
+     for s, nx, ny, nz in ((S.Weno5, 7, 7, 7), (S.Weno5, 60, 8, 7), (S.Weno5, 61, 7, 8), (S.Weno5, 62, 9, 7),
+                           (S.Weno3, 5, 6, 5), (S.Weno3, 63, 5, 6), (S.FirstOrder, 61, 5, 4))]
+    + [(f"sedov-{nx}x{ny}x{nz}-{s.name}", pda.Euler3d.SedovSymmetry, s, (nx, ny, nz), ())
+       for s, nx, ny, nz in ((S.Weno5, 7, 7, 7), (S.Weno5, 66, 11, 9), (S.Weno5, 130, 8, 9), (S.Weno3, 65, 6, 7),
+                             (S.FirstOrder, 64, 4, 5))])
+
+
+@pytest.mark.parametrize("case", MARCH_3D_CASES, ids=[c[0] for c in MARCH_3D_CASES])
+def test_velocity_march_3d_line_ends(case, oracle, torch):
+    name, enum, scheme, n, per = case
+    print(f"[gpu-strips] 3D velocity {name}", flush=True)
+    b = (-1, 1) * 3 if per else (0, 1.2) * 3
+    case = (name, enum, scheme, n, b, {S.FirstOrder: 3, S.Weno3: 5, S.Weno5: 7}[scheme], per, 0, None)
+    mesh, prob = cases.make(case)
+    U = cases.perturbed_state(prob, 6)
+    Ud = torch.from_numpy(U).cuda()
+    out = []
+    for h in (0, 1, 3):
+        prob.set_velocity_strip_height(h)
+        V = prob.createRightHandSide()
+        prob.rightHandSide(Ud, 0.0, V)
+        torch.cuda.synchronize()
+        out.append(V.cpu().numpy())
+    err = cases.rel_err(out[0], oracle.velocity(oracle.from_mesh(mesh), cases.oracle_problem(case), U))
+    print(f"[gpu-strips] 3D velocity {name}: {err:.2e}", flush=True)
+    assert err <= TOL, err
+    assert np.array_equal(out[0], out[1]) and np.array_equal(out[0], out[2])
+
+
 def test_riemann_1024_workload(oracle, torch):
     """The measured 1024^2 workload: WENO5 velocity (problem A) at the strip
     heights the step loop chooses from, first-order jacobian() (problem B)
