@@ -43,49 +43,36 @@ __device__ __forceinline__ int64_t xcd_contiguous(int64_t b, int64_t n) {
 // row r + 1.
 template <int W> __host__ __device__ constexpr int vcc_width() { return 64 - 2 * W; }
 
-// state of cell (i, j) of a 2D grid, each index possibly outside the grid
-// and mapped along its axis: periodic wrap, or the mirror cell times the side's
-// ghost sign (the GHOST_MIRROR rule, whose ghost values do not depend on the
-// reading row)
-template <int M>
-__device__ __forceinline__ void load_cell_mapped2(const View &P, const Box &B, const double *__restrict__ U,
-                                                  int64_t i, int64_t j, double *q) {
-  double sg[M];
-#pragma unroll
-  for (int k = 0; k < M; ++k) sg[k] = 1.;
-  int64_t c[2] = {i, j};
-#pragma unroll
-  for (int a = 0; a < 2; ++a) {
-    const int64_t n = B.n[a];
-    int side = -1;
-    if (c[a] < 0) {
-      if (B.mode[a] == 1) c[a] += n;
-      else { c[a] = -1 - c[a]; side = 0; }
-    } else if (c[a] >= n) {
-      if (B.mode[a] == 1) c[a] -= n;
-      else { c[a] = 2 * n - 1 - c[a]; side = 1; }
-    }
-    if (side >= 0) {
-#pragma unroll
-      for (int k = 0; k < M; ++k) sg[k] *= P.gsign[a][side][k];
-    }
+// Cell index c along axis A, possibly outside the grid, mapped by the axis's
+// mode: periodic wrap, or the mirror cell times the side's ghost sign (the
+// GHOST_MIRROR rule, whose ghost values do not depend on the reading row).
+struct Mapped {
+  int at, side; // side -1: no ghost sign
+};
+template <int A> __device__ __forceinline__ Mapped map_axis(const Box &B, int c) {
+  const int n = int(B.n[A]);
+  Mapped m{c, -1};
+  if (B.mode[A] == 1) {
+    m.at = c < 0 ? c + n : (c >= n ? c - n : c);
+  } else {
+    m.side = c < 0 ? 0 : (c >= n ? 1 : -1);
+    m.at = c < 0 ? -1 - c : (c >= n ? 2 * n - 1 - c : c);
   }
-  const int64_t cell = c[1] * B.n[0] + c[0];
-#pragma unroll
-  for (int k = 0; k < M; ++k) q[k] = sg[k] * U[cell * M + k];
+  return m;
 }
 
 // value of lane l - 1 (lane_prev) or l + 1 (lane_next) of the wavefront,
-// by DPP wavefront shifts of the two halves; lane 0 (lane 63) gets 0
+// by DPP wavefront shifts of the two halves; lane 0 (lane 63) gets 0 (by bound
+// control: a 0 to keep would be one more move per half)
 __device__ __forceinline__ double lane_dpp(double v, int ctrl_is_next) {
   const long long b = __double_as_longlong(v);
   int lo, hi;
   if (ctrl_is_next) {
-    lo = __builtin_amdgcn_update_dpp(0, int(b), 0x130, 0xf, 0xf, false);        // wave_shl:1
-    hi = __builtin_amdgcn_update_dpp(0, int(b >> 32), 0x130, 0xf, 0xf, false);
+    lo = __builtin_amdgcn_update_dpp(0, int(b), 0x130, 0xf, 0xf, true);        // wave_shl:1
+    hi = __builtin_amdgcn_update_dpp(0, int(b >> 32), 0x130, 0xf, 0xf, true);
   } else {
-    lo = __builtin_amdgcn_update_dpp(0, int(b), 0x138, 0xf, 0xf, false);        // wave_shr:1
-    hi = __builtin_amdgcn_update_dpp(0, int(b >> 32), 0x138, 0xf, 0xf, false);
+    lo = __builtin_amdgcn_update_dpp(0, int(b), 0x138, 0xf, 0xf, true);        // wave_shr:1
+    hi = __builtin_amdgcn_update_dpp(0, int(b >> 32), 0x138, 0xf, 0xf, true);
   }
   return __longlong_as_double((long long)(unsigned(lo)) | ((long long)hi << 32));
 }
@@ -123,26 +110,49 @@ __device__ __forceinline__ void vel_cc_body(const View &P, const Box &B, int row
   const int64_t seg = bid % nseg, strip = bid / nseg;
   const int64_t iseg = B.lo[0] + seg * NC;
   const int ncell = int(bw - seg * NC < NC ? bw - seg * NC : NC);
-  const int64_t j0 = B.lo[1] + strip * rows_per_strip;
-  const int64_t j1 = j0 + rows_per_strip < B.hi[1] ? j0 + rows_per_strip : B.hi[1];
+  const int j0 = int(B.lo[1] + strip * rows_per_strip);
+  const int j1 = j0 + rows_per_strip < int(B.hi[1]) ? j0 + rows_per_strip : int(B.hi[1]);
   // lane l holds column iseg - W + l; lanes past the last column that the
   // segment's cells read hold that column again
   const int lc = lane < ncell + 2 * W - 1 ? lane : ncell + 2 * W - 1;
-  const int64_t i = iseg - W + lc;
+  const int i = int(iseg) - W + lc;
+  // The column is mapped once (only wavefronts at a mirror edge have ghost signs
+  // to apply), a row by scalar instructions as it is loaded: mapped per lane and
+  // row, with the row's sources read again from memory, a shallow-water step of
+  // the loop had 944 instructions, 772 now (96 instances x 10 RK4 steps 6.49 ->
+  // 4.68 ms).
+  const Mapped ix = map_axis<0>(B, i);
+  const bool xghost = __any(ix.side >= 0);
+  const double *col = U + int64_t(ix.at) * M;
+  auto load_row = [&](int j, double (&q)[M]) {
+    const Mapped jy = map_axis<1>(B, j);
+    const double *u = col + int64_t(jy.at) * nx * M;
+#pragma unroll
+    for (int k = 0; k < M; ++k) q[k] = u[k];
+    if (xghost) {
+#pragma unroll
+      for (int k = 0; k < M; ++k)
+        q[k] *= ix.side < 0 ? 1. : (ix.side == 0 ? P.gsign[0][0][k] : P.gsign[0][1][k]);
+    }
+    if (jy.side >= 0) {
+#pragma unroll
+      for (int k = 0; k < M; ++k) q[k] *= P.gsign[1][jy.side][k];
+    }
+  };
   const bool own = lane >= W && lane < W + ncell;
   const double hx = P.hinv[0], hy = P.hinv[1];
   // win[p] = row r + 2 - W + p at step r (W = 1: row r + 1); nxt = the
   // row that enters the window at the next step, loaded one step ahead
   double win[NR][M], nxt[M];
 #pragma unroll
-  for (int p = 0; p < NR; ++p) load_cell_mapped2<M>(P, B, U, i, j0 - W + p, win[p]);
-  load_cell_mapped2<M>(P, B, U, i, j0 - 1 + W, nxt);
+  for (int p = 0; p < NR; ++p) load_row(j0 - W + p, win[p]);
+  load_row(j0 - 1 + W, nxt);
   double qhi[M], fb[M];  // high-side y value of row r; flux of the face below row r
   // The loop is neither unrolled nor peeled: each face kind has one copy of
   // its code, so a face's value does not depend on the step that forms it
   // (the first two steps of a strip form the faces below it).
 #pragma clang loop unroll(disable)
-  for (int64_t r = j0 - 2; r < j1; ++r) {
+  for (int r = j0 - 2; r < j1; ++r) {
     if (r > j0 - 2) {
 #pragma unroll
       for (int p = 0; p + 1 < NR; ++p)
@@ -150,7 +160,7 @@ __device__ __forceinline__ void vel_cc_body(const View &P, const Box &B, int row
         for (int k = 0; k < M; ++k) win[p][k] = win[p + 1][k];
 #pragma unroll
       for (int k = 0; k < M; ++k) win[NR - 1][k] = nxt[k];
-      if (r + 1 < j1) load_cell_mapped2<M>(P, B, U, i, r + 1 + W, nxt);
+      if (r + 1 < j1) load_row(r + 1 + W, nxt);
     }
     // y face values of cell (i, r + 1)
     double yhi[M], ylo[M];
@@ -166,11 +176,26 @@ __device__ __forceinline__ void vel_cc_body(const View &P, const Box &B, int row
       Ph::template flux<1>(P, qhi, ylo, fa);
       if (r >= j0) {
         // x face values of cell (i, r), the stencil from the lanes beside
-        double xhi[M], xlo[M];
+        double xhi[M], xlo[M], mid[M];
+#pragma unroll
+        for (int k = 0; k < M; ++k) mid[k] = W >= 2 ? win[W >= 2 ? W - 2 : 0][k] : qhi[k];
+        // the stage's terms, read here for the latency to pass under the x part
+        const int64_t e0 = soff + (int64_t(r) * nx + i) * M;
+        double xt[4][M];
+        if constexpr (STG && M <= 3) {
+          if (own) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+              if (q < S.nx) {
+#pragma unroll
+                for (int k = 0; k < M; ++k) xt[q][k] = S.x[q][e0 + k];
+              }
+          }
+        }
 #pragma unroll
         for (int k = 0; k < M; ++k) {
           double s[NR];
-          s[W - 1] = W >= 2 ? win[W >= 2 ? W - 2 : 0][k] : qhi[k];
+          s[W - 1] = mid[k];
 #pragma unroll
           for (int o = 1; o < W; ++o) {
             s[W - 1 - o] = lane_prev(s[W - o]);
@@ -190,15 +215,24 @@ __device__ __forceinline__ void vel_cc_body(const View &P, const Box &B, int row
           acc[k] += hy * (fb[k] - fa[k]);
         }
         if (own) {
-          const int64_t c = r * nx + i;
-          Sources<Ph>::apply(P, c, false, U, int32_t(c), acc, nullptr);
+          const int64_t c = int64_t(r) * nx + i;
+          if constexpr (std::is_same<Ph, PhSwe>::value) Sources<Ph>::velocity(P, mid, acc);
+          else Sources<Ph>::apply(P, c, false, U, int32_t(c), acc, nullptr);
           if constexpr (STG) {
 #pragma unroll
             for (int k = 0; k < M; ++k) {
-              const int64_t e = soff + c * M + k;
+              const int64_t e = e0 + k;
               if (S.kout) S.kout[e] = acc[k];
-              double o = S.c[0] * S.x[0][e];
-              for (int q = 1; q < S.nx; ++q) o += S.c[q] * S.x[q][e];
+              double o;
+              if constexpr (M <= 3) {
+                o = S.c[0] * xt[0][k];
+#pragma unroll
+                for (int q = 1; q < 4; ++q)
+                  if (q < S.nx) o += S.c[q] * xt[q][k];
+              } else {
+                o = S.c[0] * S.x[0][e];
+                for (int q = 1; q < S.nx; ++q) o += S.c[q] * S.x[q][e];
+              }
               o += S.cv * acc[k];
               S.out[e] = o;
             }

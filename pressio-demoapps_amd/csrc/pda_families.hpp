@@ -107,12 +107,19 @@ template <class Ph> struct Sources {
 
 // Coriolis forcing, impl/swe_2d_prob_class.hpp:984-1012
 template <> struct Sources<PhSwe> {
+  // the velocity's part from the row's state; the two quotients share their
+  // reciprocal
+  __device__ static void velocity(const View &P, const double *q, double *v) {
+    const double f = P.p[1];
+    v[1] -= phys::fdiv(f * q[2], q[0]);
+    v[2] += phys::fdiv(f * q[1], q[0]);
+  }
   __device__ static void apply(const View &P, int64_t, bool, const double *U, int32_t self,
                                double *v, double *J) {
     const double f = P.p[1];
     const double h = U[3 * int64_t(self)], hu = U[3 * int64_t(self) + 1], hv = U[3 * int64_t(self) + 2];
-    v[1] -= f * hv / h;
-    v[2] += f * hu / h;
+    const double q[3] = {h, hu, hv};
+    velocity(P, q, v);
     if (J) {
       J[1 * 3 + 0] += f * hv / (h * h);
       J[1 * 3 + 2] += -f / h;

@@ -462,8 +462,9 @@ __device__ __forceinline__ void swe_flux(const double *qL, const double *qR, dou
   FL[0] = hL * unL; FL[1] = hL * unL * uL + (A == 0 ? pL : 0.); FL[2] = hL * unL * vL + (A == 1 ? pL : 0.);
   FR[0] = hR * unR; FR[1] = hR * unR * uR + (A == 0 ? pR : 0.); FR[2] = hR * unR * vR + (A == 1 ? pR : 0.);
   const double hm = 0.5 * (hL + hR);
-  const double sL = fsqrt(hL), sR = fsqrt(hR);
-  const double um = fdiv(unL * sL + unR * sR, sL + sR + kEs);
+  // the Roe average's weights sqrt(h), both divided by sqrt(hL)
+  const double RT = fsqrt(hR * iL);
+  const double um = fdiv(unL + RT * unR, 1. + RT);
   const double c = fsqrt(g * hm);
   // sqrt(x * x) is |x| exactly in IEEE arithmetic (no overflow here)
   const double smax = fabs(um) + fabs(c);
