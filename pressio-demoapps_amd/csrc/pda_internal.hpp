@@ -220,7 +220,7 @@ int launch_velocity_stage(const pda_problem_s &p, const double *U, const RkStage
 // (Uin != Uout)
 constexpr int STEPS1D_MAX = 8;
 bool steps1d_fits(const pda_problem_s &p, int scheme, bool *periodic);
-int steps1d_per_launch(const pda_problem_s &p, int scheme);
+int steps1d_per_launch(const pda_problem_s &p, int scheme, bool periodic);
 int launch_steps1d(const pda_problem_s &p, int scheme, const double *Uin, double *Uout, int nsteps, double dt,
                    bool periodic, hipStream_t s);
 int launch_jacobian(const pda_problem_s &p, const double *U, double t, double *J,

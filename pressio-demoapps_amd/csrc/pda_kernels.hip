@@ -49,22 +49,29 @@ __global__ void __launch_bounds__(64) k_velocity_stage(View P, const double *__r
 // in LDS with H cells on each side, H = W x the number of stages it runs:
 // each stage's values are valid on a region W cells narrower per side than
 // the stage before, so after the last stage the owned cells are exact.  A
-// stage is one dependent chain per lane with little beside it on the CU, so
-// it is spread thin: four lanes per row, lane (f, s) reconstructing side s
-// (0 minus, 1 plus) of face f (0 left, 1 right) of the row with the generic
-// row code's stencil and ghost rule (the plus side is the minus side of the
-// reversed stencil, so the lanes share one instruction stream); the pair
-// exchanges its sides and the faces their fluxes by DPP, and lane q < M forms
-// dof q of the stage, as k_velocity_stage does, term by term.  Where a lane
+// stage is one dependent chain per lane with little beside it on the CU, so it
+// is spread thin, one wave per SIMD: two lanes per face, lane s
+// reconstructing side s (0 minus, 1 plus) with the generic row code's stencil
+// and ghost rule (the plus side is the minus side of the reversed stencil, so
+// the lanes share one instruction stream) and exchanging it with the other.  A
+// row's pair of lanes has its left face; the right face's flux comes from the
+// next pair, by DPP.  That is the next row's left face, except where the face
+// reads ghosts, whose values depend on the row that reads them: there the row
+// has a second pair, for its right face.  A wave owns 31 pairs; its last pair
+// repeats the next wave's first.  Lane s forms dofs s and s + 2 of the
+// row's stage, as k_velocity_stage does, term by term.  Where a lane
 // reads does not change from stage to stage: its cells' places in LDS are
 // found once per launch.  Ghosts: the opposite rule (a row reads position
 // g - d < 0 as cell g + d - 1, g + d >= n as g - d + 1; the 1D problems have no
 // sign to apply), or periodic wrap.  The state is read from Uin and
-// written to Uout (workgroups read each other's cells).  The region is 128
-// rows (two waves per SIMD of the CU).  1000 cells, WENO5, SSPRK3: 4.8 us per
-// step, 8.6 us with two lanes per row that each reconstructed both sides of
-// a face and looked up every cell's place in every stage.
-constexpr int S1_ROWS = 128, S1_LPR = 4;
+// written to Uout (workgroups read each other's cells).
+// 1000 cells, WENO5, SSPRK3: 2.85 us per step; with four lanes per row, each
+// face evaluated by both its rows and two waves per SIMD bound by issue, 3.9.
+// 10^6 cells 67 us (162).
+constexpr int S1_WAVES = 4, S1_OWN = 31, S1_PAIRS = S1_WAVES * S1_OWN, S1_STRIDE = 128;
+// rows of a region: every row a pair, and the second pairs of the rows at the
+// ends of an open grid (W - 1 at the low end, W at the high end)
+constexpr int s1_rows(int w, bool periodic) { return S1_PAIRS - (periodic ? 0 : 2 * w - 1); }
 
 struct Steps1dCoef {
   double c[4][4];  // per stage: coefficients of the stage's terms
@@ -80,15 +87,25 @@ template <int CTRL> __device__ __forceinline__ double quad_swap(double v) {
   return __longlong_as_double((long long)(unsigned(lo)) | ((long long)hi << 32));
 }
 
+// value of lane l + 2 (the next pair's), by two DPP wavefront shifts of each half
+__device__ __forceinline__ double next_pair(double v) {
+  const long long b = __double_as_longlong(v);
+  int lo = __builtin_amdgcn_update_dpp(0, int(b), 0x130, 0xf, 0xf, true); // wave_shl:1
+  int hi = __builtin_amdgcn_update_dpp(0, int(b >> 32), 0x130, 0xf, 0xf, true);
+  lo = __builtin_amdgcn_update_dpp(0, lo, 0x130, 0xf, 0xf, true);
+  hi = __builtin_amdgcn_update_dpp(0, hi, 0x130, 0xf, 0xf, true);
+  return __longlong_as_double((long long)(unsigned(lo)) | ((long long)hi << 32));
+}
+
 template <class Ph, int W, int SCHEME>
-__global__ void __launch_bounds__(S1_LPR * S1_ROWS) k_steps1d(View P, int64_t n, int periodic, int own, int H,
+__global__ void __launch_bounds__(S1_WAVES * 64) k_steps1d(View P, int64_t n, int periodic, int own, int H,
                                                              int nsteps, const double *__restrict__ Uin,
                                                              double *__restrict__ Uout, Steps1dCoef C) {
-  constexpr int M = Ph::M, R = S1_ROWS, NP = 2 * W - 1;
-  static_assert(M <= S1_LPR, "a lane per dof");
+  constexpr int M = Ph::M, R = S1_STRIDE, NP = 2 * W - 1;
+  static_assert(M == 3, "dofs s and s + 2 of lane s");
   extern __shared__ double lds[];
   const int64_t a0 = int64_t(blockIdx.x) * own, base = a0 - H;
-  const int rows = own + 2 * H; // <= R
+  const int rows = own + 2 * H; // <= s1_rows
   // buffers of M x R doubles ([dof][row]): 0 the step's state, 1 and 2 stage
   // states, 3..5 the RK4 stage velocities
   auto buf = [&](int b) { return lds + b * (R * M); };
@@ -105,24 +122,45 @@ __global__ void __launch_bounds__(S1_LPR * S1_ROWS) k_steps1d(View P, int64_t n,
     }
     buf(0)[k * R + i] = v;
   }
-  const int i = int(threadIdx.x) / S1_LPR, q4 = int(threadIdx.x) % S1_LPR, f = q4 >> 1, sd = q4 & 1;
-  const int64_t g = base + i;
-  const bool store = i < rows && (periodic || (g >= 0 && g < n)) && q4 < M;
-  const int kq = q4 < M ? q4 : 0; // this lane's dof
-  const double hf = f ? -P.hinv[0] : P.hinv[0];
+  // the lane's face: the right one (kind 1) or the left one of row g, the
+  // pairs counted from the region's first cell of the grid
+  const int sd = int(threadIdx.x) & 1, pl = (int(threadIdx.x) & 63) >> 1;
+  const int64_t sp = int64_t(threadIdx.x >> 6) * S1_OWN + pl;
+  int64_t g = base + sp;
+  int kind = 0;
+  if (!periodic) {
+    const int64_t g0 = base > 0 ? base : 0, hi = n - W; // rows from hi on have two pairs, as the first W - 1 do
+    const int64_t q = sp + g0 + (g0 < W - 1 ? g0 : W - 1) + (g0 > hi ? g0 - hi : 0);
+    if (q < 2 * (W - 1)) {
+      g = q >> 1;
+      kind = int(q & 1);
+    } else if (q - (W - 1) < hi) {
+      g = q - (W - 1);
+    } else {
+      const int64_t t = q - (W - 1) - hi;
+      g = hi + (t >> 1);
+      kind = int(t & 1);
+    }
+  }
+  const int64_t il = g - base;
+  const bool store = kind == 0 && pl < S1_OWN && il < rows && (periodic || g < n);
+  const int i = int(il < rows ? il : rows - 1);
   // the lane's 2W-1 cells, from the one upwind of the face's farthest on
   int at[NP];
 #pragma unroll
   for (int j = 0; j < NP; ++j) {
     const int p = sd ? 2 * W - 1 - j : j; // point of the face's 2W cells
-    int64_t src = g + f - W + p;
+    int64_t src = g + kind - W + p;
     if (!periodic) src = src < 0 ? 2 * g - src - 1 : (src >= n ? 2 * g - src + 1 : src);
     const int64_t li = src - base;
     at[j] = int(li < 0 ? 0 : (li >= rows ? rows - 1 : li));
   }
   __syncthreads();
-  // dof kq of the velocity of row i from state X (every lane takes part in
-  // the exchanges)
+  // dofs sd and (lane 0 of the pair) 2 of the velocity of row i from state X
+  // (every lane takes part in the exchanges)
+  struct Two {
+    double a, b;
+  };
   auto vel = [&](const double *X) {
     double q[M][NP];
 #pragma unroll
@@ -145,22 +183,13 @@ __global__ void __launch_bounds__(S1_LPR * S1_ROWS) k_steps1d(View P, int64_t n,
       up[k] = sd ? v : o;
     }
     Ph::template flux<0>(P, um, up, F);
-    // left minus right flux: this lane's face minus the other, turned round in
-    // the lanes of the right face
-    double acc = 0.;
-#pragma unroll
-    for (int k = 0; k < M; ++k) {
-      const double d = F[k] - quad_swap<0x4E>(F[k]);
-      acc = k == kq ? d : acc;
-    }
-    acc = 0. + hf * acc;
-    return acc;
+    const double fa = sd ? F[1] : F[0], fb = F[2];
+    return Two{0. + P.hinv[0] * (fa - next_pair(fa)), 0. + P.hinv[0] * (fb - next_pair(fb))};
   };
-  const int e = kq * R + (i < rows ? i : 0);
+  const int e = sd * R + i, e2 = 2 * R + i;
   // out = c0 x0 + ... + cv v, the terms in k_velocity_stage's order
-  auto comb = [&](double *out, int st, int nx, const double *x0, const double *x1, const double *x2,
-                  const double *x3, double acc) {
-    if (!store) return;
+  auto comb1 = [&](double *out, int e, int st, int nx, const double *x0, const double *x1, const double *x2,
+                   const double *x3, double acc) {
     double o = C.c[st][0] * x0[e];
     if (nx > 1) o += C.c[st][1] * x1[e];
     if (nx > 2) o += C.c[st][2] * x2[e];
@@ -168,11 +197,19 @@ __global__ void __launch_bounds__(S1_LPR * S1_ROWS) k_steps1d(View P, int64_t n,
     o += C.cv[st] * acc;
     out[e] = o;
   };
-  auto keep = [&](double *kb, double acc) {
-    if (store) kb[e] = acc;
+  auto comb = [&](double *out, int st, int nx, const double *x0, const double *x1, const double *x2,
+                  const double *x3, Two acc) {
+    if (!store) return;
+    comb1(out, e, st, nx, x0, x1, x2, x3, acc.a);
+    if (sd == 0) comb1(out, e2, st, nx, x0, x1, x2, x3, acc.b);
+  };
+  auto keep = [&](double *kb, Two acc) {
+    if (!store) return;
+    kb[e] = acc.a;
+    if (sd == 0) kb[e2] = acc.b;
   };
   for (int s = 0; s < nsteps; ++s) {
-    double acc;
+    Two acc;
     if constexpr (SCHEME == PDA_SSPRK3) {
       acc = vel(buf(0));  // u1 = u + dt f(u)
       comb(buf(1), 0, 1, buf(0), nullptr, nullptr, nullptr, acc);
@@ -201,7 +238,10 @@ __global__ void __launch_bounds__(S1_LPR * S1_ROWS) k_steps1d(View P, int64_t n,
       __syncthreads();
     }
   }
-  if (store && i >= H && i < H + own && g < n) Uout[g * M + kq] = buf(0)[e];
+  if (store && i >= H && i < H + own && g < n) {
+    Uout[g * M + sd] = buf(0)[e];
+    if (sd == 0) Uout[g * M + 2] = buf(0)[e2];
+  }
 }
 
 template <class Ph, int W, bool WV>
@@ -1146,20 +1186,22 @@ bool steps1d_fits(const pda_problem_s &p, int scheme, bool *periodic_out) {
   return open && p.view.ghost_rule == GHOST_OPPOSITE;
 }
 
-// Steps per launch: more steps pay the launch (about 5 us, against 1.1 us for a
-// stage) less often, but leave a workgroup fewer owned rows of its 128 (SSPRK3
-// WENO5: 6 steps, 20 owned rows), so more workgroups.  The least time per
-// step, with the workgroups running in rounds of two per CU: the most steps
-// up to about 10^4 cells, fewer beyond.
-int steps1d_per_launch(const pda_problem_s &p, int scheme) {
+// Steps per launch: more steps pay the launch (about 4 us, against 0.7 us for a
+// WENO5 stage) less often, but leave a workgroup fewer owned rows of its 119
+// or 124 (SSPRK3 WENO5: 6 steps, 11 owned rows), so more workgroups; the second
+// workgroup of a CU makes a stage 1.6 times as long, every further one adds as
+// much.  The least time per step: the most steps up to about 3 10^3 cells,
+// fewer beyond.
+int steps1d_per_launch(const pda_problem_s &p, int scheme, bool periodic) {
   const int nst = scheme == PDA_RK4 ? 4 : 3;
   int best = 1;
   double best_cost = 1e300;
   for (int k = 1; k <= STEPS1D_MAX; ++k) {
-    const int own = S1_ROWS - 2 * nst * p.w * k;
-    if (own < 16 && k > 1) break;
+    const int own = s1_rows(p.w, periodic) - 2 * nst * p.w * k;
+    if (own < 8 && k > 1) break;
     const int64_t nwg = (p.mesh->n_sample + own - 1) / own;
-    const double cost = double((nwg + 511) / 512) * (5. + 1.1 * nst * k) / k;
+    const double per_cu = double((nwg + 255) / 256);
+    const double cost = (4. + 0.7 * std::max(1., 0.8 * per_cu) * nst * k) / k;
     if (cost < best_cost) {
       best_cost = cost;
       best = k;
@@ -1170,17 +1212,17 @@ int steps1d_per_launch(const pda_problem_s &p, int scheme) {
 
 int launch_steps1d(const pda_problem_s &p, int scheme, const double *Uin, double *Uout, int nsteps, double dt,
                    bool periodic, hipStream_t s) {
-  const int kmax = steps1d_per_launch(p, scheme);
+  const int kmax = steps1d_per_launch(p, scheme, periodic);
   if (nsteps < 1 || nsteps > kmax) {
     set_error("steps1d: steps per launch out of range");
     return PDA_E_INVALID_ARG;
   }
   const int nst = scheme == PDA_RK4 ? 4 : 3, nbuf = scheme == PDA_RK4 ? 6 : 3;
-  const int H = nst * p.w * kmax, own = S1_ROWS - 2 * H;
+  const int H = nst * p.w * kmax, own = s1_rows(p.w, periodic) - 2 * H;
   const int64_t n = p.mesh->n_sample;
   constexpr int M = PhEuler1::M;
-  const unsigned threads = S1_LPR * S1_ROWS;
-  const size_t lds = sizeof(double) * size_t(nbuf) * size_t(S1_ROWS) * M;
+  const unsigned threads = S1_WAVES * 64;
+  const size_t lds = sizeof(double) * size_t(nbuf) * size_t(S1_STRIDE) * M;
   const dim3 grid{unsigned((n + own - 1) / own), 1, 1};
   if (own < 1 || lds > 64 * 1024) {
     set_error("steps1d: region too large");

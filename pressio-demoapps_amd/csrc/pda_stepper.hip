@@ -271,7 +271,7 @@ int pda_stepper_advance(pda_stepper st, double *d_U, double t0, double dt, int64
     // stepper's buffer (a launch's workgroups read cells that other
     // workgroups of it write); one copy back when the count of launches is
     // odd.  use_graph does not change this path.
-    const int kmax = steps1d_per_launch(*st->prob, st->scheme);
+    const int kmax = steps1d_per_launch(*st->prob, st->scheme, st->periodic1d);
     double *a = d_U, *b = st->aux.as<double>();
     for (int64_t done = 0; done < nsteps;) {
       const int k = int(std::min<int64_t>(nsteps - done, kmax));

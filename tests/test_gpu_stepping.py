@@ -241,6 +241,20 @@ def test_1d_steps_per_launch(case, scheme, oracle, torch):
     assert err <= 1e-11
 
 
+# open grids whose doubled rows at either end (those that read ghosts) fall on a
+# wavefront's 31 rows, on a region's edge, or meet; periodic ones likewise
+ONE_D_EDGES = ([(f"sod-{n}-{s.name}", pda.Euler1d.Sod, s, (n,), (-0.5, 0.5), st, (), 0, None)
+                for s, st, ns in ((S.Weno5, 7, (7, 8, 29, 30, 31, 119, 131)), (S.Weno3, 5, (5, 6, 30, 61, 92)),
+                                  (S.FirstOrder, 3, (3, 31, 123))) for n in ns]
+               + [(f"periodic-{n}-Weno5", pda.Euler1d.PeriodicSmooth, S.Weno5, (n,), (-1.0, 1.0), 7, True, 0, None)
+                  for n in (7, 31, 125)])
+
+
+@pytest.mark.parametrize("case", ONE_D_EDGES, ids=[c[0] for c in ONE_D_EDGES])
+def test_1d_steps_at_region_edges(case, oracle, torch):
+    test_1d_steps_per_launch(case, "SSPRK3", oracle, torch)
+
+
 @pytest.mark.parametrize("scheme", ["SSPRK3", "RK4"])
 def test_1d_steps_per_launch_of_large_grids(scheme, torch):
     """Grids where a launch takes fewer steps (its workgroups run in several
