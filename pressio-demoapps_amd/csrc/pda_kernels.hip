@@ -2,8 +2,8 @@
 // mesh: full, sample/stencil, 1D/2D/3D): velocity (residual) and Jacobian
 // assembly into the fixed CSR pattern, plus the launch logic that pairs them
 // with the structured box kernels.  The per-row device code is in
-// pda_rows.hpp.
-#include "pda_rows.hpp"
+// pda_rows.hpp and pda_staged.hpp.
+#include "pda_staged.hpp"
 
 namespace pda {
 namespace {
@@ -12,14 +12,7 @@ using namespace fam;
 template <class Ph, int W>
 __global__ void __launch_bounds__(64) k_velocity(View P, const double *__restrict__ U,
                                                    double *__restrict__ V) {
-  constexpr int M = Ph::M, D = Ph::DIM;
-  double acc[M];
-  const int64_t r = rows::velocity_lanes<Ph, W>(P, int64_t(blockIdx.x), U, acc);
-  if (r < 0) return;
-  const int a = int(threadIdx.x) % D; // the row's lanes share its stores
-#pragma unroll
-  for (int k = 0; k < M; ++k)
-    if (k % D == a) V[r * M + k] = acc[k];
+  rows::velocity_rows<Ph, W>(P, int64_t(blockIdx.x), U, V);
 }
 
 // velocity with an explicit stage fused into the store (RkStage)
@@ -251,214 +244,36 @@ __global__ void __launch_bounds__(64) k_jacobian(View P, const double *__restric
 }
 
 // ------------------------------- first-order Euler Jacobian, staged rows
-// Rows of the first-order Euler Jacobian (Euler has no source term) with
-// four lanes per row and 16 rows per wavefront.  Lane a < D evaluates the two
-// faces of axis a.  The Euler flux along axis a is the flux along x with
-// momentum components 1 and 1+a exchanged, so every lane runs the x-face
-// code on exchanged states and writes entry (k, j) of its blocks to
-// (p(k), p(j)), p the 1 <-> 1+a exchange: one instruction stream for all
-// axes.  A row's blocks are assembled in LDS in CSR order (scalar row k,
-// block slot, column), the diagonal block adding the axes in order as the
-// generic row code does, and the wavefront then copies each staged row to
-// its contiguous CSR values with coalesced streaming stores (one thread per
-// row would scatter every store over 64 rows); 16 rows consecutive in the
-// CSR leave as one range of 16-byte stores.  Used where no structured box
-// kernel applies (sample meshes, 2D meshes given as a graph) and for the
-// boundary rows of a structured 3D full mesh.  Bound by latency: a wavefront
-// alone takes 11 us (three dependent loads, two faces of divisions and square
-// roots, the stage, the copy) and the stage's 23 KB leave 7 of them per CU; 5 %
-// sample mesh of 128^3 50.6 us (147 MB of values), 61.7 us with a ghost branch
-// per block entry and the rows' CSR offsets fetched one by one at the copy.
-// Near-boundary rows: a
-// missing neighbour along axis a reads the ghost state sign_k U_k of the row's own cell (the first
-// ghost layer of every ghost rule), writes no block, and adds fac_j JL (left
-// side) or -fac_j JR (right side) of that face, times h, to the axis's
-// diagonal part, fac the row's BC factors (the terms of
-// impl/mixin_directional_flux_balance_jacobian.hpp:312-369, with the factors
-// of impl/euler_3d_prob_class.hpp:626-651).
-constexpr int SJ_LANES = 4, SJ_ROWS = 64 / SJ_LANES;
-
-__device__ __forceinline__ int exch(int k, int a) { return k == 1 ? 1 + a : (k == 1 + a ? 1 : k); }
-
-// ghost sign of native dof exch(k, a) on side `side` of axis a
-template <int D>
-__device__ __forceinline__ double ghost_sign(const View &P, int a, int side, int k) {
-  const double s0 = P.gsign[0][side][exch(k, 0)];
-  const double s1 = D > 1 ? P.gsign[1][side][exch(k, 1)] : 0.;
-  const double s2 = D > 2 ? P.gsign[2][side][exch(k, 2)] : 0.;
-  return a == 0 ? s0 : (a == 1 ? s1 : s2);
-}
-
 template <int D>
 __global__ void __launch_bounds__(64) k_jac_fo_euler_staged(View P, const double *__restrict__ U,
                                                               double *__restrict__ J) {
-  using Ph = PhEuler<D>;
-  constexpr int M = D + 2, NB = 1 + 2 * D, RS = NB * M, PER = M * RS;
-  __shared__ double stage[SJ_ROWS * PER];
-  __shared__ int64_t base_of[SJ_ROWS]; // first CSR value of the row, -1: no row
-  __shared__ int blk_of[SJ_ROWS];      // its column blocks
-  const int lane = threadIdx.x, g = lane / SJ_LANES, a = lane % SJ_LANES;
-  const int64_t t = int64_t(blockIdx.x) * SJ_ROWS + g;
-  int64_t r = -1;
-  if (t < P.nvisit) {
-    const int64_t rr = P.rows ? P.rows[t] : t;
-    r = rr;
-  }
-  // the row's place in the CSR, in each of its lanes
-  const int64_t base = r >= 0 ? P.rowbase[r] : -1;
-  const int nblk = r >= 0 ? P.nblk[r] : 0;
-  if (a == 0) {
-    base_of[g] = base;
-    blk_of[g] = nblk;
-  }
-  const bool act = r >= 0 && a < D;
-  double *st = stage + g * PER;
-  typename Ph::Side Ln, Lp, Rn, Rp;
-  int sL = 0, sR = 0, s0 = 0;
-  bool gl = false, gr_ = false; // no neighbour on the left / right
-  double fac[M];                // BC factors of native dof exch(j, a)
-  double h = 0.;
-  if (act) {
-    int64_t cells[3];
-    {
-      const int32_t *gr = P.graph + r * P.ncols;
-      const uint8_t *sl = P.slot + r * P.npos;
-      const int cl = colof<D>(a, 0, 0), cr = colof<D>(a, 1, 0);
-      const int32_t il = gr[cl], ir = gr[cr];
-      gl = il < 0;
-      gr_ = ir < 0;
-      cells[0] = gl ? gr[0] : il;
-      cells[1] = gr[0];
-      cells[2] = gr_ ? gr[0] : ir;
-      sL = gl ? 0 : sl[cl];
-      sR = gr_ ? 0 : sl[cr];
-      s0 = sl[0];
-    }
-    double q[3][M];
-#pragma unroll
-    for (int c = 0; c < 3; ++c)
-#pragma unroll
-      for (int k = 0; k < M; ++k) q[c][k] = U[cells[c] * M + exch(k, a)];
-#pragma unroll
-    for (int k = 0; k < M; ++k) {
-      if (gl) q[0][k] = ghost_sign<D>(P, a, 0, k) * q[0][k];
-      if (gr_) q[2][k] = ghost_sign<D>(P, a, 1, k) * q[2][k];
-      fac[k] = 0.;
-    }
-    const int64_t gi = P.ghost_row[r];
-    if ((gl || gr_) && gi >= 0) {
-      const double *f = P.bcf + (gi * D + a) * M;
-#pragma unroll
-      for (int k = 0; k < M; ++k) fac[k] = f[exch(k, a)];
-    }
-    Ph::template sides<0>(P, q[0], q[1], Ln, Lp);
-    Ph::template sides<0>(P, q[1], q[2], Rn, Rp);
-    h = P.hinv[a];
-  }
-  // a fence between the face math and the stage stores keeps the entry
-  // evaluations from being hoisted into it (2D: 148 -> 126 registers)
-  wave_sync();
-  auto put = [&](int slot, const typename Ph::Side &S, bool minus) {
-#pragma unroll
-    for (int k = 0; k < M; ++k)
-#pragma unroll
-      for (int j = 0; j < M; ++j) {
-        const double v = Ph::template entry<0>(P, S, k, j);
-        st[exch(k, a) * RS + exch(j, a) + slot * M] = 0. + (minus ? -v : v) * h;
-      }
-  };
-  if (act && !gl) put(sL, Ln, false);
-  if (act && !gr_) put(sR, Rp, true);
-  // every lane forms its axis's part of the diagonal block at once; the
-  // axes then add their parts in order, one axis at a time, in LDS
-  double dg[M][M];
-  wave_sync();
-  if (act) {
-#pragma unroll
-    for (int k = 0; k < M; ++k)
-#pragma unroll
-      for (int j = 0; j < M; ++j)
-        dg[k][j] = (Ph::template entry<0>(P, Lp, k, j) - Ph::template entry<0>(P, Rn, k, j)) * h;
-  }
-  if (act && gl) {
-#pragma unroll
-    for (int k = 0; k < M; ++k)
-#pragma unroll
-      for (int j = 0; j < M; ++j) dg[k][j] += (fac[j] * Ph::template entry<0>(P, Ln, k, j)) * h;
-  }
-  if (act && gr_) {
-#pragma unroll
-    for (int k = 0; k < M; ++k)
-#pragma unroll
-      for (int j = 0; j < M; ++j) dg[k][j] += (fac[j] * -Ph::template entry<0>(P, Rp, k, j)) * h;
-  }
-#pragma unroll
-  for (int ax = 0; ax < D; ++ax) {
-    wave_sync();
-    if (act && a == ax) {
-#pragma unroll
-      for (int k = 0; k < M; ++k)
-#pragma unroll
-        for (int j = 0; j < M; ++j) {
-          const int o = exch(k, a) * RS + s0 * M + exch(j, a);
-          st[o] = (ax == 0 ? 0. : st[o]) + dg[k][j];
-        }
-    }
-  }
-  wave_sync();
-  // Copy-out from the row table in LDS alone: the rows' CSR offsets were
-  // loaded with their states (not here, one row after the other).  Whole
-  // rows leave as one flattened loop over their values: 16-byte stores where
-  // every row starts on an even value (2D, and 3D rows consecutive in the CSR
-  // after a leading value), else 8-byte ones.
-  const int64_t rb0 = base_of[0];
-  const bool whole = __all(base >= 0 && nblk == NB);
-  const bool run = __all(base == rb0 + int64_t(g) * PER);
-  if (whole && run) {
-    constexpr int TOT = SJ_ROWS * PER;
-    const int head = int(rb0 & 1); // a leading value that is not 16-byte aligned
-    double *dst = J + rb0;
-    if (head && lane == 0) store_stream(dst, stage[0]);
-    const int npairs = (TOT - head) / 2;
-    double2 *d2 = reinterpret_cast<double2 *>(dst + head);
-#pragma unroll 4
-    for (int q = lane; q < npairs; q += 64)
-      store_stream(d2 + q, make_double2(stage[head + 2 * q], stage[head + 2 * q + 1]));
-    if (((TOT - head) & 1) && lane == 0) store_stream(dst + TOT - 1, stage[TOT - 1]);
-    return;
-  }
-  if (whole) {
-    if constexpr (PER % 2 == 0) {
-#pragma unroll 4
-      for (int q = lane; q < SJ_ROWS * (PER / 2); q += 64) {
-        const int gg = q / (PER / 2), e = 2 * (q - gg * (PER / 2));
-        const double *src = stage + gg * PER + e;
-        store_stream(reinterpret_cast<double2 *>(J + base_of[gg] + e), make_double2(src[0], src[1]));
-      }
-    } else {
-#pragma unroll 4
-      for (int q = lane; q < SJ_ROWS * PER; q += 64) {
-        const int gg = q / PER;
-        store_stream(J + base_of[gg] + (q - gg * PER), stage[q]);
-      }
-    }
-    return;
-  }
-#pragma clang loop unroll(disable)
-  for (int gg = 0; gg < SJ_ROWS; ++gg) {
-    const int64_t rb = base_of[gg];
-    if (rb < 0) continue;
-    double *dst = J + rb;
-    const double *src = stage + gg * PER;
-    // a near-boundary row holds nblk of the NB block slots per scalar row
-    const int rs = blk_of[gg] * M;
-    for (int e = lane; e < M * rs; e += 64) {
-      int k = 0;
-#pragma unroll
-      for (int q = 1; q < M; ++q) k += e >= q * rs;
-      store_stream(dst + e, src[k * RS + (e - k * rs)]);
-    }
-  }
+  __shared__ rows::StagedLds<D> L;
+  rows::jac_fo_euler_staged<D>(P, int64_t(blockIdx.x), U, J, L);
+}
+
+// Near-boundary rows of a WENO problem, velocity and Jacobian: the Jacobian's
+// rows are first order there and staged, by the first njac workgroups; the
+// others take the velocity's rows.  The rows are few, so the launch lasts as
+// long as one wavefront: 5,340 rows of 2D Euler WENO5 9.4 us, 15.6 with one
+// thread per row (2 KB of registers spilled).
+template <int D, int W>
+__global__ void __launch_bounds__(64) k_near_euler(View P, int njac, const double *__restrict__ U,
+                                                     double *__restrict__ V, double *__restrict__ J) {
+  __shared__ rows::StagedLds<D> L;
+  if (int(blockIdx.x) < njac) rows::jac_fo_euler_staged<D>(P, int64_t(blockIdx.x), U, J, L);
+  else rows::velocity_rows<PhEuler<D>, W>(P, int64_t(blockIdx.x) - njac, U, V);
+}
+
+// the near-boundary rows of a WENO problem (without merged columns)
+template <int D>
+int jac_near_euler(const View &v, int w, const double *U, double *V, double *J, hipStream_t s) {
+  const unsigned nj = unsigned((v.nvisit + rows::SJ_ROWS - 1) / rows::SJ_ROWS);
+  const unsigned nv = unsigned((v.nvisit + rows::vel_rows<D>() - 1) / rows::vel_rows<D>());
+  if (!V) hipLaunchKernelGGL((k_jac_fo_euler_staged<D>), dim3(nj), dim3(64), 0, s, v, U, J);
+  else if (w == 2) hipLaunchKernelGGL((k_near_euler<D, 2>), dim3(nj + nv), dim3(64), 0, s, v, int(nj), U, V, J);
+  else hipLaunchKernelGGL((k_near_euler<D, 3>), dim3(nj + nv), dim3(64), 0, s, v, int(nj), U, V, J);
+  PDA_HIP_CHECK(hipGetLastError());
+  return PDA_OK;
 }
 
 // ------------------------------------ WENO3/WENO5 Jacobian, staged rows
@@ -1280,8 +1095,16 @@ int launch_jacobian(const pda_problem_s &p, const double *U, double, double *J, 
       PDA_HIP_CHECK(hipGetLastError());
     }
     if (!p.view.dup && p.w > 1 && p.family != PDA_ADR2D) {
-      // WENO Jacobian: staged inner rows, then the near-boundary rows (first
-      // order with BC factors) with the generic row code; for the 2D
+      // the near-boundary rows (first order with BC factors): staged for 2D and
+      // 3D Euler, the generic row code for the others
+      auto near_rows = [&]() -> int {
+        if (p.n_near == 0) return PDA_OK;
+        const View v = generic_view(p, &p.d_near_rows, p.n_near);
+        if (p.family == PDA_EULER2D) return jac_near_euler<2>(v, p.w, U, V, J, s);
+        if (p.family == PDA_EULER3D) return jac_near_euler<3>(v, p.w, U, V, J, s);
+        return jac_generic(v, p, U, V, J, s);
+      };
+      // WENO Jacobian: staged inner rows, then the near-boundary rows; for the 2D
       // two- and three-dof families, the box's rows with each face once
       // (when the box holds no near-boundary row) and the staged kernel on
       // the rows outside it
@@ -1319,8 +1142,7 @@ int launch_jacobian(const pda_problem_s &p, const double *U, double, double *J, 
                                            : jac_weno_staged<PhEuler2>(vr, p.w, U, V, J, s);
             if (rc) return rc;
           }
-          if (p.n_near == 0) return PDA_OK;
-          return jac_generic(generic_view(p, &p.d_near_rows, p.n_near), p, U, V, J, s);
+          return near_rows();
         }
       }
       const View v = generic_view(p, nullptr, 0);
@@ -1333,8 +1155,7 @@ int launch_jacobian(const pda_problem_s &p, const double *U, double, double *J, 
         case PDA_BURGERS2D: rc = jac_weno_staged<PhBurgers>(v, p.w, U, V, J, s); break;
         default: set_error("jacobian: unsupported family"); return PDA_E_UNSUPPORTED;
       }
-      if (rc || p.n_near == 0) return rc;
-      return jac_generic(generic_view(p, &p.d_near_rows, p.n_near), p, U, V, J, s);
+      return rc ? rc : near_rows();
     }
     if (!V && !p.view.dup && p.w == 1 && (p.family == PDA_EULER2D || p.family == PDA_EULER3D)) {
       // first-order Euler Jacobian alone
@@ -1345,13 +1166,13 @@ int launch_jacobian(const pda_problem_s &p, const double *U, double, double *J, 
         const int rc = launch_jacobian_fo_euler3d_box(p, U, J, s);
         if (rc || p.h_rem_rows.empty()) return rc;
         const View vr = generic_view(p, &p.d_rem_rows, int64_t(p.h_rem_rows.size()));
-        hipLaunchKernelGGL((k_jac_fo_euler_staged<3>), dim3(unsigned((vr.nvisit + SJ_ROWS - 1) / SJ_ROWS)),
+        hipLaunchKernelGGL((k_jac_fo_euler_staged<3>), dim3(unsigned((vr.nvisit + rows::SJ_ROWS - 1) / rows::SJ_ROWS)),
                            dim3(64), 0, s, vr, U, J);
         PDA_HIP_CHECK(hipGetLastError());
         return PDA_OK;
       }
       // every row, near-boundary rows included, staged four lanes per row
-      const unsigned nb = unsigned((v.nvisit + SJ_ROWS - 1) / SJ_ROWS);
+      const unsigned nb = unsigned((v.nvisit + rows::SJ_ROWS - 1) / rows::SJ_ROWS);
       if (p.family == PDA_EULER2D)
         hipLaunchKernelGGL((k_jac_fo_euler_staged<2>), dim3(nb), dim3(64), 0, s, v, U, J);
       else hipLaunchKernelGGL((k_jac_fo_euler_staged<3>), dim3(nb), dim3(64), 0, s, v, U, J);

@@ -116,6 +116,20 @@ __device__ __forceinline__ int64_t velocity_lanes(const View &P, int64_t wg, con
   return r;
 }
 
+// the velocity of workgroup wg's rows; the row's lanes share its stores
+template <class Ph, int W>
+__device__ __forceinline__ void velocity_rows(const View &P, int64_t wg, const double *__restrict__ U,
+                                              double *__restrict__ V) {
+  constexpr int M = Ph::M, D = Ph::DIM;
+  double acc[M];
+  const int64_t r = velocity_lanes<Ph, W>(P, wg, U, acc);
+  if (r < 0) return;
+  const int a = int(threadIdx.x) % D;
+#pragma unroll
+  for (int k = 0; k < M; ++k)
+    if (k % D == a) V[r * M + k] = acc[k];
+}
+
 // ---------------------------------------------------------------- jacobian
 // interior row, one axis
 template <class Ph, int W, int A, bool WV>
