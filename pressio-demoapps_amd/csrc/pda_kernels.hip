@@ -243,6 +243,105 @@ __global__ void __launch_bounds__(64) k_jacobian(View P, const double *__restric
   rows::jacobian_row<Ph, W, WV>(P, int64_t(blockIdx.x) * blockDim.x + threadIdx.x, U, V, J);
 }
 
+// -------------------------------- advection-diffusion-reaction Jacobian rows
+// Rows of the scalar family's Jacobian (and, with WV, its velocity), inner and
+// near-boundary ones: two lanes per row, lane a forming axis a's entries and
+// its part of the diagonal (the terms of jac_axis_inner and jac_axis_near; the
+// flux takes the minus side alone, whose derivative by the plus side is 0).
+// The rows' values are put together in LDS and leave as contiguous runs.
+// Bound by latency (61,103 rows are two wavefronts per SIMD): 301 x 203 WENO5
+// 7.2 us, 11 with one thread per row, both sides' gradients and a store of
+// 8 bytes per value.
+template <int W, bool WV>
+__global__ void __launch_bounds__(64) k_jac_adr(View P, const double *__restrict__ U, double *__restrict__ V,
+                                                  double *__restrict__ J) {
+#pragma clang fp contract(off)
+  using Ph = PhAdr;
+  constexpr int NB = 1 + 4 * W, RPW = 32;
+  __shared__ double stage[RPW * NB];
+  __shared__ int64_t base_of[RPW]; // first CSR value of the row, -1: no row
+  __shared__ int blk_of[RPW];
+  const int lane = threadIdx.x, g = lane >> 1, a = lane & 1;
+  const int64_t t = int64_t(blockIdx.x) * RPW + g;
+  const int64_t r = t < P.nvisit ? (P.rows ? int64_t(P.rows[t]) : t) : -1;
+  const int32_t *gr = P.graph + (r >= 0 ? r : 0) * P.ncols;
+  const uint8_t *sl = P.slot + (r >= 0 ? r : 0) * P.npos;
+  double *st = stage + g * NB;
+  bool near = false;
+  double self = 0., acc[1] = {0.};
+  if (a == 0) {
+    base_of[g] = r >= 0 ? P.rowbase[r] : -1;
+    blk_of[g] = r >= 0 ? P.nblk[r] : 0;
+  }
+  if (r >= 0) {
+    const int64_t gi = P.ghost_row[r];
+    near = gi >= 0;
+    const double h = a ? P.hinv[1] : P.hinv[0], c = a ? P.p[1] : P.p[0];
+    const double diff = Sources<Ph>::offdiag(P, near, a, 0, 0);
+    const int cl = colof<2>(a, 0, 0), cr = colof<2>(a, 1, 0);
+    if (W == 1 || near) {
+      self = -c * h;
+      if (gr[cl] != -1) st[sl[cl]] = c * h + diff;
+      else self += (P.bcf[gi * 2 + a] * c) * h;
+      if (gr[cr] != -1) st[sl[cr]] = diff;
+    } else if constexpr (W > 1) {
+      int32_t src[2 * W + 1];
+      int minus, plus;
+      stencil_cells<2, W>(P, gr, a, src, minus, plus);
+      double q[2 * W + 1], lm, rm, unused, gl[2 * W], gr_[2 * W], ug[2 * W];
+#pragma unroll
+      for (int p = 0; p <= 2 * W; ++p) q[p] = U[src[p]];
+      if constexpr (W == 2) {
+        phys::weno3_grad(q, lm, unused, gl, ug);
+        phys::weno3_grad(q + 1, rm, unused, gr_, ug);
+      } else {
+        phys::weno5_grad(q, lm, unused, gl, ug);
+        phys::weno5_grad(q + 1, rm, unused, gr_, ug);
+      }
+#pragma unroll
+      for (int p = 0; p <= 2 * W; ++p) {
+        double v = 0.;
+        if (p < 2 * W) v += c * gl[p < 2 * W ? p : 0] * h;
+        if (p > 0) v -= c * gr_[p > 0 ? p - 1 : 0] * h;
+        if (p == W - 1 || p == W + 1) v += diff;
+        if (p == W) self = v;
+        else st[sl[p > W ? cr + 4 * (p - W - 1) : cl + 4 * (W - 1 - p)]] = v;
+      }
+    }
+    if constexpr (WV) rows::velocity_axis<Ph, W>(P, gr, near, a, U, acc);
+  }
+  double diag = __shfl(self, lane & ~1, 64) + __shfl(self, lane | 1, 64);
+  if constexpr (WV) acc[0] = __shfl(acc[0], lane & ~1, 64) + __shfl(acc[0], lane | 1, 64);
+  if (r >= 0 && a == 0) {
+    Sources<Ph>::apply(P, r, near, U, gr[0], acc, &diag);
+    st[sl[0]] = diag;
+    if constexpr (WV) V[r] = acc[0];
+  }
+  wave_sync();
+#pragma unroll
+  for (int q = lane; q < RPW * NB; q += 64) {
+    const int gg = q / NB, e = q - gg * NB;
+    const int64_t rb = base_of[gg];
+    if (rb >= 0 && e < blk_of[gg]) store_stream(J + rb + e, stage[q]);
+  }
+}
+
+int launch_jac_adr(const View &v, int w, const double *U, double *V, double *J, hipStream_t s) {
+  if (v.nvisit == 0) return PDA_OK;
+  const unsigned nb = unsigned((v.nvisit + 31) / 32);
+  if (V) {
+    if (w == 1) hipLaunchKernelGGL((k_jac_adr<1, true>), dim3(nb), dim3(64), 0, s, v, U, V, J);
+    else if (w == 2) hipLaunchKernelGGL((k_jac_adr<2, true>), dim3(nb), dim3(64), 0, s, v, U, V, J);
+    else hipLaunchKernelGGL((k_jac_adr<3, true>), dim3(nb), dim3(64), 0, s, v, U, V, J);
+  } else {
+    if (w == 1) hipLaunchKernelGGL((k_jac_adr<1, false>), dim3(nb), dim3(64), 0, s, v, U, V, J);
+    else if (w == 2) hipLaunchKernelGGL((k_jac_adr<2, false>), dim3(nb), dim3(64), 0, s, v, U, V, J);
+    else hipLaunchKernelGGL((k_jac_adr<3, false>), dim3(nb), dim3(64), 0, s, v, U, V, J);
+  }
+  PDA_HIP_CHECK(hipGetLastError());
+  return PDA_OK;
+}
+
 // ------------------------------- first-order Euler Jacobian, staged rows
 template <int D>
 __global__ void __launch_bounds__(64) k_jac_fo_euler_staged(View P, const double *__restrict__ U,
@@ -910,7 +1009,8 @@ static int jac_generic(const View &v, const pda_problem_s &p, const double *U, d
     case PDA_EULER3D: return jac_dispatch<PhEuler3>(v, p.w, U, V, J, s);
     case PDA_SWE2D: return jac_dispatch<PhSwe>(v, p.w, U, V, J, s);
     case PDA_BURGERS2D: return jac_dispatch<PhBurgers>(v, p.w, U, V, J, s);
-    case PDA_ADR2D: return jac_dispatch<PhAdr>(v, p.w, U, V, J, s);
+    case PDA_ADR2D: // merged columns are summed by one thread per row
+      return v.dup ? jac_dispatch<PhAdr>(v, p.w, U, V, J, s) : launch_jac_adr(v, p.w, U, V, J, s);
     default: set_error("jacobian: unsupported family"); return PDA_E_UNSUPPORTED;
   }
 }

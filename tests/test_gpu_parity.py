@@ -280,3 +280,20 @@ def test_random_shapes_match_oracle(case, oracle, torch):
     e = (cases.rel_err(Vg, Vo), cases.rel_err(V2g, V2o), cases.rel_err(Jg, Jo), cases.rel_err(Jvg, Jo))
     print(f"[gpu-parity] {case[0]}: V {e[0]:.2e} V(J path) {e[1]:.2e} J {e[2]:.2e} J alone {e[3]:.2e}", flush=True)
     assert max(e) <= TOL, e
+
+
+@pytest.mark.parametrize("n", [(7, 7), (8, 9), (33, 31), (64, 8)])
+@pytest.mark.parametrize("scheme", [S.FirstOrder, S.Weno3, S.Weno5], ids=lambda s: s.name)
+def test_adr_rows_of_partial_wavefronts(scheme, n, oracle, torch):
+    """The scalar family's Jacobian rows, 32 to a wavefront: one box cell, a
+    last wavefront with a few rows or with all of them; with and without the
+    velocity, pattern and values as the oracle's."""
+    print(f"[gpu-parity] adr {n} {scheme.name}", flush=True)
+    case = (f"adr-{n}", pda.AdvectionDiffusionReaction2d.ProblemA, scheme, n, (0, 1, 0, 1), 7, (), 0, None)
+    mesh, prob = cases.make(case)
+    U = cases.perturbed_state(prob, 2)
+    Vg, V2g, Jg, Jvg, rp, ci = _run_gpu(prob, U, torch)
+    V2o, rpo, cio, Jo = oracle.velocity_and_jacobian(oracle.from_mesh(mesh), cases.oracle_problem(case), U)
+    assert np.array_equal(rp, rpo) and np.array_equal(ci, cio)
+    assert max(cases.rel_err(Vg, V2o), cases.rel_err(V2g, V2o)) <= TOL
+    assert max(cases.rel_err(Jg, Jo), cases.rel_err(Jvg, Jo)) <= TOL
