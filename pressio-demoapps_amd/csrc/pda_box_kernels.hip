@@ -1093,9 +1093,30 @@ int64_t jacobian_strip_height(const Box &B) {
 // with 16 (at its best height, 4), measured with one lane per x face
 constexpr int J3SEG = 21;
 
-// default strip height (planes per workgroup) of that march, the fastest
-// at 256^3 (5.02 ms per jacobian() at 6, 5.11 at 5, 5.28 at 8, 5.46 at 2)
-constexpr int64_t J3_STRIP = 6;
+// Default strip height (planes per workgroup) of that march, us per jacobian():
+// - one plane where the states stay in the last-level cache (256 MB): workgroups
+//   in flight then write one range of the CSR, and the neighbouring planes'
+//   states are read from that cache (128^3 633, 694 at 6 planes; 160^3 1214, 1376;
+//   64^3 96, 108);
+// - four where they do not (192^3 2089, 2514 at 1, 2122 at 6; 256^3 4701, 5495,
+//   5018);
+// - the fewest rounds of the 1,280 workgroups that are resident where there are
+//   hardly more, a round lasting two planes' time and its own (24^3 1 plane 23, 39
+//   at 6; 32^3 2 planes 29; 40^3 3 planes 36, 41 at 1 and at 6).
+int64_t jacobian3d_strip_height(const Box &B) {
+  const int64_t bz = B.hi[2] - B.lo[2];
+  const int64_t lines = (B.hi[0] - B.lo[0] + J3SEG - 1) / J3SEG * (B.hi[1] - B.lo[1]);
+  if (lines * bz > 3072) return B.n[0] * B.n[1] * B.n[2] > int64_t(5000000) ? 4 : 1;
+  int64_t best = 1, cost = INT64_MAX;
+  for (int64_t h = 1; h <= bz; ++h) {
+    const int64_t c = (lines * ((bz + h - 1) / h) + 1279) / 1280 * (2 + h);
+    if (c < cost) {
+      cost = c;
+      best = h;
+    }
+  }
+  return best;
+}
 
 int launch_jacobian_fo_euler3d_box(const pda_problem_s &p, const double *U, double *J, hipStream_t s) {
   const Box &B = p.box;
@@ -1104,7 +1125,7 @@ int launch_jacobian_fo_euler3d_box(const pda_problem_s &p, const double *U, doub
       set_error("first-order 3D Jacobian march: box stencil leaves the grid");
       return PDA_E_INVALID_ARG;
     }
-  int64_t rps = J3_STRIP;
+  int64_t rps = jacobian3d_strip_height(B);
   if (p.jac_rps > 0) rps = p.jac_rps; // pda_problem_set_jacobian_strip_height
   const int64_t nseg = (B.hi[0] - B.lo[0] + J3SEG - 1) / J3SEG;
   const int64_t nstrip = (B.hi[2] - B.lo[2] + rps - 1) / rps;
