@@ -1012,7 +1012,6 @@ static int jac_box(const pda_problem_s &p, const double *U, double *J, double *V
   const Box &B = p.box;
   if constexpr (std::is_same<Ph, PhEuler2>::value) {
     if (V == nullptr) {
-      // strips of rows_per_strip rows: ~16k one-wave groups for the 1024^2 grid
       const int64_t nseg = (B.hi[0] - B.lo[0] + ESEG - 1) / ESEG;
       const int64_t bh = B.hi[1] - B.lo[1];
       int64_t rps = jacobian_strip_height(B);
@@ -1058,7 +1057,9 @@ static int64_t velocity_waves(const Box &B, int dim, int w) {
 // default strip height of the single-problem velocity march.  Each strip
 // evaluates extra rows of y values, so taller strips do less work but
 // give fewer waves; 2D grids aim at ~3 waves per SIMD (1024^2: 6 rows,
-// 3,078 waves on 1,024 SIMDs).  3D waves run two to a SIMD for the same time
+// 3,078 waves on 1,024 SIMDs; on states that are not in the caches 165 us with
+// the Jacobian at 6 rows, 177 at 10, whose 1,836 waves are 4 us faster on
+// states that are).  3D waves run two to a SIMD for the same time
 // each, so the height is the one with the fewest rows (a strip's own and half
 // a row for the values before its first) over the rounds of 2,048 waves (128^3:
 // 16 rows, 1,952 waves, 152 us; 150 to 190 at the others from 2 to 18, 217 at 24).
@@ -1079,12 +1080,18 @@ int64_t velocity_strip_height(const Box &B, int dim, int w) {
   return rps < 1 ? 1 : (rps > 64 ? 64 : rps);
 }
 
-// default strip height of the first-order 2D Euler Jacobian march: about
-// 16k one-wave groups (2 rows per strip at 1024^2)
+// Default strip height of the first-order 2D Euler Jacobian march (us with the
+// velocity before it):
+// - single rows where the states stay in the last-level cache (256 MB), so that
+//   the workgroups in flight write one range of the CSR (1024^2 167, 178 at 2
+//   rows; jacobian() alone at 2048^2 460, 493), else four (3000 x 2900 1056, 1175);
+// - where there are hardly more workgroups than the 2,048 resident ones, rows
+//   enough for about 1,024 (300 x 280 27.4 at 3 rows, 30.7 at 1; 150 x 300 23.0 at
+//   2, 24.6 at 1).
 int64_t jacobian_strip_height(const Box &B) {
-  const int64_t nseg = (B.hi[0] - B.lo[0] + ESEG - 1) / ESEG;
-  const int64_t rps = ((B.hi[1] - B.lo[1]) * nseg) / 16384;
-  return rps < 1 ? 1 : (rps > 64 ? 64 : rps);
+  const int64_t lines = (B.hi[0] - B.lo[0] + ESEG - 1) / ESEG * (B.hi[1] - B.lo[1]);
+  if (lines <= 3072) return (lines + 1023) / 1024;
+  return B.n[0] * B.n[1] > 6000000 ? 4 : 1;
 }
 
 // cells per x segment of the first-order 3D Euler Jacobian march: 3 x 21
