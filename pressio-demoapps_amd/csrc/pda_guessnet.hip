@@ -853,6 +853,11 @@ int backward(pda_guessnet_s &net, hipStream_t st) {
 int loss(pda_guessnet_s &net, const double *costs, bool want, hipStream_t st) {
   Costs c;
   for (int j = 0; j < NOUT; ++j) c.c[j] = costs[j];
+  if (want && !net.loss_ready) { // the first loss that is asked for; a network that only predicts has none
+    if (!net.hloss)
+      PDA_HIP_CHECK(hipHostMalloc(reinterpret_cast<void **>(&net.hloss), sizeof(double), hipHostMallocDefault));
+    PDA_HIP_CHECK(hipEventCreateWithFlags(&net.loss_ready, hipEventDisableTiming));
+  }
   const int rc = policy(net, &c, st, want ? net.hloss : nullptr);
   if (!rc && want) PDA_HIP_CHECK(hipEventRecord(net.loss_ready, st));
   return rc;
@@ -932,9 +937,6 @@ int pda_guessnet_create(int nx, int ny, pda_guessnet *out) {
   if (e == hipSuccess) e = net->pol.alloc(sizeof(double) * POL_LEN);
   if (e == hipSuccess) e = net->lg.alloc(sizeof(double) * (1 + NOUT));
   if (e == hipSuccess) e = net->dy.alloc(sizeof(float) * C);
-  if (e == hipSuccess)
-    e = hipHostMalloc(reinterpret_cast<void **>(&net->hloss), sizeof(double), hipHostMallocDefault);
-  if (e == hipSuccess) e = hipEventCreateWithFlags(&net->loss_ready, hipEventDisableTiming);
   if (e == hipSuccess) e = hipMemset(net->pol.ptr, 0, sizeof(double) * POL_LEN);
   if (e == hipSuccess) e = hipMemset(net->w.ptr, 0, sizeof(float) * wo);
   if (e == hipSuccess) e = hipMemset(net->m1.ptr, 0, sizeof(float) * wo);
