@@ -34,15 +34,27 @@ constexpr int MAXB = 1024; // most blocks (partial sums) of the reducing kernels
 // RHO, ALPHA and DONE, the update kernel W and NITER.
 enum { S_RHO = 0, S_RHO_NEXT, S_ALPHA, S_W, S_RR, S_BB, S_TOL2, S_DONE, S_DONE_NEXT, S_NITER, S_COUNT };
 
-__device__ __forceinline__ double block_sum(double v, double *sh) {
-  for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+// a and b become their sums over the block, the same in every thread
+__device__ __forceinline__ void block_sums(double &a, double &b, double *sh) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+    const double ta = __shfl_xor(a, o, 64), tb = __shfl_xor(b, o, 64);
+    a += ta;
+    b += tb;
+  }
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   __syncthreads();
-  if (l == 0) sh[w] = v;
+  if (l == 0) {
+    sh[w] = a;
+    sh[TB / 64 + w] = b;
+  }
   __syncthreads();
-  double s = 0.;
-  for (int i = 0; i < TB / 64; ++i) s += sh[i];
-  return s; // the same in every thread
+  a = b = 0.;
+#pragma unroll
+  for (int i = 0; i < TB / 64; ++i) {
+    a += sh[i];
+    b += sh[TB / 64 + i];
+  }
 }
 
 // The sums of n pairs of partial sums, in a fixed order, the same in every
@@ -55,13 +67,13 @@ __device__ __forceinline__ void sum_pairs(const double *__restrict__ part, int n
     a += part[2 * i];
     b += part[2 * i + 1];
   }
-  s1 = block_sum(a, sh);
-  s2 = block_sum(b, sh);
+  block_sums(a, b, sh);
+  s1 = a;
+  s2 = b;
 }
 
 __device__ __forceinline__ void put_pair(double *part, double s1, double s2, double *sh) {
-  s1 = block_sum(s1, sh);
-  s2 = block_sum(s2, sh);
+  block_sums(s1, s2, sh);
   if (threadIdx.x == 0) {
     part[2 * blockIdx.x] = s1;
     part[2 * blockIdx.x + 1] = s2;
@@ -71,7 +83,7 @@ __device__ __forceinline__ void put_pair(double *part, double s1, double s2, dou
 // the norms of up to two vectors from their partial sums, into host memory
 __global__ void __launch_bounds__(TB) k_norms_out(const double *__restrict__ pa, const double *__restrict__ pb, int n,
                                                   double *__restrict__ host) {
-  __shared__ double sh[TB / 64];
+  __shared__ double sh[2 * (TB / 64)];
   double s1, s2;
   sum_pairs(pa, n, sh, s1, s2);
   if (threadIdx.x == 0) host[0] = sqrt(s1);
@@ -156,8 +168,8 @@ __global__ void __launch_bounds__(TB) k_form(Blocks K, const double *__restrict_
 // (r0 . v) from its partial sums, and x = r - alpha v is formed as it is
 // gathered, for 50 MB more from L2 but without a launch and a vector for it.
 // Bound by the matrix, which stays in the last-level cache: 512 x 512 Burgers
-// (12 2 x 2 blocks a cell, 113 MB with their columns) 17.1 us (7.3 TB/s) and
-// 19.3 SECOND; 16 lanes per cell over the Jacobian's own CSR blocks 23.8, with
+// (12 2 x 2 blocks a cell, 113 MB with their columns) 17.0 us (7.4 TB/s) and
+// 18.9 SECOND; 16 lanes per cell over the Jacobian's own CSR blocks 23.8, with
 // 14.4 us of launches that applied Minv beside each product.
 // Partial sums of (r0 . y), or with SECOND of (y . x, y . y).
 template <int M, bool SECOND>
@@ -167,7 +179,7 @@ __global__ void __launch_bounds__(TB) k_spmv(const double *__restrict__ A, const
                                              double *__restrict__ y, int64_t per_block,
                                              const double *__restrict__ part_in, int npart,
                                              double *__restrict__ part, double *__restrict__ scal) {
-  __shared__ double sh[TB / 64];
+  __shared__ double sh[2 * (TB / 64)];
   constexpr int V = Ell<M>::V, PAIRS = Ell<M>::PAIRS;
   double alpha = 0.;
   if constexpr (SECOND) {
@@ -292,7 +304,7 @@ __global__ void __launch_bounds__(TB) k_block_inv(Blocks K, const double *__rest
 __global__ void __launch_bounds__(TB) k_start(const double *__restrict__ R, double *__restrict__ x,
                                               double *__restrict__ r, double *__restrict__ r0, int64_t n,
                                               double *__restrict__ part, double *__restrict__ scal) {
-  __shared__ double sh[TB / 64];
+  __shared__ double sh[2 * (TB / 64)];
   double s = 0.;
   for (int64_t i = int64_t(blockIdx.x) * TB + threadIdx.x; i < n; i += int64_t(gridDim.x) * TB) {
     const double b = -R[i];
@@ -326,7 +338,7 @@ __global__ void __launch_bounds__(TB) k_p(const double *__restrict__ r, double *
                                            const double *__restrict__ v, int64_t n,
                                            const double *__restrict__ part, int npart, double *__restrict__ scal,
                                            int first, double rtol) {
-  __shared__ double sh[TB / 64];
+  __shared__ double sh[2 * (TB / 64)];
   if (scal[S_DONE] != 0.) return; // written by earlier kernels: the same in every block
   const double alpha = scal[S_ALPHA], w = scal[S_W], rho = scal[S_RHO];
   double s1, s2;
@@ -344,18 +356,26 @@ __global__ void __launch_bounds__(TB) k_p(const double *__restrict__ r, double *
   }
   if (done) return;
   const double beta = (s1 / rho) * (alpha / w);
-  for (int64_t i = int64_t(blockIdx.x) * TB + threadIdx.x; i < n; i += int64_t(gridDim.x) * TB)
-    p[i] = first ? r[i] : r[i] + beta * (p[i] - w * v[i]);
+  auto next = [&](double ri, double pi, double vi) { return first ? ri : ri + beta * (pi - w * vi); };
+  const double2 *r2 = reinterpret_cast<const double2 *>(r), *v2 = reinterpret_cast<const double2 *>(v);
+  double2 *p2 = reinterpret_cast<double2 *>(p);
+  for (int64_t i = int64_t(blockIdx.x) * TB + threadIdx.x; i < n / 2; i += int64_t(gridDim.x) * TB) {
+    const double2 a = r2[i], b = p2[i], c = v2[i];
+    p2[i] = make_double2(next(a.x, b.x, c.x), next(a.y, b.y, c.y));
+  }
+  if ((n & 1) && blockIdx.x == 0 && threadIdx.x == 0) p[n - 1] = next(r[n - 1], p[n - 1], v[n - 1]);
 }
 
 // w = (t . s) / (t . t) from their partial sums; s = r - alpha v;
-// x += alpha p + w s; r = s - w t; partial sums of (r0 . r, r . r)
+// x += alpha p + w s; r = s - w t; partial sums of (r0 . r, r . r).  Two entries
+// per lane in 16-byte accesses, both sums of a block reduced together: 8.2 us at
+// 512 x 512 x 2 unknowns (33 MB, in the last-level cache), 8.8 entry by entry.
 __global__ void __launch_bounds__(TB) k_xr(double *__restrict__ x, double *__restrict__ r,
                                             const double *__restrict__ p, const double *__restrict__ v,
                                             const double *__restrict__ t, const double *__restrict__ r0, int64_t n,
                                             const double *__restrict__ part_in, int npart,
                                             double *__restrict__ part, double *__restrict__ scal) {
-  __shared__ double sh[TB / 64];
+  __shared__ double sh[2 * (TB / 64)];
   if (scal[S_DONE_NEXT] != 0.) return; // the last residual's partial sums stay
   const double alpha = scal[S_ALPHA];
   double ts, tt;
@@ -366,14 +386,25 @@ __global__ void __launch_bounds__(TB) k_xr(double *__restrict__ x, double *__res
     scal[S_NITER] += 1.; // read by no other block
   }
   double s1 = 0., s2 = 0.;
-  for (int64_t i = int64_t(blockIdx.x) * TB + threadIdx.x; i < n; i += int64_t(gridDim.x) * TB) {
-    const double si = r[i] - alpha * v[i];
-    x[i] += alpha * p[i] + w * si;
-    const double ri = si - w * t[i];
-    r[i] = ri;
-    s1 += r0[i] * ri;
+  auto update = [&](double &xi, double &ri, double pi, double vi, double ti, double qi) {
+    const double si = ri - alpha * vi;
+    xi += alpha * pi + w * si;
+    ri = si - w * ti;
+    s1 += qi * ri;
     s2 += ri * ri;
+  };
+  double2 *x2 = reinterpret_cast<double2 *>(x), *r2 = reinterpret_cast<double2 *>(r);
+  const double2 *p2 = reinterpret_cast<const double2 *>(p), *v2 = reinterpret_cast<const double2 *>(v);
+  const double2 *t2 = reinterpret_cast<const double2 *>(t), *q2 = reinterpret_cast<const double2 *>(r0);
+  for (int64_t i = int64_t(blockIdx.x) * TB + threadIdx.x; i < n / 2; i += int64_t(gridDim.x) * TB) {
+    double2 a = x2[i], b = r2[i];
+    const double2 pi = p2[i], vi = v2[i], ti = t2[i], qi = q2[i];
+    update(a.x, b.x, pi.x, vi.x, ti.x, qi.x);
+    update(a.y, b.y, pi.y, vi.y, ti.y, qi.y);
+    x2[i] = a;
+    r2[i] = b;
   }
+  if ((n & 1) && blockIdx.x == 0 && threadIdx.x == 0) update(x[n - 1], r[n - 1], p[n - 1], v[n - 1], t[n - 1], r0[n - 1]);
   put_pair(part, s1, s2, sh);
 }
 
@@ -381,7 +412,7 @@ __global__ void __launch_bounds__(TB) k_xr(double *__restrict__ x, double *__res
 enum { H_DONE = 0, H_NITER, H_RR, H_BB, H_COUNT };
 __global__ void __launch_bounds__(TB) k_check(const double *__restrict__ part, int npart,
                                               const double *__restrict__ scal, double *__restrict__ host) {
-  __shared__ double sh[TB / 64];
+  __shared__ double sh[2 * (TB / 64)];
   double s1, s2;
   sum_pairs(part, npart, sh, s1, s2);
   if (threadIdx.x != 0) return;
@@ -397,7 +428,7 @@ __global__ void __launch_bounds__(TB) k_residual(double *__restrict__ R, const d
                                                  const double *__restrict__ x2, double c2,
                                                  const double *__restrict__ F, double cf, int64_t n,
                                                  double *__restrict__ part) {
-  __shared__ double sh[TB / 64];
+  __shared__ double sh[2 * (TB / 64)];
   double s = 0.;
   for (int64_t i = int64_t(blockIdx.x) * TB + threadIdx.x; i < n; i += int64_t(gridDim.x) * TB) {
     double v = cnp1 * Y[i];
@@ -416,7 +447,7 @@ template <int M>
 __global__ void __launch_bounds__(TB) k_unscale(const double *__restrict__ Minv, const double *__restrict__ x,
                                                 double *__restrict__ dx, double *__restrict__ Y, int64_t ncell,
                                                 double *__restrict__ part) {
-  __shared__ double sh[TB / 64];
+  __shared__ double sh[2 * (TB / 64)];
   double s = 0.;
   for (int64_t c = int64_t(blockIdx.x) * TB + threadIdx.x; c < ncell; c += int64_t(gridDim.x) * TB) {
 #pragma unroll
