@@ -71,7 +71,7 @@ __host__ __device__ constexpr int ksteps(int cin) { return cin == C ? 9 : 3; }
 // third of a hidden layer's vector work).  z is kept above -87, where the
 // value is 1e-38, so that exp stays finite and the step defined.
 __device__ __forceinline__ float sigmoid(float z) {
-  const float d = 1.f + __expf(-fmaxf(z, -87.f));
+  const float d = 1.f + __expf(-__builtin_amdgcn_fmed3f(z, -87.f, 3.4e38f)); // fmaxf's two instructions in one
   const float r = __builtin_amdgcn_rcpf(d);
   return __fmaf_rn(r, __fmaf_rn(-d, r, 1.f), r);
 }
@@ -252,7 +252,10 @@ __global__ void __launch_bounds__(256) k_conv(ConvArgs A, Features T) {
           for (int i = 0; i < 4; ++i) {
             z[i] += bias[nt][i];
             o[i] = __bf16(silu(z[i]));
-            ysum[nt][i] += float(o[i]);
+          }
+          if (MODE == MODE_HIDDEN && A.csum) { // the last hidden layer
+#pragma unroll
+            for (int i = 0; i < 4; ++i) ysum[nt][i] += float(o[i]);
           }
           if (A.Z) *reinterpret_cast<f32x4 *>(A.Z + p * C + c) = z;
           *reinterpret_cast<bf16x4 *>(A.Y + p * C + c) = o;
