@@ -61,6 +61,37 @@ template <int A> __device__ __forceinline__ Mapped map_axis(const Box &B, int c)
   return m;
 }
 
+// a lane's column, mapped, and where its row 0 lies; ghost: some lane of the
+// wavefront has ghost signs
+struct Column {
+  const double *u;
+  int at, side;
+  bool ghost;
+};
+template <int M>
+__device__ __forceinline__ Column map_column(const Box &B, const double *__restrict__ U, int c) {
+  const Mapped m = map_axis<0>(B, c);
+  return {U + int64_t(m.at) * M, m.at, m.side, __any(m.side >= 0) != 0};
+}
+// state of the cell of column i in row j, both mapped
+template <int M>
+__device__ __forceinline__ void load_cell_mapped2(const View &P, const Box &B, const double *__restrict__ U,
+                                                  const Column &i, int64_t j, double *q) {
+  const Mapped jy = map_axis<1>(B, int(j));
+  const double *u = i.u + int64_t(jy.at) * B.n[0] * M;
+#pragma unroll
+  for (int k = 0; k < M; ++k) q[k] = u[k];
+  if (i.ghost) {
+    asm volatile(""); // a branch: as selects, every wavefront would wait for its loads here
+#pragma unroll
+    for (int k = 0; k < M; ++k) q[k] *= i.side < 0 ? 1. : (i.side == 0 ? P.gsign[0][0][k] : P.gsign[0][1][k]);
+  }
+  if (jy.side >= 0) {
+#pragma unroll
+    for (int k = 0; k < M; ++k) q[k] *= P.gsign[1][jy.side][k];
+  }
+}
+
 // value of lane l - 1 (lane_prev) or l + 1 (lane_next) of the wavefront,
 // by DPP wavefront shifts of the two halves; lane 0 (lane 63) gets 0 (by bound
 // control: a 0 to keep would be one more move per half)
@@ -115,44 +146,26 @@ __device__ __forceinline__ void vel_cc_body(const View &P, const Box &B, int row
   // lane l holds column iseg - W + l; lanes past the last column that the
   // segment's cells read hold that column again
   const int lc = lane < ncell + 2 * W - 1 ? lane : ncell + 2 * W - 1;
-  const int i = int(iseg) - W + lc;
   // The column is mapped once (only wavefronts at a mirror edge have ghost signs
   // to apply), a row by scalar instructions as it is loaded: mapped per lane and
   // row, with the row's sources read again from memory, a shallow-water step of
   // the loop had 944 instructions, 772 now (96 instances x 10 RK4 steps 6.49 ->
-  // 4.68 ms).
-  const Mapped ix = map_axis<0>(B, i);
-  const bool xghost = __any(ix.side >= 0);
-  const double *col = U + int64_t(ix.at) * M;
-  auto load_row = [&](int j, double (&q)[M]) {
-    const Mapped jy = map_axis<1>(B, j);
-    const double *u = col + int64_t(jy.at) * nx * M;
-#pragma unroll
-    for (int k = 0; k < M; ++k) q[k] = u[k];
-    if (xghost) {
-#pragma unroll
-      for (int k = 0; k < M; ++k)
-        q[k] *= ix.side < 0 ? 1. : (ix.side == 0 ? P.gsign[0][0][k] : P.gsign[0][1][k]);
-    }
-    if (jy.side >= 0) {
-#pragma unroll
-      for (int k = 0; k < M; ++k) q[k] *= P.gsign[1][jy.side][k];
-    }
-  };
+  // 4.26 ms).
+  const Column i = map_column<M>(B, U, int(iseg) - W + lc);
   const bool own = lane >= W && lane < W + ncell;
   const double hx = P.hinv[0], hy = P.hinv[1];
   // win[p] = row r + 2 - W + p at step r (W = 1: row r + 1); nxt = the
   // row that enters the window at the next step, loaded one step ahead
   double win[NR][M], nxt[M];
 #pragma unroll
-  for (int p = 0; p < NR; ++p) load_row(j0 - W + p, win[p]);
-  load_row(j0 - 1 + W, nxt);
+  for (int p = 0; p < NR; ++p) load_cell_mapped2<M>(P, B, U, i, j0 - W + p, win[p]);
+  load_cell_mapped2<M>(P, B, U, i, j0 - 1 + W, nxt);
   double qhi[M], fb[M];  // high-side y value of row r; flux of the face below row r
   // The loop is neither unrolled nor peeled: each face kind has one copy of
   // its code, so a face's value does not depend on the step that forms it
   // (the first two steps of a strip form the faces below it).
 #pragma clang loop unroll(disable)
-  for (int r = j0 - 2; r < j1; ++r) {
+  for (int64_t r = j0 - 2; r < j1; ++r) {
     if (r > j0 - 2) {
 #pragma unroll
       for (int p = 0; p + 1 < NR; ++p)
@@ -160,7 +173,7 @@ __device__ __forceinline__ void vel_cc_body(const View &P, const Box &B, int row
         for (int k = 0; k < M; ++k) win[p][k] = win[p + 1][k];
 #pragma unroll
       for (int k = 0; k < M; ++k) win[NR - 1][k] = nxt[k];
-      if (r + 1 < j1) load_row(r + 1 + W, nxt);
+      if (r + 1 < j1) load_cell_mapped2<M>(P, B, U, i, r + 1 + W, nxt);
     }
     // y face values of cell (i, r + 1)
     double yhi[M], ylo[M];
@@ -180,7 +193,7 @@ __device__ __forceinline__ void vel_cc_body(const View &P, const Box &B, int row
 #pragma unroll
         for (int k = 0; k < M; ++k) mid[k] = W >= 2 ? win[W >= 2 ? W - 2 : 0][k] : qhi[k];
         // the stage's terms, read here for the latency to pass under the x part
-        const int64_t e0 = soff + (int64_t(r) * nx + i) * M;
+        const int64_t e0 = soff + (r * nx + i.at) * M;
         double xt[4][M];
         if constexpr (STG && M <= 3) {
           if (own) {
@@ -215,7 +228,7 @@ __device__ __forceinline__ void vel_cc_body(const View &P, const Box &B, int row
           acc[k] += hy * (fb[k] - fa[k]);
         }
         if (own) {
-          const int64_t c = int64_t(r) * nx + i;
+          const int64_t c = r * nx + i.at;
           if constexpr (std::is_same<Ph, PhSwe>::value) Sources<Ph>::velocity(P, mid, acc);
           else Sources<Ph>::apply(P, c, false, U, int32_t(c), acc, nullptr);
           if constexpr (STG) {
@@ -262,7 +275,8 @@ __device__ __forceinline__ void vel_cc_body(const View &P, const Box &B, int row
 // value from the cell below and from the cell above, as planes are not carried.
 // Bound by FP64 issue: 1,750 FP64 instructions a row of 62 cells against 5,300
 // evaluating every face's two sides by themselves; WENO5 at 128^3 179 us (244).
-constexpr int V3OWN = 62; // cells a wavefront owns of its 64
+constexpr int VSEG = 63;         // a wavefront's last lane; it and lane 0 overlap the neighbouring wavefronts
+constexpr int V3OWN = VSEG - 1;  // cells it owns
 
 // cell index c along axis A, wrapped where the box covers a periodic axis whole
 // (the box keeps every stencil inside the grid otherwise)
@@ -281,7 +295,8 @@ __device__ __forceinline__ void vel_cc3_body(const View &P, const Box &B, int ro
   static_assert(Ph::DIM == 3, "3D march");
   constexpr int M = Ph::M, NR = 2 * W - 1;
   const int lane = threadIdx.x;
-  const int nx = int(B.n[0]), ny = int(B.n[1]);
+  const int64_t nx = B.n[0];
+  const int ny = int(B.n[1]);
   const int bw = int(B.hi[0] - B.lo[0]), line = bw + 2;
   const int64_t ncell = int64_t(line) * (B.hi[2] - B.lo[2]);
   const int64_t nwave = (ncell - 2 + V3OWN - 1) / V3OWN;
@@ -290,17 +305,19 @@ __device__ __forceinline__ void vel_cc3_body(const View &P, const Box &B, int ro
   const int j1 = j0 + rows_per_strip < int(B.hi[1]) ? j0 + rows_per_strip : int(B.hi[1]);
   const int64_t s0 = wave * V3OWN + lane, s = s0 < ncell ? s0 : ncell - 1;
   const int plane = int(s / line), e = int(s - int64_t(plane) * line);
-  const int i = int(B.lo[0]) + e - 1, kz = int(B.lo[2]) + plane;
+  const int kz = int(B.lo[2]) + plane, xe = int(B.lo[0]) + e - 1;
+  const int64_t i = wrap_axis<0>(B, xe);
+  // a column inside the grid for every lane's reads, whatever the box
+  const int64_t ic = i < nx ? i : nx - 1;
   const bool own = lane >= 1 && lane <= V3OWN && s0 < ncell && e >= 1 && e <= bw;
   const double hx = P.hinv[0], hy = P.hinv[1], hz = P.hinv[2];
   // places of the x and z stencils relative to the lane's cell of the row, in cells
-  const int ic = wrap_axis<0>(B, i);
   int dx[NR];
   int dz[2 * W + 1];
 #pragma unroll
-  for (int p = 0; p < NR; ++p) dx[p] = wrap_axis<0>(B, i + p - (W - 1)) - ic;
+  for (int p = 0; p < NR; ++p) dx[p] = wrap_axis<0>(B, xe + p - (W - 1)) - int(ic);
 #pragma unroll
-  for (int p = 0; p <= 2 * W; ++p) dz[p] = (wrap_axis<2>(B, kz + p - W) - kz) * nx * ny;
+  for (int p = 0; p <= 2 * W; ++p) dz[p] = (wrap_axis<2>(B, kz + p - W) - kz) * int(nx) * ny;
   const double *col = U + (int64_t(kz) * nx * ny + ic) * M; // row 0 of the lane's column
   const int64_t row = int64_t(nx) * M;
   auto load = [&](const double *u, double (&q)[M]) {
