@@ -98,7 +98,13 @@ __global__ void __launch_bounds__(256) k_apply_rows(View P, const int32_t *__res
       if (w > 1) {
 #pragma unroll
         for (int q = 0; q < w / 2; ++q) {
-          const double keep = up ? acc[w / 2 + q] : acc[q], give = up ? acc[q] : acc[w / 2 + q];
+          double lo = acc[q], hi = acc[w / 2 + q];
+          // both read before the choice: the compiler otherwise chooses the index
+          // and searches acc for it (at 16 sums 1,300 more instructions: five
+          // row-major columns of first-order Burgers on 500 x 512 cells 180 us
+          // with the Jacobian, 56 now)
+          asm volatile("" : "+v"(lo), "+v"(hi));
+          const double keep = up ? hi : lo, give = up ? lo : hi;
           acc[q] = keep + __shfl_xor(give, o, 64);
         }
         if (up) first += w / 2;
