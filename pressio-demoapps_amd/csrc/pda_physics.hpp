@@ -59,11 +59,13 @@ __device__ __forceinline__ double frsqrt(double x) {
 // to 1e-12 (differentiated as WENO5 below, the gradients are a thousand times
 // nearer to extended precision and up to 3e-12 from the reference's).  The
 // quotients are fdiv's, rounded as the IEEE sequence rounds them but for rare
-// last places.
+// last places.  S and the numerators over S^2 carry powers of two (exact, no
+// other bits), as S^2 is 1 / B^4 and would leave the normal range at cell
+// differences of 1e38; with them the gradients hold to 2e41.
 __device__ __forceinline__ void weno3_grad(const double *q, double &un, double &up,
                                            double *gn, double *gp) {
 #pragma clang fp contract(off)
-  constexpr double eps = 1.e-6, c13 = 1. / 3., c23 = 2. / 3.;
+  constexpr double eps = 1.e-6, c13 = 1. / 3., c23 = 2. / 3., KS = 0x1p46, KS2 = 0x1p92;
   {
     const double qim1 = q[0], qi = q[1], qip1 = q[2];
     const double p0 = (-qim1 + 3. * qi) * 0.5, p1 = (qi + qip1) * 0.5;
@@ -74,12 +76,13 @@ __device__ __forceinline__ void weno3_grad(const double *q, double &un, double &
     const double s = fdiv(1., a0 + a1);
     const double e0 = B0 + eps, e1 = B1 + eps;
     const double e03 = e0 * e0 * e0, e13 = e1 * e1 * e1;
-    const double S = fdiv(2., 3. * (e1 * e1)) + fdiv(1., 3. * (e0 * e0));
+    const double S = fdiv(2. * KS, 3. * (e1 * e1)) + fdiv(KS, 3. * (e0 * e0));
     const double S2 = S * S;
     const double x0 = fdiv(4. * d0, 3. * e03), x1 = fdiv(8. * d1, 3. * e13);
     const double da0[3] = {-x0, x0, 0.};
     const double da1[3] = {0., -x1, x1};
-    const double ds[3] = {fdiv(4. * d0, 3. * e03 * S2), -fdiv(x0 - x1, S2), -fdiv(8. * d1, 3. * S2 * e13)};
+    const double ds[3] = {fdiv((4. * KS2) * d0, 3. * e03 * S2), -fdiv(KS2 * (x0 - x1), S2),
+                          -fdiv((8. * KS2) * d1, 3. * S2 * e13)};
     const double dp0[3] = {-0.5, 1.5, 0.}, dp1[3] = {0., 0.5, 0.5};
     const double w0 = a0 * s, w1 = a1 * s;
     for (int i = 0; i < 3; ++i) {
@@ -101,12 +104,13 @@ __device__ __forceinline__ void weno3_grad(const double *q, double &un, double &
     const double w0 = a0 * s, w1 = a1 * s;
     const double e0 = B0 + eps, e1 = B1 + eps;
     const double e03 = e0 * e0 * e0, e13 = e1 * e1 * e1;
-    const double S = fdiv(1., 3. * (e1 * e1)) + fdiv(2., 3. * (e0 * e0));
+    const double S = fdiv(KS, 3. * (e1 * e1)) + fdiv(2. * KS, 3. * (e0 * e0));
     const double S2 = S * S;
     const double x0 = fdiv(8. * d0, 3. * e03), x1 = fdiv(4. * d1, 3. * e13);
     const double da0[3] = {-x0, x0, 0.};
     const double da1[3] = {0., -x1, x1};
-    const double ds[3] = {fdiv(8. * d0, 3. * e03 * S2), -fdiv(x0 - x1, S2), -fdiv(4. * d1, 3. * S2 * e13)};
+    const double ds[3] = {fdiv((8. * KS2) * d0, 3. * e03 * S2), -fdiv(KS2 * (x0 - x1), S2),
+                          -fdiv((4. * KS2) * d1, 3. * S2 * e13)};
     const double dp0[3] = {0.5, 0.5, 0.}, dp1[3] = {0., 1.5, -0.5};
     for (int i = 0; i < 3; ++i) {
       double v = (da0[i] * s + ds[i] * a0) * p0 + dp0[i] * w0;
@@ -239,6 +243,9 @@ __device__ __forceinline__ void weno3_cell_1div(double a, double b, double c, do
 // reciprocals and about 90 operations a value instead of eight divisions and
 // about 260.  The 2D Euler WENO5 Jacobian with velocity of 509 x 387 cells is
 // bound by FP64 issue: 109 us (138 in the reference's form).
+// The products of the E_k carry 2^-250 (two multiplications, no other bits): of
+// the eighth degree in the differences, they would overflow at 1e34 to 1e38,
+// where the reference's form holds to 1e39; with it the gradients hold to 1e50.
 
 // q = cells i-2 .. i+2: the value of cell i at the face towards i+1 (w5_hi's,
 // bit for bit) and its gradient by the five cells
@@ -252,7 +259,8 @@ __device__ __forceinline__ double weno5_side_grad(double q0, double q1, double q
   const double E0 = __fma_rn(k0, t0, __fma_rn(a0, a0, eps4));
   const double E1 = __fma_rn(k1, t1, __fma_rn(a1, a1, eps4));
   const double E2 = __fma_rn(k2, t2, __fma_rn(a2, a2, eps4));
-  const double p0 = E1 * E2, p1 = E0 * E2, p2 = E0 * E1;
+  const double E0s = 0x1p-250 * E0, E2s = 0x1p-250 * E2;
+  const double p0 = E1 * E2s, p1 = E0 * E2s, p2 = E0s * E1;
   const double s0 = p0 * p0, s1 = 6. * (p1 * p1), m2 = 3. * (p2 * p2);
   const double iD = frcp((s0 + s1) + m2), iE = -4. * frcp(p0 * E0);
   const double c0 = __fma_rn(5., e2, -2. * e1), c1 = __fma_rn(2., e3, e2), c2 = __fma_rn(4., e3, -e4);
