@@ -415,8 +415,8 @@ __device__ __forceinline__ void vel_cc3_body(const View &P, const Box &B, int ro
               below[k] = c[0];
               above[k] = c[2];
             } else if constexpr (W == 2) {
-              below[k] = phys::w3_hi(c[0], c[1], c[2], phys::w3_d(c[0], c[1]), phys::w3_d(c[1], c[2]));
-              above[k] = phys::w3_lo(c[2], c[3], c[4], phys::w3_d(c[2], c[3]), phys::w3_d(c[3], c[4]));
+              below[k] = phys::weno3_side_1div(c[0], c[1], c[2]);
+              above[k] = phys::weno3_side_1div(c[4], c[3], c[2]);
             } else {
               below[k] = phys::weno5_side_1div(c[0], c[1], c[2], c[3], c[4]);
               above[k] = phys::weno5_side_1div(c[6], c[5], c[4], c[3], c[2]);

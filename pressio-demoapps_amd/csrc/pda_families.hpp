@@ -421,6 +421,7 @@ struct FaceGrads {
   double glm[M][2 * W], glp[M][2 * W], grm[M][2 * W], grp[M][2 * W];
 };
 
+// (in the wide form, which leaves the bits as they are)
 template <int M, int W>
 __device__ __forceinline__ void reconstruct(const double st[][M], Faces<M, W> &f) {
 #pragma unroll
@@ -431,14 +432,13 @@ __device__ __forceinline__ void reconstruct(const double st[][M], Faces<M, W> &f
     if constexpr (W == 1) {
       f.lm[k] = q[0]; f.lp[k] = q[1]; f.rm[k] = q[1]; f.rp[k] = q[2];
     } else if constexpr (W == 2) {
-      double un, up;
-      phys::weno3_1div(q, f.lm[k], up);
-      phys::weno3_cell_1div(q[1], q[2], q[3], f.rm[k], f.lp[k]);
-      phys::weno3_1div(q + 1, un, f.rp[k]);
+      f.lm[k] = phys::weno3_side_1div<true>(q[0], q[1], q[2]);
+      phys::weno3_cell_1div<true>(q[1], q[2], q[3], f.rm[k], f.lp[k]);
+      f.rp[k] = phys::weno3_side_1div<true>(q[4], q[3], q[2]);
     } else {
-      f.lm[k] = phys::weno5_side_1div(q[0], q[1], q[2], q[3], q[4]);
-      phys::weno5_cell_1div(q[1], q[2], q[3], q[4], q[5], f.rm[k], f.lp[k]);
-      f.rp[k] = phys::weno5_side_1div(q[6], q[5], q[4], q[3], q[2]);
+      f.lm[k] = phys::weno5_side_1div<true>(q[0], q[1], q[2], q[3], q[4]);
+      phys::weno5_cell_1div<true>(q[1], q[2], q[3], q[4], q[5], f.rm[k], f.lp[k]);
+      f.rp[k] = phys::weno5_side_1div<true>(q[6], q[5], q[4], q[3], q[2]);
     }
   }
 }

@@ -167,9 +167,9 @@ __global__ void __launch_bounds__(S1_WAVES * 64) k_steps1d(View P, int64_t n, in
       if constexpr (W == 1) {
         v = q[k][0];
       } else if constexpr (W == 2) {
-        v = phys::w3_hi(q[k][0], q[k][1], q[k][2], phys::w3_d(q[k][0], q[k][1]), phys::w3_d(q[k][1], q[k][2]));
+        v = phys::weno3_side_1div<true>(q[k][0], q[k][1], q[k][2]);
       } else {
-        v = phys::weno5_side_1div(q[k][0], q[k][1], q[k][2], q[k][3], q[k][4]);
+        v = phys::weno5_side_1div<true>(q[k][0], q[k][1], q[k][2], q[k][3], q[k][4]);
       }
       const double o = quad_swap<0xB1>(v);
       um[k] = sd ? o : v;

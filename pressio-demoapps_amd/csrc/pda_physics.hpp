@@ -137,10 +137,18 @@ __device__ __forceinline__ void weno3_grad(const double *q, double &un, double &
 // same for a window read from either side, so a face value does not depend on
 // which of the forms below gives it.  58 operations for the two values of a cell
 // (85 as weighted candidates with the B's and their squares formed apart).
+// The products of the E's are of the eighth degree in the differences, and with
+// the differences they multiply they overflow, which gives NaN, where those
+// reach about 2e33.  WIDE: the products carry 2^-350 (two multiplications, exact:
+// no other bits), which moves that to 6e56 and keeps every term normal for
+// differences down to 1e-75.  The general row kernels and the 1D steps take it (the
+// form with a division per weight held to 1e77 there); the box kernels, bound by
+// FP64 issue, do not (their earlier weights, of the same degree, held to 6e33).
 struct W5 {
   double e1, e2, e3, e4; // the differences
   double s0, s1, s2;     // Prod E^2 without window 0, 6 times without 1, without 2
 };
+template <bool WIDE = false>
 __device__ __forceinline__ W5 w5_window(double q0, double q1, double q2, double q3, double q4) {
   constexpr double eps4 = 4.e-6, c133 = 13. / 3.;
   W5 w;
@@ -153,7 +161,9 @@ __device__ __forceinline__ W5 w5_window(double q0, double q1, double q2, double 
   const double E0 = __fma_rn(c133 * t0, t0, __fma_rn(a0, a0, eps4));
   const double E1 = __fma_rn(c133 * t1, t1, __fma_rn(a1, a1, eps4));
   const double E2 = __fma_rn(c133 * t2, t2, __fma_rn(a2, a2, eps4));
-  const double p0 = E1 * E2, p1 = E0 * E2, p2 = E0 * E1;
+  constexpr double scale = WIDE ? 0x1p-350 : 1.;
+  const double E0s = scale * E0, E2s = scale * E2;
+  const double p0 = E1 * E2s, p1 = E0 * E2s, p2 = E0s * E1;
   w.s0 = p0 * p0;
   w.s1 = 6. * (p1 * p1);
   w.s2 = p2 * p2;
@@ -178,26 +188,20 @@ __device__ __forceinline__ double w5_lo(const W5 &w, double q2) {
   return __fma_rn(-c16, w_quot(n, (w.s2 + w.s1) + m0), q2);
 }
 // the left-biased value: of cell q2 at the face towards q3
+template <bool WIDE = false>
 __device__ __forceinline__ double weno5_side_1div(double q0, double q1, double q2, double q3,
                                                   double q4) {
-  return w5_hi(w5_window(q0, q1, q2, q3, q4), q2);
-}
-
-// q = {q_{i-2}, ..., q_{i+3}}; un, up: left and right states of face i+1/2
-__device__ __forceinline__ void weno5_1div(const double *q, double &un, double &up) {
-  un = weno5_side_1div(q[0], q[1], q[2], q[3], q[4]);
-  // mirrored stencil: the right state of the face is the left-biased
-  // reconstruction of the reversed sequence
-  up = weno5_side_1div(q[5], q[4], q[3], q[2], q[1]);
+  return w5_hi(w5_window<WIDE>(q0, q1, q2, q3, q4), q2);
 }
 
 // Both face values of one cell from q = cells i-2 .. i+2: hi = the left
-// state of face i+1/2, lo = the right state of face i-1/2.  Bit-identical to
-// the two weno5_side_1div calls of weno5_1div at those faces; the windows are
-// formed once.
+// state of face i+1/2, lo = the right state of face i-1/2 (the left-biased value
+// of the reversed cells).  Bit-identical to the two weno5_side_1div calls at
+// those faces; the windows are formed once.
+template <bool WIDE = false>
 __device__ __forceinline__ void weno5_cell_1div(double q0, double q1, double q2, double q3,
                                                 double q4, double &hi, double &lo) {
-  const W5 w = w5_window(q0, q1, q2, q3, q4);
+  const W5 w = w5_window<WIDE>(q0, q1, q2, q3, q4);
   hi = w5_hi(w, q2);
   lo = w5_lo(w, q2);
 }
@@ -205,11 +209,14 @@ __device__ __forceinline__ void weno5_cell_1div(double q0, double q1, double q2,
 // WENO3 counterparts (impl/weno3.hpp:56-132): D = (eps + B)^2 of the two-cell
 // window (a, b) with B = (a - b)^2, the same in either direction, and the
 // values as corrections: the candidates at the face of b towards c are
-// b + (b - a) / 2 and b + (c - b) / 2 with weights 1/3 and 2/3.
+// b + (b - a) / 2 and b + (c - b) / 2 with weights 1/3 and 2/3.  WIDE: D carries
+// 2^-300, and the values hold over the whole range of D (differences of 1e77;
+// 1e61 without).
+template <bool WIDE = false>
 __device__ __forceinline__ double w3_d(double a, double b) {
-  constexpr double eps = 1.e-6;
+  constexpr double eps = 1.e-6, scale = WIDE ? 0x1p-300 : 1.;
   const double d = a - b, E = __fma_rn(d, d, eps);
-  return E * E;
+  return E * (scale * E);
 }
 // the face values of cell b (neighbours a below, c above) from the windows'
 // D: hi at the face towards c, lo at the face towards a
@@ -220,13 +227,15 @@ __device__ __forceinline__ double w3_hi(double a, double b, double c, double Dab
 __device__ __forceinline__ double w3_lo(double a, double b, double c, double Dab, double Dbc) {
   return w3_hi(c, b, a, Dbc, Dab);
 }
-__device__ __forceinline__ void weno3_1div(const double *q, double &un, double &up) {
-  un = w3_hi(q[0], q[1], q[2], w3_d(q[0], q[1]), w3_d(q[1], q[2]));
-  up = w3_lo(q[1], q[2], q[3], w3_d(q[1], q[2]), w3_d(q[2], q[3]));
+// the left-biased value: of cell b at the face towards c
+template <bool WIDE = false>
+__device__ __forceinline__ double weno3_side_1div(double a, double b, double c) {
+  return w3_hi(a, b, c, w3_d<WIDE>(a, b), w3_d<WIDE>(b, c));
 }
-// both face values of cell b, bit-identical to weno3_1div's at its faces
+// both face values of cell b, bit-identical to weno3_side_1div's at its faces
+template <bool WIDE = false>
 __device__ __forceinline__ void weno3_cell_1div(double a, double b, double c, double &hi, double &lo) {
-  const double Dab = w3_d(a, b), Dbc = w3_d(b, c);
+  const double Dab = w3_d<WIDE>(a, b), Dbc = w3_d<WIDE>(b, c);
   hi = w3_hi(a, b, c, Dab, Dbc);
   lo = w3_lo(a, b, c, Dab, Dbc);
 }
@@ -244,8 +253,8 @@ __device__ __forceinline__ void weno3_cell_1div(double a, double b, double c, do
 // about 260.  The 2D Euler WENO5 Jacobian with velocity of 509 x 387 cells is
 // bound by FP64 issue: 109 us (138 in the reference's form).
 // The products of the E_k carry 2^-250 (two multiplications, no other bits): of
-// the eighth degree in the differences, they would overflow at 1e34 to 1e38,
-// where the reference's form holds to 1e39; with it the gradients hold to 1e50.
+// the eighth degree in the differences, they would overflow at 2e33 to 1e38,
+// where the reference's form holds to 1e39; with it the gradients hold to 8e49.
 
 // q = cells i-2 .. i+2: the value of cell i at the face towards i+1 (w5_hi's,
 // bit for bit) and its gradient by the five cells
