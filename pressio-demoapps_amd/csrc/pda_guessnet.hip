@@ -122,8 +122,8 @@ __device__ __forceinline__ bf16x8 features(const Features &T, int64_t p) {
 //                csum[c][block])
 //   MODE_OUT:    out[p][c] = acc + bias for c < NOUT (FP32)
 //   MODE_BWD:    dZprev[p][c] = acc * SiLU'(Zprev[p][c]) (bf16), no bias
-// A workgroup of four waves owns a tile of CT_W columns x 4 RW rows (RW rows
-// per wave).  The tile and its halo are staged in LDS once, [pixel][channel]
+// A workgroup of four waves owns a tile of 128 RW pixels, TW columns x 128 RW / TW
+// rows (tile_of's choice), 32 RW consecutive ones per wave.  The tile and its halo are staged in LDS once, [pixel][channel]
 // as in memory, so a pixel operand is one 16-byte LDS read for every tap and
 // no lane computes addresses or wraps per tap; the layer's weights stay in
 // registers.  M = output channels and N = pixels, so that a lane ends with
@@ -134,8 +134,6 @@ __device__ __forceinline__ bf16x8 features(const Features &T, int64_t p) {
 // every lane gathered its pixels per tap from memory.  Loading the tile in a
 // loop that waits for each 16 bytes took 17.4 us.
 enum { MODE_FIRST = 0, MODE_HIDDEN = 1, MODE_OUT = 2, MODE_BWD = 3 };
-constexpr int CT_W = 32; // columns of a tile
-
 struct ConvArgs {
   const __bf16 *X, *Wp;
   const float *bias;
@@ -147,15 +145,15 @@ struct ConvArgs {
   float *csum;
 };
 
-template <int MODE, int RW>
+template <int MODE, int RW, int TW>
 __global__ void __launch_bounds__(256) k_conv(ConvArgs A, Features T) {
   constexpr int CIN = MODE == MODE_FIRST ? CIN0 : C, NT = MODE == MODE_OUT ? 1 : 2, KS = ksteps(CIN);
-  constexpr int TR = 4 * RW, XW = CT_W + 2, NV = CIN / 8, NPT = CT_W / 16;
+  constexpr int TR = 128 * RW / TW, XW = TW + 2, NV = CIN / 8, NPT = 2; // NPT: MFMA pixel tiles of 32 pixels
   __shared__ __align__(16) __bf16 sx[(TR + 2) * XW * CIN];
   __shared__ float ssum[4][C];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 15, g = lane >> 4;
   const int H = A.H, W = A.W;
-  const int x0 = (int(blockIdx.x) % A.ntx) * CT_W, y0 = (int(blockIdx.x) / A.ntx) * TR;
+  const int x0 = (int(blockIdx.x) % A.ntx) * TW, y0 = (int(blockIdx.x) / A.ntx) * TR;
   // every load of the tile in flight before the first LDS store
   constexpr int TOT = (TR + 2) * XW * NV, PER = (TOT + 255) / 256;
   bf16x8 stg[PER];
@@ -170,7 +168,7 @@ __global__ void __launch_bounds__(256) k_conv(ConvArgs A, Features T) {
     const int64_t p = int64_t(y) * W + x;
     if constexpr (MODE == MODE_FIRST) {
       stg[k] = features(T, p);
-      if (A.X0 && px >= 1 && px <= CT_W && row >= 1 && row <= TR && x0 - 1 + px < W && y0 - 1 + row < H)
+      if (A.X0 && px >= 1 && px <= TW && row >= 1 && row <= TR && x0 - 1 + px < W && y0 - 1 + row < H)
         *reinterpret_cast<bf16x8 *>(A.X0 + p * CIN) = stg[k];
     } else {
       stg[k] = *reinterpret_cast<const bf16x8 *>(A.X + p * CIN + 8 * v);
@@ -201,7 +199,10 @@ __global__ void __launch_bounds__(256) k_conv(ConvArgs A, Features T) {
   __syncthreads();
 #pragma unroll 1
   for (int rr = 0; rr < RW; ++rr) {
-    const int row = wave * RW + rr, y = y0 + row;
+    // pixel i of the 32: tile column (32 (wave RW + rr) + i) % TW of that row
+    const int p0 = 32 * (wave * RW + rr);
+    auto row_of = [&](int pt) { return (p0 + 16 * pt + r) / TW; };
+    auto col_of = [&](int pt) { return (16 * pt + r) % TW; };
     f32x4 acc[NPT][NT];
 #pragma unroll
     for (int pt = 0; pt < NPT; ++pt)
@@ -214,8 +215,7 @@ __global__ void __launch_bounds__(256) k_conv(ConvArgs A, Features T) {
       const int tap = CIN == C ? s : (4 * s + g < 9 ? 4 * s + g : 8);
 #pragma unroll
       for (int pt = 0; pt < NPT; ++pt) {
-        const int px = 16 * pt + r;
-        bf16x8 a = *reinterpret_cast<const bf16x8 *>(sx + ((row + tap / 3) * XW + px + tap % 3) * CIN +
+        bf16x8 a = *reinterpret_cast<const bf16x8 *>(sx + ((row_of(pt) + tap / 3) * XW + col_of(pt) + tap % 3) * CIN +
                                                      (CIN == C ? 8 * g : 0));
         if constexpr (CIN != C) {
           if (4 * s + g >= 9)
@@ -229,7 +229,7 @@ __global__ void __launch_bounds__(256) k_conv(ConvArgs A, Features T) {
     }
 #pragma unroll
     for (int pt = 0; pt < NPT; ++pt) {
-      const int x = x0 + 16 * pt + r;
+      const int x = x0 + col_of(pt), y = y0 + row_of(pt);
       if (x >= W || y >= H) continue;
       const int64_t p = int64_t(y) * W + x;
 #pragma unroll
@@ -281,16 +281,34 @@ __global__ void __launch_bounds__(256) k_conv(ConvArgs A, Features T) {
   }
 }
 
-// rows per wave: 4 where that still gives the chip a workgroup per CU (fewer
-// halo pixels, 1.20 times the tile against 1.59, and the weights loaded for
-// more pixels: a hidden layer at 512 x 512 takes 16.3 us with 4 rows, 16.9 with
-// 2, 18.0 with 1), else 1
-inline int conv_rows(int H, int W) {
-  return int64_t((W + CT_W - 1) / CT_W) * ((H + 15) / 16) >= 256 ? 4 : 1;
+// The tile's shape.  RW: 4 where that still gives the chip a workgroup per CU
+// (fewer halo pixels, 1.20 times the tile against 1.59, and the weights loaded for
+// more pixels: a hidden layer at 512 x 512 takes 16.3 us with 4, 16.9 with 2, 18.0
+// with 1), else 1, and 1 too on grids so low that it stages fewer pixels.  TW: 32
+// columns, or 8 where those stage at most three quarters of the pixels, as on
+// grids of fewer columns than 32, most of whose tile would be columns that are
+// not there (predict on 8 x 65536 pixels 156 -> 84 us, 4 x 131072 270 -> 117,
+// 131072 x 4 162 -> 105; pixels in linear order, gathered per tap, 133).
+struct Tile {
+  int rw, tw, ntx, nty;
+};
+inline Tile tile_of(int H, int W) {
+  auto shape = [&](int rw, int tw) {
+    const int tr = 128 * rw / tw;
+    return Tile{rw, tw, (W + tw - 1) / tw, (H + tr - 1) / tr};
+  };
+  auto blocks = [](const Tile &t) { return int64_t(t.ntx) * t.nty; };
+  auto staged = [&](const Tile &t) { return blocks(t) * (t.tw + 2) * (128 * t.rw / t.tw + 2); };
+  auto pick = [&](int tw) {
+    const Tile big = shape(4, tw), small = shape(1, tw);
+    return blocks(big) >= 256 && staged(big) <= staged(small) ? big : small;
+  };
+  const Tile wide = pick(32), narrow = pick(8);
+  return 4 * staged(narrow) <= 3 * staged(wide) ? narrow : wide;
 }
 inline int conv_blocks(int H, int W) {
-  const int tr = 4 * conv_rows(H, W);
-  return ((W + CT_W - 1) / CT_W) * ((H + tr - 1) / tr);
+  const Tile t = tile_of(H, W);
+  return t.ntx * t.nty;
 }
 
 // Backward-weight of a hidden layer: dW[tap][cout][cin] = sum_p dZ[p][cout]
@@ -767,12 +785,15 @@ int policy(pda_guessnet_s &net, const Costs *costs, hipStream_t st, double *host
 
 template <int MODE>
 void conv(const pda_guessnet_s &net, ConvArgs A, const Features &T, hipStream_t st) {
+  const Tile t = tile_of(net.H, net.W);
   A.H = net.H;
   A.W = net.W;
-  A.ntx = (net.W + CT_W - 1) / CT_W;
-  const dim3 grid{unsigned(conv_blocks(net.H, net.W)), 1, 1};
-  if (conv_rows(net.H, net.W) == 4) hipLaunchKernelGGL((k_conv<MODE, 4>), grid, dim3(256), 0, st, A, T);
-  else hipLaunchKernelGGL((k_conv<MODE, 1>), grid, dim3(256), 0, st, A, T);
+  A.ntx = t.ntx;
+  const dim3 grid{unsigned(t.ntx) * unsigned(t.nty), 1, 1};
+  if (t.tw == 32 && t.rw == 4) hipLaunchKernelGGL((k_conv<MODE, 4, 32>), grid, dim3(256), 0, st, A, T);
+  else if (t.tw == 32) hipLaunchKernelGGL((k_conv<MODE, 1, 32>), grid, dim3(256), 0, st, A, T);
+  else if (t.rw == 4) hipLaunchKernelGGL((k_conv<MODE, 4, 8>), grid, dim3(256), 0, st, A, T);
+  else hipLaunchKernelGGL((k_conv<MODE, 1, 8>), grid, dim3(256), 0, st, A, T);
 }
 
 // forward through the hidden layers from the velocity history, with the
