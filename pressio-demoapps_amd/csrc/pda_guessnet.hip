@@ -313,7 +313,11 @@ inline int conv_blocks(int H, int W) {
 
 // Backward-weight of a hidden layer: dW[tap][cout][cin] = sum_p dZ[p][cout]
 // X[p + tap][cin] and db[cout] = sum_p dZ[p][cout], as MFMAs with M = cout,
-// N = cin, K = pixels.  A workgroup takes a band of WG_SEG columns and marches
+// N = cin, K = pixels.  A workgroup takes a band of WG_SEG columns (every
+// nband-th one on grids of more bands than WG_MAX, so that the workgroups' sums
+// are bounded: 44 MB, 177 on 131072 x 4 with a workgroup for every band; MANY, a
+// kernel of its own: a loop over the bands in the other cost it 8 registers and
+// 7 % of a training step) and marches
 // up its share of the grid rows, WG_ROWS rows at a time: those rows of dZ and
 // the WG_ROWS + 2 rows of X that the taps read are staged in LDS once, in the
 // layout they have in memory ([pixel][channel]), and the operands, which need
@@ -355,28 +359,29 @@ __host__ __device__ constexpr int wg_ntiles(int cin) { return cin == C ? 6 : 2; 
 __host__ __device__ constexpr int wg_sums(int cin) { return 3 * wg_ntiles(cin) * 2 * 256 + C; }
 
 struct WgradGrid {
-  int nseg, rows_per_wg, nwg; // bands, grid rows of a workgroup, workgroups
+  int nseg, nband, rows_per_wg, nwg; // bands, bands taken at a time, grid rows of a workgroup, workgroups
 };
 inline WgradGrid wgrad_grid(int H, int W) {
   WgradGrid G;
   G.nseg = (W + WG_SEG - 1) / WG_SEG;
-  const int per = std::max(1, WG_MAX / G.nseg);           // workgroups a band may take
+  G.nband = std::min(G.nseg, WG_MAX);
+  const int per = WG_MAX / G.nband; // workgroups a band may take
   G.rows_per_wg = ((H + per - 1) / per + WG_ROWS - 1) / WG_ROWS * WG_ROWS;
-  G.nwg = G.nseg * ((H + G.rows_per_wg - 1) / G.rows_per_wg);
+  G.nwg = G.nband * ((H + G.rows_per_wg - 1) / G.rows_per_wg);
   return G;
 }
 
-template <int CIN>
+template <int CIN, bool MANY>
 __global__ void __launch_bounds__(WG_THREADS) k_conv_wgrad(const __bf16 *__restrict__ dZ,
                                                           const __bf16 *__restrict__ X, int H, int W,
-                                                          int nseg, int rows_per_wg, float *__restrict__ part) {
+                                                          int nband, int rows_per_wg,
+                                                          float *__restrict__ part) {
   constexpr int NT = wg_ntiles(CIN);
   __shared__ __align__(16) __bf16 sz[WG_ROWS * WG_SEG * C];
   __shared__ __align__(16) __bf16 sx[(WG_ROWS + 2) * (WG_SEG + 2) * CIN];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int g = lane >> 4, i16 = lane & 15;
-  const int x0 = (int(blockIdx.x) % nseg) * WG_SEG;
-  const int yb = (int(blockIdx.x) / nseg) * rows_per_wg;
+  const int yb = (int(blockIdx.x) / nband) * rows_per_wg;
   const int ye = yb + rows_per_wg < H ? yb + rows_per_wg : H;
   f32x4 acc[NT][2], accb[2];
 #pragma unroll
@@ -391,7 +396,8 @@ __global__ void __launch_bounds__(WG_THREADS) k_conv_wgrad(const __bf16 *__restr
     ones[j] = __bf16(1.f);
     zero[j] = __bf16(0.f);
   }
-  for (int y0 = yb; y0 < ye; y0 += WG_ROWS) {
+  int x0 = (int(blockIdx.x) % nband) * WG_SEG;
+  for (int y0 = yb; y0 < ye;) {
     constexpr int ZV = WG_ROWS * WG_SEG * (C / 8), XW = WG_SEG + 2, XV = (WG_ROWS + 2) * XW * (CIN / 8);
     constexpr int ZP = (ZV + WG_THREADS - 1) / WG_THREADS, XP = (XV + WG_THREADS - 1) / WG_THREADS;
     bf16x8 dz[ZP], dx[XP]; // every load in flight before the first LDS store
@@ -454,6 +460,11 @@ __global__ void __launch_bounds__(WG_THREADS) k_conv_wgrad(const __bf16 *__restr
         }
       }
     __syncthreads();
+    y0 += WG_ROWS;
+    if (MANY && y0 >= ye && x0 + nband * WG_SEG < W) { // the next of its bands
+      x0 += nband * WG_SEG;
+      y0 = yb;
+    }
   }
   float *dst = part + int64_t(blockIdx.x) * wg_sums(CIN);
 #pragma unroll
@@ -849,12 +860,12 @@ int backward(pda_guessnet_s &net, hipStream_t st) {
     const int cin = cin_of(l);
     L.part[l] = part;
     L.gw[l] = gW + net.woff[l];
-    if (cin == C)
-      hipLaunchKernelGGL((k_conv_wgrad<C>), dim3(G.nwg), dim3(WG_THREADS), 0, st, dz, net.Y[l - 1].as<__bf16>(),
-                         net.H, net.W, G.nseg, G.rows_per_wg, part);
-    else
-      hipLaunchKernelGGL((k_conv_wgrad<CIN0>), dim3(G.nwg), dim3(WG_THREADS), 0, st, dz, net.X0.as<__bf16>(),
-                         net.H, net.W, G.nseg, G.rows_per_wg, part);
+    const auto go = [&](auto kernel, const __bf16 *x) {
+      hipLaunchKernelGGL(kernel, dim3(G.nwg), dim3(WG_THREADS), 0, st, dz, x, net.H, net.W, G.nband, G.rows_per_wg, part);
+    };
+    const bool many = G.nseg > G.nband;
+    if (cin == C) go(many ? k_conv_wgrad<C, true> : k_conv_wgrad<C, false>, net.Y[l - 1].as<__bf16>());
+    else go(many ? k_conv_wgrad<CIN0, true> : k_conv_wgrad<CIN0, false>, net.X0.as<__bf16>());
     part += int64_t(G.nwg) * wg_sums(cin);
     PDA_HIP_CHECK(hipGetLastError());
     if (l == 0) break;

@@ -34,10 +34,12 @@ def _net(nx, ny, w, scales):
 
 
 # (columns, rows, repeats in x, repeats in y): 8-column tiles with one and four
-# rows per wave, a tile wider than the grid, partial tiles, grids lower than a tile
+# rows per wave, a tile wider than the grid, partial tiles, grids lower than a
+# tile; the last one's repetition has more bands of columns than the backward
+# pass has workgroups
 @pytest.mark.parametrize("nx,ny,rx,ry", [(4, 128, 8, 1), (4, 32768, 8, 1), (5, 512, 32, 1), (8, 64, 4, 1),
                                          (8, 16384, 8, 1), (12, 128, 8, 1), (40, 512, 4, 1), (512, 4, 1, 8),
-                                         (16384, 4, 1, 8), (4096, 12, 1, 4)])
+                                         (16384, 4, 1, 8), (4096, 12, 1, 4), (32768, 4, 2, 1)])
 def test_narrow_grid_equals_its_periodic_repetition(nx, ny, rx, ry, torch):
     print(f"[gpu-nn-tiles] {nx} x {ny}", flush=True)
     rng = np.random.default_rng(nx + ny)
@@ -83,3 +85,19 @@ def test_cost_of_narrow_and_low_grids(torch):
         us = cost(nx, ny)
         print(f"[gpu-nn-tiles] {nx} x {ny}: {us:.0f} us, 1024 x 512: {wide:.0f} us", flush=True)
         assert us <= 1.4 * wide
+
+
+def test_memory_of_a_wide_grid(torch):
+    """The backward pass's partial sums are bounded: a grid of 131072 columns takes
+    what the same pixels take as 1024 columns, to 32 MB of 430 (177 MB of partial
+    sums with a workgroup for every band of 64 columns, 44 with 512 at most)."""
+    def taken(nx, ny):
+        torch.cuda.synchronize()
+        before = torch.cuda.mem_get_info()[0]
+        net = pda.GuessNet(nx, ny)
+        return before - torch.cuda.mem_get_info()[0], net
+
+    a, keep = taken(1024, 512)
+    b, other = taken(131072, 4)
+    print(f"[gpu-nn-tiles] 1024 x 512: {a / 1e6:.0f} MB, 131072 x 4: {b / 1e6:.0f} MB", flush=True)
+    assert a > 300e6 and b <= a + 32e6
