@@ -8,7 +8,8 @@
 // default linear solver wraps, solvers_linear_traits.hpp:95-105) and a
 // block-Jacobi preconditioner (the m x m diagonal blocks, inverted per cell),
 // applied from the right: the matrix of the iteration is I + B with the blocks
-// B_ij = cf J_ij (cf J_jj + cnp1 I)^-1, formed once per Newton iteration.
+// B_ij = cf J_ij (cf J_jj + cnp1 I)^-1, formed once per Newton iteration, beside
+// the Jacobian slot by slot, or in its place where memory is short.
 //
 // Stop rules:
 //   PDA_STOP_CORRECTION -- pressio's default: stop when the l2 norm of the
@@ -124,9 +125,12 @@ __global__ void __launch_bounds__(TB) k_ell_cols(Blocks K, int M, int32_t *__res
 // cell, a lane per block, so that a cell's values are read as they lie; a block
 // of threads writes 16 consecutive cells of every slot.  Bound by the matrix
 // read and written: 512 x 512 Burgers (222 MB) 54 us, repaid within three iterations.
+// IN_PLACE: in the place of the Jacobian's blocks, for steppers without room for a
+// second matrix (a block is read and written by its lane alone; the diagonal
+// blocks stay).
 constexpr int FL = 16;
-template <int M>
-__global__ void __launch_bounds__(TB) k_form(Blocks K, const double *__restrict__ J, double cf,
+template <int M, bool IN_PLACE>
+__global__ void __launch_bounds__(TB) k_form(Blocks K, double *__restrict__ J, double cf,
                                              const double *__restrict__ Minv, double *__restrict__ A) {
   constexpr int V = Ell<M>::V, PAIRS = Ell<M>::PAIRS;
   const int64_t c = (int64_t(blockIdx.x) * TB + threadIdx.x) / FL;
@@ -140,7 +144,7 @@ __global__ void __launch_bounds__(TB) k_form(Blocks K, const double *__restrict_
 #pragma unroll
     for (int k = 0; k < M * M; ++k) o[k] = 0.;
     if (b < nb) {
-      const double *Jr = J + rb + b * M;
+      double *Jr = J + rb + b * M;
       const double *Mi = Minv + int64_t(K.bcol[c * K.maxb + b]) * M * M;
 #pragma unroll
       for (int k = 0; k < M; ++k) {
@@ -152,7 +156,14 @@ __global__ void __launch_bounds__(TB) k_form(Blocks K, const double *__restrict_
 #pragma unroll
           for (int i = 0; i < M; ++i) o[k * M + j] += a[i] * Mi[i * M + j];
       }
+      if constexpr (IN_PLACE) {
+#pragma unroll
+        for (int k = 0; k < M; ++k)
+#pragma unroll
+          for (int j = 0; j < M; ++j) Jr[int64_t(k) * nb * M + j] = o[k * M + j];
+      }
     }
+    if constexpr (IN_PLACE) continue;
 #pragma unroll
     for (int h = 0; h < PAIRS; ++h)
 #pragma unroll
@@ -172,9 +183,10 @@ __global__ void __launch_bounds__(TB) k_form(Blocks K, const double *__restrict_
 // 18.9 SECOND; 16 lanes per cell over the Jacobian's own CSR blocks 23.8, with
 // 14.4 us of launches that applied Minv beside each product.
 // Partial sums of (r0 . y), or with SECOND of (y . x, y . y).
-template <int M, bool SECOND>
-__global__ void __launch_bounds__(TB) k_spmv(const double *__restrict__ A, const int32_t *__restrict__ col,
-                                             int slots, int64_t ncell, const double *__restrict__ x,
+// IN_PLACE: the blocks lie in the Jacobian's CSR (k_form), their columns in K.
+template <int M, bool SECOND, bool IN_PLACE>
+__global__ void __launch_bounds__(TB) k_spmv(Blocks K, const double *__restrict__ A,
+                                             const int32_t *__restrict__ col, int slots, int64_t ncell, const double *__restrict__ x,
                                              const double *__restrict__ xv, const double *__restrict__ r0,
                                              double *__restrict__ y, int64_t per_block,
                                              const double *__restrict__ part_in, int npart,
@@ -212,15 +224,32 @@ __global__ void __launch_bounds__(TB) k_spmv(const double *__restrict__ A, const
       if constexpr (SECOND) own[k] -= alpha * xv[c * M + k];
       acc[k] = own[k];
     }
+    int nb = 0, d = 0;
+    if constexpr (IN_PLACE) {
+      nb = K.nblk[c];
+      d = int((K.diag[c] - K.rowbase[c]) / M);
+      slots = nb - 1;
+    }
 #pragma unroll 4
     for (int e = 0; e < slots; ++e) {
-      const int64_t j = int64_t(col[e * ncell + c]) * M;
-      const double *a = A + (int64_t(e) * PAIRS * ncell + c) * V;
+      int64_t j;
       double u[M], b[M * M];
+      if constexpr (IN_PLACE) {
+        const int q = e < d ? e : e + 1;
+        const double *a = A + K.rowbase[c] + q * M;
+        j = int64_t(K.bcol[c * K.maxb + q]) * M;
 #pragma unroll
-      for (int h = 0; h < PAIRS; ++h)
+        for (int k = 0; k < M; ++k)
 #pragma unroll
-        for (int v = 0; v < V; ++v) b[h * V + v] = a[h * ncell * V + v];
+          for (int i = 0; i < M; ++i) b[k * M + i] = a[int64_t(k) * nb * M + i];
+      } else {
+        const double *a = A + (int64_t(e) * PAIRS * ncell + c) * V;
+        j = int64_t(col[e * ncell + c]) * M;
+#pragma unroll
+        for (int h = 0; h < PAIRS; ++h)
+#pragma unroll
+          for (int v = 0; v < V; ++v) b[h * V + v] = a[h * ncell * V + v];
+      }
 #pragma unroll
       for (int k = 0; k < M; ++k) {
         u[k] = x[j + k];
@@ -488,6 +517,7 @@ struct pda_implicit_s {
   static constexpr int FIRST_POLL = 16; // the first poll comes no later, each further one by twice the count
   pda::DevBuf J, F, Fn, R, Y, Yn, dx, x, r, r0, p, v, t, Minv, scal;
   pda::DevBuf ell, ellcol;  // the iteration's matrix and its column cells
+  bool in_place = false;    // without them: the matrix in the Jacobian's place
   pda::DevBuf part[5];      // partial sums: r0.v, (t.s, t.t), (r0.r, r.r), R.R, dx.dx
   pda::DevBuf diag;         // first value of every cell's diagonal block
   double *host = nullptr;   // pinned: what the host reads after a synchronization
@@ -529,12 +559,14 @@ Blocks blocks_of(const pda_implicit_s &ip) {
 }
 
 // one BiCGSTAB iteration; every kernel is a no-op once the convergence flag is set
-template <int M> void bicgstab_iteration(pda_implicit_s &ip, hipStream_t st, bool first, double rtol) {
+template <int M, bool IN_PLACE>
+void bicgstab_iteration_in(pda_implicit_s &ip, hipStream_t st, bool first, double rtol) {
   const int64_t n = ip.n, nc = ip.ncell;
   const int slots = ip.prob->maxb - 1;
   double *r = ip.r.as<double>(), *r0 = ip.r0.as<double>(), *pp = ip.p.as<double>();
   double *v = ip.v.as<double>(), *t = ip.t.as<double>(), *scal = ip.scal.as<double>();
-  const double *A = ip.ell.as<double>();
+  const double *A = IN_PLACE ? ip.J.as<double>() : ip.ell.as<double>();
+  const Blocks K = blocks_of(ip);
   const int32_t *col = ip.ellcol.as<int32_t>();
   double *pr0v = ip.part[P_R0V].as<double>(), *pts = ip.part[P_TS].as<double>(), *prr = ip.part[P_RR].as<double>();
   const unsigned gv = grid_strided(n);
@@ -542,11 +574,16 @@ template <int M> void bicgstab_iteration(pda_implicit_s &ip, hipStream_t st, boo
   const int64_t per = ((nc + MAXB - 1) / MAXB + TB - 1) / TB * TB;
   const unsigned gs = unsigned((nc + per - 1) / per);
   hipLaunchKernelGGL(k_p, dim3(gv), dim3(TB), 0, st, r, pp, v, n, prr, int(gv), scal, first ? 1 : 0, rtol);
-  hipLaunchKernelGGL((k_spmv<M, false>), dim3(gs), dim3(TB), 0, st, A, col, slots, nc, pp, nullptr, r0, v, per,
-                     nullptr, 0, pr0v, scal);
-  hipLaunchKernelGGL((k_spmv<M, true>), dim3(gs), dim3(TB), 0, st, A, col, slots, nc, r, v, nullptr, t, per, pr0v,
-                     int(gs), pts, scal);
+  hipLaunchKernelGGL((k_spmv<M, false, IN_PLACE>), dim3(gs), dim3(TB), 0, st, K, A, col, slots, nc, pp, nullptr, r0, v,
+                     per, nullptr, 0, pr0v, scal);
+  hipLaunchKernelGGL((k_spmv<M, true, IN_PLACE>), dim3(gs), dim3(TB), 0, st, K, A, col, slots, nc, r, v, nullptr, t, per,
+                     pr0v, int(gs), pts, scal);
   hipLaunchKernelGGL(k_xr, dim3(gv), dim3(TB), 0, st, ip.x.as<double>(), r, pp, v, t, r0, n, pts, int(gs), prr, scal);
+}
+
+template <int M> void bicgstab_iteration(pda_implicit_s &ip, hipStream_t st, bool first, double rtol) {
+  if (ip.in_place) bicgstab_iteration_in<M, true>(ip, st, first, rtol);
+  else bicgstab_iteration_in<M, false>(ip, st, first, rtol);
 }
 
 // (cnp1 I + cf J) dx = -R, Y += dx where Y is given, partial sums of dx . dx.  newton: index of the Newton iteration, whose
@@ -565,8 +602,8 @@ int bicgstab_m(pda_implicit_s &ip, double cf, double cnp1, double *Y, hipStream_
   const unsigned gv = grid_strided(n), gc = grid_of(nc);
   hipLaunchKernelGGL((k_block_inv<M>), dim3(gc), dim3(TB), 0, st, blocks_of(ip), ip.J.as<double>(), cf, cnp1,
                      ip.Minv.as<double>());
-  hipLaunchKernelGGL((k_form<M>), dim3(grid_of(nc * FL)), dim3(TB), 0, st, blocks_of(ip), ip.J.as<double>(), cf,
-                     ip.Minv.as<double>(), ip.ell.as<double>());
+  hipLaunchKernelGGL((ip.in_place ? k_form<M, true> : k_form<M, false>), dim3(grid_of(nc * FL)), dim3(TB), 0, st,
+                     blocks_of(ip), ip.J.as<double>(), cf, ip.Minv.as<double>(), ip.ell.as<double>());
   hipLaunchKernelGGL(k_start, dim3(gv), dim3(TB), 0, st, ip.R.as<double>(), ip.x.as<double>(), ip.r.as<double>(),
                      ip.r0.as<double>(), n, prr, scal);
   PDA_HIP_CHECK(hipGetLastError());
@@ -672,9 +709,6 @@ int pda_implicit_create(pda_problem p, int scheme, pda_implicit *out) {
   for (auto *d : vecs)
     if (e == hipSuccess) e = d->alloc(vb);
   if (e == hipSuccess) e = ip->Minv.alloc(sizeof(double) * size_t(ip->ncell) * p->m * p->m);
-  const size_t blocks = size_t(ip->ncell) * size_t(std::max(1, p->maxb - 1));
-  if (e == hipSuccess) e = ip->ell.alloc(sizeof(double) * blocks * p->m * p->m);
-  if (e == hipSuccess) e = ip->ellcol.alloc(sizeof(int32_t) * blocks);
   for (auto &d : ip->part)
     if (e == hipSuccess) e = d.alloc(sizeof(double) * 2 * pda::MAXB);
   if (e == hipSuccess) e = hipHostMalloc(reinterpret_cast<void **>(&ip->host), sizeof(double) * 8, hipHostMallocDefault);
@@ -691,14 +725,28 @@ int pda_implicit_create(pda_problem p, int scheme, pda_implicit *out) {
         return PDA_E_STATE;
       }
     e = ip->diag.upload(dg);
-    if (e == hipSuccess) {
+  }
+  if (e == hipSuccess) e = ip->scal.alloc(sizeof(double) * pda::S_COUNT);
+  if (e == hipSuccess) {
+    // the iteration's matrix last: where it would take more than half of the
+    // memory that is left, the stepper does without (k_form's IN_PLACE), at 8
+    // bytes a nonzero instead of 16
+    const size_t blocks = size_t(ip->ncell) * size_t(std::max(1, p->maxb - 1));
+    const size_t ell = sizeof(double) * blocks * p->m * p->m, cols = sizeof(int32_t) * blocks;
+    size_t left = 0, total = 0;
+    ip->in_place = hipMemGetInfo(&left, &total) != hipSuccess || left / 2 < ell + cols ||
+                   ip->ell.alloc(ell) != hipSuccess || ip->ellcol.alloc(cols) != hipSuccess;
+    if (ip->in_place) {
+      ip->ell.reset();
+      ip->ellcol.reset();
+      (void)hipGetLastError(); // a failed allocation is not the caller's error
+    } else {
       hipLaunchKernelGGL(k_ell_cols, dim3(grid_of(ip->ncell)), dim3(TB), 0, nullptr, blocks_of(*ip), p->m,
                          ip->ellcol.as<int32_t>());
       e = hipGetLastError();
+      if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
     }
-    if (e == hipSuccess) e = hipStreamSynchronize(nullptr);
   }
-  if (e == hipSuccess) e = ip->scal.alloc(sizeof(double) * pda::S_COUNT);
   if (e != hipSuccess) {
     set_error(std::string("pda_implicit_create: ") + hipGetErrorString(e));
     delete ip;
