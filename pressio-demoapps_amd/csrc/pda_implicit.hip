@@ -752,7 +752,6 @@ int pda_implicit_create(pda_problem p, int scheme, pda_implicit *out) {
     delete ip;
     return PDA_E_HIP;
   }
-  p->applied = true; // pda_apply_jacobian_noalloc may follow
   *out = ip;
   return PDA_OK;
 }

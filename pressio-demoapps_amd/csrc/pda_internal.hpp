@@ -186,7 +186,6 @@ struct pda_problem_s {
   std::vector<uint8_t> h_slot;
   std::vector<double> h_bcf;
   bool on_device = false;
-  bool applied = false;              // pda_apply_jacobian has been called
   // structured fast path
   pda::Box box;
   std::vector<int32_t> h_rem_rows;   // rows outside the box

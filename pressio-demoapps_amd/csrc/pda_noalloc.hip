@@ -65,9 +65,9 @@ int pda_apply_jacobian_noalloc(pda_problem p, const double *d_U, double t, const
   }
   // the problem's index tables are uploaded by the allocating entry points on
   // first use; this one only reads them
-  if (!p->on_device || !(p->d_rowptr.ptr || p->applied)) {
+  if (!p->on_device) {
     set_error("pda_apply_jacobian_noalloc: the problem's device tables are not built; call "
-              "pda_jacobian_pattern (or pda_apply_jacobian) once before");
+              "pda_jacobian_pattern or any evaluation once before");
     return PDA_E_STATE;
   }
   double *J = nullptr;

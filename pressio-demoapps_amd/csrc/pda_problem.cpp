@@ -755,7 +755,6 @@ int pda_apply_jacobian(pda_problem p, const double *d_U, double t, const double 
   // on the host) is not made for this
   int rc = ensure_device(*p);
   if (rc) return rc;
-  p->applied = true;
   if (p->d_scratch_v.bytes < sizeof(double) * size_t(p->nnz))
     PDA_HIP_CHECK(p->d_scratch_v.alloc(sizeof(double) * size_t(p->nnz)));
   rc = launch_jacobian(*p, d_U, t, p->d_scratch_v.as<double>(), nullptr, hipStream_t(stream));
