@@ -172,15 +172,15 @@ __device__ __forceinline__ void jac_fo_euler_staged(const View &P, int64_t wg, c
   // Copy-out from the row table in LDS alone: the rows' CSR offsets were
   // loaded with their states (not here, one row after the other).  Whole
   // rows leave as one flattened loop over their values: 16-byte stores where
-  // every row starts on an even value (2D, and 3D rows consecutive in the CSR
-  // after a leading value), else 8-byte ones.
+  // every row starts on a 16-byte boundary (2D, if J does, and rows consecutive in
+  // the CSR after a leading value), else 8-byte ones.
   const int64_t rb0 = base_of[0];
   const bool whole = __all(base >= 0 && nblk == NB);
   const bool run = __all(base == rb0 + int64_t(g) * PER);
   if (whole && run) {
     constexpr int TOT = SJ_ROWS * PER;
-    const int head = int(rb0 & 1); // a leading value that is not 16-byte aligned
     double *dst = J + rb0;
+    const int head = int(reinterpret_cast<uintptr_t>(dst) >> 3 & 1); // a leading value that is not 16-byte aligned
     if (head && lane == 0) store_stream(dst, stage[0]);
     const int npairs = (TOT - head) / 2;
     double2 *d2 = reinterpret_cast<double2 *>(dst + head);
@@ -191,7 +191,7 @@ __device__ __forceinline__ void jac_fo_euler_staged(const View &P, int64_t wg, c
     return;
   }
   if (whole) {
-    if constexpr (PER % 2 == 0) {
+    if (PER % 2 == 0 && reinterpret_cast<uintptr_t>(J) % 16 == 0) {
 #pragma unroll 4
       for (int q = lane; q < SJ_ROWS * (PER / 2); q += 64) {
         const int gg = q / (PER / 2), e = 2 * (q - gg * (PER / 2));
