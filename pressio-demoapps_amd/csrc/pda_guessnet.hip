@@ -1101,6 +1101,14 @@ int pda_guessnet_train_step(pda_guessnet net, const double *const *d_f, double n
   if (!rc) rc = check_costs(costs, "pda_guessnet_train_step");
   if (rc) return rc;
   hipStream_t st = hipStream_t(stream);
+  if (lossv) { // refused before the step is counted
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    PDA_HIP_CHECK(hipStreamIsCapturing(st, &cs));
+    if (cs != hipStreamCaptureStatusNone) {
+      set_error("pda_guessnet_train_step: the loss cannot be read while the stream is captured");
+      return PDA_E_HIP;
+    }
+  }
   rc = forward(*net, feature_args(*net, F, nu), true, false, st);
   if (!rc) rc = loss(*net, costs, lossv != nullptr, st);
   if (!rc) rc = backward(*net, st);
