@@ -307,7 +307,7 @@ __device__ __forceinline__ void vel_cc3_body(const View &P, const Box &B, int ro
   const int plane = int(s / line), e = int(s - int64_t(plane) * line);
   const int kz = int(B.lo[2]) + plane, xe = int(B.lo[0]) + e - 1;
   const int64_t i = wrap_axis<0>(B, xe);
-  // a column inside the grid for every lane's reads, whatever the box
+  // i itself for the boxes that are built: wrapped, or inside with its neighbours
   const int64_t ic = i < nx ? i : nx - 1;
   const bool own = lane >= 1 && lane <= V3OWN && s0 < ncell && e >= 1 && e <= bw;
   const double hx = P.hinv[0], hy = P.hinv[1], hz = P.hinv[2];
