@@ -71,9 +71,9 @@ struct Steps1dCoef {
   double cv[4];    // per stage: coefficient of the velocity
 };
 
-// value of the lane whose index differs in bit 0 (quad_perm 1,0,3,2) or bit 1
-// (quad_perm 2,3,0,1)
-template <int CTRL> __device__ __forceinline__ double quad_swap(double v) {
+// value of the other lane of the pair (quad_perm 1,0,3,2)
+__device__ __forceinline__ double pair_swap(double v) {
+  constexpr int CTRL = 0xB1;
   const long long b = __double_as_longlong(v);
   const int lo = __builtin_amdgcn_update_dpp(0, int(b), CTRL, 0xf, 0xf, false);
   const int hi = __builtin_amdgcn_update_dpp(0, int(b >> 32), CTRL, 0xf, 0xf, false);
@@ -171,7 +171,7 @@ __global__ void __launch_bounds__(S1_WAVES * 64) k_steps1d(View P, int64_t n, in
       } else {
         v = phys::weno5_side_1div<true>(q[k][0], q[k][1], q[k][2], q[k][3], q[k][4]);
       }
-      const double o = quad_swap<0xB1>(v);
+      const double o = pair_swap(v);
       um[k] = sd ? o : v;
       up[k] = sd ? v : o;
     }

@@ -33,7 +33,8 @@ namespace rows {
 // of impl/euler_3d_prob_class.hpp:626-651).
 constexpr int SJ_LANES = 4, SJ_ROWS = 64 / SJ_LANES;
 
-__device__ __forceinline__ int exch(int k, int a) { return k == 1 ? 1 + a : (k == 1 + a ? 1 : k); }
+// the axis frame's dof k (AxisPerm, the same for every dimension)
+__device__ __forceinline__ int exch(int k, int a) { return AxisPerm<PhEuler3>::p(k, a); }
 
 // ghost sign of native dof exch(k, a) on side `side` of axis a
 template <int D>
