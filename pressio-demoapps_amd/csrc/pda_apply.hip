@@ -12,19 +12,21 @@ namespace {
 // M ncols values of B for its M*M own.
 //
 // k_apply_cols, many columns of a row-major B: L lanes per cell, a lane
-// holding VW columns of its M results; the block's values are the same for
-// the L lanes (one broadcast load), its M rows of B contiguous runs over
+// holding VW columns of its M results, and 256 / L cells of a block of threads
+// (inv = 2^16 / L rounded up, so that thread t's cell is t inv >> 16: exact for t <
+// 256 and L <= 64); the block's values are the same for the L lanes (one broadcast load), its M rows of B contiguous runs over
 // them.  10 % sample mesh of 512 x 400, WENO3, 32 columns: 133 -> 36 us
 // (186 MB of B and AJ: 5.1 TB/s) against a thread per entry of AJ walking the
 // scalar CSR, which read every value and column index ncols times.
 template <int M, int VW>
 __global__ void __launch_bounds__(256) k_apply_cols(View P, const int32_t *__restrict__ bcol, int maxb,
                                                     const double *__restrict__ J, const double *__restrict__ B,
-                                                    int64_t ncols, int L, double *__restrict__ AJ) {
+                                                    int64_t ncols, int L, int inv, double *__restrict__ AJ) {
   typedef double vec __attribute__((ext_vector_type(VW)));
-  const int64_t r = int64_t(blockIdx.x) * (256 / L) + threadIdx.x / L;
-  if (r >= P.nrows) return;
-  const int64_t c0 = (int64_t(blockIdx.y) * L + threadIdx.x % L) * VW;
+  const int g = int(threadIdx.x) * inv >> 16, cells = 256 * inv >> 16; // its cell; cells of the block
+  const int64_t r = int64_t(blockIdx.x) * cells + g;
+  if (g >= cells || r >= P.nrows) return;
+  const int64_t c0 = (int64_t(blockIdx.y) * L + (int(threadIdx.x) - g * L)) * VW;
   if (c0 >= ncols) return;
   const int nb = P.nblk[r];
   const int32_t *bc = bcol + r * maxb;
@@ -136,12 +138,14 @@ static int apply_m(const pda_problem_s &p, const double *J, const double *B, int
   if (layout == 1 && ncols >= 8) {
     // two columns per lane where every row of B and AJ is 16-byte aligned
     const int vw = ncols % 2 == 0 && (reinterpret_cast<uintptr_t>(B) | reinterpret_cast<uintptr_t>(AJ)) % 16 == 0 ? 2 : 1;
-    const int64_t lanes = (ncols + vw - 1) / vw;
-    int L = 4;
-    while (L < 64 && L < lanes) L *= 2;
-    const dim3 grid{unsigned((v.nrows + 256 / L - 1) / (256 / L)), unsigned((lanes + L - 1) / L), 1};
-    if (vw == 2) hipLaunchKernelGGL((k_apply_cols<M, 2>), grid, dim3(256), 0, s, v, bc, p.maxb, J, B, ncols, L, AJ);
-    else hipLaunchKernelGGL((k_apply_cols<M, 1>), grid, dim3(256), 0, s, v, bc, p.maxb, J, B, ncols, L, AJ);
+    // the lanes in equal parts of at most 64, no more than they are: rounded up to
+    // a power of two, 33 columns left 31 of 64 lanes idle (scalar family on 600 x
+    // 500 cells, first order: 135 us with the Jacobian, 88 now)
+    const int64_t lanes = (ncols + vw - 1) / vw, parts = (lanes + 63) / 64;
+    const int L = int((lanes + parts - 1) / parts), inv = (65536 + L - 1) / L;
+    const dim3 grid{unsigned((v.nrows + 256 / L - 1) / (256 / L)), unsigned(parts), 1};
+    if (vw == 2) hipLaunchKernelGGL((k_apply_cols<M, 2>), grid, dim3(256), 0, s, v, bc, p.maxb, J, B, ncols, L, inv, AJ);
+    else hipLaunchKernelGGL((k_apply_cols<M, 1>), grid, dim3(256), 0, s, v, bc, p.maxb, J, B, ncols, L, inv, AJ);
     PDA_HIP_CHECK(hipGetLastError());
     return PDA_OK;
   }
