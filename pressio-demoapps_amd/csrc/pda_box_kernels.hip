@@ -274,7 +274,9 @@ __device__ __forceinline__ void vel_cc_body(const View &P, const Box &B, int row
 // cell is reconstructed once per axis; the z faces take one more one-sided
 // value from the cell below and from the cell above, as planes are not carried.
 // Bound by FP64 issue: 1,750 FP64 instructions a row of 62 cells against 5,300
-// evaluating every face's two sides by themselves; WENO5 at 128^3 179 us (244).
+// evaluating every face's two sides by themselves.  WENO5 at 128^3: 172 us in a
+// pass with the Jacobian (median of a kernel trace; 158 the least, 187 called over
+// and over, by the clock); in the run that compared them 179, 244 face by face.
 constexpr int VSEG = 63;         // a wavefront's last lane; it and lane 0 overlap the neighbouring wavefronts
 constexpr int V3OWN = VSEG - 1;  // cells it owns
 
@@ -1078,8 +1080,9 @@ static int64_t velocity_waves(const Box &B, int dim, int w) {
 // the Jacobian at 6 rows, 177 at 10, whose 1,836 waves are 4 us faster on
 // states that are).  3D waves run two to a SIMD for the same time
 // each, so the height is the one with the fewest rows (a strip's own and half
-// a row for the values before its first) over the rounds of 2,048 waves (128^3:
-// 16 rows, 1,952 waves, 152 us; 150 to 190 at the others from 2 to 18, 217 at 24).
+// a row for the values before its first) over the rounds of 2,048 waves (128^3, the
+// heights in turn in one run: 16 rows, 1,952 waves, 152 us; 150 to 190 at the others
+// from 2 to 18, 217 at 24).
 int64_t velocity_strip_height(const Box &B, int dim, int w) {
   const int64_t nw = velocity_waves(B, dim, w), bh = B.hi[1] - B.lo[1];
   if (dim == 3) {

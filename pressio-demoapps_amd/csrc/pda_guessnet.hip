@@ -128,7 +128,7 @@ __device__ __forceinline__ bf16x8 features(const Features &T, int64_t p) {
 // no lane computes addresses or wraps per tap; the layer's weights stay in
 // registers.  M = output channels and N = pixels, so that a lane ends with
 // four consecutive channels of one pixel: 8-byte (Y) and 16-byte (Z) accesses
-// instead of one per value.  At 512 x 512 a hidden layer takes 16.3 us (33.5 MB
+// instead of one per value.  At 512 x 512 a hidden layer takes 15.9 us (33.5 MB
 // in and out: 7 us at the copy rate; SiLU's vector instructions: 4 us; the two
 // phases overlap little, as all 512 workgroups run at once), 24.2 us when
 // every lane gathered its pixels per tap from memory.  Loading the tile in a
@@ -283,8 +283,8 @@ __global__ void __launch_bounds__(256) k_conv(ConvArgs A, Features T) {
 
 // The tile's shape.  RW: 4 where that still gives the chip a workgroup per CU
 // (fewer halo pixels, 1.20 times the tile against 1.59, and the weights loaded for
-// more pixels: a hidden layer at 512 x 512 takes 16.3 us with 4, 16.9 with 2, 18.0
-// with 1), else 1, and 1 too on grids so low that it stages fewer pixels.  TW: 32
+// more pixels: a hidden layer at 512 x 512 took 16.3 us with 4, 16.9 with 2, 18.0
+// with 1 in one run), else 1, and 1 too on grids so low that it stages fewer pixels.  TW: 32
 // columns, or 8 where those stage at most three quarters of the pixels, as on
 // grids of fewer columns than 32, most of whose tile would be columns that are
 // not there (predict on 8 x 65536 pixels 156 -> 84 us, 4 x 131072 270 -> 117,
