@@ -58,7 +58,7 @@ __global__ void __launch_bounds__(64) k_velocity_stage(View P, const double *__r
 // g - d < 0 as cell g + d - 1, g + d >= n as g - d + 1; the 1D problems have no
 // sign to apply), or periodic wrap.  The state is read from Uin and
 // written to Uout (workgroups read each other's cells).
-// 1000 cells, WENO5, SSPRK3: 2.85 us per step; with four lanes per row, each
+// 1000 cells, WENO5, SSPRK3: 2.8 us per step; with four lanes per row, each
 // face evaluated by both its rows and two waves per SIMD bound by issue, 3.9.
 // 10^6 cells 67 us (162).
 constexpr int S1_WAVES = 4, S1_OWN = 31, S1_PAIRS = S1_WAVES * S1_OWN, S1_STRIDE = 128;
