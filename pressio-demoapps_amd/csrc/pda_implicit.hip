@@ -514,7 +514,7 @@ struct pda_implicit_s {
   double lin_rtol = 1e-14;
   int lin_max = 0;          // 0: 2 * unknowns (Eigen's default)
   int check_every = 4;      // iterations of the recorded graph
-  static constexpr int FIRST_POLL = 16; // the first poll comes no later, each further one by twice the count
+  static constexpr int FIRST_POLL = 24; // the first poll comes no later, each further one by twice the count
   pda::DevBuf J, F, Fn, R, Y, Yn, dx, x, r, r0, p, v, t, Minv, scal;
   pda::DevBuf ell, ellcol;  // the iteration's matrix and its column cells
   bool in_place = false;    // without them: the matrix in the Jacobian's place
